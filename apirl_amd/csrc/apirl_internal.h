@@ -240,6 +240,8 @@ hipError_t launch_project(const apirl_plan* p, const float* img, float* sino, in
                           int nsubsets, int precision, const FusedRatio* fused, int* nblocks_out,
                           hipStream_t st);
 bool path_forward_ok(const apirl_plan* p, int precision);
+// Floats of the path forward projector's z-fastest image copy (apirl_plan::d_imgT).
+size_t path_image_floats(const Geo& g);
 int project_partials(const apirl_plan* p, int subset, int nsubsets, bool path);
 hipError_t launch_backproject(const apirl_plan* p, const float* sino, const float* est,
                               float* img, int subset, int nsubsets, int kind, int mode,

@@ -660,8 +660,10 @@ apirl_status plan_create_impl(apirl_ctx* ctx, const apirl_image_desc* image,
   // The gather's tile order for the default depth (without it the column kernel
   // keeps the grid's order).
   (void)ensure_tile_map(p);
-  // Transposed image for the forward projector's x-major rays.
-  if (hipMalloc(&p->d_imgT, (size_t)im.nx * im.ny * im.nz * sizeof(float)) != hipSuccess) {
+  // The forward projector's image copy (z fastest, or transposed for x-major rays).
+  const size_t copy_floats =
+      geo.dims == 3 ? apirl::path_image_floats(geo) : (size_t)im.nx * im.ny * im.nz;
+  if (hipMalloc(&p->d_imgT, copy_floats * sizeof(float)) != hipSuccess) {
     p->d_imgT = nullptr;
     (void)hipGetLastError();
   }

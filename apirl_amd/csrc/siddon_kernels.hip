@@ -15,6 +15,7 @@
 #include <cmath>
 
 #include "apirl_internal.h"
+#include "alpha_exact.h"
 #include "siddon_f64.h"
 
 namespace apirl {
@@ -24,7 +25,8 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kNumXcd = 8;  // MI355X: 8 XCDs of 32 CUs
 constexpr int kUnroll = 8;  // Siddon steps per batch of voxel loads
-constexpr int kPathUnroll = 12;  // the same for project_paths_kernel (12: 0.86 ms per C2 subset; 8: 0.90, 16: 0.88)
+constexpr int kPathUnroll = 12;  // the same for project_paths_kernel's step-by-step batches
+constexpr int kPathCols = 8;     // columns per batch of project_paths_kernel's column walk
 // Marks a batch slot without a term: no Siddon weight is NaN-boxed like this value.
 
 // Per-ray traversal state (Siddon.cpp:253-340).
@@ -949,203 +951,337 @@ __global__ __launch_bounds__(kBlock) void update_group_kernel(BatchHeader* __res
 inline unsigned grid_for(long n) { return (unsigned)((n + kBlock - 1) / kBlock); }
 
 
-// ---- Path forward projector (3D, APIRL_PREC_REFERENCE, one LOR per bin) ------------
+// ---- Path forward projector (3D, one LOR per bin, every precision but F64) ---------
 //
 // The rays of one (angle, radial bin) in every sinogram share their transaxial path:
 // the reference's loop takes its x and y steps in the same order whatever its z steps
 // (Siddon.cpp:318-339: a z step is taken only below both, and x before y on ties).
 // project_paths_kernel takes one (angle, bin) per workgroup, first writes that path to
-// LDS (the columns the loop visits and the alpha at which it leaves each, one thread
-// running the loop's x / y additions), then takes the sinograms one per lane: each
-// lane runs the reference's loop, taking a z step when its next z crossing is below
-// the column's exit alpha and the path's next column otherwise, and adds w * voxel in
-// the loop's order, so the bin is
-// the reference's float sum, bit for bit (as project_kernel's).  Voxels come from a
-// copy of the image with z fastest, where the lanes, at one column and neighbouring
-// slices, read neighbouring words.
+// LDS (the columns the loop visits and the alpha at which it leaves each), then takes
+// the sinograms one per lane: each lane runs the reference's loop, taking a z step when
+// its next z crossing is below the column's exit alpha and the path's next column
+// otherwise, and adds w * voxel in the loop's order, so the bin is the reference's float
+// sum, bit for bit (as project_kernel's).  Voxels come from a copy of the image with z
+// fastest, where the lanes, at one column and neighbouring slices, read neighbouring
+// words; kPathGuard zeros lie between its columns.
+//
+// VALU issue bounds it.  While every lane of a wavefront is well inside the image, the
+// wavefront therefore walks kPathCols columns at a time, the same ones for all of its
+// lanes: their exit alphas and addresses are one LDS read for the wavefront, a column
+// costs each lane its slice's address, two products and a sum, and the one z step a lane
+// may take among them is put in by selects.  Its loads also touch the lines of one column
+// instead of those of several, as they do where each lane steps on its own (the form kept
+// for the path's ends, and from the first batch on in which a lane would take two z
+// steps).  Fused, 12-angle subset of the 256x256x81 / 344x252x837 workload: 0.86 -> 0.68
+// ms (3.3e8 VALU wave-instructions, 0.54 ms of issue); the whole 192x192x233 sinogram of
+// a 128x128x47 image: 1.24 -> 0.74 ms; F64_SETUP, 12 angles of 344x252x357 on 172x172x65:
+// 0.26 -> 0.22 ms.  Stepping every lane by itself with the same 12 instructions a step
+// measured 0.74, 0.80 and 0.23 ms; 6 columns a batch 0.68, 0.75 and 0.22 ms.
 
 struct FwdStep {
-  float ae;     // alpha at which the loop leaves this column by an x or y step
-  int base;     // (j nx + i) nz: the column's first voxel in the z-fastest copy
-  short i, j;   // the column (may lie outside the image at the path's ends)
-  int run;      // columns inside the image from this one on, this one included
+  float ae;       // alpha at which the loop leaves this column by an x or y step
+  unsigned base;  // byte address of the column's slice 0 in the z-fastest copy
 };
-static_assert(sizeof(FwdStep) == 16, "FwdStep is 16 bytes");
+static_assert(sizeof(FwdStep) == 8, "FwdStep is one 8-byte LDS read");
+
+// Zeros before, between and after the columns of the z-fastest copy: a batch that starts
+// inside the image takes at most kPathUnroll - 1 slices past a face, where it reads zeros
+// (a term the reference does not add; adding w * 0 leaves the sum as it is).
+constexpr int kPathGuard = kPathUnroll;
+inline int path_pitch(const Geo& g) { return g.nz + kPathGuard; }
 
 // Path length kept per (angle, bin): the transaxial list plus a few columns (a rounding
 // can trade a z step of the list for an x or y step).
 __host__ __device__ inline int fwd_path_len(const Geo& g) { return g.nx + g.ny + 4; }
-// LDS of project_paths_kernel: the list (one entry more) and the two crossing chains
+// LDS of project_paths_kernel: the list (one entry more, and two before it), its columns
+// and the two crossing chains
 inline size_t fwd_path_lds(const Geo& g) {
-  return (size_t)(fwd_path_len(g) + 1) * (sizeof(FwdStep) + 2 * sizeof(float));
+  return 2 * sizeof(FwdStep) +
+         (size_t)(fwd_path_len(g) + 1) * (sizeof(FwdStep) + sizeof(int) + 2 * sizeof(float));
+}
+// Wavefronts of project_paths_kernel's workgroup: four, or fewer when that many passes of
+// 64 sinograms do not need four (73 sinograms: two; 357: three, two passes each).
+inline int fwd_path_waves(const Geo& g) {
+  const int passes = (g.nsino + 63) / 64, rounds = (passes + 3) / 4;
+  return (passes + rounds - 1) / rounds;
 }
 
-// out[(j nx + i) nz + k] = in[(k ny + j) nx + i] through a 32 (i) x 32 (k) LDS tile.
+// out[(j nx + i) pitch + kPathGuard + k] = in[(k ny + j) nx + i] through a 32 (i) x 32 (k)
+// LDS tile; slices nz .. pitch - 1 write the zeros before the next column.
 __global__ __launch_bounds__(kBlock) void transpose_zfast_kernel(const float* __restrict__ in,
                                                                  float* __restrict__ out, int nx,
-                                                                 int ny, int nz) {
+                                                                 int ny, int nz, int pitch) {
   __shared__ float tile[32][33];
   const int i0 = blockIdx.x * 32, j = blockIdx.y, k0 = blockIdx.z * 32;
   const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;  // 32 x 8
   const long nxy = (long)nx * ny;
   for (int r = ty; r < 32; r += 8) {
     const int k = k0 + r, i = i0 + tx;
-    if (k < nz && i < nx) tile[r][tx] = in[(long)k * nxy + (long)j * nx + i];
+    tile[r][tx] = k < nz && i < nx ? in[(long)k * nxy + (long)j * nx + i] : 0.f;
   }
   __syncthreads();
   for (int r = ty; r < 32; r += 8) {
     const int i = i0 + r, k = k0 + tx;
-    if (i < nx && k < nz) out[((long)j * nx + i) * nz + k] = tile[tx][r];
+    if (i < nx && k < pitch) out[((long)j * nx + i) * pitch + kPathGuard + k] = tile[tx][r];
   }
+  if (blockIdx.x == 0 && j == 0 && k0 == 0 && threadIdx.x < kPathGuard) out[threadIdx.x] = 0.f;
 }
 
-template <bool FUSED>
-__global__ __launch_bounds__(kBlock) void project_paths_kernel(
+template <bool FUSED, int PREC>
+__global__ __launch_bounds__(kBlock, PREC == APIRL_PREC_REFERENCE ? 8 : 7) void project_paths_kernel(
     Geo g, const RayXY* __restrict__ rays, const float2* __restrict__ zab,
     const float* __restrict__ img, const float* __restrict__ imgZ, float* __restrict__ sino,
-    int nang_sub, int subset, int nsubsets, FusedRatio fr, int qmax) {
-  extern __shared__ FwdStep sp[];
+    int nang_sub, int subset, int nsubsets, FusedRatio fr, int qmax, int pitch) {
+  constexpr bool kSum2 = PREC != APIRL_PREC_REFERENCE;     // Kahan-compensated sum
+  constexpr bool kStrict = PREC == APIRL_PREC_F64_SETUP;   // in-image voxels only
+  extern __shared__ __align__(16) FwdStep sraw[];
+  FwdStep* const sp = sraw + 2;  // entry -1 holds the alpha of the path's entry
   __shared__ int s_qin[2];  // first and last list entries inside the image
+  const int nt = blockDim.x;
   const int pair = blockIdx.x;
   const int ka = pair / g.nr, rr = pair % g.nr;
   const int a = subset + nsubsets * ka;
-  const RayXY t = rays[(long)a * g.nr + rr];
-  // The list has qmax + 1 entries (a fast batch that starts kPathUnroll columns before the
+  RayXY t = rays[(long)a * g.nr + rr];
+  SetupXY64 xy64;
+  if (PREC == APIRL_PREC_F64_SETUP) {
+    // the transaxial setup in double from the float LOR (siddon_f64.h), rounded to float
+    setup_xy_f64(g, t.p0x, t.p0y, t.vx, t.vy, xy64);
+    t.ax = (float)xy64.ax;
+    t.ay = (float)xy64.ay;
+    t.axu = (float)xy64.axu;
+    t.ayu = (float)xy64.ayu;
+    t.i0 = xy64.i0;
+    t.j0 = xy64.j0;
+  }
+  const int iinc = PREC == APIRL_PREC_F64_SETUP ? xy64.iinc : ray_iinc(t.flags);
+  const int jinc = PREC == APIRL_PREC_F64_SETUP ? xy64.jinc : ray_jinc(t.flags);
+  // The list has qmax + 1 entries (a batch that starts kPathUnroll columns before the
   // list's end reads the entry after it).  The loop's x crossings X[m] (X[0] = ax,
   // X[m + 1] = X[m] + axu, in float as the loop adds them) and y crossings Y[k] are
-  // two chains, one lane each; the loop takes the x step at X[m] when X[m] <= the
-  // pending Y, so it takes X[m] at step m + #{k: Y[k] < X[m]} and Y[k] at step
+  // two chains, half of the threads each: a thread takes a run of its chain, from the
+  // closed form of the additions before it (alpha_exact.h; two threads adding them one
+  // after the other had the rest wait).  The loop takes the x step at X[m] when X[m] <=
+  // the pending Y, so it takes X[m] at step m + #{k: Y[k] < X[m]} and Y[k] at step
   // k + #{m: X[m] <= Y[k]} (a stable merge of the two sorted chains, x first on ties):
   // each step's entry is written by the crossing the loop takes there.
-  float* xs = (float*)(sp + qmax + 1);
+  int* ij = (int*)(sp + qmax + 1);  // (j << 16) | (i & 0xffff) of each entry's column
+  float* xs = (float*)(ij + qmax + 1);
   float* ys = xs + (qmax + 1);
-  if (threadIdx.x < 2) {
-    const bool isx = threadIdx.x == 0;
-    float v = isx ? t.ax : t.ay;
+  {
+    const int half = nt / 2;
+    const bool isx = (int)threadIdx.x < half;
+    const int per = (qmax + half) / half;
+    const int m0 = ((int)threadIdx.x - (isx ? 0 : half)) * per;
+    const int m1 = m0 + per < qmax + 1 ? m0 + per : qmax + 1;
     const float u = isx ? t.axu : t.ayu;
+    float v = isx ? t.ax : t.ay;
     float* arr = isx ? xs : ys;
-    for (int m = 0; m <= qmax; m++) {
-      arr[m] = v;
-      v = v + u;
+    if (m0 < m1) {
+      if (m0 > 0) v = u < 3.0e38f ? alpha_after(v, u, m0) : v + u;  // inf or NaN stays
+      for (int m = m0; m < m1; m++) {
+        arr[m] = v;
+        v = v + u;
+      }
     }
   }
   if (threadIdx.x == 0) {
     s_qin[0] = qmax + 1;
     s_qin[1] = -1;
+    sp[-1].ae = PREC == APIRL_PREC_F64_SETUP ? (float)xy64.amin : t.amin;
   }
   __syncthreads();
-  {
-    const int iinc = ray_iinc(t.flags), jinc = ray_jinc(t.flags);
-    for (int c = threadIdx.x; c < 2 * (qmax + 1); c += kBlock) {
-      const bool isx = c <= qmax;
-      const int m = isx ? c : c - (qmax + 1);
-      const float v = isx ? xs[m] : ys[m];
-      const float* other = isx ? ys : xs;
-      int lo = 0, hi = qmax + 1;  // other[0 .. lo) come before v
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        const float o = other[mid];
-        const bool before = isx ? (o < v) : (o <= v);
-        lo = before ? mid + 1 : lo;
-        hi = before ? hi : mid;
-      }
-      const int q = m + lo;
-      if (q <= qmax) {
-        const int mx = isx ? m : lo, my = isx ? lo : m;
-        const int i = t.i0 + mx * iinc, j = t.j0 + my * jinc;
-        sp[q].ae = v;
-        sp[q].i = (short)i;
-        sp[q].j = (short)j;
-        sp[q].base = (j * g.nx + i) * g.nz;
-        // the entries inside the image are one run: i and j each move one way, so each
-        // stays in range over one interval of entries
-        if ((unsigned)i < (unsigned)g.nx && (unsigned)j < (unsigned)g.ny) {
-          atomicMin(&s_qin[0], q);
-          atomicMax(&s_qin[1], q);
-        }
+  for (int c = threadIdx.x; c < 2 * (qmax + 1); c += nt) {
+    const bool isx = c <= qmax;
+    const int m = isx ? c : c - (qmax + 1);
+    const float v = isx ? xs[m] : ys[m];
+    const float* other = isx ? ys : xs;
+    int lo = 0, hi = qmax + 1;  // other[0 .. lo) come before v
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      const float o = other[mid];
+      const bool before = isx ? (o < v) : (o <= v);
+      lo = before ? mid + 1 : lo;
+      hi = before ? hi : mid;
+    }
+    const int q = m + lo;
+    if (q <= qmax) {
+      const int mx = isx ? m : lo, my = isx ? lo : m;
+      const int i = t.i0 + mx * iinc, j = t.j0 + my * jinc;
+      FwdStep e;
+      e.ae = v;
+      e.base = ((unsigned)(j * g.nx + i) * (unsigned)pitch + (unsigned)kPathGuard) * 4u;
+      sp[q] = e;
+      ij[q] = (j << 16) | (i & 0xffff);
+      // the entries inside the image are one run: i and j each move one way, so each
+      // stays in range over one interval of entries
+      if ((unsigned)i < (unsigned)g.nx && (unsigned)j < (unsigned)g.ny) {
+        atomicMin(&s_qin[0], q);
+        atomicMax(&s_qin[1], q);
       }
     }
   }
   __syncthreads();
-  {
-    const int qa = s_qin[0], qb = s_qin[1];
-    for (int q = threadIdx.x; q <= qmax; q += kBlock)
-      sp[q].run = q >= qa && q <= qb ? qb - q + 1 : 0;
-  }
+  const int qa = s_qin[0], qb = s_qin[1];
+  // da[q]: the alpha the loop spends in a column without a z step (over the chain xs, which
+  // the merge has read)
+  float* da = xs;
+  for (int q = threadIdx.x; q <= qmax; q += nt) da[q] = sp[q].ae - sp[q - 1].ae;
   __syncthreads();
+  const char* const zbytes = (const char*)imgZ;
   const int nxy = g.nx * g.ny, npix = nxy * g.nz;
   double lik = 0.0;
-  for (int s = threadIdx.x; s < g.nsino; s += kBlock) {
+  for (int s = threadIdx.x; s < g.nsino; s += nt) {
     const float2 zz = zab[s];
     Ray ray;
-    const bool valid = setup_ray<3>(g, t, zz.x, zz.y, ray);
-    float acc = 0.f;
+    bool valid = setup_ray<3>(g, t, zz.x, zz.y, ray);
+    if (PREC == APIRL_PREC_F64_SETUP) {
+      // the axial setup in double too (project_ray's F64_SETUP)
+      SetupZ64 zs;
+      setup_z_f64(g, xy64, zz.x, t.vx, t.vy, (double)(zz.y - zz.x), zs);
+      ray.az = (float)zs.az;
+      ray.azu = (float)zs.azu;
+      ray.ac = (float)xy64.amin;
+      ray.L = (float)zs.L;
+      ray.k = zs.k0;
+      ray.kinc = zs.kinc;
+      ray.n = abs(xy64.i1 - xy64.i0) + abs(xy64.j1 - xy64.j0) + abs(zs.k1 - zs.k0);
+    }
+    RaySum<kSum2> acc;
     if (valid) {
-      // Steps are taken kPathUnroll at a time: the batch's voxel loads are issued together,
-      // then added in the loop's order.
-      int q = 0, k = ray.k;
-      FwdStep e = sp[0];
+      // state: the next z crossing, the last crossing taken, the slice (kb: its byte offset
+      // in a column) and the columns left (q); n - left steps are taken so far
       float Zn = ray.az, ac = ray.ac;
-      for (int m0 = 0; m0 < ray.n; m0 += kPathUnroll) {
+      const float azu = ray.azu, L = ray.L;
+      const int kinc = ray.kinc, kstep = kinc * 4, nzb = g.nz * 4;
+      int kb = ray.k * 4, left = ray.n, q = 0;
+      // slices to the face ahead; a compensated sum is changed by a zero term, so there no
+      // batch may pass a face: the crossing into the slice beyond (half an increment early,
+      // for the rounding) has to come after the batch's last column
+      auto within = [&](int steps) -> bool {
+        if (!kSum2) return true;
+        const int room = (kinc > 0 ? nzb - 4 - kb : kb) >> 2;
+        const int last = q + steps - 1 < qmax ? q + steps - 1 : qmax;
+        return (kinc == 0) | (room >= steps - 1) |
+               (Zn + ((float)room - 0.5f) * azu >= sp[last].ae);
+      };
+      // kPathCols columns at a time, the same ones for every lane, as long as no lane takes
+      // more than one z step among them: column c, whose exit alpha is the first above Zn
+      while (q >= qa && q + kPathCols - 1 <= qb) {
+        const float aend = sp[q + kPathCols - 1].ae, Z1 = Zn + azu;
+        const int kb1 = kb + kstep;
+        if (!__all((Zn >= ac) & (Z1 >= aend) & (left > kPathCols) &
+                   ((unsigned)kb < (unsigned)nzb) & within(kPathCols)))
+          break;
+        float p[kPathCols], d[kPathCols];
+        bool zs[kPathCols];  // the z step comes before the column's exit
+        int c = 0;
+#pragma unroll
+        for (int u = 0; u < kPathCols; u++) {
+          const FwdStep e = sp[q + u];
+          d[u] = da[q + u];
+          zs[u] = Zn < e.ae;
+          p[u] = *(const float*)(zbytes + (e.base + (unsigned)(zs[u] ? kb1 : kb)));
+          c += zs[u] ? 0 : 1;
+        }
+        c = q + (c < kPathCols ? c : kPathCols - 1);
+        const FwdStep ez = sp[c];
+        const float pz = *(const float*)(zbytes + (ez.base + (unsigned)kb));
+        const float wz = (Zn - sp[c - 1].ae) * L, dc = ez.ae - Zn;
+#pragma unroll
+        for (int u = 0; u < kPathCols; u++) {
+          const bool atz = zs[u] && !(u > 0 && zs[u > 0 ? u - 1 : 0]);
+          acc.add_if(atz, wz * pz);
+          acc.add(((atz ? dc : d[u]) * L) * p[u]);
+        }
+        const bool crossed = zs[kPathCols - 1];
+        Zn = crossed ? Z1 : Zn;
+        kb = crossed ? kb1 : kb;
+        ac = aend;
+        q += kPathCols;
+        left -= kPathCols + (crossed ? 1 : 0);
+      }
+      // Step by step, kPathUnroll at a time: the batch's voxel loads are issued together,
+      // then added in the loop's order.
+      for (; left > 0; left -= kPathUnroll) {
         float wv[kPathUnroll], pv[kPathUnroll];
-        // a batch whose kPathUnroll steps all stay in the image (the path's next kPathUnroll
-        // columns inside; the slice inside and kPathUnroll - 1 z steps from the face it
-        // moves towards) needs no read test; the wavefront takes it when every lane can
-        const int kfar = k + (kPathUnroll - 1) * ray.kinc;
-        const bool fast = (m0 + kPathUnroll <= ray.n) & (e.run >= kPathUnroll) & (k >= 0) &
-                          (k < g.nz) & (kfar >= 0) & (kfar < g.nz);
-        if (__all(fast)) {
+        // A batch whose columns are all inside the image (its entries are among qa .. qb)
+        // and that starts at a slice inside needs no read test: past a face it reads the
+        // zeros.  The wavefront takes this form when every lane can.
+        const int steps = left < kPathUnroll ? left : kPathUnroll;
+        if (__all((q >= qa) & (q + steps - 1 <= qb) & ((unsigned)kb < (unsigned)nzb) &
+                  within(kPathUnroll))) {
+          const FwdStep* ep = sp + q;
+          if (__all(left >= kPathUnroll)) {
 #pragma unroll
-          for (int u = 0; u < kPathUnroll; u++) {
-            const bool zst = Zn < e.ae;
-            const float an = zst ? Zn : e.ae;
-            wv[u] = (an - ac) * ray.L;
-            ac = an;
-            pv[u] = imgZ[(unsigned)(e.base + k)];  // inside the image: non-negative
-            Zn = zst ? Zn + ray.azu : Zn;
-            k += zst ? ray.kinc : 0;
-            q += zst ? 0 : 1;
-            e = sp[q];
+            for (int u = 0; u < kPathUnroll; u++) {
+              const FwdStep e = *ep;
+              const bool zst = Zn < e.ae;
+              const float an = zst ? Zn : e.ae;
+              wv[u] = (an - ac) * L;
+              ac = an;
+              pv[u] = *(const float*)(zbytes + (e.base + (unsigned)kb));
+              Zn = Zn + (zst ? azu : 0.f);
+              kb += zst ? kstep : 0;
+              ep += zst ? 0 : 1;
+            }
+#pragma unroll
+            for (int u = 0; u < kPathUnroll; u++) acc.add(wv[u] * pv[u]);
+          } else {
+            // some lane's last steps: the same, each step taken while it is left
+#pragma unroll
+            for (int u = 0; u < kPathUnroll; u++) {
+              const FwdStep e = *ep;
+              const bool zst = Zn < e.ae, on = u < left;
+              const float an = zst ? Zn : e.ae;
+              wv[u] = (an - ac) * L;
+              ac = an;
+              pv[u] = *(const float*)(zbytes + (on ? e.base + (unsigned)kb : 0u));
+              Zn = Zn + (zst ? azu : 0.f);
+              kb += zst ? kstep : 0;
+              ep += (zst | !on) ? 0 : 1;
+            }
+#pragma unroll
+            for (int u = 0; u < kPathUnroll; u++) acc.add_if(u < left, wv[u] * pv[u]);
           }
-#pragma unroll
-          for (int u = 0; u < kPathUnroll; u++) acc = acc + wv[u] * pv[u];
+          q = (int)(ep - sp);
           continue;
         }
         bool tv[kPathUnroll];
+        int k = kb >> 2;
+        q = q < qmax ? q : qmax - 1;
 #pragma unroll
         for (int u = 0; u < kPathUnroll; u++) {
+          const FwdStep e = sp[q];
           const bool zst = Zn < e.ae;
           const float an = zst ? Zn : e.ae;
-          wv[u] = (an - ac) * ray.L;
+          wv[u] = (an - ac) * L;
           ac = an;
           // the reference's read test (upper bounds and a non-negative linear index)
-          const int ci = e.i, cj = e.j;
+          const int c = ij[q], ci = (short)(c & 0xffff), cj = c >> 16;
           const int li = k * nxy + cj * g.nx + ci;
-          const bool ok = (ci < g.nx) & (cj < g.ny) & (k < g.nz) & (li >= 0) & (li < npix) &
-                          (m0 + u < ray.n);
-          const bool inside = (ci >= 0) & (cj >= 0);
+          const bool inside = (ci >= 0) & (cj >= 0) & (k >= 0);
+          bool ok = (ci < g.nx) & (cj < g.ny) & (k < g.nz) & (u < left);
+          ok &= kStrict ? inside : (li >= 0) & (li < npix);
           tv[u] = ok;
-          pv[u] = ok ? (inside ? imgZ[e.base + k] : img[li]) : 0.f;
-          Zn = zst ? Zn + ray.azu : Zn;
-          k += zst ? ray.kinc : 0;
+          pv[u] = ok ? (inside ? *(const float*)(zbytes + (e.base + (unsigned)(k * 4))) : img[li])
+                     : 0.f;
+          Zn = Zn + (zst ? azu : 0.f);
+          k += zst ? kinc : 0;
           q += zst ? 0 : 1;
-          e = sp[q < qmax ? q : qmax - 1];
+          q = q < qmax ? q : qmax - 1;
         }
 #pragma unroll
-        for (int u = 0; u < kPathUnroll; u++) {
-          const float term = wv[u] * pv[u];
-          const float nacc = acc + term;
-          acc = tv[u] ? nacc : acc;
-        }
+        for (int u = 0; u < kPathUnroll; u++) acc.add_if(tv[u], wv[u] * pv[u]);
+        kb = k * 4;
       }
     }
     const long idx = ((long)s * nang_sub + ka) * g.nr + rr;
     if (!FUSED) {
-      if (valid) sino[idx] = acc;
+      if (valid) sino[idx] = acc.s;
     } else {
       // fused EM epilogue, as project_ray's (Sinogram3D.cpp:584-607, 830-870)
       const long full = ((long)s * g.nang + a) * g.nr + rr;
-      float est = valid ? acc : 0.f;
+      float est = valid ? acc.s : 0.f;
       if (fr.additive)
         est = est + fr.additive[fr.additive_local ? ((long)s * g.nang + ka) * g.nr + rr : full];
       const float y = fr.meas[full];
@@ -1157,10 +1293,10 @@ __global__ __launch_bounds__(kBlock) void project_paths_kernel(
   if (FUSED && fr.lik_partials) {
     // deterministic block reduction of the likelihood partials (fixed tree)
     __shared__ double red[kBlock];
-    red[threadIdx.x] = lik;
+    for (int i = threadIdx.x; i < kBlock; i += nt) red[i] = i == (int)threadIdx.x ? lik : 0.0;
     __syncthreads();
     for (int off = kBlock / 2; off > 0; off >>= 1) {
-      if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
+      for (int i = threadIdx.x; i < off; i += nt) red[i] += red[i + off];
       __syncthreads();
     }
     if (threadIdx.x == 0) fr.lik_partials[blockIdx.x] = red[0];
@@ -1171,8 +1307,14 @@ __global__ __launch_bounds__(kBlock) void project_paths_kernel(
 
 bool path_forward_ok(const apirl_plan* p, int precision) {
   const Geo& g = p->geo;
-  return g.dims == 3 && precision == APIRL_PREC_REFERENCE && g.ns * g.nas == 1 && g.walk24 &&
-         p->d_imgT != nullptr && fwd_path_lds(g) <= 48 * 1024;
+  // the columns of an entry are kept in 16 bits each, a voxel's byte address in 32
+  return g.dims == 3 && precision != APIRL_PREC_F64_ALPHA && g.ns * g.nas == 1 && g.walk24 &&
+         g.nx < 16384 && g.ny < 16384 && p->d_imgT != nullptr &&
+         path_image_floats(g) < ((size_t)1 << 30) && fwd_path_lds(g) <= 48 * 1024;
+}
+
+size_t path_image_floats(const Geo& g) {
+  return (size_t)g.nx * g.ny * path_pitch(g) + kPathGuard;
 }
 
 int project_partials(const apirl_plan* p, int subset, int nsubsets, bool path) {
@@ -1196,20 +1338,27 @@ hipError_t launch_project(const apirl_plan* p, const float* img, float* sino, in
   if (path_forward_ok(p, precision)) {
     // the path forward projector: the image with z fastest (into the plan's
     // transposed-image buffer), one workgroup per (angle, bin) of the subset
-    const int npair = nang_sub * g.nr, qmax = fwd_path_len(g);
+    const int npair = nang_sub * g.nr, qmax = fwd_path_len(g), pitch = path_pitch(g);
     if (nblocks_out) *nblocks_out = npair;
-    const dim3 tg((g.nx + 31) / 32, g.ny, (g.nz + 31) / 32);
+    const dim3 tg((g.nx + 31) / 32, g.ny, (pitch + 31) / 32);
     hipLaunchKernelGGL(transpose_zfast_kernel, tg, dim3(kBlock), 0, st, img, p->d_imgT, g.nx,
-                       g.ny, g.nz);
-    const size_t lds = fwd_path_lds(g);  // 12.4 KB for 256 x 256
-    if (f)
-      hipLaunchKernelGGL(project_paths_kernel<true>, dim3(npair), dim3(kBlock), lds, st, g,
-                         p->d_rays, p->d_zab, img, p->d_imgT, sino, nang_sub, subset, nsubsets, fr,
-                         qmax);
-    else
-      hipLaunchKernelGGL(project_paths_kernel<false>, dim3(npair), dim3(kBlock), lds, st, g,
-                         p->d_rays, p->d_zab, img, p->d_imgT, sino, nang_sub, subset, nsubsets, fr,
-                         qmax);
+                       g.ny, g.nz, pitch);
+    const size_t lds = fwd_path_lds(g);  // 10.4 KB for 256 x 256
+    const dim3 wg(64 * fwd_path_waves(g));
+#define APIRL_LAUNCH_PATHS(F, PR)                                                             \
+  hipLaunchKernelGGL((project_paths_kernel<F, PR>), dim3(npair), wg, lds, st, g, p->d_rays,   \
+                     p->d_zab, img, p->d_imgT, sino, nang_sub, subset, nsubsets, fr, qmax, pitch)
+    if (precision == APIRL_PREC_KAHAN) {
+      if (f) APIRL_LAUNCH_PATHS(true, APIRL_PREC_KAHAN);
+      else APIRL_LAUNCH_PATHS(false, APIRL_PREC_KAHAN);
+    } else if (precision == APIRL_PREC_F64_SETUP) {
+      if (f) APIRL_LAUNCH_PATHS(true, APIRL_PREC_F64_SETUP);
+      else APIRL_LAUNCH_PATHS(false, APIRL_PREC_F64_SETUP);
+    } else {
+      if (f) APIRL_LAUNCH_PATHS(true, APIRL_PREC_REFERENCE);
+      else APIRL_LAUNCH_PATHS(false, APIRL_PREC_REFERENCE);
+    }
+#undef APIRL_LAUNCH_PATHS
     return hipGetLastError();
   }
   const float* imgT = nullptr;
