@@ -29,7 +29,7 @@ struct alignas(16) RayXY {
   int i0, j0;      // entry voxel indices (may be -1 or n)
   int nxy;         // |imax - imin| + |jmax - jmin|
   int flags;       // see RAY_* below
-  int pad;
+  float len;       // sqrtf(lxy): the ray length of a 2D LOR
 };
 static_assert(sizeof(RayXY) == 64, "RayXY must be one 64-byte line");
 
@@ -406,6 +406,7 @@ struct GatherArgs {
   const float* upd_sens;
   float upd_thr;
   int upd_strict;
+  int maxc;  // 2D: upper bound on a voxel's candidate bins of one angle
 };
 
 struct BatchHeader {
@@ -447,7 +448,7 @@ struct ZsJob {  // axial records of one subset for the gather
   long nrays;
   long first;
 };
-struct GJob {  // gather backprojection of one subset (16 x 16 slice tiles)
+struct GJob {  // gather backprojection of one subset (3D: 16 x 16 column tiles; 2D: 8 x 8 patches)
   GatherArgs A;
   int ntx, nty;
   long first;
@@ -465,9 +466,11 @@ constexpr int kGroupBlock = 256;  // threads per workgroup of the grouped launch
 inline long group_blocks(long n) { return (n + kGroupBlock - 1) / kGroupBlock; }
 // Voxels per lane along z of the grouped 3D gather (the column kernel's default).
 constexpr int kGroupZV = 3;
+constexpr int kPatch2 = 8;  // the 2D gather's voxel patches are kPatch2 x kPatch2
 inline long gather_tile_blocks(const Geo& g) {
-  const int nzg = g.dims == 3 ? (g.nz + kGroupZV - 1) / kGroupZV : g.nz;
-  return (long)((g.nx + 15) / 16) * ((g.ny + 15) / 16) * nzg;
+  if (g.dims == 2)
+    return (long)((g.nx + kPatch2 - 1) / kPatch2) * ((g.ny + kPatch2 - 1) / kPatch2);
+  return (long)((g.nx + 15) / 16) * ((g.ny + 15) / 16) * ((g.nz + kGroupZV - 1) / kGroupZV);
 }
 
 hipError_t launch_group_clear(BatchHeader* hdr, const ClearJob* jobs, int grid,

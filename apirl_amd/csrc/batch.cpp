@@ -530,8 +530,9 @@ apirl_status apirl_batch_step(apirl_batch* b, int* active) {
       const int ph = j->is2d ? PH_GATHER2 : PH_GATHER3;
       GJob& q = (j->is2d ? g2 : g3)[hdr->count[ph]++];
       q.A = A;
-      q.ntx = (g.nx + 15) / 16;
-      q.nty = (g.ny + 15) / 16;
+      const int edge = j->is2d ? kPatch2 : 16;
+      q.ntx = (g.nx + edge - 1) / edge;
+      q.nty = (g.ny + edge - 1) / edge;
       q.first = hdr->total[ph];
       hdr->total[ph] += gather_tile_blocks(g);
     }

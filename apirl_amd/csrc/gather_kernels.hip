@@ -825,6 +825,150 @@ __global__ __launch_bounds__(kGBlock) void gather_kernel(GatherArgs A) {
   gather_voxel<DIMS, PREC>(A, s_zab, i, j, k);
 }
 
+// ---- 2D gather, reference arithmetic ------------------------------------------------
+//
+// A workgroup takes a patch of 8 x 8 voxels, one per lane.  Its first nw wavefronts take
+// one angle each per round and write every candidate bin's term (0 where the bin does not
+// cross the voxel) to LDS; the next wavefront adds the terms of the round before to the 64
+// sums, in the reference's order (angle, radial bin).  The terms of an angle do not depend
+// on the sums, so an image too small to fill the GPU with one lane per voxel (gather_kernel:
+// 256 wavefronts for 128 x 128, each waiting for the loads of 192 angles in turn) runs 16
+// times the wavefronts with the same sums, bit for bit.  The rays that can cross the patch
+// (17 of an angle there) are staged in LDS by coalesced loads, with their entry crossings of
+// the patch's columns and rows: read by each lane at its own candidates, they took 38 cache
+// lines per load and bounded the kernel.  128x128 from 192 angles x 192 bins: 569 -> 48 us
+// (72 without the staging); 256x256 from 252 x 344: 642 -> 139 us; 64x64 from 48 x 64: 85 ->
+// 14 us.
+constexpr int kPatch = kPatch2;
+constexpr int kG2Waves = 16;   // wavefronts of the workgroup, one of them sums
+constexpr int kG2Rays = 20;    // rays staged at a time, by each wavefront
+// a staged ray: words 4 .. 15 of its RayXY (the bin value in place of lxy) and its crossings
+// into the patch's columns and rows
+constexpr int kG2RayWords = 12 + 2 * kPatch;
+constexpr int kG2LdsFloats = 16 * 1024;  // 64 KiB: the staged rays and two rounds of terms
+// Wavefronts that compute terms for plans with up to maxc candidates per (voxel, angle);
+// 0: the terms of one angle do not fit (over 120 bins per voxel).
+__host__ __device__ inline int gather2_waves(int maxc) {
+  const int fit = kG2LdsFloats / (kG2Rays * kG2RayWords + 2 * kWave * (maxc > 0 ? maxc : 1));
+  return fit < kG2Waves - 1 ? fit : kG2Waves - 1;
+}
+inline size_t gather2_lds(int nw, int maxc) {
+  return (size_t)nw * (kG2Rays * kG2RayWords + 2 * kWave * maxc) * sizeof(float);
+}
+
+// Orders a wavefront's LDS accesses before and after this point (lanes read what
+// other lanes of the wavefront wrote).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The terms of angle ka for the voxels of patch (px, py), this lane's (i, j): T[c * 64] for
+// candidate c < maxc.  st: the wavefront's kG2Rays staged rays.
+__device__ __forceinline__ void gather2_terms(const GatherArgs& A, int ka, int px, int py, int i,
+                                              int j, float inv_dr, float* st, float* T) {
+  const Geo& g = A.g;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int a = A.subset + A.nsubsets * ka;
+  const float xc = -g.R + g.dx * ((float)i + 0.5f), yc = -g.R + g.dy * ((float)j + 0.5f);
+  int jlo, jhi, lo1, hi1;
+  candidate_bins<kGridUniform>(A, a, xc, yc, inv_dr, jlo, jhi, lo1, hi1);
+  // the patch's bins: its half-width, a hundredth of a bin and 2 um more than its voxels' own
+  // ranges, whose rounding is far below that
+  const float2 cs = A.angcs[a];
+  const float sp = (-g.R + g.dx * (float)(px * kPatch + kPatch / 2)) * cs.x +
+                   (-g.R + g.dy * (float)(py * kPatch + kPatch / 2)) * cs.y;
+  const float hp = 0.5f * kPatch * (g.dx * fabsf(cs.x) + g.dy * fabsf(cs.y)) +
+                   0.5f * fabsf(g.dx - g.dy) + g.rmargin + 0.01f * g.dr + 2e-3f;
+  int p0 = (int)ceilf((sp - hp - g.r0) * inv_dr), p1 = (int)floorf((sp + hp - g.r0) * inv_dr);
+  p0 = __builtin_amdgcn_readfirstlane(p0 < 0 ? 0 : p0);
+  p1 = __builtin_amdgcn_readfirstlane(p1 > g.nr - 1 ? g.nr - 1 : p1);
+  const float* bins = A.kind == BP_PLAIN ? A.sino + (long)ka * g.nr
+                                         : (A.kind == BP_MULT ? A.sino + (long)a * g.nr : nullptr);
+  for (int c = 0; c < A.maxc; c++) T[c * kWave] = 0.f;
+  for (int r0 = p0; r0 <= p1; r0 += kG2Rays) {
+    const int nr = p1 - r0 + 1 < kG2Rays ? p1 - r0 + 1 : kG2Rays;
+    wave_lds_sync();  // the rays staged before are read
+    if (lane < 3 * kG2Rays && lane / 3 < nr) {
+      const int r = lane / 3, q = lane - 3 * r;
+      float4 v = reinterpret_cast<const float4*>(A.rays + (long)a * g.nr + r0 + r)[1 + q];
+      if (q == 1) v.z = bins ? bins[r0 + r] : 1.f;
+      *reinterpret_cast<float4*>(st + r * kG2RayWords + 4 * q) = v;
+    }
+    const float* xytab = A.xytab + ((long)a * g.nr + r0) * (g.nx + g.ny);
+    for (int q = lane; q < nr * 2 * kPatch; q += kWave) {
+      const int r = q / (2 * kPatch), w = q % (2 * kPatch);
+      int e = w < kPatch ? px * kPatch + w : py * kPatch + w - kPatch;
+      e = w < kPatch ? (e < g.nx ? e : g.nx - 1) : g.nx + (e < g.ny ? e : g.ny - 1);
+      st[r * kG2RayWords + 12 + w] = xytab[(long)r * (g.nx + g.ny) + e];
+    }
+    wave_lds_sync();
+    const int rlo = jlo > r0 ? jlo : r0, rhi = jhi < r0 + nr - 1 ? jhi : r0 + nr - 1;
+    for (int rr = rlo; rr <= rhi; rr++) {
+      const float* s = st + (rr - r0) * kG2RayWords;
+      const float4 q1 = *reinterpret_cast<const float4*>(s);
+      const float4 q2 = *reinterpret_cast<const float4*>(s + 4);
+      const float4 q3 = *reinterpret_cast<const float4*>(s + 8);
+      const float xyi = s[12 + (i & (kPatch - 1))], xyj = s[12 + kPatch + (j & (kPatch - 1))];
+      const float amin = q1.x, ax = q1.z, ay = q1.w, axu = q2.x, ayu = q2.y, b = q2.z, len = q3.w;
+      const int i0 = __float_as_int(q2.w), j0 = __float_as_int(q3.x);
+      const int nxy = __float_as_int(q3.y), flags = __float_as_int(q3.z);
+      // the tests of gather_voxel as one predicate
+      const int iinc = ray_iinc(flags), jinc = ray_jinc(flags);
+      const int na = __mul24(i - i0, iinc), nb = __mul24(j - j0, jinc), m = na + nb;
+      bool ok = (flags & RAY_VALID) != 0;
+      ok &= (i == i0) | ((iinc != 0) & (na >= 0));
+      ok &= (j == j0) | ((jinc != 0) & (nb >= 0));
+      ok &= m < nxy;
+      const float Xp = na > 0 ? xyi : -FLT_MAX, Xn = na > 0 ? xyi + axu : ax;
+      const float Yp = nb > 0 ? xyj : -FLT_MAX, Yn = nb > 0 ? xyj + ayu : ay;
+      ok &= ((na <= 0) | (Xp <= Yn)) & ((nb <= 0) | (Yp < Xn));
+      const float ac = m > 0 ? (Xp > Yp ? Xp : Yp) : amin;
+      const float an = Xn < Yn ? Xn : Yn;
+      const float w = (an - ac) * len;
+      if (ok) T[(rr - jlo) * kWave] = w * b * 1.0f;  // SiddonProjector.cpp:72
+    }
+  }
+}
+
+// Patch (px, py) by the whole workgroup (more than nw wavefronts, 1 <= nw <=
+// gather2_waves(A.maxc)); lds: gather2_lds(nw, A.maxc) bytes.
+__device__ __forceinline__ void gather2_patch(const GatherArgs& A, int nw, int px, int py,
+                                              float* lds) {
+  const Geo& g = A.g;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & (kWave - 1);
+  const int ir = px * kPatch + (lane & (kPatch - 1)), jr = py * kPatch + lane / kPatch;
+  const bool in = ir < g.nx && jr < g.ny;
+  const int i = ir < g.nx ? ir : g.nx - 1, j = jr < g.ny ? jr : g.ny - 1;
+  const long v = (long)j * g.nx + i;
+  const float inv_dr = 1.0f / g.dr;
+  float* T = lds + nw * kG2Rays * kG2RayWords;
+  const int buf = nw * A.maxc * kWave, rounds = (A.nang_sub + nw - 1) / nw;
+  float acc = wave == nw && !A.upd_sens ? A.img[v] : 0.f;
+  for (int it = 0; it <= rounds; it++) {
+    if (wave < nw) {
+      const int ka = it * nw + wave;
+      if (ka < A.nang_sub)
+        gather2_terms(A, ka, px, py, i, j, inv_dr, lds + wave * kG2Rays * kG2RayWords,
+                      T + (it & 1) * buf + wave * A.maxc * kWave + lane);
+    } else if (wave == nw && it > 0) {
+      const float* s = T + ((it - 1) & 1) * buf + lane;
+      const int left = A.nang_sub - (it - 1) * nw, n = (left < nw ? left : nw) * A.maxc;
+#pragma unroll 8
+      for (int q = 0; q < n; q++) acc = acc + s[q * kWave];
+    }
+    __syncthreads();
+  }
+  if (wave == nw && in) store_voxel(A, v, acc);
+}
+
+__global__ __launch_bounds__(kG2Waves * kWave, 8) void gather2_kernel(GatherArgs A, int nw) {
+  extern __shared__ __align__(16) float g2lds[];
+  gather2_patch(A, nw, blockIdx.x, blockIdx.y, g2lds);
+}
+
 // ---- grouped (multi-job) launches --------------------------------------------
 #include "group_common.h"
 
@@ -846,14 +990,13 @@ __global__ __launch_bounds__(kGBlock) void zsetup_group_kernel(BatchHeader* __re
   }
 }
 
-// Each virtual block is one 16 x 16 tile of one job (tile-major), of one slice in 2D
-// and of kGroupZV slices in 3D (the column kernel's shape); 3D jobs reload the axial
-// and crossing-slot tables into LDS when the workgroup moves to another job.
-template <int DIMS>
-__global__ __launch_bounds__(kGBlock) void gather_group_kernel(BatchHeader* __restrict__ hdr,
+// Each virtual block is one 16 x 16 tile of kGroupZV slices of one job (the column
+// kernel's shape, tile-major); the axial and crossing-slot tables are reloaded into LDS
+// when the workgroup moves to another job.
+__global__ __launch_bounds__(kGBlock) void gather3_group_kernel(BatchHeader* __restrict__ hdr,
                                                                const GJob* __restrict__ jobs) {
   extern __shared__ float2 s_zab[];
-  const int ph = DIMS == 2 ? PH_GATHER2 : PH_GATHER3;
+  const int ph = PH_GATHER3;
   const int n = hdr->count[ph];
   const long total = hdr->total[ph];
   const int grab = grab_size(hdr);
@@ -866,7 +1009,7 @@ __global__ __launch_bounds__(kGBlock) void gather_group_kernel(BatchHeader* __re
       const GJob& J = jobs[jj];
       const int ns = J.A.g.nsino;
       int4* s_slot = (int4*)((char*)s_zab + column_lds_off(ns));
-      if (DIMS == 3 && loaded != jj) {
+      if (loaded != jj) {
         __syncthreads();
         for (int q = threadIdx.x; q < ns; q += kGBlock) {
           s_zab[q] = J.A.zab[q];
@@ -885,11 +1028,33 @@ __global__ __launch_bounds__(kGBlock) void gather_group_kernel(BatchHeader* __re
       const int i = bx * kTile + (threadIdx.x % kTile);
       const int j = by * kTile + (threadIdx.x / kTile);
       if (i < J.A.g.nx && j < J.A.g.ny) {
-        if constexpr (DIMS == 3)
-          gather_column<APIRL_PREC_REFERENCE, kGroupZV>(J.A, s_zab, s_slot, J.A.segs, i, j,
-                                                        kg * kGroupZV);
-        else
-          gather_voxel<DIMS, APIRL_PREC_REFERENCE>(J.A, s_zab, i, j, kg);
+        gather_column<APIRL_PREC_REFERENCE, kGroupZV>(J.A, s_zab, s_slot, J.A.segs, i, j,
+                                                      kg * kGroupZV);
+      }
+    }
+  }
+}
+
+// Each virtual block is one 8 x 8 patch of one 2D job, by the whole workgroup.
+__global__ __launch_bounds__(kG2Waves * kWave) void gather2_group_kernel(
+    BatchHeader* __restrict__ hdr, const GJob* __restrict__ jobs) {
+  extern __shared__ __align__(16) float g2lds[];
+  const int n = hdr->count[PH_GATHER2];
+  const long total = hdr->total[PH_GATHER2];
+  const int grab = grab_size(hdr);
+  for (;;) {
+    const long v0 = grab_vb(&hdr->next[PH_GATHER2], grab);
+    if (v0 >= total) break;
+    for (long vb = v0; vb < v0 + grab && vb < total; vb++) {
+      const GJob& J = jobs[find_job(jobs, n, vb)];
+      const int lb = (int)(vb - J.first), px = lb % J.ntx, py = lb / J.ntx;
+      const int nw = gather2_waves(J.A.maxc);
+      if (nw > 0) {
+        gather2_patch(J.A, nw, px, py, g2lds);
+      } else if (threadIdx.x < kWave) {  // more candidates per angle than the LDS holds
+        const int i = px * kPatch2 + threadIdx.x % kPatch2, j = py * kPatch2 + threadIdx.x / kPatch2;
+        if (i < J.A.g.nx && j < J.A.g.ny)
+          gather_voxel<2, APIRL_PREC_REFERENCE>(J.A, nullptr, i, j, 0);
       }
     }
   }
@@ -942,6 +1107,13 @@ void launch_gather3(const GatherArgs& A, int zlanes, int zvox, hipStream_t st) {
 template <int PREC>
 void launch_gather2(const GatherArgs& A, hipStream_t st) {
   const Geo& g = A.g;
+  if (PREC == APIRL_PREC_REFERENCE && gather2_waves(A.maxc) > 0) {
+    const int nw = gather2_waves(A.maxc) < A.nang_sub ? gather2_waves(A.maxc) : A.nang_sub;
+    hipLaunchKernelGGL(gather2_kernel,
+                       dim3((g.nx + kPatch2 - 1) / kPatch2, (g.ny + kPatch2 - 1) / kPatch2),
+                       dim3((nw + 1) * kWave), gather2_lds(nw, A.maxc), st, A, nw);
+    return;
+  }
   const dim3 grid((g.nx + kTile - 1) / kTile, (g.ny + kTile - 1) / kTile, g.nz);
   hipLaunchKernelGGL((gather_kernel<2, PREC>), grid, dim3(kGBlock), 0, st, A);
 }
@@ -1175,14 +1347,6 @@ __device__ __forceinline__ void tile_lane(const TileRay& R, const float* pae,
     ae = zst ? ae : ae1;
     cidx = zst ? cidx : c1 * zs;
   }
-}
-
-// Orders a wavefront's LDS accesses before and after this point (lanes read what
-// other lanes of the wavefront wrote).
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // One in-flight ray of a wavefront, in LDS: its entry and path (the lanes walking
@@ -1973,6 +2137,9 @@ void gather_args_for(const apirl_plan* p, int subset, int nsubsets, int kind, co
   }
   A.zr = zr;
   A.nz_pair = nz_pair;
+  // bins within the column's half-width (candidate_bins) of its centre, on a uniform grid
+  A.maxc = (int)std::min(1e6, std::floor((1.41421357 * std::max(g.dx, g.dy) + 2.0 * g.rmargin) /
+                                             g.dr * 1.0001 + 1e-3) + 1);
   A.upd_sens = nullptr;
   A.upd_thr = 0.f;
   A.upd_strict = 0;
@@ -1981,8 +2148,9 @@ void gather_args_for(const apirl_plan* p, int subset, int nsubsets, int kind, co
 hipError_t launch_group_gather(BatchHeader* hdr, const ZsJob* zs, const GJob* g2,
                                const GJob* g3, int grid, int max_nsino, hipStream_t st) {
   hipLaunchKernelGGL(zsetup_group_kernel, dim3(grid), dim3(kGBlock), 0, st, hdr, zs);
-  hipLaunchKernelGGL(gather_group_kernel<2>, dim3(grid), dim3(kGBlock), 0, st, hdr, g2);
-  hipLaunchKernelGGL(gather_group_kernel<3>, dim3(grid), dim3(kGBlock),
+  hipLaunchKernelGGL(gather2_group_kernel, dim3(grid), dim3(kG2Waves * kWave),
+                     kG2LdsFloats * sizeof(float), st, hdr, g2);
+  hipLaunchKernelGGL(gather3_group_kernel, dim3(grid), dim3(kGBlock),
                      column_lds_bytes(max_nsino), st, hdr, g3);
   return hipGetLastError();
 }

@@ -211,6 +211,7 @@ void build_ray_table_pts(const apirl_image_desc& img, bool is2d, const std::vect
       t.axu = fabsf(dx / vx);
       t.ayu = fabsf(dy / vy);
       t.lxy = ex * ex + ey * ey;
+      t.len = sqrtf(t.lxy);
       t.i0 = imin; t.j0 = jmin;
       t.nxy = rejected ? 0 : std::abs(imax - imin) + std::abs(jmax - jmin);
       t.flags = ray_flags(iinc, jinc, 1, rejected) | (fabsf(vx) > fabsf(vy) ? RAY_XMAJOR : 0);

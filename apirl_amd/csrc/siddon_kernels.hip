@@ -45,7 +45,7 @@ __device__ __forceinline__ bool setup_ray(const Geo& g, const RayXY& t, float za
   float az = FLT_MAX, azu = 0.f, L;
   int k = 0, kinc = 0, n = t.nxy;
   if (DIMS == 2) {
-    L = sqrtf(t.lxy);
+    L = t.len;
   } else {
     const float vz = zb - za;
     const float z1 = za + vz * t.amin;
