@@ -134,13 +134,12 @@ struct apirl_plan {
   int gather_zvox = 3;             // 3D gather voxels per lane along z (1..4, tiles only)
   int gather_xcd = APIRL_GATHER_XCD_WEDGES;  // column kernel's tile order
   int tile_zs = 0;                 // tile backprojector's slab depth (0: about 5 slices)
-  int* d_tile_order = nullptr;     // its item order (built for tile_order_n items)
-  int tile_order_n = 0;
+  int* d_tile_order = nullptr;     // its tiles, nearest the image centre first
+  float* d_zinc = nullptr;         // [nsino] z-crossing increment |dz / Vz|, negative for Vz < 0
+  bool slices16 = false;           // every slice index of its rays fits 16 bits
   // its geometry per (LOR form, subset, subsets), kept from the first call on, within
-  // tile_geo_budget bytes in all (apirl_tuning.tile_cache_mb); `ready` once the launches
-  // that build it are enqueued on `stream`, whose event `ev` follows them; `list` the
-  // sinogram lists of its (item, ray) pairs (lists: 0 not tried, 1 kept, -1 beyond the
-  // budget)
+  // tile_geo_budget bytes in all (apirl_tuning.tile_cache_mb); `ready` once the launch
+  // that builds it is enqueued on `stream`, whose event `ev` follows it
   struct TileGeo {
     int form, subset, nsubsets;
     void* d;
@@ -148,9 +147,6 @@ struct apirl_plan {
     bool ready;
     hipStream_t stream;
     hipEvent_t ev;
-    unsigned short* list;
-    size_t list_bytes;
-    int lists;
   };
   std::vector<TileGeo> tile_geo;
   size_t tile_geo_used = 0;
@@ -236,9 +232,11 @@ struct FusedRatio {
 // 3D, reference precision, one LOR per bin (path_forward_ok): the path forward
 // projector, which writes project_partials(.., true) likelihood partials (one per
 // subset (angle, bin)) instead of one per 256 bins.
+// image_copy: where the projector's copy of the image goes (path_image_floats floats in 3D,
+// the image's in 2D) instead of the plan's own buffer, for work on a stream of its own.
 hipError_t launch_project(const apirl_plan* p, const float* img, float* sino, int subset,
                           int nsubsets, int precision, const FusedRatio* fused, int* nblocks_out,
-                          hipStream_t st);
+                          hipStream_t st, float* image_copy = nullptr);
 bool path_forward_ok(const apirl_plan* p, int precision);
 // Floats of the path forward projector's z-fastest image copy (apirl_plan::d_imgT).
 size_t path_image_floats(const Geo& g);
@@ -273,7 +271,9 @@ void free_os_parts(apirl_plan* p);
 // block partials into `partials`, then a fixed-order sum into *out.
 hipError_t launch_likelihood(const float* x, const float* y, long n, int positive_only,
                              double* partials, double* out, hipStream_t st);
-hipError_t launch_min_nz_max(const float* x, size_t n, float* d_out2, hipStream_t st);
+// d_out: [min_nz, max] and 2 kMinMaxBlocks floats of scratch.
+constexpr int kMinMaxBlocks = 512;
+hipError_t launch_min_nz_max(const float* x, size_t n, float* d_out, hipStream_t st);
 hipError_t launch_count_intersections(const apirl_plan* p, int subset, int nsubsets,
                                       unsigned long long* d_out, hipStream_t st);
 
@@ -288,30 +288,27 @@ hipError_t launch_backproject_gather(const apirl_plan* p, const float* sino, flo
                                      int subset, int nsubsets, int kind, int precision,
                                      void* scratch, size_t scratch_bytes, hipStream_t st,
                                      const EmFuse* fuse = nullptr);
-// Tile-walk backprojector (APIRL_BP_TILE); tile_misfit says why a plan cannot take it
-// (null when it can).  Its geometry for one subset (the candidate rays of every tile
-// and their paths; tile_geo_bytes) depends on the plan's LOR form alone: with `geo`
-// null it is built in the scratch on every call; otherwise it lives in `geo`, built
-// there when `geo_ready` is false and reused as it stands when true (with `list`, the
-// sinogram lists launch_tile_lists kept for it, when not null).  The scratch
-// (tile_scratch_bytes, with the geometry when `geo` is null) holds the call's axial
-// records with their bin values and its live-ray lists.
+// Tile-walk backprojector; tile_misfit says why a plan cannot take it (null when it can).
+// Its geometry for one subset (the rays of every tile and their paths; tile_geo_bytes)
+// depends on the plan's LOR form alone: with `geo` null it is built in the scratch on every
+// call; otherwise it lives in `geo`, built there when `geo_ready` is false and reused as it
+// stands when true.  The scratch (tile_scratch_bytes, with the geometry when `geo` is null)
+// holds the call's axial records with their bin values and the sums of its chunks.
 hipError_t launch_backproject_tile(const apirl_plan* p, const float* sino, float* img,
                                    int subset, int nsubsets, int kind, void* scratch,
                                    size_t scratch_bytes, hipStream_t st, const EmFuse* fuse,
-                                   void* geo, bool geo_ready,
-                                   const unsigned short* list = nullptr);
-// The sinogram lists of every (item, candidate ray) of a kept geometry (built):
-// with list null, counts them (*total: the device address of their number, a long
-// long, valid once the stream reaches it); otherwise writes them to list (2 bytes
-// each).  launch_backproject_tile then reads them instead of listing.
-hipError_t launch_tile_lists(const apirl_plan* p, int subset, int nsubsets, void* geo,
-                             unsigned short* list, long long** total, hipStream_t st);
+                                   void* geo, bool geo_ready);
 const char* tile_misfit(const apirl_plan* p);
+// A batched 3D job's backprojections (one LOR per bin), as apirl_backproject runs them for
+// APIRL_BP_GATHER, on any stream with a scratch of the job's own.  job_scratch_bytes: what a
+// subset needs; prepare also builds the tile order and takes the memory of its kept geometry.
+size_t job_scratch_bytes(apirl_plan* p, int subset, int nsubsets, bool prepare);
+hipError_t job_backproject(apirl_plan* p, const float* sino, float* img, int subset, int nsubsets,
+                           int kind, const EmFuse* fuse, void* scratch, size_t scratch_bytes,
+                           hipStream_t st);
 size_t tile_geo_bytes(const apirl_plan* p, int subset, int nsubsets);
 size_t tile_scratch_bytes(const apirl_plan* p, int subset, int nsubsets, bool with_geo);
-int tile_items(const apirl_plan* p);
-// item order of the tile backprojector: the tiles nearest the image centre first
+// the tiles, the ones nearest the image centre first
 void build_tile_order(const apirl_plan* p, std::vector<int>& order);
 size_t gather_scratch_bytes(const apirl_plan* p, int subset, int nsubsets);
 // The 3D gather's 32-bit record and table offsets hold for this subset (fewer than
@@ -343,7 +340,7 @@ void build_gather_tables(const apirl_plan& p, std::vector<float2>& angcs,
 enum { BP_PLAIN = 0, BP_ONES = 1, BP_DIVIDE = 2, BP_MULT = 3 };
 
 // ---- batched jobs (batch.cpp, grouped kernels) --------------------------------
-// A round runs one OSEM / MLEM sub-iteration of every active job with one launch
+// A round runs one OSEM / MLEM sub-iteration of every active 2D job with one launch
 // per phase; each launch walks a job table in device memory.  Every job owns a
 // contiguous run of "virtual blocks" (first .. next job's first) of that phase;
 // the launches are persistent (fixed grid) and their workgroups take virtual blocks
@@ -410,83 +407,38 @@ struct GatherArgs {
 };
 
 struct BatchHeader {
-  long total[8];                // virtual blocks of each phase (BatchPhase)
-  int count[8];                 // jobs in each phase's table
-  unsigned long long next[8];   // work counters (uploaded as 0 with every round's table)
+  long total[2];                // virtual blocks of each phase (BatchPhase)
+  int count[2];                 // jobs in each phase's table
+  unsigned long long next[2];   // work counters (uploaded as 0 with every round's table)
   int grab;                     // virtual blocks a workgroup takes per counter draw (>= 1)
   int pad;
 };
-enum BatchPhase { PH_CLEAR = 0, PH_PROJ2, PH_PROJ3, PH_ZSETUP, PH_GATHER2, PH_GATHER3, PH_UPDATE };
+enum BatchPhase { PH_PROJ2 = 0, PH_GATHER2 };
 
-struct ClearJob {  // zero n floats (or ints) at p
-  float* p;
-  long n;
-  long first;
-};
 struct ProjJob {  // fused projection + ratio of one subset (likelihood not taken)
   Geo g;
   const RayXY* rays;
-  const float2* zab;
-  const int* zorder;
   const float* img;
   FusedRatio fr;
   int nang_sub, subset, nsubsets, pad;
   long nrays;
   long first;
 };
-struct ZsJob {  // axial records of one subset for the gather
-  Geo g;
-  const RayXY* rays;
-  const float2* zab;
-  const float* sino;
-  ZRay* out;
-  int* nz_pair;
-  float* ztab;
-  const int* zsoff;
-  int zblock, pad;
-  int kind, nang_sub, subset, nsubsets;
-  long nrays;
-  long first;
-};
-struct GJob {  // gather backprojection of one subset (3D: 16 x 16 column tiles; 2D: 8 x 8 patches)
+struct GJob {  // gather backprojection of one subset with the update fused in (8 x 8 patches)
   GatherArgs A;
   int ntx, nty;
   long first;
 };
-struct UpdJob {  // x := (s cmp thr) ? x b / s : 0
-  float* x;
-  const float* b;
-  const float* s;
-  long n;
-  float thr;
-  int strict;
-  long first;
-};
 constexpr int kGroupBlock = 256;  // threads per workgroup of the grouped launches
 inline long group_blocks(long n) { return (n + kGroupBlock - 1) / kGroupBlock; }
-// Voxels per lane along z of the grouped 3D gather (the column kernel's default).
-constexpr int kGroupZV = 3;
 constexpr int kPatch2 = 8;  // the 2D gather's voxel patches are kPatch2 x kPatch2
-inline long gather_tile_blocks(const Geo& g) {
-  if (g.dims == 2)
-    return (long)((g.nx + kPatch2 - 1) / kPatch2) * ((g.ny + kPatch2 - 1) / kPatch2);
-  return (long)((g.nx + 15) / 16) * ((g.ny + 15) / 16) * ((g.nz + kGroupZV - 1) / kGroupZV);
+inline long gather_patches(const Geo& g) {
+  return (long)((g.nx + kPatch2 - 1) / kPatch2) * ((g.ny + kPatch2 - 1) / kPatch2);
 }
 
-hipError_t launch_group_clear(BatchHeader* hdr, const ClearJob* jobs, int grid,
-                              hipStream_t st);
-hipError_t launch_group_project(BatchHeader* hdr, const ProjJob* jobs2,
-                                const ProjJob* jobs3, int grid, hipStream_t st);
-hipError_t launch_group_update(BatchHeader* hdr, const UpdJob* jobs, int grid,
-                               hipStream_t st);
-hipError_t launch_group_gather(BatchHeader* hdr, const ZsJob* zs, const GJob* g2,
-                               const GJob* g3, int grid, int max_nsino, hipStream_t st);
+hipError_t launch_group_project(BatchHeader* hdr, const ProjJob* jobs, int grid, hipStream_t st);
+hipError_t launch_group_gather(BatchHeader* hdr, const GJob* jobs, int grid, hipStream_t st);
 void gather_args_for(const apirl_plan* p, int subset, int nsubsets, int kind, const float* sino,
                      float* img, void* scratch, GatherArgs& A, ZRay*& zr, int*& nz_pair);
-// LDS bytes of the 3D gather launches for nsino sinograms (axial table, slot offsets
-// and first slices of the z-crossing table)
-inline size_t gather_lds_bytes(int nsino) {
-  return (size_t)nsino * sizeof(float2) + (size_t)(2 * nsino + 1) * sizeof(int);
-}
 
 }  // namespace apirl

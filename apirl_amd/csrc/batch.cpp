@@ -1,11 +1,11 @@
 // Batched OSEM / MLEM jobs: many reconstructions of different geometries advance
-// together, one sub-iteration of every active job per round.  Jobs of at least
-// kLargeVoxels voxels run their sub-iteration with the single-job kernels after the
-// grouped launches; the others share the round's seven grouped launches (clear, fused projection + ratio for 2D and 3D jobs, axial setup,
-// gather backprojection for 2D and 3D jobs, update) that read per-job descriptors
-// from a table in device memory; the launches are persistent (fixed grid), so the
-// whole round is captured once into a hipGraph and replayed, and jobs join or leave
-// between rounds by rewriting the table (continuous batching).
+// together, one sub-iteration of every active job per round.  The 2D jobs share the
+// round's two grouped launches (fused projection + ratio, gather backprojection with the
+// update fused in) that read per-job descriptors from a table in device memory; the
+// launches are persistent (fixed grid), so the pair is captured once into a hipGraph and
+// replayed, and jobs join or leave between rounds by rewriting the table (continuous
+// batching).  A 3D job's sub-iteration fills the GPU with its own launches, which are
+// enqueued after the grouped ones, with buffers of the job's own.
 //
 // Each job computes exactly what apirl_em_reconstruct computes for it with
 // APIRL_BP_GATHER and APIRL_PREC_REFERENCE (same per-ray and per-voxel code, fixed
@@ -42,17 +42,15 @@ struct BJob {
   // device state owned by the job
   float* sens = nullptr;     // S images
   float* ratio = nullptr;    // largest subset sinogram
-  float* bp = nullptr;       // backprojection
-  void* zscr = nullptr;      // gather axial records + non-zero flags (3D)
+  float* bp = nullptr;       // backprojection (oversampled bins: one LOR after the other)
+  void* zscr = nullptr;      // 3D: backprojection scratch
   size_t zscr_bytes = 0;
-  bool large = false;        // runs its sub-iterations with the single-job kernels
-  bool tile = false;         //   and, large, the tile backprojector (else the gather)
+  float* copy = nullptr;     // 3D: the projector's copy of the image
   std::vector<std::pair<void*, size_t>> bufs;
 };
 
-// A 3D job of at least this many voxels fills the GPU with its own launches, so its
-// sub-iterations are enqueued with the single-job kernels (which read the plan's
-// transposed image copy and need no job table) after each grouped round.
+// 3D jobs of at least this many voxels are named after the tile form
+// (apirl_batch_job_backprojector).
 constexpr size_t kLargeVoxels = size_t(1) << 21;
 
 template <class T>
@@ -77,8 +75,7 @@ struct apirl_batch {
   char* h_tab[2] = {nullptr, nullptr};
   hipEvent_t copy_ev[2] = {nullptr, nullptr};
   int cur = 0;
-  size_t off_clear = 0, off_p2 = 0, off_p3 = 0, off_zs = 0, off_g2 = 0, off_g3 = 0,
-         off_upd = 0, tab_bytes = 0;
+  size_t off_p2 = 0, off_g2 = 0, tab_bytes = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   std::multimap<size_t, void*> pool;  // released device buffers, reused by size
@@ -108,7 +105,7 @@ void* balloc(apirl_batch* b, size_t bytes) {
 void release_bufs(apirl_batch* b, BJob* j) {
   for (auto& pr : j->bufs) b->pool.emplace(pr.second, pr.first);
   j->bufs.clear();
-  j->sens = j->ratio = j->bp = nullptr;
+  j->sens = j->ratio = j->bp = j->copy = nullptr;
   j->zscr = nullptr;
 }
 
@@ -118,23 +115,22 @@ size_t max_subset_bins(const apirl_plan* p, int S) {
   return m;
 }
 
-size_t max_gather_scratch(const apirl_plan* p, int S) {
+size_t job_scratch(apirl_plan* p, int S, bool prepare) {
   size_t m = 0;
-  for (int s = 0; s < S; s++) m = std::max(m, gather_scratch_bytes(p, s, S));
+  for (int s = 0; s < S; s++) m = std::max(m, job_scratch_bytes(p, s, S, prepare));
   return m;
 }
 
-// The direct path's gather backprojection of a job's ratio into its bp: the plan's
-// own, or for oversampled bins those of its plans of one LOR per bin, in turn.
-hipError_t backproject_job(const BJob* j, int s, hipStream_t st) {
-  const apirl_plan* p = j->plan;
+// The 3D backprojection of a job: the plan's own, or for oversampled bins those of its plans
+// of one LOR per bin, in turn (fuse needs one LOR per bin).
+hipError_t backproject_job(const BJob* j, const float* sino, float* img, int s, int kind,
+                           const EmFuse* fuse, hipStream_t st) {
+  apirl_plan* p = j->plan;
   if (p->geo.ns * p->geo.nas == 1)
-    return launch_backproject_gather(p, j->ratio, j->bp, s, j->S, BP_PLAIN, APIRL_PREC_REFERENCE,
-                                     j->zscr, j->zscr_bytes, st);
-  for (const apirl_plan* h : p->os_parts) {
-    const hipError_t e = launch_backproject_gather(h, j->ratio, j->bp, s, j->S, BP_PLAIN,
-                                                   APIRL_PREC_REFERENCE, j->zscr, j->zscr_bytes,
-                                                   st);
+    return job_backproject(p, sino, img, s, j->S, kind, fuse, j->zscr, j->zscr_bytes, st);
+  for (apirl_plan* h : p->os_parts) {
+    const hipError_t e =
+        job_backproject(h, sino, img, s, j->S, kind, nullptr, j->zscr, j->zscr_bytes, st);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -142,20 +138,10 @@ hipError_t backproject_job(const BJob* j, int s, hipStream_t st) {
 
 hipError_t enqueue_round(apirl_batch* b) {
   BatchHeader* hdr = (BatchHeader*)b->d_tab;
-  hipError_t e;
-  if ((e = launch_group_clear(hdr, (const ClearJob*)(b->d_tab + b->off_clear), b->grid,
-                              b->stream)) != hipSuccess)
-    return e;
-  if ((e = launch_group_project(hdr, (const ProjJob*)(b->d_tab + b->off_p2),
-                                (const ProjJob*)(b->d_tab + b->off_p3), b->grid, b->stream)) !=
-      hipSuccess)
-    return e;
-  if ((e = launch_group_gather(hdr, (const ZsJob*)(b->d_tab + b->off_zs),
-                               (const GJob*)(b->d_tab + b->off_g2),
-                               (const GJob*)(b->d_tab + b->off_g3), b->grid, b->max_nsino,
-                               b->stream)) != hipSuccess)
-    return e;
-  return launch_group_update(hdr, (const UpdJob*)(b->d_tab + b->off_upd), b->grid, b->stream);
+  const hipError_t e = launch_group_project(hdr, (const ProjJob*)(b->d_tab + b->off_p2), b->grid,
+                                            b->stream);
+  if (e != hipSuccess) return e;
+  return launch_group_gather(hdr, (const GJob*)(b->d_tab + b->off_g2), b->grid, b->stream);
 }
 
 hipError_t capture(apirl_batch* b) {
@@ -190,20 +176,10 @@ apirl_status apirl_batch_create(apirl_ctx* ctx, int max_jobs, int max_sinograms,
   b->cap = max_jobs;
   b->max_nsino = max_sinograms;
   size_t off = align_up<char>(sizeof(BatchHeader));
-  b->off_clear = off;
-  off += align_up<char>(sizeof(ClearJob) * 2 * max_jobs);
   b->off_p2 = off;
   off += align_up<char>(sizeof(ProjJob) * max_jobs);
-  b->off_p3 = off;
-  off += align_up<char>(sizeof(ProjJob) * max_jobs);
-  b->off_zs = off;
-  off += align_up<char>(sizeof(ZsJob) * max_jobs);
   b->off_g2 = off;
   off += align_up<char>(sizeof(GJob) * max_jobs);
-  b->off_g3 = off;
-  off += align_up<char>(sizeof(GJob) * max_jobs);
-  b->off_upd = off;
-  off += align_up<char>(sizeof(UpdJob) * max_jobs);
   b->tab_bytes = off;
   if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
       hipMalloc(&b->d_tab, off) != hipSuccess ||
@@ -257,14 +233,16 @@ int apirl_batch_job_backprojector(const apirl_plan* p) {
 size_t apirl_batch_job_bytes(const apirl_plan* p, int subsets) {
   if (!p || subsets < 1) return 0;
   const size_t nvox = apirl_plan_image_voxels(p);
-  size_t bytes = (size_t)subsets * nvox * sizeof(float) + nvox * sizeof(float) +
+  size_t bytes = (size_t)subsets * nvox * sizeof(float) +
                  max_subset_bins(p, subsets) * sizeof(float);
   if (p->geo.dims == 3) {
-    // oversampled bins: the largest gather scratch of the plans of one LOR per bin
-    // once they are built (the job's submission builds them), the plan's own before
-    size_t z = max_gather_scratch(p, subsets);
-    for (const apirl_plan* h : p->os_parts) z = std::max(z, max_gather_scratch(h, subsets));
-    bytes += z;
+    // oversampled bins: the largest scratch of the plans of one LOR per bin once they are
+    // built (the job's submission builds them), the plan's own before
+    size_t z = 0;
+    if (p->os_parts.empty()) z = job_scratch(const_cast<apirl_plan*>(p), subsets, false);
+    for (apirl_plan* h : p->os_parts) z = std::max(z, job_scratch(h, subsets, false));
+    bytes += z + path_image_floats(p->geo) * sizeof(float);
+    if (p->geo.ns * p->geo.nas > 1) bytes += nvox * sizeof(float);
   }
   return bytes;
 }
@@ -341,12 +319,12 @@ apirl_status apirl_batch_submit(apirl_batch* b, const apirl_job_desc* d, int* jo
   j->x = d->d_out;
   j->nvox = apirl_plan_image_voxels(p);
   j->strict = (!j->osem && j->is2d) ? 1 : 0;
+  apirl::ActiveForm form_scope(p, j->form);
   const size_t sens_b = (size_t)j->S * j->nvox * sizeof(float);
   const size_t ratio_b = max_subset_bins(p, j->S) * sizeof(float);
-  const size_t bp_b = j->nvox * sizeof(float);
   size_t z_b = 0;
   if (!j->is2d)
-    for (apirl_plan* q : gplans) z_b = std::max(z_b, max_gather_scratch(q, j->S));
+    for (apirl_plan* q : gplans) z_b = std::max(z_b, job_scratch(q, j->S, true));
   auto get = [&](size_t n) -> void* {
     void* q = balloc(b, n);
     if (q) j->bufs.emplace_back(q, n);
@@ -354,15 +332,11 @@ apirl_status apirl_batch_submit(apirl_batch* b, const apirl_job_desc* d, int* jo
   };
   j->sens = (float*)get(sens_b);
   j->ratio = (float*)get(ratio_b);
-  j->bp = (float*)get(bp_b);
+  if (os) j->bp = (float*)get(j->nvox * sizeof(float));
   if (z_b) j->zscr = get(z_b);
   j->zscr_bytes = z_b;
-  j->large = (!j->is2d && j->nvox >= kLargeVoxels) || os;
-  {
-    apirl::ActiveForm fs(p, j->form);
-    j->tile = apirl_batch_job_backprojector(p) == APIRL_BP_TILE;
-  }
-  if (!j->sens || !j->ratio || !j->bp || (z_b && !j->zscr) ||
+  if (!j->is2d) j->copy = (float*)get(path_image_floats(p->geo) * sizeof(float));
+  if (!j->sens || !j->ratio || (os && !j->bp) || (z_b && !j->zscr) || (!j->is2d && !j->copy) ||
       hipEventCreateWithFlags(&j->done_ev, hipEventDisableTiming) != hipSuccess) {
     release_bufs(b, j);
     delete j;
@@ -385,12 +359,23 @@ apirl_status apirl_batch_submit(apirl_batch* b, const apirl_job_desc* d, int* jo
   c->stream = b->stream;
   apirl_status st = APIRL_OK;
   j->thr.assign(j->S, 0.f);
-  apirl::ActiveForm form_scope(p, j->form);
   for (int s = 0; s < j->S && st == APIRL_OK; s++) {
-    st = apirl_sensitivity(p, d->d_mult, j->sens + (size_t)s * j->nvox, s, j->S,
-                           j->tile ? APIRL_BP_TILE : APIRL_BP_GATHER, j->osem);
-    if (st == APIRL_OK && !j->osem)
-      st = apirl_mlem_threshold(c, j->sens + (size_t)s * j->nvox, j->nvox, &j->thr[s]);
+    float* sens = j->sens + (size_t)s * j->nvox;
+    if (j->is2d) {
+      st = apirl_sensitivity(p, d->d_mult, sens, s, j->S, APIRL_BP_GATHER, j->osem);
+    } else {
+      // as apirl_sensitivity computes it, in the job's own scratch
+      hipError_t e = hipMemsetAsync(sens, 0, j->nvox * sizeof(float), b->stream);
+      if (e == hipSuccess)
+        e = backproject_job(j, d->d_mult, sens, s, d->d_mult ? BP_MULT : BP_ONES, nullptr,
+                            b->stream);
+      if (e == hipSuccess && j->osem) e = launch_force_positive(sens, j->nvox, b->stream);
+      if (e != hipSuccess) {
+        c->err = std::string("sensitivity: ") + hipGetErrorString(e);
+        st = APIRL_ERR_HIP;
+      }
+    }
+    if (st == APIRL_OK && !j->osem) st = apirl_mlem_threshold(c, sens, j->nvox, &j->thr[s]);
   }
   if (st == APIRL_OK &&
       hipMemcpyAsync(j->x, d->d_init, j->nvox * sizeof(float), hipMemcpyDeviceToDevice,
@@ -424,15 +409,10 @@ apirl_status apirl_batch_step(apirl_batch* b, int* active) {
   BatchHeader* hdr = (BatchHeader*)h;
   std::memset(hdr, 0, sizeof(BatchHeader));
   hdr->grab = b->grab;
-  ClearJob* cl = (ClearJob*)(h + b->off_clear);
   ProjJob* p2 = (ProjJob*)(h + b->off_p2);
-  ProjJob* p3 = (ProjJob*)(h + b->off_p3);
-  ZsJob* zs = (ZsJob*)(h + b->off_zs);
   GJob* g2 = (GJob*)(h + b->off_g2);
-  GJob* g3 = (GJob*)(h + b->off_g3);
-  UpdJob* up = (UpdJob*)(h + b->off_upd);
   std::vector<BJob*> finishing;
-  std::vector<std::pair<BJob*, int>> direct;  // large jobs and their subset this round
+  std::vector<std::pair<BJob*, int>> direct;  // 3D jobs and their subset this round
   // The jobs' virtual blocks are laid out, and so drawn, in this order: submission,
   // or the round's largest sub-iteration first (rays traced plus voxels) so that the
   // small jobs fill the end of each phase.  Results do not depend on it.
@@ -453,7 +433,7 @@ apirl_status apirl_batch_step(apirl_batch* b, int* active) {
     const apirl_plan* p = j->plan;
     const Geo& g = p->geo;
     const int s = j->s, S = j->S;
-    if (j->large) {
+    if (!j->is2d) {
       direct.emplace_back(j, s);
       if (++j->s == S) {
         j->s = 0;
@@ -463,33 +443,11 @@ apirl_status apirl_batch_step(apirl_batch* b, int* active) {
     }
     const int nang_sub = subset_num_angles(g.nang, S, s);
     const long nrays = (long)g.nsino * nang_sub * g.nr;
-    // clear the backprojection (and the gather's non-zero flags)
+    // fused projection + ratio (Sinogram2D.cpp:234-266)
     {
-      ClearJob& c = cl[hdr->count[PH_CLEAR]++];
-      c.p = j->bp;
-      c.n = (long)j->nvox;
-      c.first = hdr->total[PH_CLEAR];
-      hdr->total[PH_CLEAR] += group_blocks(c.n);
-    }
-    GatherArgs A;
-    ZRay* zr = nullptr;
-    int* nzp = nullptr;
-    gather_args_for(p, s, S, BP_PLAIN, j->ratio, j->bp, j->zscr, A, zr, nzp);
-    if (!j->is2d) {
-      ClearJob& c = cl[hdr->count[PH_CLEAR]++];
-      c.p = (float*)nzp;
-      c.n = (long)nang_sub * g.nr;
-      c.first = hdr->total[PH_CLEAR];
-      hdr->total[PH_CLEAR] += group_blocks(c.n);
-    }
-    // fused projection + ratio (Sinogram3D.cpp:830-856, 857+)
-    {
-      const int ph = j->is2d ? PH_PROJ2 : PH_PROJ3;
-      ProjJob& q = (j->is2d ? p2 : p3)[hdr->count[ph]++];
+      ProjJob& q = p2[hdr->count[PH_PROJ2]++];
       q.g = g;
       q.rays = p->d_rays;
-      q.zab = p->d_zab;
-      q.zorder = j->is2d ? nullptr : p->d_zorder;
       q.img = j->x;
       q.fr = FusedRatio();
       q.fr.meas = j->meas;
@@ -497,55 +455,28 @@ apirl_status apirl_batch_step(apirl_batch* b, int* active) {
       q.fr.additive_local = j->add_local;
       q.fr.ratio = j->ratio;
       q.fr.lik_partials = nullptr;
-      q.fr.lik_positive_only = j->is2d ? 1 : 0;
+      q.fr.lik_positive_only = 1;
       q.nang_sub = nang_sub;
       q.subset = s;
       q.nsubsets = S;
       q.pad = 0;
       q.nrays = nrays;
-      q.first = hdr->total[ph];
-      hdr->total[ph] += group_blocks(nrays);
+      q.first = hdr->total[PH_PROJ2];
+      hdr->total[PH_PROJ2] += group_blocks(nrays);
     }
-    if (!j->is2d) {
-      ZsJob& z = zs[hdr->count[PH_ZSETUP]++];
-      z.g = g;
-      z.rays = p->d_rays;
-      z.zab = p->d_zab;
-      z.sino = j->ratio;
-      z.out = zr;
-      z.nz_pair = nzp;
-      z.ztab = A.ztab;
-      z.zsoff = A.zsoff;
-      z.zblock = A.zblock;
-      z.pad = 0;
-      z.kind = BP_PLAIN;
-      z.nang_sub = nang_sub;
-      z.subset = s;
-      z.nsubsets = S;
-      z.nrays = nrays;
-      z.first = hdr->total[PH_ZSETUP];
-      hdr->total[PH_ZSETUP] += group_blocks(nrays);
-    }
+    // gather backprojection, each voxel's update applied to it
     {
-      const int ph = j->is2d ? PH_GATHER2 : PH_GATHER3;
-      GJob& q = (j->is2d ? g2 : g3)[hdr->count[ph]++];
-      q.A = A;
-      const int edge = j->is2d ? kPatch2 : 16;
-      q.ntx = (g.nx + edge - 1) / edge;
-      q.nty = (g.ny + edge - 1) / edge;
-      q.first = hdr->total[ph];
-      hdr->total[ph] += gather_tile_blocks(g);
-    }
-    {
-      UpdJob& u = up[hdr->count[PH_UPDATE]++];
-      u.x = j->x;
-      u.b = j->bp;
-      u.s = j->sens + (size_t)s * j->nvox;
-      u.n = (long)j->nvox;
-      u.thr = j->thr[s];
-      u.strict = j->strict;
-      u.first = hdr->total[PH_UPDATE];
-      hdr->total[PH_UPDATE] += group_blocks(u.n);
+      GJob& q = g2[hdr->count[PH_GATHER2]++];
+      ZRay* unused_zr = nullptr;
+      int* unused_nz = nullptr;
+      gather_args_for(p, s, S, BP_PLAIN, j->ratio, j->x, nullptr, q.A, unused_zr, unused_nz);
+      q.A.upd_sens = j->sens + (size_t)s * j->nvox;
+      q.A.upd_thr = j->thr[s];
+      q.A.upd_strict = j->strict;
+      q.ntx = (g.nx + kPatch2 - 1) / kPatch2;
+      q.nty = (g.ny + kPatch2 - 1) / kPatch2;
+      q.first = hdr->total[PH_GATHER2];
+      hdr->total[PH_GATHER2] += gather_patches(g);
     }
     // advance the job
     if (++j->s == S) {
@@ -571,8 +502,8 @@ apirl_status apirl_batch_step(apirl_batch* b, int* active) {
     if (e != hipSuccess)
       return bfail(b, APIRL_ERR_HIP, std::string("round launch failed: ") + hipGetErrorString(e));
   }
-  // large jobs: the sub-iteration apirl_em_reconstruct runs for them (fused projection
-  // and ratio, gather backprojection, update), on the batch stream
+  // 3D jobs: the sub-iteration apirl_em_reconstruct runs for them (fused projection and
+  // ratio, backprojection with the update fused in), on the batch stream
   for (auto& pr : direct) {
     BJob* j = pr.first;
     const int s = pr.second;
@@ -584,40 +515,33 @@ apirl_status apirl_batch_step(apirl_batch* b, int* active) {
     fr.ratio = j->ratio;
     fr.lik_partials = nullptr;
     fr.lik_positive_only = 0;
-    if ((e = launch_project(j->plan, j->x, nullptr, s, j->S, APIRL_PREC_REFERENCE, &fr, nullptr,
-                            b->stream)) != hipSuccess)
-      return bfail(b, APIRL_ERR_HIP, std::string("large-job launch failed: ") +
-                                         hipGetErrorString(e));
-    if (j->tile) {
-      // the tile backprojection with the update fused in, as apirl_em_reconstruct runs
-      // it with APIRL_BP_TILE (on the batch stream; the plan keeps its geometry)
-      apirl_ctx* c = b->ctx;
-      hipStream_t saved = c->stream;
-      c->stream = b->stream;
-      const apirl_status st = apirl_backproject_update(
-          j->plan, j->ratio, j->x, j->sens + (size_t)s * j->nvox, j->thr[s], j->strict, s, j->S,
-          APIRL_BP_TILE, APIRL_PREC_REFERENCE);
-      c->stream = saved;
-      if (st != APIRL_OK)
-        return bfail(b, st, std::string("large-job tile backprojection failed: ") + c->err);
-      continue;
+    const float* sens = j->sens + (size_t)s * j->nvox;
+    // more scratch than at submission only when the plan's tuning has changed since
+    size_t need = 0;
+    if (j->plan->geo.ns * j->plan->geo.nas == 1) need = job_scratch_bytes(j->plan, s, j->S, true);
+    else
+      for (apirl_plan* q : j->plan->os_parts)
+        need = std::max(need, job_scratch_bytes(q, s, j->S, true));
+    if (need > j->zscr_bytes) {
+      void* z = balloc(b, need);
+      if (!z) return bfail(b, APIRL_ERR_NOMEM, "cannot allocate the job's device state");
+      j->bufs.emplace_back(z, need);
+      j->zscr = z;
+      j->zscr_bytes = need;
     }
-    if (j->plan->geo.ns * j->plan->geo.nas == 1) {
-      // the update fused into the gather, as apirl_em_reconstruct runs it
-      const EmFuse fz{j->sens + (size_t)s * j->nvox, j->thr[s], j->strict};
-      if ((e = launch_backproject_gather(j->plan, j->ratio, j->x, s, j->S, BP_PLAIN,
-                                         APIRL_PREC_REFERENCE, j->zscr, j->zscr_bytes, b->stream,
-                                         &fz)) != hipSuccess)
-        return bfail(b, APIRL_ERR_HIP, std::string("large-job launch failed: ") +
-                                           hipGetErrorString(e));
-      continue;
+    e = launch_project(j->plan, j->x, nullptr, s, j->S, APIRL_PREC_REFERENCE, &fr, nullptr,
+                       b->stream, j->copy);
+    if (e == hipSuccess && !j->bp) {
+      const EmFuse fz{sens, j->thr[s], j->strict};
+      e = backproject_job(j, j->ratio, j->x, s, BP_PLAIN, &fz, b->stream);
+    } else if (e == hipSuccess) {
+      e = hipMemsetAsync(j->bp, 0, j->nvox * sizeof(float), b->stream);
+      if (e == hipSuccess) e = backproject_job(j, j->ratio, j->bp, s, BP_PLAIN, nullptr, b->stream);
+      if (e == hipSuccess)
+        e = launch_em_update(j->x, j->bp, sens, j->nvox, j->thr[s], j->strict, b->stream);
     }
-    if ((e = hipMemsetAsync(j->bp, 0, j->nvox * sizeof(float), b->stream)) != hipSuccess ||
-        (e = backproject_job(j, s, b->stream)) != hipSuccess ||
-        (e = launch_em_update(j->x, j->bp, j->sens + (size_t)s * j->nvox, j->nvox, j->thr[s],
-                              j->strict, b->stream)) != hipSuccess)
-      return bfail(b, APIRL_ERR_HIP, std::string("large-job launch failed: ") +
-                                         hipGetErrorString(e));
+    if (e != hipSuccess)
+      return bfail(b, APIRL_ERR_HIP, std::string("3D job launch failed: ") + hipGetErrorString(e));
   }
   for (BJob* j : finishing) {
     (void)hipEventRecord(j->done_ev, b->stream);

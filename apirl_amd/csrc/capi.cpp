@@ -2,6 +2,7 @@
 // and the device-resident MLEM / OSEM drivers.
 #include <cfloat>
 #include <cmath>
+#include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <algorithm>
@@ -178,19 +179,11 @@ bool ensure_f64s_tables(apirl_plan* p) {
   return ok;
 }
 
-// The tile backprojector's item order for the plan's current slab depth, built on
-// first use (and again when the slab depth changes the item count).
+// The tile backprojector's tile order, built on first use.
 bool ensure_tile_order(apirl_plan* p) {
-  const int n = apirl::tile_items(p);
-  if (p->d_tile_order && p->tile_order_n == n) return true;
+  if (p->d_tile_order) return true;
   std::vector<int> order;
   apirl::build_tile_order(p, order);
-  if (p->d_tile_order) {
-    if (hipStreamSynchronize(p->ctx->stream) != hipSuccess) return false;
-    (void)hipFree(p->d_tile_order);
-  }
-  p->d_tile_order = nullptr;
-  p->tile_order_n = 0;
   if (hipMalloc(&p->d_tile_order, order.size() * sizeof(int)) != hipSuccess ||
       hipMemcpy(p->d_tile_order, order.data(), order.size() * sizeof(int),
                 hipMemcpyHostToDevice) != hipSuccess) {
@@ -199,27 +192,31 @@ bool ensure_tile_order(apirl_plan* p) {
     p->d_tile_order = nullptr;
     return false;
   }
-  p->tile_order_n = n;
   return true;
 }
 
-// The kept tile geometry of (the plan's LOR form, subset, subsets): found, or allocated
-// within the plan's budget (not ready until a call has built it).  Null when it does
-// not fit the budget or the stream is being captured (a capture would only record the
-// launches that build it): the call then builds it in its scratch.
-apirl_plan::TileGeo* tile_geo_for(apirl_plan* p, int subset, int nsubsets) {
+// Work enqueued on the stream is being captured into a graph (or its state is unknown).
+bool capturing(hipStream_t st) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(p->ctx->stream, &cs) != hipSuccess ||
-      cs != hipStreamCaptureStatusNone) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
+  if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+// The kept tile geometry of (the plan's LOR form, subset, subsets) for work on stream st:
+// found, or allocated within the plan's budget (not ready until a call has built it).  Null
+// when it does not fit the budget; the call then builds it in its scratch.  During a capture
+// (which would only record the launch that builds it, and cannot wait for another stream's)
+// only geometry that is ready on the same stream is taken.
+apirl_plan::TileGeo* tile_geo_for(apirl_plan* p, int subset, int nsubsets, hipStream_t st) {
+  const bool cap = capturing(st);
   for (apirl_plan::TileGeo& e : p->tile_geo)
-    if (e.form == p->scanner && e.subset == subset && e.nsubsets == nsubsets) return &e;
+    if (e.form == p->scanner && e.subset == subset && e.nsubsets == nsubsets)
+      return !cap || (e.ready && e.stream == st) ? &e : nullptr;
+  if (cap) return nullptr;
   const size_t bytes = apirl::tile_geo_bytes(p, subset, nsubsets);
   if (bytes == 0 || p->tile_geo_used + bytes > p->tile_geo_budget) return nullptr;
-  apirl_plan::TileGeo e{p->scanner, subset, nsubsets, nullptr, bytes, false, nullptr, nullptr,
-                        nullptr, 0, 0};
+  apirl_plan::TileGeo e{p->scanner, subset, nsubsets, nullptr, bytes, false, nullptr, nullptr};
   if (hipMalloc(&e.d, bytes) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
@@ -238,11 +235,40 @@ void free_tile_geo(apirl_plan* p) {
   for (apirl_plan::TileGeo& e : p->tile_geo) {
     (void)hipEventSynchronize(e.ev);
     (void)hipFree(e.d);
-    if (e.list) (void)hipFree(e.list);
     (void)hipEventDestroy(e.ev);
   }
   p->tile_geo.clear();
   p->tile_geo_used = 0;
+}
+
+// The tile backprojection of one subset on stream st with the geometry tg (null: built in the
+// scratch); the item order is built.
+hipError_t tile_run(apirl_plan* p, const float* sino, float* img, int subset, int nsubsets,
+                    int kind, const apirl::EmFuse* fuse, apirl_plan::TileGeo* tg, void* scratch,
+                    size_t scratch_bytes, hipStream_t st) {
+  hipError_t e;
+  if (tg && tg->ready && tg->stream != st &&
+      (e = hipStreamWaitEvent(st, tg->ev, 0)) != hipSuccess)
+    return e;
+  if ((e = apirl::launch_backproject_tile(p, sino, img, subset, nsubsets, kind, scratch,
+                                          scratch_bytes, st, fuse, tg ? tg->d : nullptr,
+                                          tg && tg->ready)) != hipSuccess)
+    return e;
+  if (tg && !tg->ready) {
+    tg->ready = true;
+    tg->stream = st;
+    return hipEventRecord(tg->ev, st);
+  }
+  return hipSuccess;
+}
+
+// A plan's backprojections in the reference arithmetic, whichever form is asked for, are run
+// by the tile backprojector where it takes the plan: it adds the same float terms, in double,
+// in a fixed order.  12-angle subset of the 256x256x81 / 344x252x837 workload, every bin
+// non-zero: 1.8 ms, the gather's column kernel 4.2 ms, the scatter's atomics 22 ms; 12 angles
+// of 122x84x73 on 64x64x17: 0.05, 0.40 and 0.20 ms.
+bool tile_takes(const apirl_plan* p, int subset, int nsubsets) {
+  return p->gather_ok && !apirl::gather_misfit(p, subset, nsubsets) && !apirl::tile_misfit(p);
 }
 
 // Backprojection of one subset in either form.
@@ -250,6 +276,42 @@ void free_tile_geo(apirl_plan* p) {
 // 24-bit index walk).
 bool os_precision_ok(const apirl_plan* p, int precision) {
   return p->geo.ns * p->geo.nas == 1 || (precision == APIRL_PREC_REFERENCE && p->geo.walk24);
+}
+
+// The plan's backprojection scratch holds at least `need` bytes.
+bool ensure_gscratch(apirl_plan* p, size_t need) {
+  if (need <= p->gscratch_bytes) return true;
+  if (p->d_gscratch) {
+    if (hipStreamSynchronize(p->ctx->stream) != hipSuccess) return false;
+    (void)hipFree(p->d_gscratch);
+  }
+  p->d_gscratch = nullptr;
+  p->gscratch_bytes = 0;
+  if (hipMalloc(&p->d_gscratch, need) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  p->gscratch_bytes = need;
+  return true;
+}
+
+// The tile backprojection with the plan's scratch.  done stays false when it cannot be had
+// (no memory, or a capture that would have to allocate): the caller's own form then runs.
+apirl_status tile_backproject(apirl_plan* p, const float* sino, float* img, int subset,
+                              int nsubsets, int kind, const apirl::EmFuse* fuse, bool& done) {
+  apirl_ctx* c = p->ctx;
+  apirl_plan::TileGeo* tg = tile_geo_for(p, subset, nsubsets, c->stream);
+  const size_t need = apirl::tile_scratch_bytes(p, subset, nsubsets, tg == nullptr);
+  if ((need > p->gscratch_bytes || !p->d_tile_order) && capturing(c->stream))
+    return fail(c, APIRL_ERR_NOMEM, "the gather scratch cannot be allocated during a capture");
+  if (!ensure_gscratch(p, need))
+    return fail(c, APIRL_ERR_NOMEM, "cannot allocate the gather scratch");
+  if (!ensure_tile_order(p))
+    return fail(c, APIRL_ERR_NOMEM, "cannot allocate the tile backprojector's item order");
+  done = true;
+  APIRL_HIP(c, tile_run(p, sino, img, subset, nsubsets, kind, fuse, tg, p->d_gscratch,
+                        p->gscratch_bytes, c->stream));
+  return APIRL_OK;
 }
 
 // fuse (gather form, one LOR per bin): img is the EM image, updated by each voxel's
@@ -265,6 +327,12 @@ apirl_status backproject_any(apirl_plan* p, const float* sino, const float* est,
     if (precision != APIRL_PREC_REFERENCE)
       return fail(c, APIRL_ERR_UNSUPPORTED,
                   "the scatter backprojector has the reference precision only");
+    if (kind != apirl::BP_DIVIDE && tile_takes(p, subset, nsubsets)) {
+      // DivideAndBackproject keeps its own bounds rule (BP_DIVIDE in the scatter kernel)
+      bool done = false;
+      const apirl_status st = tile_backproject(p, sino, img, subset, nsubsets, kind, nullptr, done);
+      if (done) return st;
+    }
     if (!p->d_replicas && !p->replicas_failed) {
       // the per-XCD scatter targets (16 image copies), zeroed here and re-zeroed by
       // the reduction after every use; without them the atomics go to the image
@@ -314,21 +382,6 @@ apirl_status backproject_any(apirl_plan* p, const float* sino, const float* est,
   if (const char* why = apirl::gather_misfit(p, subset, nsubsets))
     return fail(c, APIRL_ERR_UNSUPPORTED,
                 std::string("gather: ") + why + " (use the scatter form)");
-  apirl_plan::TileGeo* tg = mode == APIRL_BP_TILE ? tile_geo_for(p, subset, nsubsets) : nullptr;
-  const size_t need = mode == APIRL_BP_TILE
-                          ? apirl::tile_scratch_bytes(p, subset, nsubsets, tg == nullptr)
-                          : apirl::gather_scratch_bytes(p, subset, nsubsets);
-  if (need > p->gscratch_bytes) {
-    if (p->d_gscratch) {
-      APIRL_HIP(c, hipStreamSynchronize(c->stream));
-      (void)hipFree(p->d_gscratch);
-    }
-    p->d_gscratch = nullptr;
-    p->gscratch_bytes = 0;
-    if (hipMalloc(&p->d_gscratch, need) != hipSuccess)
-      return fail(c, APIRL_ERR_NOMEM, "cannot allocate the gather scratch");
-    p->gscratch_bytes = need;
-  }
   if (kind == apirl::BP_DIVIDE) {
     // DivideAndBackproject gathered: each bin's value by the reference's rule, then a
     // plain backprojection of it (the bins the rule zeroes add nothing, as the bins
@@ -349,48 +402,17 @@ apirl_status backproject_any(apirl_plan* p, const float* sino, const float* est,
     sino = p->d_divbins;
     kind = apirl::BP_PLAIN;
   }
+  if (precision == APIRL_PREC_REFERENCE && tile_takes(p, subset, nsubsets)) {
+    bool done = false;
+    const apirl_status st = tile_backproject(p, sino, img, subset, nsubsets, kind, fuse, done);
+    if (done || mode == APIRL_BP_TILE) return st;
+  }
+  if (!ensure_gscratch(p, apirl::gather_scratch_bytes(p, subset, nsubsets)))
+    return fail(c, APIRL_ERR_NOMEM, "cannot allocate the gather scratch");
   if (!ensure_tile_map(p))
     return fail(c, APIRL_ERR_NOMEM, "cannot allocate the gather's tile map");
   if (precision == APIRL_PREC_F64_SETUP && p->geo.dims == 3 && p->gather_zlanes <= 1)
     (void)ensure_f64s_tables(p);  // without them the one-voxel F64_SETUP kernel runs
-  if (mode == APIRL_BP_TILE) {
-    if (!ensure_tile_order(p))
-      return fail(c, APIRL_ERR_NOMEM, "cannot allocate the tile backprojector's item order");
-    if (tg && tg->ready && tg->stream != c->stream)
-      APIRL_HIP(c, hipStreamWaitEvent(c->stream, tg->ev, 0));
-    APIRL_HIP(c, apirl::launch_backproject_tile(p, sino, img, subset, nsubsets, kind,
-                                                p->d_gscratch, p->gscratch_bytes, c->stream,
-                                                fuse, tg ? tg->d : nullptr, tg && tg->ready,
-                                                tg && tg->lists == 1 ? tg->list : nullptr));
-    if (tg && !tg->ready) {
-      tg->ready = true;
-      tg->stream = c->stream;
-      // the sinogram lists of its (item, ray) pairs: counted, then kept if they fit
-      long long* dtot = nullptr;
-      long long total = 0;
-      APIRL_HIP(c, apirl::launch_tile_lists(p, subset, nsubsets, tg->d, nullptr, &dtot,
-                                            c->stream));
-      APIRL_HIP(c, hipMemcpyAsync(&total, dtot, sizeof(total), hipMemcpyDeviceToHost,
-                                  c->stream));
-      APIRL_HIP(c, hipStreamSynchronize(c->stream));
-      const size_t lb = (size_t)(total > 0 ? total : 0) * sizeof(unsigned short);
-      tg->lists = -1;
-      if (lb > 0 && p->tile_geo_used + lb <= p->tile_geo_budget) {
-        if (hipMalloc(&tg->list, lb) == hipSuccess) {
-          p->tile_geo_used += lb;
-          tg->list_bytes = lb;
-          tg->lists = 1;
-          APIRL_HIP(c, apirl::launch_tile_lists(p, subset, nsubsets, tg->d, tg->list, nullptr,
-                                                c->stream));
-        } else {
-          (void)hipGetLastError();
-          tg->list = nullptr;
-        }
-      }
-      APIRL_HIP(c, hipEventRecord(tg->ev, c->stream));
-    }
-    return APIRL_OK;
-  }
   APIRL_HIP(c, apirl::launch_backproject_gather(p, sino, img, subset, nsubsets, kind, precision,
                                                 p->d_gscratch, p->gscratch_bytes, c->stream,
                                                 fuse));
@@ -428,7 +450,7 @@ apirl_status apirl_ctx_create(int device, apirl_ctx** out) {
   apirl_ctx* c = new apirl_ctx();
   c->device = device;
   DeviceGuard g(device);
-  if (hipMalloc(&c->d_fred, 64 * sizeof(float)) != hipSuccess ||
+  if (hipMalloc(&c->d_fred, (2 + 2 * apirl::kMinMaxBlocks) * sizeof(float)) != hipSuccess ||
       hipMalloc(&c->d_ured, 8 * sizeof(unsigned long long)) != hipSuccess) {
     delete c;
     return APIRL_ERR_NOMEM;
@@ -576,6 +598,26 @@ apirl_status plan_create_impl(apirl_ctx* ctx, const apirl_image_desc* image,
       return fail(ctx, APIRL_ERR_NOMEM, "cannot upload the ring table");
     }
   }
+  // The tile backprojector's z-crossing increments and the range of the rays' slices
+  // (their alphas lie in [0, 1]).
+  if (sd.dims == 3) {
+    std::vector<float> zinc(sd.nsino);
+    double zlo = 0, zhi = 0;
+    for (int q = 0; q < sd.nsino; q++) {
+      const float vz = p->zab[q].y - p->zab[q].x;
+      zinc[q] = vz < 0 ? -fabsf(im.dz / vz) : fabsf(im.dz / vz);
+      zlo = std::min(zlo, (double)std::min(p->zab[q].x, p->zab[q].y));
+      zhi = std::max(zhi, (double)std::max(p->zab[q].x, p->zab[q].y));
+    }
+    p->slices16 = (zhi - zlo) / im.dz < 32000.0;
+    if (hipMalloc(&p->d_zinc, zinc.size() * sizeof(float)) != hipSuccess ||
+        hipMemcpy(p->d_zinc, zinc.data(), zinc.size() * sizeof(float), hipMemcpyHostToDevice) !=
+            hipSuccess) {
+      if (p->d_zinc) (void)hipFree(p->d_zinc);
+      p->d_zinc = nullptr;
+      (void)hipGetLastError();
+    }
+  }
   // Forward-projection order: sinograms by mean axial coordinate (stable).
   if (sd.dims == 3) {
     std::vector<int> order(sd.nsino);
@@ -680,6 +722,28 @@ apirl_status apirl_plan_create(apirl_ctx* ctx, const apirl_image_desc* image,
 extern "C++" {
 namespace apirl {
 
+size_t job_scratch_bytes(apirl_plan* p, int subset, int nsubsets, bool prepare) {
+  if (!tile_takes(p, subset, nsubsets)) return gather_scratch_bytes(p, subset, nsubsets);
+  if (!prepare) return tile_scratch_bytes(p, subset, nsubsets, false);
+  if (!ensure_tile_order(p)) return SIZE_MAX;  // not to be had
+  return tile_scratch_bytes(p, subset, nsubsets,
+                            tile_geo_for(p, subset, nsubsets, p->ctx->stream) == nullptr);
+}
+
+hipError_t job_backproject(apirl_plan* p, const float* sino, float* img, int subset, int nsubsets,
+                           int kind, const EmFuse* fuse, void* scratch, size_t scratch_bytes,
+                           hipStream_t st) {
+  if (tile_takes(p, subset, nsubsets)) {
+    if (!p->d_tile_order) return hipErrorInvalidValue;  // job_scratch_bytes builds it
+    apirl_plan::TileGeo* tg = tile_geo_for(p, subset, nsubsets, st);
+    if (scratch_bytes >= tile_scratch_bytes(p, subset, nsubsets, tg == nullptr))
+      return tile_run(p, sino, img, subset, nsubsets, kind, fuse, tg, scratch, scratch_bytes, st);
+    return hipErrorInvalidValue;
+  }
+  return launch_backproject_gather(p, sino, img, subset, nsubsets, kind, APIRL_PREC_REFERENCE,
+                                   scratch, scratch_bytes, st, fuse);
+}
+
 void free_os_parts(apirl_plan* p) {
   for (apirl_plan* h : p->os_parts) apirl_plan_destroy(h);
   p->os_parts.clear();
@@ -755,6 +819,7 @@ apirl_status apirl_plan_destroy(apirl_plan* p) {
   for (int* m : p->d_tilemap)
     if (m) (void)hipFree(m);
   if (p->d_tile_order) (void)hipFree(p->d_tile_order);
+  if (p->d_zinc) (void)hipFree(p->d_zinc);
   free_tile_geo(p);
   if (p->d_zsoff) (void)hipFree(p->d_zsoff);
   delete p;
@@ -880,11 +945,9 @@ apirl_status apirl_plan_set_tuning(apirl_plan* p, const apirl_tuning* t) {
       return fail(p->ctx, APIRL_ERR_INVALID, "unknown gather_xcd");
     p->gather_xcd = t->gather_xcd;
   }
-  bool zs_changed = false;
   if (t->tile_zs) {
     if (t->tile_zs < 1 || t->tile_zs > 256)
       return fail(p->ctx, APIRL_ERR_INVALID, "tile_zs must be in 1..256");
-    zs_changed = t->tile_zs != p->tile_zs;
     p->tile_zs = t->tile_zs;
   }
   DeviceGuard g(p->ctx->device);
@@ -894,7 +957,6 @@ apirl_status apirl_plan_set_tuning(apirl_plan* p, const apirl_tuning* t) {
     p->tile_geo_budget = t->tile_cache_mb < 0 ? 0 : (size_t)t->tile_cache_mb << 20;
     if (p->tile_geo_used > p->tile_geo_budget) free_tile_geo(p);
   }
-  if (zs_changed) free_tile_geo(p);  // the kept lists are per slab
   if (!ensure_tile_map(p))
     return fail(p->ctx, APIRL_ERR_NOMEM, "cannot allocate the gather's tile map");
   for (apirl_plan* h : p->os_parts) {  // the oversampled plan's gathers follow it
@@ -902,7 +964,6 @@ apirl_status apirl_plan_set_tuning(apirl_plan* p, const apirl_tuning* t) {
     h->gather_zvox = p->gather_zvox;
     h->gather_xcd = p->gather_xcd;
     h->tile_zs = p->tile_zs;
-    if (zs_changed) free_tile_geo(h);
     const size_t share = p->tile_geo_budget / p->os_parts.size();
     if (h->tile_geo_budget != share) {
       h->tile_geo_budget = share;

@@ -845,7 +845,8 @@ constexpr int kG2Rays = 20;    // rays staged at a time, by each wavefront
 // a staged ray: words 4 .. 15 of its RayXY (the bin value in place of lxy) and its crossings
 // into the patch's columns and rows
 constexpr int kG2RayWords = 12 + 2 * kPatch;
-constexpr int kG2LdsFloats = 16 * 1024;  // 64 KiB: the staged rays and two rounds of terms
+constexpr int kG2LdsFloats = 16 * 1024 - 64;  // 64 KiB less the batch's block number: the
+                                              // staged rays and two rounds of terms
 // Wavefronts that compute terms for plans with up to maxc candidates per (voxel, angle);
 // 0: the terms of one angle do not fit (over 120 bins per voxel).
 __host__ __device__ inline int gather2_waves(int maxc) {
@@ -969,71 +970,8 @@ __global__ __launch_bounds__(kG2Waves * kWave, 8) void gather2_kernel(GatherArgs
   gather2_patch(A, nw, blockIdx.x, blockIdx.y, g2lds);
 }
 
-// ---- grouped (multi-job) launches --------------------------------------------
+// ---- grouped (multi-job) launch -----------------------------------------------
 #include "group_common.h"
-
-__global__ __launch_bounds__(kGBlock) void zsetup_group_kernel(BatchHeader* __restrict__ hdr,
-                                                               const ZsJob* __restrict__ jobs) {
-  const int n = hdr->count[PH_ZSETUP];
-  const long total = hdr->total[PH_ZSETUP];
-  const int grab = grab_size(hdr);
-  for (;;) {
-    const long v0 = grab_vb(&hdr->next[PH_ZSETUP], grab);
-    if (v0 >= total) break;
-    for (long vb = v0; vb < v0 + grab && vb < total; vb++) {
-      const ZsJob& J = jobs[find_job(jobs, n, vb)];
-      const long idx = (vb - J.first) * kGBlock + threadIdx.x;
-      if (idx < J.nrays)
-        zsetup_one(J.g, J.rays, J.zab, J.sino, J.kind, J.nang_sub, J.subset, J.nsubsets, J.out,
-                   J.nz_pair, J.ztab, J.zsoff, J.zblock, idx);
-    }
-  }
-}
-
-// Each virtual block is one 16 x 16 tile of kGroupZV slices of one job (the column
-// kernel's shape, tile-major); the axial and crossing-slot tables are reloaded into LDS
-// when the workgroup moves to another job.
-__global__ __launch_bounds__(kGBlock) void gather3_group_kernel(BatchHeader* __restrict__ hdr,
-                                                               const GJob* __restrict__ jobs) {
-  extern __shared__ float2 s_zab[];
-  const int ph = PH_GATHER3;
-  const int n = hdr->count[ph];
-  const long total = hdr->total[ph];
-  const int grab = grab_size(hdr);
-  int loaded = -1;
-  for (;;) {
-    const long v0 = grab_vb(&hdr->next[ph], grab);
-    if (v0 >= total) break;
-    for (long vb = v0; vb < v0 + grab && vb < total; vb++) {
-      const int jj = find_job(jobs, n, vb);
-      const GJob& J = jobs[jj];
-      const int ns = J.A.g.nsino;
-      int4* s_slot = (int4*)((char*)s_zab + column_lds_off(ns));
-      if (loaded != jj) {
-        __syncthreads();
-        for (int q = threadIdx.x; q < ns; q += kGBlock) {
-          s_zab[q] = J.A.zab[q];
-          if (J.A.zsoff) {
-            const int so = J.A.zsoff[q], so1 = J.A.zsoff[q + 1], km = J.A.zsoff[ns + 1 + q];
-            s_slot[q] = make_int4(so - km, so, so1 - 1 < so ? so : so1 - 1, 0);
-          }
-        }
-        __syncthreads();
-        loaded = jj;
-      }
-      const long lb = vb - J.first;
-      const int bx = (int)(lb % J.ntx);
-      const int by = (int)((lb / J.ntx) % J.nty);
-      const int kg = (int)(lb / ((long)J.ntx * J.nty));
-      const int i = bx * kTile + (threadIdx.x % kTile);
-      const int j = by * kTile + (threadIdx.x / kTile);
-      if (i < J.A.g.nx && j < J.A.g.ny) {
-        gather_column<APIRL_PREC_REFERENCE, kGroupZV>(J.A, s_zab, s_slot, J.A.segs, i, j,
-                                                      kg * kGroupZV);
-      }
-    }
-  }
-}
 
 // Each virtual block is one 8 x 8 patch of one 2D job, by the whole workgroup.
 __global__ __launch_bounds__(kG2Waves * kWave) void gather2_group_kernel(
@@ -1042,9 +980,7 @@ __global__ __launch_bounds__(kG2Waves * kWave) void gather2_group_kernel(
   const int n = hdr->count[PH_GATHER2];
   const long total = hdr->total[PH_GATHER2];
   const int grab = grab_size(hdr);
-  for (;;) {
-    const long v0 = grab_vb(&hdr->next[PH_GATHER2], grab);
-    if (v0 >= total) break;
+  for (long v0 = first_vb(grab); v0 < total; v0 = next_vb(&hdr->next[PH_GATHER2], grab, total))
     for (long vb = v0; vb < v0 + grab && vb < total; vb++) {
       const GJob& J = jobs[find_job(jobs, n, vb)];
       const int lb = (int)(vb - J.first), px = lb % J.ntx, py = lb / J.ntx;
@@ -1057,7 +993,6 @@ __global__ __launch_bounds__(kG2Waves * kWave) void gather2_group_kernel(
           gather_voxel<2, APIRL_PREC_REFERENCE>(J.A, nullptr, i, j, 0);
       }
     }
-  }
 }
 
 inline unsigned ggrid(long n) { return (unsigned)((n + kGBlock - 1) / kGBlock); }
@@ -1079,7 +1014,8 @@ void launch_gather_column(const GatherArgs& A, hipStream_t st) {
 template <int PREC>
 void launch_gather3(const GatherArgs& A, int zlanes, int zvox, hipStream_t st) {
   const Geo& g = A.g;
-  const size_t lds = gather_lds_bytes(g.nsino);
+  const size_t lds =
+      (size_t)g.nsino * sizeof(float2) + (size_t)(2 * g.nsino + 1) * sizeof(int);
   if (PREC != APIRL_PREC_F64_ALPHA && PREC != APIRL_PREC_F64_SETUP && zlanes <= 1 &&
       zvox >= 1) {
     constexpr int P =
@@ -1123,21 +1059,22 @@ void launch_gather2(const GatherArgs& A, hipStream_t st) {
 //
 // A wavefront owns an item: kTW x kTW voxel columns (a tile) times a slab of slices,
 // summed in its own LDS.  For every ray (angle, radial bin) of the subset that crosses
-// the tile, the wavefront finds once where the rays of all sinograms enter the tile
-// (they share the transaxial path) and its lanes take the sinograms whose rays can
-// reach the slab there, one ray per lane.  Each lane resumes the reference's Siddon
-// loop (Siddon.cpp:310-340) at the tile's entry: the x / y crossings are the loop's
-// accumulated float values from the plan's table, its z crossings come from the
-// first one by the loop's own additions.  It walks to the tile's exit, adding
-// (alpha - alpha_c) L b (SiddonProjector.cpp:546) to the voxels it visits inside the
-// slab, while its step count stays below the list length |di| + |dj| + |dk|
-// (:220, the dropped exit voxel), and only there: the voxels, weights and terms are
-// the reference's floats, bit for bit.  Each voxel's terms are summed in double in
+// the tile (its entry and path there are found once per subset: the rays of all sinograms
+// share them) its lanes take the sinograms whose rays can reach the slab there, one ray
+// per lane.  Each lane resumes the reference's Siddon loop (Siddon.cpp:310-340) at the
+// tile's entry: the x / y crossings are the loop's accumulated float values from the plan's
+// table, its z crossings come from the first one by the loop's own additions.  It walks to
+// the tile's exit, adding (alpha - alpha_c) L b (SiddonProjector.cpp:546) to the voxels it
+// visits inside the slab, while its step count stays below the list length
+// |di| + |dj| + |dk| (:220, the dropped exit voxel), and only there: the voxels, weights and
+// terms are the reference's floats, bit for bit.  Each voxel's terms are summed in double in
 // the wavefront's order, which depends on the data only (one wavefront per item), so
 // repeated runs are bit-identical, and rounded to float once.
+//
+// An image of few tiles is split further: each (tile, slab) into chunks of the tile's rays,
+// whose sums go to memory in double and are added in chunk order.
 
 constexpr int kTW = 8;      // item tile width in columns (kTW * kTW = one lane per column)
-constexpr int kTWaves = 4;  // items (wavefronts) per workgroup
 
 struct TileEntry {
   int i, j;      // column and row of the ray's first voxel in the tile
@@ -1147,27 +1084,39 @@ struct TileEntry {
   float aout;    // alpha near the tile's exit (sinogram candidates only)
 };
 
-// A candidate ray of a tile, found once per subset by tile_rays_kernel for every
-// slab of the tile: its entry and the length of its transaxial path there.
+// A ray that enters a tile: the loop's state there and the transaxial part of its walk
+// through the tile, the same for every sinogram: the columns it visits in order, for each
+// the alpha at which the loop leaves it by an x or y crossing (the smaller accumulated
+// crossing there; x before y on ties, Siddon.cpp:318-331) and the bytes from the column's
+// sums to the next one's.  At most 2 kTW - 1 columns; the last one's step leaves the slab for
+// good, and two entries follow that lead nowhere, so a walk may go on a step past its end.
+constexpr int kTPath = 2 * kTW + 2;
+constexpr int kTileAway = 1 << 29;
+struct TileStep {
+  float ae;
+  int step;
+};
 struct alignas(16) TileRay {
-  TileEntry E;
-  int pair;      // ka * nr + r, or -1: no ray (or one that misses the tile)
-  int ncol;      // columns on its path through the tile
-  int nxy;       // the ray's transaxial list length |di| + |dj|
-  int pad[2];
+  float ce, aout;  // alpha at the entry (alpha_c) and where the walk leaves the tile
+  int pair;        // ka * nr + r
+  int mxy;         // x and y crossings the loop has taken at the entry
+  int nxy;         // the ray's transaxial list length |di| + |dj|
+  int ncol;        // columns on its path through the tile
+  int col0;        // byte offset of the first column's sums
+  int pad;
+  TileStep path[kTPath];
 };
-static_assert(sizeof(TileRay) == 48, "TileRay is three 16-byte loads");
+static_assert(sizeof(TileRay) == 32 + 8 * kTPath, "TileRay is whole 16-byte words");
 
-// The transaxial part of a candidate ray's walk through its tile, the same for every
-// sinogram: the columns it visits in order and, for each, the alpha at which the
-// loop leaves it by an x or y crossing (the smaller accumulated crossing there; x
-// before y on ties, Siddon.cpp:318-331).  At most 2 kTW - 1 columns.
-constexpr int kTPath = 2 * kTW;
-struct alignas(16) TilePath {
-  float ae[kTPath];
-  unsigned char col[kTPath];  // (j - tj0) kTW + (i - ti0)
+// Axial record of one ray with its bin value, (angle, r, sinogram) order: with the
+// sinogram's crossing increment (apirl_plan::d_zinc) what a lane needs beside the TileRay.
+struct alignas(16) TileZ {
+  float az0;  // first z crossing
+  float L;    // ray length
+  float b;    // bin value
+  int k01;    // entry and exit slice, 16 bits each
 };
-static_assert(sizeof(TilePath) == 80, "TilePath is five 16-byte loads");
+static_assert(sizeof(TileZ) == 16, "TileZ is one 16-byte load");
 
 // Crossings p after which index i0 + inc p enters [lo, hi] (pin) and first lies
 // beyond it (pout); false when it never lies in it.
@@ -1284,104 +1233,126 @@ __device__ __forceinline__ void tile_bins(const GatherArgs& A, int a, float xc, 
   lut_bins(A, so, hwo, lo1, hi1);
 }
 
-// One lane: the ray of record z from the tile's entry E to its exit, its terms added
-// to the item's sums acc[column * zs + slice - kz0] for slices kz0..kz1.  One loop
-// iteration is one step of the reference's loop, its branch taken by selects.
-__device__ __forceinline__ void tile_lane(const TileRay& R, const float* pae,
-                                          const unsigned char* pcol, const ZRay& z, int kz0,
-                                          int kz1, int zs, double* acc) {
-  const TileEntry& E = R.E;
-  const int nxy = R.nxy, ncol = R.ncol;
-  const int kinc = z.kinc;
-  const float azu = z.azu, L = z.L, b = z.b;
-  const int N = nxy + abs((int)z.k1 - z.k0);
-  int m = E.mxy, k = z.k0;
+// Byte distance of neighbouring slices' sums in an item: one word pair more than the tile's
+// columns, so that lanes on one column and neighbouring slices take different LDS banks.
+constexpr int kTPitch = (kTW * kTW + 1) * 8;
+
+typedef __attribute__((address_space(3))) double LdsDouble;
+typedef __attribute__((address_space(3))) const TileStep LdsTileStep;
+typedef __attribute__((address_space(3))) const char LdsByte;
+
+// One step of the reference's loop in an item: the term goes to the sum of the lane's voxel
+// (at LDS address v; only where that lies in the slab, below lim), then the lane moves on
+// along its path (at LDS address ep).  14 VALU instructions with the end test of every
+// second step.
+__device__ __forceinline__ void tile_step(unsigned& ep, float& Zn, float& ac, unsigned& v,
+                                          float azu, float L, float b, int kstep, unsigned lim) {
+  LdsTileStep* p = (LdsTileStep*)(uintptr_t)ep;
+  const float ae = p->ae;
+  const int step = p->step;
+  const bool zst = Zn < ae;  // Siddon.cpp:318-339: x, then y, then z on ties
+  const float an = zst ? Zn : ae;
+  const float term = (an - ac) * L * b;  // the reference's float term (geomFactor 1)
+  if (v < lim)
+    __hip_atomic_fetch_add((LdsDouble*)(uintptr_t)v, (double)term, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_WAVEFRONT);
+  ac = an;
+  Zn = Zn + (zst ? azu : 0.f);
+  v += (unsigned)(zst ? kstep : step);
+  ep += zst ? 0u : (unsigned)sizeof(TileStep);
+}
+
+// One lane: the ray (R, z, zinc) from the tile's entry to its exit, its terms added to the
+// item's sums (slice kz0 + q of column c at LDS address q kTPitch + 8 c, below lim: the sums
+// are the first thing in the workgroup's LDS).
+__device__ __forceinline__ void tile_lane(const TileRay& R, const TileZ& z, float zinc, int kz0,
+                                          unsigned lim) {
+  const float azu = fabsf(zinc), ce = R.ce;
+  const int kinc = zinc > 0.f ? 1 : -1;  // no z step where Vz is 0: az0 is FLT_MAX
+  int k = (short)(z.k01 & 0xffff);
+  int left = R.nxy + abs((z.k01 >> 16) - k) - R.mxy;
   float Zn = z.az0;
   // z crossings taken before the entry: those below its alpha (a z crossing at the
   // alpha of an x or y crossing is taken after it, Siddon.cpp:318-339), by the
   // loop's own additions, four at a time
-  if (m > 0 && kinc != 0) {
-    while (m < N) {
+  if (R.mxy > 0) {
+    while (left > 0 && Zn < ce) {
       const float z1 = Zn + azu, z2 = z1 + azu, z3 = z2 + azu;
-      if (z3 < E.ce) {
-        Zn = z3 + azu;
-        k += 4 * kinc;
-        m += 4;
-        continue;
-      }
-      const int c = (Zn < E.ce ? 1 : 0) + (z1 < E.ce ? 1 : 0) + (z2 < E.ce ? 1 : 0);
-      Zn = c == 0 ? Zn : (c == 1 ? z1 : (c == 2 ? z2 : z3));
+      const int c = 1 + (z1 < ce ? 1 : 0) + (z2 < ce ? 1 : 0) + (z3 < ce ? 1 : 0);
+      Zn = c == 1 ? z1 : (c == 2 ? z2 : (c == 3 ? z3 : z3 + azu));
       k += c * kinc;
-      m += c;
-      break;
+      left -= c;
+      if (c < 4) break;
     }
   }
-  // slice relative to the slab and its end in the direction of travel (a lane that
-  // reaches it adds nothing more); the column comes from the path, whose x / y steps
-  // are the same for every lane
-  const int nzs = kz1 - kz0 + 1;
-  int kl = k - kz0;
-  const int kend = kinc > 0 ? nzs : -1;
-  if (kinc == 0 ? (unsigned)kl >= (unsigned)nzs : (kinc > 0 ? kl >= nzs : kl < 0)) return;
-  int q = 0;
-  float ae = pae[0];
-  int cidx = pcol[0] * zs;
-  float ac = E.ce;
-  for (int left = N - m; left > 0; left--) {
-    // the next column's entry, read before this step's add so that the wait for it
-    // does not include the add (entry q + 1 < kTPath always exists)
-    const float ae1 = pae[q + 1];
-    const int c1 = pcol[q + 1];
-    const bool zst = Zn < ae;  // Siddon.cpp:318-339: x, then y, then z on ties
-    const float an = zst ? Zn : ae;
-    if ((unsigned)kl < (unsigned)nzs) {
-      const float term = (an - ac) * L * b;  // the reference's float term (geomFactor 1)
-      __hip_atomic_fetch_add(acc + cidx + kl, (double)term, __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_WAVEFRONT);
+  unsigned v = (unsigned)((k - kz0) * kTPitch + R.col0);
+  const int kstep = kinc * kTPitch;
+  unsigned ep = (unsigned)(size_t)(LdsByte*)(const char*)R.path;
+  const unsigned eend = ep + R.ncol * (unsigned)sizeof(TileStep);
+  float ac = ce;
+  // far from the list's end the walk cannot reach it in the next kTFar steps
+  constexpr int kTFar = 2 * kTPath;
+  if (left >= kTFar) {
+    left -= kTFar;
+    for (int m = 0; m < kTFar; m += 2) {
+      tile_step(ep, Zn, ac, v, azu, z.L, z.b, kstep, lim);
+      tile_step(ep, Zn, ac, v, azu, z.L, z.b, kstep, lim);
+      if (ep >= eend) return;
     }
-    ac = an;
-    Zn = zst ? Zn + azu : Zn;
-    kl += zst ? kinc : 0;
-    q += zst ? 0 : 1;
-    if ((q == ncol) | (kl == kend)) break;
-    ae = zst ? ae : ae1;
-    cidx = zst ? cidx : c1 * zs;
   }
+  for (; left > 0 && ep < eend; left--)
+    tile_step(ep, Zn, ac, v, azu, z.L, z.b, kstep, lim);
 }
 
-// One in-flight ray of a wavefront, in LDS: its entry and path (the lanes walking
-// its sinograms read both).
-struct alignas(16) TileSlot {
-  TileRay R;
-  TilePath P;
-};
-static_assert(sizeof(TileSlot) == 128, "TileSlot is 32 words");
-constexpr int kTSlots = 8;    // rays in flight per wavefront
-constexpr int kTRing = 128;   // pending (ray, sinogram) entries per wavefront
+constexpr int kTSlots = 4;    // rays in flight per wavefront
+constexpr int kTQueue = 128;  // pending (ray, sinogram) entries per wavefront
 
-// Bytes of one wavefront's LDS: the item's sums (double: LDS adds of doubles run
-// about 20 times faster than of floats here, and sum more exactly), the rays in
-// flight, and the ring of pending (ray, sinogram) entries.
-__host__ __device__ inline int tile_wave_bytes(int zs, int nsino) {
-  (void)nsino;
-  return kTW * kTW * zs * 8 + kTSlots * (int)sizeof(TileSlot) + kTRing * 4;
+// LDS of one item: its sums (double: LDS adds of doubles run about 20 times faster than of
+// floats here, and sum more exactly), the rays in flight, and the queue of pending (ray,
+// sinogram) entries.
+__host__ __device__ inline int tile_acc_bytes(int zs) { return (zs * kTPitch + 15) / 16 * 16; }
+inline size_t tile_lds_bytes(int zs) {
+  return (size_t)tile_acc_bytes(zs) + kTSlots * sizeof(TileRay) + kTQueue * 4;
 }
 
+// Columns a ray visits in the tile [ti0, ti1] x [tj0, tj1] from its entry E on, by the loop's
+// x / y steps; step(q, ae, bx) for each: the alpha at which it leaves the q-th, by an x step or
+// by a y step.
+template <class Step>
+__device__ __forceinline__ int tile_path(const RayXY& t, const TileEntry& E, int ti0, int ti1,
+                                         int tj0, int tj1, Step&& step) {
+  const int iinc = ray_iinc(t.flags), jinc = ray_jinc(t.flags);
+  float Xn = E.Xn, Yn = E.Yn;
+  int i = E.i, j = E.j, q = 0;
+  while (q < kTPath - 2) {
+    const bool bx = Xn <= Yn;
+    step(q, Xn < Yn ? Xn : Yn, bx);
+    q++;
+    if (bx) {
+      i += iinc;
+      Xn = Xn + t.axu;
+    } else {
+      j += jinc;
+      Yn = Yn + t.ayu;
+    }
+    if (i < ti0 || i > ti1 || j < tj0 || j > tj1) break;
+  }
+  return q;
+}
 
-// Candidate ray c of angle ka for tile `tile` (slot (tile * nang_sub + ka) * maxc + c):
-// the c-th bin of the angle's candidate range, kept when its bins are not all zero,
-// its LOR is valid and its path enters the tile.  The slots of one (tile, angle) are
-// in bin order.
-__global__ __launch_bounds__(kGBlock) void tile_rays_kernel(GatherArgs A, int maxc, long nslots,
-                                                            TileRay* __restrict__ out,
-                                                            TilePath* __restrict__ paths) {
-  const long idx = (long)blockIdx.x * kGBlock + threadIdx.x;
-  if (idx >= nslots) return;
+// The rays of one tile per workgroup: candidate c of angle ka (the c-th bin of the angle's
+// candidate range) is kept when its LOR is valid and its path enters the tile.  The kept rays
+// go to the front of the tile's slots, the longest paths first and in (angle, bin) order among
+// equal ones: the lanes of a pass then walk about equally far.
+__global__ __launch_bounds__(kGBlock) void tile_rays_kernel(GatherArgs A, int maxc, int nslot,
+                                                            TileRay* __restrict__ rays,
+                                                            int* __restrict__ pairs,
+                                                            int* __restrict__ count) {
+  constexpr int kWaves = kGBlock / kWave;
+  __shared__ int place[kTPath];            // next slot of each path length
+  __shared__ int wcount[kWaves][kTPath];
   const Geo& g = A.g;
-  const int c = (int)(idx % maxc);
-  const long t2 = idx / maxc;
-  const int ka = (int)(t2 % A.nang_sub);
-  const int tile = (int)(t2 / A.nang_sub);
+  const int tile = blockIdx.x, wave = threadIdx.x / kWave;
   const int ntx = (g.nx + kTW - 1) / kTW;
   const int ti0 = (tile % ntx) * kTW, tj0 = (tile / ntx) * kTW;
   const int ti1 = (ti0 + kTW < g.nx ? ti0 + kTW : g.nx) - 1;
@@ -1390,393 +1361,309 @@ __global__ __launch_bounds__(kGBlock) void tile_rays_kernel(GatherArgs A, int ma
   const float yt = -g.R + g.dy * 0.5f * (float)(tj0 + tj1 + 1);
   const float hx = 0.5f * g.dx * (float)(ti1 - ti0 + 1);
   const float hy = 0.5f * g.dy * (float)(tj1 - tj0 + 1);
-  const int a = A.subset + A.nsubsets * ka;
-  int lo0, hi0, lo1, hi1;
-  tile_bins(A, a, xt, yt, hx, hy, 1.0f / g.dr, lo0, hi0, lo1, hi1);
-  const int jlo = lo0 < lo1 ? lo0 : lo1, jhi = hi0 > hi1 ? hi0 : hi1;
-  const int rr = jlo + c;
-  TileRay R;
-  R.pair = -1;
-  if (rr <= jhi && (!grid_lut<kGridAny>(A) || in_parity_range(rr, lo0, hi0, lo1, hi1))) {
-    const int pair = ka * g.nr + rr;
-    const RayXY t = A.rays[(long)a * g.nr + rr];
-    if ((t.flags & RAY_VALID) &&
-        tile_entry(g, t, A.xytab + ((long)a * g.nr + rr) * (g.nx + g.ny), ti0, ti1, tj0, tj1,
-                   R.E)) {
-      R.pair = pair;
-      R.nxy = t.nxy;
-      // the path: the loop's x / y steps from the entry until it leaves the tile
-      TilePath P;
-      const int iinc = ray_iinc(t.flags), jinc = ray_jinc(t.flags);
-      float Xn = R.E.Xn, Yn = R.E.Yn;
-      int i = R.E.i, j = R.E.j, q = 0;
-      while (q < kTPath) {
-        P.col[q] = (unsigned char)((j - tj0) * kTW + (i - ti0));
-        P.ae[q] = Xn < Yn ? Xn : Yn;
-        q++;
-        if (Xn <= Yn) {
-          i += iinc;
-          Xn = Xn + t.axu;
-        } else {
-          j += jinc;
-          Yn = Yn + t.ayu;
-        }
-        if (i < ti0 || i > ti1 || j < tj0 || j > tj1) break;
-      }
-      for (int r = q; r < kTPath; r++) {
-        P.col[r] = 0;
-        P.ae[r] = 0.f;
-      }
-      R.ncol = q;
-      paths[idx] = P;
-    }
-  }
-  out[idx] = R;
-}
-
-// The candidate rays of each tile that enter it, moved to the front of its slots in
-// slot order (one wavefront per tile); count[tile] says how many.
-__global__ __launch_bounds__(kGBlock) void tile_compact_kernel(TileRay* __restrict__ trays,
-                                                               TilePath* __restrict__ paths,
-                                                               int nslot, int ntiles,
-                                                               int* __restrict__ count) {
-  const int tile = blockIdx.x * kTWaves + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & (kWave - 1);
-  if (tile >= ntiles) return;
-  TileRay* tr = trays + (long)tile * nslot;
-  TilePath* tp = paths + (long)tile * nslot;
-  int n = 0;
-  for (int c0 = 0; c0 < nslot; c0 += kWave) {
-    TileRay R;
-    TilePath P;
-    R.pair = -1;
-    if (c0 + lane < nslot) R = tr[c0 + lane];
-    const bool keep = R.pair >= 0;
-    if (keep) P = tp[c0 + lane];
-    const unsigned long long bal = __ballot(keep);
-    __builtin_amdgcn_wave_barrier();  // every lane has read its slot before any is written
-    if (keep) {
-      const int d = n + __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
-                                                  __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0));
-      tr[d] = R;
-      tp[d] = P;
-    }
-    n += __popcll(bal);
-  }
-  if (lane == 0) count[tile] = n;
-}
-
-// The tile backprojector's axial records, out[(ka nr + r) nsino + s] (zray_setup and
-// the bin value), through a 32 (r) x 32 (s) LDS tile of the bin values so that the
-// sinogram is read along r and the records are written along s; nz_pair[ka nr + r]
-// set where a valid LOR's bin is non-zero (one atomic per 32 sinograms).
-__global__ __launch_bounds__(kGBlock) void tile_zsetup_kernel(GatherArgs A,
-                                                              ZRay* __restrict__ out,
-                                                              int* __restrict__ nz_pair) {
-  __shared__ float tb[32][33];
-  const Geo& g = A.g;
-  const int r0 = blockIdx.x * 32, ka = blockIdx.y, s0 = blockIdx.z * 32;
-  const int a = A.subset + A.nsubsets * ka;
-  const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;  // 32 x 8
-  for (int q = ty; q < 32; q += 8) {
-    const int s = s0 + q, rr = r0 + tx;
-    float b = 1.f;
-    if (s < g.nsino && rr < g.nr) {
-      if (A.kind == BP_PLAIN) b = A.sino[((long)s * A.nang_sub + ka) * g.nr + rr];
-      else if (A.kind == BP_MULT) b = A.sino[((long)s * g.nang + a) * g.nr + rr];
-    }
-    tb[q][tx] = b;
-  }
+  RayXY t;
+  TileEntry E;
+  int pair = 0;
+  // the ray of candidate slot idx, the columns of its path (0: none)
+  auto candidate = [&](int idx) -> int {
+    if (idx >= nslot) return 0;
+    const int c = idx % maxc, ka = idx / maxc, a = A.subset + A.nsubsets * ka;
+    int lo0, hi0, lo1, hi1;
+    tile_bins(A, a, xt, yt, hx, hy, 1.0f / g.dr, lo0, hi0, lo1, hi1);
+    const int jlo = lo0 < lo1 ? lo0 : lo1, jhi = hi0 > hi1 ? hi0 : hi1;
+    const int rr = jlo + c;
+    if (rr > jhi || (grid_lut<kGridAny>(A) && !in_parity_range(rr, lo0, hi0, lo1, hi1))) return 0;
+    pair = ka * g.nr + rr;
+    t = A.rays[(long)a * g.nr + rr];
+    if (!(t.flags & RAY_VALID) ||
+        !tile_entry(g, t, A.xytab + ((long)a * g.nr + rr) * (g.nx + g.ny), ti0, ti1, tj0, tj1, E))
+      return 0;
+    return tile_path(t, E, ti0, ti1, tj0, tj1, [](int, float, bool) {});
+  };
+  if (threadIdx.x < kTPath) place[threadIdx.x] = 0;
   __syncthreads();
-  const int s = s0 + tx;
-  const float2 zz = s < g.nsino ? A.zab[s] : make_float2(0.f, 0.f);
-  for (int q = ty; q < 32; q += 8) {
-    const int rr = r0 + q;  // uniform over each half wavefront
-    bool nz = false;
-    if (rr < g.nr && s < g.nsino) {
-      const RayXY R = A.rays[(long)a * g.nr + rr];
-      ZRay z;
-      zray_setup(g, R, zz.x, zz.y, z);
-      z.b = tb[tx][q];
-      z.zcount = 0;
-      z.pad = 0;
-      out[((long)ka * g.nr + rr) * g.nsino + s] = z;
-      nz = z.b != 0.f && (R.flags & RAY_VALID);
-    }
-    const unsigned long long bal = __ballot(nz);
-    const unsigned half = (unsigned)(bal >> (threadIdx.x & 32));
-    if (tx == 0 && half != 0u) atomicOr(&nz_pair[(long)ka * g.nr + rr], 1);
+  for (int base = 0; base < nslot; base += kGBlock) {
+    const int n = candidate(base + threadIdx.x);
+    if (n > 0) atomicAdd(&place[n], 1);
   }
-}
-
-// Per tile, the positions (in trays order) of its rays with a non-zero bin, live[tile *
-// nslot + c] for c < nlive[tile] (one wavefront per tile).
-__global__ __launch_bounds__(kGBlock) void tile_live_kernel(const TileRay* __restrict__ trays,
-                                                            const int* __restrict__ count,
-                                                            const int* __restrict__ nz_pair,
-                                                            int nslot, int ntiles,
-                                                            int* __restrict__ live,
-                                                            int* __restrict__ nlive) {
-  const int tile = blockIdx.x * kTWaves + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & (kWave - 1);
-  if (tile >= ntiles) return;
-  const TileRay* tr = trays + (long)tile * nslot;
-  int* lv = live + (long)tile * nslot;
-  const int nc = count[tile];
-  int n = 0;
-  for (int c0 = 0; c0 < nc; c0 += kWave) {
-    const int c = c0 + lane;
-    const bool keep = c < nc && nz_pair[tr[c].pair] != 0;
-    const unsigned long long bal = __ballot(keep);
-    if (keep)
-      lv[n + __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
-                                       __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0))] = c;
-    n += __popcll(bal);
-  }
-  if (lane == 0) nlive[tile] = n;
-}
-
-// The sinograms whose ray (tile entry E) can reach the slab [zlo, zhi] (widened)
-// inside the tile, in segment-run order: per run, the indices whose mean z lies
-// within the slab widened by the run's slopes over the tile's alpha range (z = zmean
-// + (zb - za)(alpha - 1/2)) and its deviation from the line (one run per lane); of
-// those, the sinograms whose ray's z over that alpha range meets the slab.  The
-// wavefront calls emit(keep, s) together for each group of up to 64 tested indices.
-template <class Emit>
-__device__ __forceinline__ void tile_list_ray(const GatherArgs& A, const TileEntry& E, float zlo,
-                                              float zhi, const float2* s_zab, int lane,
-                                              Emit&& emit) {
-  const float ulo = E.ce - 0.5f, uhi = E.aout - 0.5f;
-  for (int sb = 0; sb < A.nseg; sb += kWave) {
-    int s0 = 0, cnt = 0;
-    if (sb + lane < A.nseg) {
-      const GatherSeg S = A.segs[sb + lane];
-      const float c1 = S.dmin * ulo, c2 = S.dmin * uhi, c3 = S.dmax * ulo, c4 = S.dmax * uhi;
-      const float dlo = fminf(fminf(c1, c2), fminf(c3, c4));
-      const float dhi = fmaxf(fmaxf(c1, c2), fmaxf(c3, c4));
-      const float lf = (zlo - dhi - S.devz - 0.01f - S.z0) * S.dhi - 1.f;
-      const float hf = (zhi - dlo + S.devz + 0.01f - S.z0) * S.dhi + 1.f;
-      const int l0 = lf > 0.f ? (int)lf : 0;
-      const int l1 = hf < (float)(S.count - 1) ? (int)hf : S.count - 1;
-      s0 = S.first + l0;
-      cnt = l1 >= l0 ? l1 - l0 + 1 : 0;
-    }
-    const int ns = A.nseg - sb < kWave ? A.nseg - sb : kWave;
-    for (int sg = 0; sg < ns; sg++) {
-      const int cs = __builtin_amdgcn_readlane(cnt, sg);
-      if (cs == 0) continue;
-      const int f = __builtin_amdgcn_readlane(s0, sg);
-      for (int l0 = 0; l0 < cs; l0 += kWave) {
-        const int s = f + l0 + lane;
-        bool keep = false;
-        if (l0 + lane < cs) {
-          const float2 zz = s_zab[s];
-          const float vz = zz.y - zz.x;
-          const float z1 = z_at(zz.x, vz, E.ce), z2 = z_at(zz.x, vz, E.aout);
-          keep = !(fmaxf(z1, z2) < zlo) && !(fminf(z1, z2) > zhi);
-        }
-        emit(keep, s);
-      }
-    }
-  }
-}
-
-// The slab's z range widened by the listing margin.
-__device__ __forceinline__ void tile_slab_z(const Geo& g, int kz0, int kz1, float& zlo,
-                                            float& zhi) {
-  zlo = g.offz + kz0 * g.dz - kZMargin;
-  zhi = g.offz + (kz1 + 1) * g.dz + kZMargin;
-}
-
-// The listed sinograms of every (item, candidate ray) kept for a subset, one wavefront
-// per item, rays in the tile's order.  COUNT: loff[item * (nslot + 1) + c] = entries
-// of the item before ray c (c up to the tile's ray count) and tot[item] = its total.
-// Otherwise the sinograms (16 bits each) go to list[base[item] + ...].
-template <bool COUNT>
-__global__ __launch_bounds__(kGBlock) void tile_list_kernel(
-    GatherArgs A, int zs, int nslab, int nitems, const TileRay* __restrict__ trays,
-    const int* __restrict__ tcount, int nslot, int* __restrict__ loff, int* __restrict__ tot,
-    const long long* __restrict__ base, unsigned short* __restrict__ list) {
-  extern __shared__ float2 lzab[];
-  const Geo& g = A.g;
-  for (int q = threadIdx.x; q < g.nsino; q += kGBlock) lzab[q] = A.zab[q];
-  __syncthreads();
-  const int item = blockIdx.x * kTWaves + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & (kWave - 1);
-  if (item >= nitems) return;
-  const int slab = item % nslab, tile = item / nslab;
-  const int kz0 = slab * zs, kz1 = (kz0 + zs < g.nz ? kz0 + zs : g.nz) - 1;
-  float zlo, zhi;
-  tile_slab_z(g, kz0, kz1, zlo, zhi);
-  const TileRay* tr = trays + (long)tile * nslot;
-  const int nray = tcount[tile];
-  int n = 0;
-  unsigned short* out = COUNT ? nullptr : list + base[item];
-  for (int c = 0; c < nray; c++) {
-    if (COUNT && lane == 0) loff[(long)item * (nslot + 1) + c] = n;
-    const TileEntry E = tr[c].E;
-    tile_list_ray(A, E, zlo, zhi, lzab, lane, [&](bool keep, int s) {
-      const unsigned long long bal = __ballot(keep);
-      if (!COUNT && keep)
-        out[n + __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
-                                          __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0))] =
-            (unsigned short)s;
-      n += __popcll(bal);
-    });
-  }
-  if (COUNT && lane == 0) {
-    loff[(long)item * (nslot + 1) + nray] = n;
-    tot[item] = n;
-  }
-}
-
-// base[i] = sum of tot[0 .. i), for i = 0 .. n, in one workgroup.
-__global__ __launch_bounds__(kGBlock) void tile_scan_kernel(const int* __restrict__ tot, int n,
-                                                            long long* __restrict__ base) {
-  __shared__ long long part[kGBlock];
-  const int per = (n + kGBlock - 1) / kGBlock;
-  const int b = threadIdx.x * per, e = b + per < n ? b + per : n;
-  long long sum = 0;
-  for (int i = b; i < e; i++) sum += tot[i];
-  part[threadIdx.x] = sum;
   __syncthreads();
   if (threadIdx.x == 0) {
-    long long run = 0;
-    for (int t = 0; t < kGBlock; t++) {
-      const long long v = part[t];
-      part[t] = run;
-      run += v;
+    int run = 0;
+    for (int n = kTPath - 1; n > 0; n--) {
+      const int c = place[n];
+      place[n] = run;
+      run += c;
     }
-    base[n] = run;
+    count[tile] = run;
   }
   __syncthreads();
-  long long run = part[threadIdx.x];
-  for (int i = b; i < e; i++) {
-    base[i] = run;
-    run += tot[i];
+  for (int base = 0; base < nslot; base += kGBlock) {
+    const int ncol = candidate(base + threadIdx.x);
+    int rank = 0;
+    for (int n = 1; n < kTPath; n++) {
+      const unsigned long long bal = __ballot(ncol == n);
+      if (ncol == n)
+        rank = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
+                                         __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0));
+      if (threadIdx.x % kWave == 0) wcount[wave][n] = __popcll(bal);
+    }
+    __syncthreads();
+    int d = place[ncol] + rank;
+    for (int w = 0; w < wave; w++) d += ncol > 0 ? wcount[w][ncol] : 0;
+    __syncthreads();
+    if (threadIdx.x > 0 && threadIdx.x < kTPath)
+      for (int w = 0; w < kWaves; w++) place[threadIdx.x] += wcount[w][threadIdx.x];
+    __syncthreads();
+    if (ncol == 0) continue;
+    TileRay* R = rays + (long)tile * nslot + d;
+    pairs[(long)tile * nslot + d] = pair;
+    const int iinc = ray_iinc(t.flags), jinc = ray_jinc(t.flags);
+    float last = E.ce;
+    tile_path(t, E, ti0, ti1, tj0, tj1, [&](int q, float ae, bool bx) {
+      TileStep e;
+      e.ae = last = ae;
+      e.step = q == ncol - 1 ? kTileAway : (bx ? iinc : jinc * kTW) * 8;
+      R->path[q] = e;
+    });
+    for (int r = ncol; r < kTPath; r++)
+      R->path[r] = TileStep{__int_as_float(0x7f800000), kTileAway};
+    R->ce = E.ce;
+    R->aout = fmaxf(E.aout, last);
+    R->pair = pair;
+    R->mxy = E.mxy;
+    R->nxy = t.nxy;
+    R->ncol = ncol;
+    R->col0 = ((E.j - tj0) * kTW + E.i - ti0) * 8;
+    R->pad = 0;
   }
 }
 
-// Items (tile, slab) are taken from a queue in the order of order[] (the tiles
-// nearest the image centre first, whose rays are the most), counter at *next.  The
-// rays entering tile t are trays[t * nslot + c]; those with a non-zero bin are at the
-// positions live[t * nslot + c'], c' < nlive[t].  The (ray, sinogram) pairs to walk
-// go through a ring in LDS: a pass takes 64 of them as soon as there are, so a pass
-// carries the sinograms of several rays.
-// LISTED: each (item, ray)'s sinograms are read from the lists tile_list_kernel keeps
-// (loff, base, list) instead of being listed here.
-template <bool LISTED>
-__global__ __launch_bounds__(kGBlock) void tile_bp_kernel(GatherArgs A, int zs, int nslab,
-                                                          const int* __restrict__ order,
-                                                          int nitems, int* __restrict__ next,
-                                                          const TileRay* __restrict__ trays,
-                                                          const TilePath* __restrict__ tpaths,
-                                                          int nslot,
-                                                          const int* __restrict__ live,
-                                                          const int* __restrict__ nlive,
-                                                          const int* __restrict__ loff,
-                                                          const long long* __restrict__ lbase,
-                                                          const unsigned short* __restrict__ list) {
-  extern __shared__ double tlds[];
+// The call's axial records out[(ka nr + r) nsino + s] (zray_setup and the bin value): a
+// workgroup takes kTZBins bins of one angle with all of their sinograms, 32 at a time through
+// an LDS tile, so that the sinogram is read along r and the records are written along s;
+// nzmask[(ka nr + r) nwords + s / 32]: the sinograms of a valid LOR whose bin is not zero, a
+// bit each; nz_pair[ka nr + r]: whether there is one.
+constexpr int kTZBins = 8;
+__host__ __device__ inline int tile_words(int nsino) { return (nsino + 63) / 64 * 2 + 2; }
+__global__ __launch_bounds__(kGBlock) void tile_zsetup_kernel(GatherArgs A,
+                                                              TileZ* __restrict__ out,
+                                                              unsigned* __restrict__ nzmask,
+                                                              int* __restrict__ nz_pair) {
+  __shared__ float tb[32][kTZBins + 1];
+  __shared__ int snz[kTZBins];
   const Geo& g = A.g;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & (kWave - 1);
-  const int ntx = (g.nx + kTW - 1) / kTW;
-  double* acc = (double*)((char*)tlds + (size_t)w * tile_wave_bytes(zs, g.nsino));
-  TileSlot* slots = (TileSlot*)(acc + kTW * kTW * zs);
-  unsigned* ring = (unsigned*)(slots + kTSlots);
-  // the axial table, shared by the workgroup's wavefronts, for the listing (the kept
-  // lists need none: their launch leaves it out of the LDS)
-  float2* s_zab = (float2*)((char*)tlds + (size_t)kTWaves * tile_wave_bytes(zs, g.nsino));
-  if (!LISTED)
-    for (int q = threadIdx.x; q < g.nsino; q += kGBlock) s_zab[q] = A.zab[q];
-  __syncthreads();
-  const long nxy = (long)g.nx * g.ny;
-  const int il = lane % kTW, jl = lane / kTW;
-  for (;;) {
-    int q = 0;
-    if (lane == 0) q = atomicAdd(next, 1);
-    q = __builtin_amdgcn_readfirstlane(q);
-    if (q >= nitems) return;
-    const int item = order[q];
-    const int slab = item % nslab, tile = item / nslab;
-    const int ti0 = (tile % ntx) * kTW, tj0 = (tile / ntx) * kTW;
-    const int ti1 = (ti0 + kTW < g.nx ? ti0 + kTW : g.nx) - 1;
-    const int tj1 = (tj0 + kTW < g.ny ? tj0 + kTW : g.ny) - 1;
-    const int kz0 = slab * zs, kz1 = (kz0 + zs < g.nz ? kz0 + zs : g.nz) - 1;
-    const bool incol = ti0 + il <= ti1 && tj0 + jl <= tj1;
-    const long v0 = (long)(tj0 + jl) * g.nx + ti0 + il;
-    wave_lds_sync();  // the previous item's sums are read out
-    for (int kl = 0; kl <= kz1 - kz0; kl++)
-      acc[lane * zs + kl] = (incol && !A.upd_sens) ? (double)A.img[(kz0 + kl) * nxy + v0] : 0.0;
-    wave_lds_sync();
-    float zlo, zhi;
-    tile_slab_z(g, kz0, kz1, zlo, zhi);
-    const long long ibase = LISTED ? lbase[item] : 0;
-    const TileRay* tr = trays + (long)tile * nslot;
-    const unsigned* trw = (const unsigned*)tr;
-    const unsigned* tpw = (const unsigned*)(tpaths + (long)tile * nslot);
-    const int* lv = live + (long)tile * nslot;
-    const int nray = nlive[tile];
-    int head = 0, pend = 0;  // ring entries (ray << 16 | sinogram), head .. head + pend - 1
-    int lvc = 0;             // live positions c0 .. c0 + 63, one per lane
-    // one pass: lanes l < k walk entry head + l
-    auto run_pass = [&](int k) {
-      wave_lds_sync();
-      if (lane < k) {
-        const unsigned e = ring[(head + lane) & (kTRing - 1)];
-        const TileSlot& S = slots[(e >> 16) & (kTSlots - 1)];
-        const ZRay z = load_zray(A.zr + (long)S.R.pair * g.nsino + (e & 0xffffu));
-        if (z.b != 0.f)  // SiddonProjector.cpp:496
-          tile_lane(S.R, S.P.ae, S.P.col, z, kz0, kz1, zs, acc);
+  const int r0 = blockIdx.x * kTZBins, ka = blockIdx.y;
+  const int a = A.subset + A.nsubsets * ka;
+  const int rx = threadIdx.x % kTZBins, sx = threadIdx.x / kTZBins;  // 8 bins x 32 sinograms
+  const int ty = threadIdx.x / 32, tx = threadIdx.x % 32;            // the same, s fastest
+  RayXY R = A.rays[(long)a * g.nr + (r0 + ty < g.nr ? r0 + ty : g.nr - 1)];
+  const int nwords = tile_words(g.nsino);
+  bool nz = false;
+  if (threadIdx.x < kTZBins) snz[threadIdx.x] = 0;
+  for (int s0 = 0; s0 < g.nsino; s0 += 32) {
+    __syncthreads();
+    {
+      const int s = s0 + sx, rr = r0 + rx;
+      float b = 1.f;
+      if (s < g.nsino && rr < g.nr) {
+        if (A.kind == BP_PLAIN) b = A.sino[((long)s * A.nang_sub + ka) * g.nr + rr];
+        else if (A.kind == BP_MULT) b = A.sino[((long)s * g.nang + a) * g.nr + rr];
       }
-      head = (head + k) & (kTRing - 1);
-      pend -= k;
-    };
-    for (int c = 0; c < nray; c++) {
-      // the slot of ray c is free once no pending entry belongs to ray c - kTSlots
+      tb[sx][rx] = b;
+    }
+    __syncthreads();
+    const int s = s0 + tx, rr = r0 + ty;
+    bool nzb = false;
+    if (s < g.nsino && rr < g.nr) {
+      const float2 zz = A.zab[s];
+      ZRay z;
+      zray_setup(g, R, zz.x, zz.y, z);
+      TileZ o;
+      o.az0 = z.az0;
+      o.L = z.L;
+      o.b = tb[tx][ty];
+      o.k01 = (int)(((unsigned)(int)z.k1 << 16) | ((unsigned)z.k0 & 0xffffu));
+      out[((long)ka * g.nr + rr) * g.nsino + s] = o;
+      nzb = o.b != 0.f && (R.flags & RAY_VALID);
+    }
+    const unsigned bits = (unsigned)(__ballot(nzb) >> (threadIdx.x & 32));
+    if (tx == 0 && rr < g.nr) nzmask[((long)ka * g.nr + rr) * nwords + s0 / 32] = bits;
+    nz |= bits != 0u;
+  }
+  // words that a window of 64 sinograms may reach past the last one
+  for (int w = (g.nsino + 31) / 32 + tx; w < nwords; w += 32)
+    if (r0 + ty < g.nr) nzmask[((long)ka * g.nr + r0 + ty) * nwords + w] = 0u;
+  __syncthreads();
+  if (nz) snz[ty] = 1;
+  __syncthreads();
+  if (threadIdx.x < kTZBins && r0 + (int)threadIdx.x < g.nr)
+    nz_pair[(long)ka * g.nr + r0 + threadIdx.x] = snz[threadIdx.x];
+}
+
+// Items b = (tile position * nslab + slab) * nchunk + chunk, the tiles in the order of
+// order[] (the ones nearest the image centre first, whose rays are the most), one wavefront
+// each.  The rays entering tile t are rays[t * nslot + c], c < count[t]; a chunk takes every
+// nchunk-th of them.  The (ray, sinogram) pairs to walk go through a queue in LDS: a pass takes 64 of
+// them as soon as there are, so a pass carries the sinograms of several rays.  parts: null,
+// or the chunks' sums, [nchunk][voxels].
+__global__ __launch_bounds__(kWave) void tile_bp_kernel(GatherArgs A, int zs, int nslab, int nchunk,
+                                                        const int* __restrict__ order,
+                                                        const TileRay* __restrict__ rays,
+                                                        const int* __restrict__ pairs,
+                                                        const int* __restrict__ count, int nslot,
+                                                        const TileZ* __restrict__ zrec,
+                                                        const unsigned* __restrict__ nzmask,
+                                                        const float* __restrict__ zinc,
+                                                        double* __restrict__ parts) {
+  extern __shared__ __align__(16) char tlds[];
+  const Geo& g = A.g;
+  const int lane = threadIdx.x;
+  char* acc = tlds;
+  TileRay* slots = (TileRay*)(tlds + tile_acc_bytes(zs));
+  unsigned* queue = (unsigned*)(slots + kTSlots);
+  const int ntx = (g.nx + kTW - 1) / kTW;
+  const int chunk = blockIdx.x % nchunk, ts = blockIdx.x / nchunk;
+  const int slab = ts % nslab, tile = order[ts / nslab];
+  const int ti0 = (tile % ntx) * kTW, tj0 = (tile / ntx) * kTW;
+  const int kz0 = slab * zs, kz1 = (kz0 + zs < g.nz ? kz0 + zs : g.nz) - 1, nk = kz1 - kz0 + 1;
+  const bool incol = ti0 + lane % kTW < g.nx && tj0 + lane / kTW < g.ny;
+  const long nxy = (long)g.nx * g.ny;
+  const long v0 = kz0 * nxy + (long)(tj0 + lane / kTW) * g.nx + ti0 + lane % kTW;
+  const unsigned lim = (unsigned)(nk * kTPitch);
+  double* col = (double*)acc + lane;
+  for (int q = 0; q < nk; q++)
+    col[q * (kTPitch / 8)] = (incol && !A.upd_sens && !parts) ? (double)A.img[v0 + q * nxy] : 0.0;
+  // the slab's z range widened by the search margin
+  const float zlo = g.offz + kz0 * g.dz - kZMargin, zhi = g.offz + (kz1 + 1) * g.dz + kZMargin;
+  const TileRay* tr = rays + (long)tile * nslot;
+  const int* tp = pairs + (long)tile * nslot;
+  const int nray = count[tile];
+  const int nwords = tile_words(g.nsino);
+  int pend = 0;  // pending entries (ray number << 16 | sinogram), queue[0 .. pend)
+  // one pass: the first n entries, one per lane; the ones after them move to the front
+  auto run_pass = [&](int n) {
+    wave_lds_sync();
+    const unsigned e = queue[lane];
+    const unsigned after = n == kWave ? queue[kWave + lane] : 0u;
+    if (lane < n) {
+      const TileRay& R = slots[(e >> 16) & (kTSlots - 1)];
+      const int s = (int)(e & 0xffffu);
+      const TileZ z = zrec[(long)R.pair * g.nsino + s];
+      tile_lane(R, z, zinc[s], kz0, lim);
+    }
+    pend -= n;
+    wave_lds_sync();
+    if (lane < pend) queue[lane] = after;
+  };
+  int nlive = 0;  // rays taken so far (their numbers in the queue)
+  for (int cb = chunk; cb < nray; cb += kWave * nchunk) {
+    // the chunk's next 64 rays: those with a non-zero bin
+    const int cl = cb + lane * nchunk, pr = cl < nray ? tp[cl] : -1;
+    unsigned long long live = __ballot(pr >= 0 && A.nz_pair[pr < 0 ? 0 : pr] != 0);
+    for (; live; live &= live - 1) {
+      const int c = cb + (int)__builtin_ctzll(live) * nchunk;
+      // the slot of ray number nlive is free once no pending entry belongs to the ray
+      // kTSlots before it
       while (pend > 0) {
         wave_lds_sync();
-        if ((int)(ring[head] >> 16) + kTSlots > c) break;
+        if ((((unsigned)nlive - (queue[0] >> 16)) & 0xffffu) < kTSlots) break;
         run_pass(pend < kWave ? pend : kWave);
       }
       wave_lds_sync();
-      if ((c & (kWave - 1)) == 0) lvc = c + lane < nray ? lv[c + lane] : 0;
-      const int rc = __builtin_amdgcn_readlane(lvc, c & (kWave - 1));  // in the tile's list
-      if (lane < (int)(sizeof(TileRay) / 4))
-        ((unsigned*)&slots[c & (kTSlots - 1)].R)[lane] =
-            trw[(long)rc * (sizeof(TileRay) / 4) + lane];
-      else if (lane < (int)(sizeof(TileSlot) / 4))
-        ((unsigned*)&slots[c & (kTSlots - 1)].R)[lane] =
-            tpw[(long)rc * (sizeof(TilePath) / 4) + lane - (int)(sizeof(TileRay) / 4)];
-      // the sinograms of ray c that reach the slab inside the tile go to the ring
-      auto emit = [&](bool keep, int s) {
-        const unsigned long long bal = __ballot(keep);
-        if (keep)
-          ring[(head + pend +
-                __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
-                                          __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0))) &
-               (kTRing - 1)] = ((unsigned)c << 16) | (unsigned)s;
-        pend += __popcll(bal);
-        if (pend >= kWave) run_pass(kWave);
-      };
-      if (LISTED) {
-        const int* lo = loff + (long)item * (nslot + 1) + rc;
-        const long long b0 = ibase + lo[0], b1 = ibase + lo[1];
-        for (long long l0 = b0; l0 < b1; l0 += kWave) {
-          const bool keep = l0 + lane < b1;
-          emit(keep, keep ? (int)list[l0 + lane] : 0);
+      constexpr int kWords = sizeof(TileRay) / 4;
+      if (lane < kWords)
+        ((unsigned*)&slots[nlive & (kTSlots - 1)])[lane] = ((const unsigned*)(tr + c))[lane];
+      wave_lds_sync();
+      const unsigned taglane = (((unsigned)nlive & 0xffffu) << 16) + (unsigned)lane;
+      nlive++;
+      // The sinograms whose ray can reach the slab inside the tile: runs [first, first + cnt),
+      // one per lane, of which those with a non-zero bin are queued (zero bins add nothing,
+      // SiddonProjector.cpp:496).  With one slab all of them, 64 to a run; otherwise, per
+      // segment run, the indices whose mean z lies within the slab widened by the run's slopes
+      // over the tile's alpha range (z = zmean + (zb - za)(alpha - 1/2)) and its deviation from
+      // the line.  The few that do not reach it add nothing.
+      const float ulo = tr[c].ce - 0.5f, uhi = tr[c].aout - 0.5f;
+      const unsigned* words = nzmask + (long)tr[c].pair * nwords;
+      const int nrun = nslab == 1 ? (g.nsino + kWave - 1) / kWave : A.nseg;
+      for (int rb = 0; rb < nrun; rb += kWave) {
+        int first = 0, cnt = 0;
+        if (rb + lane < nrun) {
+          if (nslab == 1) {
+            first = (rb + lane) * kWave;
+            cnt = g.nsino - first < kWave ? g.nsino - first : kWave;
+          } else {
+            const GatherSeg S = A.segs[rb + lane];
+            const float p1 = S.dmin * ulo, p2 = S.dmin * uhi, p3 = S.dmax * ulo, p4 = S.dmax * uhi;
+            const float dlo = fminf(fminf(p1, p2), fminf(p3, p4));
+            const float dhi = fmaxf(fmaxf(p1, p2), fmaxf(p3, p4));
+            // 0.01 mm and a hundredth of an index for the rounding
+            const float lf = ceilf((zlo - dhi - S.devz - 0.01f - S.z0) * S.dhi - 0.01f);
+            const float hf = floorf((zhi - dlo + S.devz + 0.01f - S.z0) * S.dhi + 0.01f);
+            const int l0 = lf > 0.f ? (lf < (float)S.count ? (int)lf : S.count) : 0;
+            const int l1 = hf < (float)(S.count - 1) ? (int)hf : S.count - 1;
+            first = S.first + l0;
+            cnt = l1 >= l0 ? l1 - l0 + 1 : 0;
+          }
         }
-      } else {
-        tile_list_ray(A, tr[rc].E, zlo, zhi, s_zab, lane, emit);
+        while (__any(cnt > 0)) {
+          // the next (up to) 64 of every run: their bits
+          unsigned lo = 0, hi = 0;
+          if (cnt > 0) {
+            const unsigned* w = words + (first >> 5);
+            const int sh = first & 31;
+            lo = __builtin_amdgcn_alignbit(w[1], w[0], sh);
+            hi = __builtin_amdgcn_alignbit(w[2], w[1], sh);
+            if (cnt < 32) lo &= (1u << cnt) - 1u;
+            hi = cnt <= 32 ? 0u : (cnt < 64 ? hi & ((1u << (cnt - 32)) - 1u) : hi);
+          }
+          unsigned long long some = __ballot((lo | hi) != 0u);
+          if (!__any(hi != 0u)) {  // runs of at most 32: the usual case, half the work
+            for (; some; some &= some - 1) {
+              const int l = __builtin_ctzll(some);
+              const unsigned m = (unsigned)__builtin_amdgcn_readlane(lo, l);
+              const int f = __builtin_amdgcn_readlane(first, l);
+              if (__builtin_amdgcn_inverse_ballot_w64((unsigned long long)m))
+                queue[__builtin_amdgcn_mbcnt_lo(m, pend)] = taglane + (unsigned)f;
+              pend += __popc(m);
+              if (pend >= kWave) run_pass(kWave);
+            }
+          } else {
+            for (; some; some &= some - 1) {
+              const int l = __builtin_ctzll(some);
+              const unsigned mlo = (unsigned)__builtin_amdgcn_readlane(lo, l);
+              const unsigned mhi = (unsigned)__builtin_amdgcn_readlane(hi, l);
+              const int f = __builtin_amdgcn_readlane(first, l);
+              if (__builtin_amdgcn_inverse_ballot_w64(mlo | (unsigned long long)mhi << 32))
+                queue[__builtin_amdgcn_mbcnt_hi(mhi, __builtin_amdgcn_mbcnt_lo(mlo, pend))] =
+                    taglane + (unsigned)f;
+              pend += __popc(mlo) + __popc(mhi);
+              if (pend >= kWave) run_pass(kWave);
+            }
+          }
+          first += kWave;
+          cnt -= kWave;
+        }
       }
     }
-    while (pend > 0) run_pass(pend < kWave ? pend : kWave);
-    wave_lds_sync();
-    if (incol)
-      for (int kl = 0; kl <= kz1 - kz0; kl++)
-        store_voxel(A, (kz0 + kl) * nxy + v0, (float)acc[lane * zs + kl]);
   }
+  while (pend > 0) run_pass(pend < kWave ? pend : kWave);
+  wave_lds_sync();
+  if (incol)
+    for (int q = 0; q < nk; q++) {
+      const double b = col[q * (kTPitch / 8)];
+      if (parts) parts[(long)chunk * nxy * g.nz + v0 + q * nxy] = b;
+      else store_voxel(A, v0 + q * nxy, (float)b);
+    }
+}
+
+// The voxels' sums over the chunks, in their order.
+__global__ __launch_bounds__(kGBlock) void tile_reduce_kernel(GatherArgs A, long nvox, int nchunk,
+                                                              const double* __restrict__ parts) {
+  const long v = (long)blockIdx.x * kGBlock + threadIdx.x;
+  if (v >= nvox) return;
+  double b = A.upd_sens ? 0.0 : (double)A.img[v];
+  for (int c = 0; c < nchunk; c++) b += parts[c * nvox + v];
+  store_voxel(A, v, (float)b);
 }
 
 }  // namespace
@@ -1839,21 +1726,16 @@ hipError_t launch_backproject_gather(const apirl_plan* p, const float* sino, flo
   return hipGetLastError();
 }
 
-// Slab depth of the tile backprojector's items: the plan's tuning, or about 5
-// slices (shallow items keep few lanes on one voxel per LDS add and leave room for
-// more wavefronts per SIMD; with the kept lists, 1.26 ms per 12-angle subset of the
-// 256x256x81 / 344x252x837 workload at 5 slices, 1.31 at 4 and 1.32 at 6).
+// Slab depth of the tile backprojector's items: the plan's tuning, or the whole image up to
+// kTSlices slices, about kTSlices - 1 otherwise (a ray is walked through every slab it
+// reaches in a tile, and deep slabs leave room for fewer wavefronts).
+constexpr int kTSlices = 13;
 int tile_slab_depth(const apirl_plan* p) {
   const int nz = p->geo.nz;
   if (p->tile_zs > 0) return p->tile_zs < nz ? p->tile_zs : nz;
-  const int nslab = (nz + 4) / 5;
+  if (nz <= kTSlices) return nz;
+  const int nslab = (nz + kTSlices - 2) / (kTSlices - 1);
   return (nz + nslab - 1) / nslab;
-}
-
-size_t tile_lds_bytes(const apirl_plan* p, bool listed) {
-  if (listed) return (size_t)kTWaves * tile_wave_bytes(tile_slab_depth(p), p->geo.nsino);
-  return (size_t)kTWaves * tile_wave_bytes(tile_slab_depth(p), p->geo.nsino) +
-         (size_t)p->geo.nsino * sizeof(float2);
 }
 
 // Upper bound on the candidate bins of one (tile, angle): the bins within the tile's
@@ -1876,18 +1758,17 @@ const char* tile_misfit(const apirl_plan* p) {
   if (p->geo.nsino >= 65536) return "the tile backprojector takes fewer than 65536 sinograms";
   if ((long)p->geo.nang * tile_max_candidates(p) >= 65536)
     return "the tile backprojector takes fewer than 65536 candidate rays per tile";
-  if (tile_lds_bytes(p, false) > 65536) return "the tile backprojector's items exceed 64 KiB of LDS";
+  if (tile_lds_bytes(tile_slab_depth(p)) > 65536)
+    return "the tile backprojector's items exceed 64 KiB of LDS";
+  if (!p->d_zinc || !p->slices16) return "the tile backprojector keeps slices in 16 bits";
   return nullptr;
 }
 
-int tile_items(const apirl_plan* p) {
-  const int zs = tile_slab_depth(p);
-  return ((p->geo.nx + kTW - 1) / kTW) * ((p->geo.ny + kTW - 1) / kTW) *
-         ((p->geo.nz + zs - 1) / zs);
+int tile_count(const apirl_plan* p) {
+  return ((p->geo.nx + kTW - 1) / kTW) * ((p->geo.ny + kTW - 1) / kTW);
 }
 
 void build_tile_order(const apirl_plan* p, std::vector<int>& order) {
-  const int zs = tile_slab_depth(p), nslab = (p->geo.nz + zs - 1) / zs;
   const int ntx = (p->geo.nx + kTW - 1) / kTW, nty = (p->geo.ny + kTW - 1) / kTW;
   std::vector<std::pair<double, int>> tiles;
   for (int ty = 0; ty < nty; ty++)
@@ -1900,17 +1781,22 @@ void build_tile_order(const apirl_plan* p, std::vector<int>& order) {
                      return a.first < b.first;
                    });
   order.clear();
-  for (const auto& t : tiles)
-    for (int s = 0; s < nslab; s++) order.push_back(t.second * nslab + s);
+  for (const auto& t : tiles) order.push_back(t.second);
 }
 
 namespace {
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
 struct TileSizes {
-  int nang_sub, maxc, ntiles;
-  long nrays, npair, nslots;
+  int nang_sub, maxc, ntiles, nslot, zs, nslab, nchunk;
+  long nrays, npair, nvox;
 };
+
+// Wavefronts the items should come to: about three for each that the GPU holds, so that the
+// last ones to finish are a small part.
+constexpr int kTWaves = 32768;
+constexpr int kTChunkRays = 8;                   // rays per chunk at least, on average
+constexpr size_t kTPartBytes = size_t(1) << 28;  // the chunks' sums at most
 
 TileSizes tile_sizes(const apirl_plan* p, int subset, int nsubsets) {
   const Geo& g = p->geo;
@@ -1918,168 +1804,112 @@ TileSizes tile_sizes(const apirl_plan* p, int subset, int nsubsets) {
   z.nang_sub = subset_num_angles(g.nang, nsubsets, subset);
   z.npair = (long)z.nang_sub * g.nr;
   z.nrays = (long)g.nsino * z.npair;
+  z.nvox = (long)g.nx * g.ny * g.nz;
   z.maxc = tile_max_candidates(p);
-  z.ntiles = ((g.nx + kTW - 1) / kTW) * ((g.ny + kTW - 1) / kTW);
-  z.nslots = (long)z.ntiles * z.nang_sub * z.maxc;
+  z.ntiles = tile_count(p);
+  z.nslot = z.nang_sub * z.maxc;
+  z.zs = tile_slab_depth(p);
+  z.nslab = (g.nz + z.zs - 1) / z.zs;
+  long c = kTWaves / ((long)z.ntiles * z.nslab);
+  c = std::min(c, (long)z.nslot / kTChunkRays);
+  c = std::min(c, (long)(kTPartBytes / (z.nvox * sizeof(double))));
+  z.nchunk = c < 1 ? 1 : (int)c;
   return z;
 }
-}  // namespace
 
-namespace {
-// geometry: [ray count per tile][candidate rays of every (tile, angle)][their paths]
-// [per item: entries before each ray, and the total][per item: first entry]
+// geometry: [ray count per tile][ray (angle, bin) pairs][rays]
 struct TileGeoPtrs {
-  int* tcount;
-  TileRay* trays;
-  TilePath* tpaths;
-  int* loff;
-  long long* lbase;
-  int* tot;
+  int* count;
+  int* pairs;
+  TileRay* rays;
   size_t bytes;
 };
 
-TileGeoPtrs tile_geo_ptrs(const apirl_plan* p, const TileSizes& z, void* geo) {
-  const int nitems = tile_items(p);
-  const int nslot = z.nang_sub * z.maxc;
+TileGeoPtrs tile_geo_ptrs(const TileSizes& z, void* geo) {
+  const size_t nslots = (size_t)z.ntiles * z.nslot;
   TileGeoPtrs q;
   char* c = (char*)geo;
   size_t o = 0;
-  q.tcount = (int*)(c + o);
+  q.count = (int*)(c + o);
   o += align256((size_t)z.ntiles * sizeof(int));
-  q.trays = (TileRay*)(c + o);
-  q.tpaths = (TilePath*)(c + o + (size_t)z.nslots * sizeof(TileRay));
-  o += align256((size_t)z.nslots * (sizeof(TileRay) + sizeof(TilePath)));
-  q.loff = (int*)(c + o);
-  o += align256((size_t)nitems * (nslot + 1) * sizeof(int));
-  q.lbase = (long long*)(c + o);
-  o += align256((size_t)(nitems + 1) * sizeof(long long));
-  q.tot = (int*)(c + o);
-  o += align256((size_t)nitems * sizeof(int));
+  q.pairs = (int*)(c + o);
+  o += align256(nslots * sizeof(int));
+  q.rays = (TileRay*)(c + o);
+  o += align256(nslots * sizeof(TileRay));
   q.bytes = o;
   return q;
 }
 }  // namespace
 
 size_t tile_geo_bytes(const apirl_plan* p, int subset, int nsubsets) {
-  return tile_geo_ptrs(p, tile_sizes(p, subset, nsubsets), nullptr).bytes;
+  return tile_geo_ptrs(tile_sizes(p, subset, nsubsets), nullptr).bytes;
 }
 
-hipError_t launch_tile_lists(const apirl_plan* p, int subset, int nsubsets, void* geo,
-                             unsigned short* list, long long** total, hipStream_t st) {
-  if (tile_misfit(p)) return hipErrorNotSupported;
-  const Geo& g = p->geo;
-  const TileSizes z = tile_sizes(p, subset, nsubsets);
-  const TileGeoPtrs q = tile_geo_ptrs(p, z, geo);
-  const int nitems = tile_items(p);
-  const int zs = tile_slab_depth(p), nslab = (g.nz + zs - 1) / zs;
-  const int nslot = z.nang_sub * z.maxc;
-  if (total) *total = q.lbase + nitems;
-  GatherArgs A;
-  ZRay* unused_zr = nullptr;
-  int* unused_nz = nullptr;
-  gather_args_for(p, subset, nsubsets, BP_ONES, nullptr, nullptr, nullptr, A, unused_zr,
-                  unused_nz);
-  const dim3 grid((nitems + kTWaves - 1) / kTWaves);
-  const size_t lds = (size_t)g.nsino * sizeof(float2);
-  if (!list) {
-    hipLaunchKernelGGL(tile_list_kernel<true>, grid, dim3(kGBlock), lds, st, A, zs, nslab, nitems,
-                       (const TileRay*)q.trays, (const int*)q.tcount, nslot, q.loff, q.tot,
-                       (const long long*)nullptr, (unsigned short*)nullptr);
-    hipLaunchKernelGGL(tile_scan_kernel, dim3(1), dim3(kGBlock), 0, st, (const int*)q.tot, nitems,
-                       q.lbase);
-  } else {
-    hipLaunchKernelGGL(tile_list_kernel<false>, grid, dim3(kGBlock), lds, st, A, zs, nslab,
-                       nitems, (const TileRay*)q.trays, (const int*)q.tcount, nslot,
-                       (int*)nullptr, (int*)nullptr, (const long long*)q.lbase, list);
-  }
-  return hipGetLastError();
-}
-
-// scratch: [ZRay x nrays, (angle, radial bin, sinogram) order][non-zero flag per
-// (angle, r), item counter][live positions per slot][live count per tile][the
-// geometry, when it is not kept]
+// scratch: [TileZ x nrays, (angle, radial bin, sinogram) order][non-zero sinograms per
+// (angle, r)][non-zero flag per (angle, r)][the chunks' sums][the geometry, when it is not
+// kept]
 size_t tile_scratch_bytes(const apirl_plan* p, int subset, int nsubsets, bool with_geo) {
   const TileSizes z = tile_sizes(p, subset, nsubsets);
-  return align256((size_t)z.nrays * sizeof(ZRay)) + align256((size_t)(z.npair + 1) * sizeof(int)) +
-         align256((size_t)z.nslots * sizeof(int)) + align256((size_t)z.ntiles * sizeof(int)) +
+  return align256((size_t)z.nrays * sizeof(TileZ)) +
+         align256((size_t)z.npair * tile_words(p->geo.nsino) * sizeof(unsigned)) +
+         align256((size_t)z.npair * sizeof(int)) +
+         (z.nchunk > 1 ? align256((size_t)z.nchunk * z.nvox * sizeof(double)) : 0) +
          (with_geo ? tile_geo_bytes(p, subset, nsubsets) : 0);
 }
 
 hipError_t launch_backproject_tile(const apirl_plan* p, const float* sino, float* img,
                                    int subset, int nsubsets, int kind, void* scratch,
                                    size_t scratch_bytes, hipStream_t st, const EmFuse* fuse,
-                                   void* geo, bool geo_ready, const unsigned short* list) {
+                                   void* geo, bool geo_ready) {
   if (kind != BP_PLAIN && kind != BP_ONES && kind != BP_MULT) return hipErrorNotSupported;
   if (tile_misfit(p)) return hipErrorNotSupported;
   const Geo& g = p->geo;
   const TileSizes z = tile_sizes(p, subset, nsubsets);
-  if (z.nrays == 0 || (long)g.nx * g.ny * g.nz == 0) return hipSuccess;
+  if (z.nrays == 0 || z.nvox == 0) return hipSuccess;
   if (scratch_bytes < tile_scratch_bytes(p, subset, nsubsets, geo == nullptr))
     return hipErrorInvalidValue;
-  const int nitems = tile_items(p);
-  if (!p->d_tile_order || p->tile_order_n != nitems) return hipErrorInvalidValue;
+  if (!p->d_tile_order) return hipErrorInvalidValue;
   char* sp = (char*)scratch;
-  ZRay* zr = (ZRay*)sp;
-  sp += align256((size_t)z.nrays * sizeof(ZRay));
+  TileZ* zr = (TileZ*)sp;
+  sp += align256((size_t)z.nrays * sizeof(TileZ));
+  unsigned* nzmask = (unsigned*)sp;
+  sp += align256((size_t)z.npair * tile_words(g.nsino) * sizeof(unsigned));
   int* nzp = (int*)sp;
-  sp += align256((size_t)(z.npair + 1) * sizeof(int));
-  int* live = (int*)sp;
-  sp += align256((size_t)z.nslots * sizeof(int));
-  int* nlive = (int*)sp;
-  sp += align256((size_t)z.ntiles * sizeof(int));
+  sp += align256((size_t)z.npair * sizeof(int));
+  double* parts = nullptr;
+  if (z.nchunk > 1) {
+    parts = (double*)sp;
+    sp += align256((size_t)z.nchunk * z.nvox * sizeof(double));
+  }
   if (!geo) {
     geo = sp;
     geo_ready = false;
-    list = nullptr;
   }
-  const TileGeoPtrs q = tile_geo_ptrs(p, z, geo);
-  int* tcount = q.tcount;
-  TileRay* trays = q.trays;
-  TilePath* tpaths = q.tpaths;
+  const TileGeoPtrs q = tile_geo_ptrs(z, geo);
   GatherArgs A;
   ZRay* unused_zr = nullptr;
   int* unused_nz = nullptr;
   gather_args_for(p, subset, nsubsets, kind, sino, img, nullptr, A, unused_zr, unused_nz);
-  A.zr = zr;
   A.nz_pair = nzp;
-  A.ztab = nullptr;  // the lanes take their z crossings by the loop's additions
   if (fuse) {
     A.upd_sens = fuse->sens;
     A.upd_thr = fuse->thr;
     A.upd_strict = fuse->strict;
   }
-  // the call's axial records with their bin values, and the (angle, r) with a
-  // non-zero bin
-  hipLaunchKernelGGL(clear_int_kernel, dim3(ggrid(z.npair + 1)), dim3(kGBlock), 0, st, nzp,
-                     z.npair + 1);
-  hipLaunchKernelGGL(tile_zsetup_kernel, dim3((g.nr + 31) / 32, z.nang_sub, (g.nsino + 31) / 32),
-                     dim3(kGBlock), 0, st, A, zr, nzp);
-  if (!geo_ready) {
-    // the subset's geometry: the candidate rays of every (tile, angle) with their
-    // paths, compacted per tile
-    hipLaunchKernelGGL(tile_rays_kernel, dim3(ggrid(z.nslots)), dim3(kGBlock), 0, st, A, z.maxc,
-                       z.nslots, trays, tpaths);
-    hipLaunchKernelGGL(tile_compact_kernel, dim3((z.ntiles + kTWaves - 1) / kTWaves),
-                       dim3(kGBlock), 0, st, trays, tpaths, z.nang_sub * z.maxc, z.ntiles, tcount);
-  }
-  // each tile's rays with a non-zero bin in this call
-  hipLaunchKernelGGL(tile_live_kernel, dim3((z.ntiles + kTWaves - 1) / kTWaves), dim3(kGBlock), 0,
-                     st, (const TileRay*)trays, (const int*)tcount, (const int*)nzp,
-                     z.nang_sub * z.maxc, z.ntiles, live, nlive);
-  const int zs = tile_slab_depth(p);
-  const int nslab = (g.nz + zs - 1) / zs;
-  const dim3 grid((unsigned)((nitems + kTWaves - 1) / kTWaves));
-  if (list && geo_ready)
-    hipLaunchKernelGGL(tile_bp_kernel<true>, grid, dim3(kGBlock), tile_lds_bytes(p, true), st, A, zs,
-                       nslab, p->d_tile_order, nitems, nzp + z.npair, (const TileRay*)trays,
-                       (const TilePath*)tpaths, z.nang_sub * z.maxc, (const int*)live,
-                       (const int*)nlive, (const int*)q.loff, (const long long*)q.lbase, list);
-  else
-    hipLaunchKernelGGL(tile_bp_kernel<false>, grid, dim3(kGBlock), tile_lds_bytes(p, false), st, A, zs,
-                       nslab, p->d_tile_order, nitems, nzp + z.npair, (const TileRay*)trays,
-                       (const TilePath*)tpaths, z.nang_sub * z.maxc, (const int*)live,
-                       (const int*)nlive, (const int*)nullptr, (const long long*)nullptr,
-                       (const unsigned short*)nullptr);
+  // the subset's geometry: the rays of every tile with their paths
+  if (!geo_ready)
+    hipLaunchKernelGGL(tile_rays_kernel, dim3(z.ntiles), dim3(kGBlock), 0, st, A, z.maxc, z.nslot,
+                       q.rays, q.pairs, q.count);
+  // the call's axial records with their bin values, and the (angle, r) with a non-zero bin
+  hipLaunchKernelGGL(tile_zsetup_kernel, dim3((g.nr + kTZBins - 1) / kTZBins, z.nang_sub),
+                     dim3(kGBlock), 0, st, A, zr, nzmask, nzp);
+  hipLaunchKernelGGL(tile_bp_kernel, dim3((unsigned)(z.ntiles * z.nslab * z.nchunk)), dim3(kWave),
+                     tile_lds_bytes(z.zs), st, A, z.zs, z.nslab, z.nchunk, p->d_tile_order,
+                     (const TileRay*)q.rays, (const int*)q.pairs, (const int*)q.count, z.nslot,
+                     (const TileZ*)zr, (const unsigned*)nzmask, p->d_zinc, parts);
+  if (parts)
+    hipLaunchKernelGGL(tile_reduce_kernel, dim3(ggrid(z.nvox)), dim3(kGBlock), 0, st, A, z.nvox,
+                       z.nchunk, (const double*)parts);
   return hipGetLastError();
 }
 
@@ -2145,13 +1975,9 @@ void gather_args_for(const apirl_plan* p, int subset, int nsubsets, int kind, co
   A.upd_strict = 0;
 }
 
-hipError_t launch_group_gather(BatchHeader* hdr, const ZsJob* zs, const GJob* g2,
-                               const GJob* g3, int grid, int max_nsino, hipStream_t st) {
-  hipLaunchKernelGGL(zsetup_group_kernel, dim3(grid), dim3(kGBlock), 0, st, hdr, zs);
+hipError_t launch_group_gather(BatchHeader* hdr, const GJob* jobs, int grid, hipStream_t st) {
   hipLaunchKernelGGL(gather2_group_kernel, dim3(grid), dim3(kG2Waves * kWave),
-                     kG2LdsFloats * sizeof(float), st, hdr, g2);
-  hipLaunchKernelGGL(gather3_group_kernel, dim3(grid), dim3(kGBlock),
-                     column_lds_bytes(max_nsino), st, hdr, g3);
+                     kG2LdsFloats * sizeof(float), st, hdr, jobs);
   return hipGetLastError();
 }
 

@@ -758,16 +758,25 @@ __global__ __launch_bounds__(kBlock) void sum_partials_kernel(const double* __re
 }
 
 // Minimum of the non-zero values and maximum (Images.cpp:397-431).  Both are
-// order-independent, so the result is exact.  out[0] = min_nz, out[1] = max; the
-// reference's maximum starts from pixel 0, so a NaN there is kept (out[2] flags it).
+// order-independent, so the result is exact.  A launch of one workgroup gives out[0] = min_nz,
+// out[1] = max; the reference's maximum starts from pixel 0, so a NaN there is kept.  A launch
+// of more leaves a pair per workgroup after them, which a second launch of one takes in place
+// of x (pairs > 0).  One workgroup took 5.7 ms for 256x256x81 voxels, the two launches TT us.
 __global__ __launch_bounds__(kBlock) void min_nz_max_kernel(const float* __restrict__ x, long n,
-                                                            float* __restrict__ out) {
+                                                            float* __restrict__ out, int pairs) {
   __shared__ float smin[kBlock], smax[kBlock];
   float mn = FLT_MAX, mx = -FLT_MAX;
-  for (long i = threadIdx.x; i < n; i += kBlock) {
-    const float v = x[i];
-    if (v != 0.f && v < mn) mn = v;
-    if (v > mx) mx = v;
+  if (pairs > 0) {
+    for (int i = threadIdx.x; i < pairs; i += kBlock) {
+      mn = fminf(mn, out[2 + 2 * i]);
+      mx = fmaxf(mx, out[3 + 2 * i]);
+    }
+  } else {
+    for (long i = (long)blockIdx.x * kBlock + threadIdx.x; i < n; i += (long)gridDim.x * kBlock) {
+      const float v = x[i];
+      if (v != 0.f && v < mn) mn = v;
+      if (v > mx) mx = v;
+    }
   }
   smin[threadIdx.x] = mn;
   smax[threadIdx.x] = mx;
@@ -780,8 +789,13 @@ __global__ __launch_bounds__(kBlock) void min_nz_max_kernel(const float* __restr
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    out[0] = smin[0];
-    out[1] = (x[0] > smax[0] || x[0] != x[0]) ? x[0] : smax[0];
+    if (gridDim.x > 1) {
+      out[2 + 2 * blockIdx.x] = smin[0];
+      out[3 + 2 * blockIdx.x] = smax[0];
+    } else {
+      out[0] = smin[0];
+      out[1] = (x[0] > smax[0] || x[0] != x[0]) ? x[0] : smax[0];
+    }
   }
 }
 
@@ -892,60 +906,19 @@ static_assert(kGroupBlock == kBlock, "grouped launches use the projector's block
 // Grouped-launch helpers (also used by gather_kernels.hip through group_common.h).
 #include "group_common.h"
 
-__global__ __launch_bounds__(kBlock) void clear_group_kernel(BatchHeader* __restrict__ hdr,
-                                                             const ClearJob* __restrict__ jobs) {
-  const int n = hdr->count[PH_CLEAR];
-  const long total = hdr->total[PH_CLEAR];
-  const int grab = grab_size(hdr);
-  for (;;) {
-    const long v0 = grab_vb(&hdr->next[PH_CLEAR], grab);
-    if (v0 >= total) break;
-    for (long vb = v0; vb < v0 + grab && vb < total; vb++) {
-      const ClearJob& J = jobs[find_job(jobs, n, vb)];
-      const long i = (vb - J.first) * kBlock + threadIdx.x;
-      if (i < J.n) J.p[i] = 0.f;
-    }
-  }
-}
-
-template <int DIMS>
 __global__ __launch_bounds__(kBlock) void project_group_kernel(BatchHeader* __restrict__ hdr,
                                                                const ProjJob* __restrict__ jobs) {
-  const int ph = DIMS == 2 ? PH_PROJ2 : PH_PROJ3;
-  const int n = hdr->count[ph];
-  const long total = hdr->total[ph];
+  const int n = hdr->count[PH_PROJ2];
+  const long total = hdr->total[PH_PROJ2];
   const int grab = grab_size(hdr);
-  for (;;) {
-    const long v0 = grab_vb(&hdr->next[ph], grab);
-    if (v0 >= total) break;
+  for (long v0 = first_vb(grab); v0 < total; v0 = next_vb(&hdr->next[PH_PROJ2], grab, total))
     for (long vb = v0; vb < v0 + grab && vb < total; vb++) {
       const ProjJob& J = jobs[find_job(jobs, n, vb)];
       const long lidx = (vb - J.first) * kBlock + threadIdx.x;
-      (void)project_ray<APIRL_PREC_REFERENCE, true, DIMS>(J.g, J.rays, J.zab, J.img, nullptr,
-                                                          J.nang_sub, J.subset, J.nsubsets,
-                                                          J.nrays, J.fr, J.zorder, nullptr, lidx);
+      (void)project_ray<APIRL_PREC_REFERENCE, true, 2>(J.g, J.rays, nullptr, J.img, nullptr,
+                                                       J.nang_sub, J.subset, J.nsubsets, J.nrays,
+                                                       J.fr, nullptr, nullptr, lidx);
     }
-  }
-}
-
-__global__ __launch_bounds__(kBlock) void update_group_kernel(BatchHeader* __restrict__ hdr,
-                                                              const UpdJob* __restrict__ jobs) {
-  const int n = hdr->count[PH_UPDATE];
-  const long total = hdr->total[PH_UPDATE];
-  const int grab = grab_size(hdr);
-  for (;;) {
-    const long v0 = grab_vb(&hdr->next[PH_UPDATE], grab);
-    if (v0 >= total) break;
-    for (long vb = v0; vb < v0 + grab && vb < total; vb++) {
-      const UpdJob& J = jobs[find_job(jobs, n, vb)];
-      const long i = (vb - J.first) * kBlock + threadIdx.x;
-      if (i < J.n) {
-        const float sv = J.s[i];
-        const bool ok = J.strict ? (sv > J.thr) : (sv >= J.thr);
-        J.x[i] = ok ? J.x[i] * J.b[i] / sv : 0.f;
-      }
-    }
-  }
 }
 
 inline unsigned grid_for(long n) { return (unsigned)((n + kBlock - 1) / kBlock); }
@@ -1326,8 +1299,9 @@ int project_partials(const apirl_plan* p, int subset, int nsubsets, bool path) {
 
 hipError_t launch_project(const apirl_plan* p, const float* img, float* sino, int subset,
                           int nsubsets, int precision, const FusedRatio* fused, int* nblocks_out,
-                          hipStream_t st) {
+                          hipStream_t st, float* image_copy) {
   const Geo& g = p->geo;
+  float* const copy = image_copy ? image_copy : p->d_imgT;
   const int nang_sub = subset_num_angles(g.nang, nsubsets, subset);
   const long nrays = (long)g.nsino * nang_sub * g.nr;
   const unsigned grid = grid_for(nrays);
@@ -1341,13 +1315,13 @@ hipError_t launch_project(const apirl_plan* p, const float* img, float* sino, in
     const int npair = nang_sub * g.nr, qmax = fwd_path_len(g), pitch = path_pitch(g);
     if (nblocks_out) *nblocks_out = npair;
     const dim3 tg((g.nx + 31) / 32, g.ny, (pitch + 31) / 32);
-    hipLaunchKernelGGL(transpose_zfast_kernel, tg, dim3(kBlock), 0, st, img, p->d_imgT, g.nx,
+    hipLaunchKernelGGL(transpose_zfast_kernel, tg, dim3(kBlock), 0, st, img, copy, g.nx,
                        g.ny, g.nz, pitch);
     const size_t lds = fwd_path_lds(g);  // 10.4 KB for 256 x 256
     const dim3 wg(64 * fwd_path_waves(g));
 #define APIRL_LAUNCH_PATHS(F, PR)                                                             \
   hipLaunchKernelGGL((project_paths_kernel<F, PR>), dim3(npair), wg, lds, st, g, p->d_rays,   \
-                     p->d_zab, img, p->d_imgT, sino, nang_sub, subset, nsubsets, fr, qmax, pitch)
+                     p->d_zab, img, copy, sino, nang_sub, subset, nsubsets, fr, qmax, pitch)
     if (precision == APIRL_PREC_KAHAN) {
       if (f) APIRL_LAUNCH_PATHS(true, APIRL_PREC_KAHAN);
       else APIRL_LAUNCH_PATHS(false, APIRL_PREC_KAHAN);
@@ -1362,10 +1336,10 @@ hipError_t launch_project(const apirl_plan* p, const float* img, float* sino, in
     return hipGetLastError();
   }
   const float* imgT = nullptr;
-  if (p->d_imgT && precision == APIRL_PREC_REFERENCE) {
+  if (copy && precision == APIRL_PREC_REFERENCE) {
     const dim3 tg((g.nx + 31) / 32, (g.ny + 31) / 32, g.nz);
-    hipLaunchKernelGGL(transpose_xy_kernel, tg, dim3(kBlock), 0, st, img, p->d_imgT, g.nx, g.ny);
-    imgT = p->d_imgT;
+    hipLaunchKernelGGL(transpose_xy_kernel, tg, dim3(kBlock), 0, st, img, copy, g.nx, g.ny);
+    imgT = copy;
   }
 #define APIRL_LAUNCH_PROJ3(PR, D)                                                           \
   if (f)                                                                                   \
@@ -1499,28 +1473,21 @@ hipError_t launch_likelihood(const float* x, const float* y, long n, int positiv
   return hipGetLastError();
 }
 
-hipError_t launch_min_nz_max(const float* x, size_t n, float* d_out2, hipStream_t st) {
+hipError_t launch_min_nz_max(const float* x, size_t n, float* d_out, hipStream_t st) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(min_nz_max_kernel, dim3(1), dim3(kBlock), 0, st, x, (long)n, d_out2);
+  // 16 values per thread and workgroup; up to two workgroups' worth in one launch
+  const size_t blocks = (n + 16 * kBlock - 1) / (16 * kBlock);
+  int pairs = 0;
+  if (blocks > 2) {
+    pairs = (int)(blocks < (size_t)kMinMaxBlocks ? blocks : (size_t)kMinMaxBlocks);
+    hipLaunchKernelGGL(min_nz_max_kernel, dim3(pairs), dim3(kBlock), 0, st, x, (long)n, d_out, 0);
+  }
+  hipLaunchKernelGGL(min_nz_max_kernel, dim3(1), dim3(kBlock), 0, st, x, (long)n, d_out, pairs);
   return hipGetLastError();
 }
 
-hipError_t launch_group_clear(BatchHeader* hdr, const ClearJob* jobs, int grid,
-                              hipStream_t st) {
-  hipLaunchKernelGGL(clear_group_kernel, dim3(grid), dim3(kBlock), 0, st, hdr, jobs);
-  return hipGetLastError();
-}
-
-hipError_t launch_group_project(BatchHeader* hdr, const ProjJob* jobs2,
-                                const ProjJob* jobs3, int grid, hipStream_t st) {
-  hipLaunchKernelGGL(project_group_kernel<2>, dim3(grid), dim3(kBlock), 0, st, hdr, jobs2);
-  hipLaunchKernelGGL(project_group_kernel<3>, dim3(grid), dim3(kBlock), 0, st, hdr, jobs3);
-  return hipGetLastError();
-}
-
-hipError_t launch_group_update(BatchHeader* hdr, const UpdJob* jobs, int grid,
-                               hipStream_t st) {
-  hipLaunchKernelGGL(update_group_kernel, dim3(grid), dim3(kBlock), 0, st, hdr, jobs);
+hipError_t launch_group_project(BatchHeader* hdr, const ProjJob* jobs, int grid, hipStream_t st) {
+  hipLaunchKernelGGL(project_group_kernel, dim3(grid), dim3(kBlock), 0, st, hdr, jobs);
   return hipGetLastError();
 }
 
