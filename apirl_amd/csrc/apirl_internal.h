@@ -229,15 +229,14 @@ struct FusedRatio {
   // Sinogram3D::addBinToBin (Sinogram3D.cpp:857-873) reads it
   int additive_local = 0;
 };
-// 3D, reference precision, one LOR per bin (path_forward_ok): the path forward
-// projector, which writes project_partials(.., true) likelihood partials (one per
-// subset (angle, bin)) instead of one per 256 bins.
+// 3D, one LOR per bin (path_forward_ok): the path forward projector, which writes
+// project_partials(.., true) likelihood partials (one per workgroup) instead of one per 256 bins.
 // image_copy: where the projector's copy of the image goes (path_image_floats floats in 3D,
 // the image's in 2D) instead of the plan's own buffer, for work on a stream of its own.
 hipError_t launch_project(const apirl_plan* p, const float* img, float* sino, int subset,
                           int nsubsets, int precision, const FusedRatio* fused, int* nblocks_out,
                           hipStream_t st, float* image_copy = nullptr);
-bool path_forward_ok(const apirl_plan* p, int precision);
+bool path_forward_ok(const apirl_plan* p, int precision, int subset, int nsubsets);
 // Floats of the path forward projector's z-fastest image copy (apirl_plan::d_imgT).
 size_t path_image_floats(const Geo& g);
 int project_partials(const apirl_plan* p, int subset, int nsubsets, bool path);

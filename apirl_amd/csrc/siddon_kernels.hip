@@ -949,7 +949,9 @@ inline unsigned grid_for(long n) { return (unsigned)((n + kBlock - 1) / kBlock);
 // ms (3.3e8 VALU wave-instructions, 0.54 ms of issue); the whole 192x192x233 sinogram of
 // a 128x128x47 image: 1.24 -> 0.74 ms; F64_SETUP, 12 angles of 344x252x357 on 172x172x65:
 // 0.26 -> 0.22 ms.  Stepping every lane by itself with the same 12 instructions a step
-// measured 0.74, 0.80 and 0.23 ms; 6 columns a batch 0.68, 0.75 and 0.22 ms.
+// measured 0.74, 0.80 and 0.23 ms; 6 columns a batch 0.68, 0.75 and 0.22 ms.  The merge looks
+// for a crossing's place from the line through the other chain: 0.74 -> 0.71 ms for the second
+// (a binary search).
 
 struct FwdStep {
   float ae;       // alpha at which the loop leaves this column by an x or y step
@@ -972,11 +974,30 @@ inline size_t fwd_path_lds(const Geo& g) {
   return 2 * sizeof(FwdStep) +
          (size_t)(fwd_path_len(g) + 1) * (sizeof(FwdStep) + sizeof(int) + 2 * sizeof(float));
 }
-// Wavefronts of project_paths_kernel's workgroup: four, or fewer when that many passes of
-// 64 sinograms do not need four (73 sinograms: two; 357: three, two passes each).
-inline int fwd_path_waves(const Geo& g) {
-  const int passes = (g.nsino + 63) / 64, rounds = (passes + 3) / 4;
-  return (passes + rounds - 1) / rounds;
+// How project_paths_kernel's sinograms are shared out: chunk of them a workgroup, parts workgroups
+// a pair. Each workgroup builds the path, so a pair takes one of at most four wavefronts, which
+// take their sinograms 64 at a time in turn (73 sinograms: two wavefronts; 357: three, two turns
+// each), unless the launch would leave part of the chip's kPathResident wavefronts idle: then in
+// fewer turns by more of them (557 sinograms of 2 x 96 bins, 65 -> 40 us; 265 of 4 x 61, 58 -> 44;
+// launches that fill the chip lose nothing or 3 % by it). Where all workgroups run at once even
+// with four wavefronts each, they have four to build the path with (nsino <= 64, 3 x 172 bins of
+// a 252 x 252 image, 97 -> 70 us; with 5000 pairs it is 55 -> 74).
+struct PathSplit {
+  int waves, chunk, parts;
+};
+constexpr int kPathResident = 8192;
+inline PathSplit fwd_path_split(const Geo& g, int npair) {
+  const int passes = (g.nsino + 63) / 64, most = (passes + 3) / 4;
+  const long fill = ((long)npair * passes + kPathResident - 1) / kPathResident;
+  const int turns = fill < most ? (fill > 0 ? (int)fill : 1) : most;
+  const int waves = (passes + turns - 1) / turns;  // of a pair
+  PathSplit s;
+  s.parts = (waves + 3) / 4;
+  s.waves = (waves + s.parts - 1) / s.parts;
+  s.chunk = s.waves * turns * 64;
+  s.parts = (g.nsino + s.chunk - 1) / s.chunk;
+  if ((long)npair * s.parts * 4 <= kPathResident) s.waves = 4;
+  return s;
 }
 
 // out[(j nx + i) pitch + kPathGuard + k] = in[(k ny + j) nx + i] through a 32 (i) x 32 (k)
@@ -1004,7 +1025,7 @@ template <bool FUSED, int PREC>
 __global__ __launch_bounds__(kBlock, PREC == APIRL_PREC_REFERENCE ? 8 : 7) void project_paths_kernel(
     Geo g, const RayXY* __restrict__ rays, const float2* __restrict__ zab,
     const float* __restrict__ img, const float* __restrict__ imgZ, float* __restrict__ sino,
-    int nang_sub, int subset, int nsubsets, FusedRatio fr, int qmax, int pitch) {
+    int nang_sub, int subset, int nsubsets, FusedRatio fr, int qmax, int pitch, int chunk) {
   constexpr bool kSum2 = PREC != APIRL_PREC_REFERENCE;     // Kahan-compensated sum
   constexpr bool kStrict = PREC == APIRL_PREC_F64_SETUP;   // in-image voxels only
   extern __shared__ __align__(16) FwdStep sraw[];
@@ -1063,19 +1084,19 @@ __global__ __launch_bounds__(kBlock, PREC == APIRL_PREC_REFERENCE ? 8 : 7) void 
     sp[-1].ae = PREC == APIRL_PREC_F64_SETUP ? (float)xy64.amin : t.amin;
   }
   __syncthreads();
+  const float inv_xu = 1.f / t.axu, inv_yu = 1.f / t.ayu;
   for (int c = threadIdx.x; c < 2 * (qmax + 1); c += nt) {
     const bool isx = c <= qmax;
     const int m = isx ? c : c - (qmax + 1);
     const float v = isx ? xs[m] : ys[m];
     const float* other = isx ? ys : xs;
-    int lo = 0, hi = qmax + 1;  // other[0 .. lo) come before v
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      const float o = other[mid];
-      const bool before = isx ? (o < v) : (o <= v);
-      lo = before ? mid + 1 : lo;
-      hi = before ? hi : mid;
-    }
+    // other[0 .. lo) come before v: the chains are lines but for their rounding, so the count
+    // is the line's or one beside it
+    const float e = (v - (isx ? t.ay : t.ax)) * (isx ? inv_yu : inv_xu) + 1.f;
+    int lo = e > 0.f ? (e < (float)(qmax + 1) ? (int)e : qmax + 1) : 0;
+    if (isx ? other[qmax] < v : other[qmax] <= v) lo = qmax + 1;  // v may be an infinity
+    while (lo > 0 && !(isx ? other[lo - 1] < v : other[lo - 1] <= v)) lo--;
+    while (lo <= qmax && (isx ? other[lo] < v : other[lo] <= v)) lo++;
     const int q = m + lo;
     if (q <= qmax) {
       const int mx = isx ? m : lo, my = isx ? lo : m;
@@ -1103,7 +1124,8 @@ __global__ __launch_bounds__(kBlock, PREC == APIRL_PREC_REFERENCE ? 8 : 7) void 
   const char* const zbytes = (const char*)imgZ;
   const int nxy = g.nx * g.ny, npix = nxy * g.nz;
   double lik = 0.0;
-  for (int s = threadIdx.x; s < g.nsino; s += nt) {
+  const int s0 = (int)blockIdx.y * chunk, s1 = s0 + chunk < g.nsino ? s0 + chunk : g.nsino;
+  for (int s = s0 + (int)threadIdx.x; s < s1; s += nt) {
     const float2 zz = zab[s];
     Ray ray;
     bool valid = setup_ray<3>(g, t, zz.x, zz.y, ray);
@@ -1272,14 +1294,28 @@ __global__ __launch_bounds__(kBlock, PREC == APIRL_PREC_REFERENCE ? 8 : 7) void 
       for (int i = threadIdx.x; i < off; i += nt) red[i] += red[i + off];
       __syncthreads();
     }
-    if (threadIdx.x == 0) fr.lik_partials[blockIdx.x] = red[0];
+    if (threadIdx.x == 0) fr.lik_partials[blockIdx.y * gridDim.x + blockIdx.x] = red[0];
   }
 }
 
 }  // namespace
 
-bool path_forward_ok(const apirl_plan* p, int precision) {
+// KAHAN and F64_SETUP walk the path with more work a column than the reference arithmetic, and a
+// ray per lane has no path to build: that is ahead where few sinograms share one (ray per lane /
+// path at 23 sinograms 137 / 341 us, at 35 84 / 146) and where the whole launch is short, by its
+// rays times the columns of a long one: 61 / 70 us at 5e7, 54 / 61 at 7e7, 60 / 63 at 9e7, against
+// 96 / 96 at 1.4e8, 111 / 98 at 1.5e8, 217 / 110 at 2.0e8, 686 / 431 at 1.0e9 (113 sinograms).
+// The reference arithmetic is ahead on the path at any number (80 / 52 us at 19 sinograms,
+// 372 / 158 at 47).
+constexpr int kPathMinSino = 112;
+constexpr double kPathMinWork = 1.0e8;
+
+bool path_forward_ok(const apirl_plan* p, int precision, int subset, int nsubsets) {
   const Geo& g = p->geo;
+  if (precision != APIRL_PREC_REFERENCE) {
+    const double rays = (double)g.nsino * subset_num_angles(g.nang, nsubsets, subset) * g.nr;
+    if (g.nsino <= kPathMinSino || rays * (g.nx + g.ny) < kPathMinWork) return false;
+  }
   // the columns of an entry are kept in 16 bits each, a voxel's byte address in 32
   return g.dims == 3 && precision != APIRL_PREC_F64_ALPHA && g.ns * g.nas == 1 && g.walk24 &&
          g.nx < 16384 && g.ny < 16384 && p->d_imgT != nullptr &&
@@ -1293,7 +1329,7 @@ size_t path_image_floats(const Geo& g) {
 int project_partials(const apirl_plan* p, int subset, int nsubsets, bool path) {
   const Geo& g = p->geo;
   const int nang_sub = subset_num_angles(g.nang, nsubsets, subset);
-  if (path) return nang_sub * g.nr;
+  if (path) return nang_sub * g.nr * fwd_path_split(g, nang_sub * g.nr).parts;
   return (int)grid_for((long)g.nsino * nang_sub * g.nr);
 }
 
@@ -1309,19 +1345,21 @@ hipError_t launch_project(const apirl_plan* p, const float* img, float* sino, in
   if (nrays == 0) return hipSuccess;
   FusedRatio fr = fused ? *fused : FusedRatio{};
   const bool f = fused != nullptr;
-  if (path_forward_ok(p, precision)) {
+  if (path_forward_ok(p, precision, subset, nsubsets)) {
     // the path forward projector: the image with z fastest (into the plan's
     // transposed-image buffer), one workgroup per (angle, bin) of the subset
     const int npair = nang_sub * g.nr, qmax = fwd_path_len(g), pitch = path_pitch(g);
-    if (nblocks_out) *nblocks_out = npair;
+    const PathSplit sp = fwd_path_split(g, npair);
+    if (nblocks_out) *nblocks_out = npair * sp.parts;
     const dim3 tg((g.nx + 31) / 32, g.ny, (pitch + 31) / 32);
     hipLaunchKernelGGL(transpose_zfast_kernel, tg, dim3(kBlock), 0, st, img, copy, g.nx,
                        g.ny, g.nz, pitch);
     const size_t lds = fwd_path_lds(g);  // 10.4 KB for 256 x 256
-    const dim3 wg(64 * fwd_path_waves(g));
+    const dim3 wg(64 * sp.waves);
 #define APIRL_LAUNCH_PATHS(F, PR)                                                             \
-  hipLaunchKernelGGL((project_paths_kernel<F, PR>), dim3(npair), wg, lds, st, g, p->d_rays,   \
-                     p->d_zab, img, copy, sino, nang_sub, subset, nsubsets, fr, qmax, pitch)
+  hipLaunchKernelGGL((project_paths_kernel<F, PR>), dim3(npair, sp.parts), wg, lds, st, g,    \
+                     p->d_rays, p->d_zab, img, copy, sino, nang_sub, subset, nsubsets, fr,    \
+                     qmax, pitch, sp.chunk)
     if (precision == APIRL_PREC_KAHAN) {
       if (f) APIRL_LAUNCH_PATHS(true, APIRL_PREC_KAHAN);
       else APIRL_LAUNCH_PATHS(false, APIRL_PREC_KAHAN);
