@@ -229,8 +229,7 @@ struct FusedRatio {
   // Sinogram3D::addBinToBin (Sinogram3D.cpp:857-873) reads it
   int additive_local = 0;
 };
-// 3D, one LOR per bin (path_forward_ok): the path forward projector, which writes
-// project_partials(.., true) likelihood partials (one per workgroup) instead of one per 256 bins.
+// The fused form writes project_partials likelihood partials, one per workgroup.
 // image_copy: where the projector's copy of the image goes (path_image_floats floats in 3D,
 // the image's in 2D) instead of the plan's own buffer, for work on a stream of its own.
 hipError_t launch_project(const apirl_plan* p, const float* img, float* sino, int subset,
@@ -239,7 +238,7 @@ hipError_t launch_project(const apirl_plan* p, const float* img, float* sino, in
 bool path_forward_ok(const apirl_plan* p, int precision, int subset, int nsubsets);
 // Floats of the path forward projector's z-fastest image copy (apirl_plan::d_imgT).
 size_t path_image_floats(const Geo& g);
-int project_partials(const apirl_plan* p, int subset, int nsubsets, bool path);
+int project_partials(const apirl_plan* p, int subset, int nsubsets, int precision);
 hipError_t launch_backproject(const apirl_plan* p, const float* sino, const float* est,
                               float* img, int subset, int nsubsets, int kind, int mode,
                               hipStream_t st);
@@ -428,8 +427,9 @@ struct GJob {  // gather backprojection of one subset with the update fused in (
   int ntx, nty;
   long first;
 };
-constexpr int kGroupBlock = 256;  // threads per workgroup of the grouped launches
-inline long group_blocks(long n) { return (n + kGroupBlock - 1) / kGroupBlock; }
+constexpr int kGroupRays = 64;       // rays of a virtual block of the grouped projection
+constexpr int kGroupProject = 512;   // and its threads
+inline long group_blocks(long n) { return (n + kGroupRays - 1) / kGroupRays; }
 constexpr int kPatch2 = 8;  // the 2D gather's voxel patches are kPatch2 x kPatch2
 inline long gather_patches(const Geo& g) {
   return (long)((g.nx + kPatch2 - 1) / kPatch2) * ((g.ny + kPatch2 - 1) / kPatch2);

@@ -1044,8 +1044,7 @@ apirl_status project_ratio_impl(apirl_plan* p, const float* d_img, const float* 
   if (!os_precision_ok(p, precision))
     return fail(c, APIRL_ERR_UNSUPPORTED, "oversampled LORs use the reference precision");
   DeviceGuard g(c->device);
-  const int nblocks = apirl::project_partials(
-      p, subset, nsubsets, apirl::path_forward_ok(p, precision, subset, nsubsets));
+  const int nblocks = apirl::project_partials(p, subset, nsubsets, precision);
   apirl::FusedRatio fr;
   fr.meas = d_meas;
   fr.additive = d_additive;

@@ -583,6 +583,178 @@ __global__ __launch_bounds__(kBlock) void project_kernel(
   }
 }
 
+// ---- 2D forward projector, reference arithmetic -------------------------------------
+//
+// A workgroup takes 64 rays, one per lane of each of its wavefronts, and every wavefront
+// kSeg2 of their steps per round: it starts a ray at its first step from the closed form of
+// the crossings' additions (alpha_exact.h), so the wavefronts walk at the same time, then they
+// add their terms to the rays' sums in turn, which are the reference's sums, bit for bit.
+// One ray per lane waits for its own loads and additions, and a 2D sinogram has few rays
+// (192 x 192: 576 wavefronts, of 256 steps).  Whole calls, their 19 us of host work included:
+// 192 x 192 bins of a 128 x 128 image 39 -> 25 us, 24 x 40 of 256 x 256 73 -> 26, 252 x 344 of
+// 128 x 128 45 -> 42, of 256 x 256 78 -> 65, of 512 x 512 149 -> 123.  32 steps a turn measured
+// 29, 27, 52, 87 and 163 us.
+constexpr int kSeg2 = 16;  // steps of a wavefront per round
+// Wavefronts of the workgroup: at most 16 where the launch's workgroups then run at once (two
+// a CU), otherwise 8, whose turns at the sums are shorter.
+constexpr int kSeg2Waves = 16;
+inline int seg2_waves(const Geo& g, long blocks) {
+  const int segs = (g.nx + g.ny + kSeg2 - 1) / kSeg2, most = blocks <= 512 ? kSeg2Waves : 8;
+  return segs < most ? segs : most;
+}
+
+// The state of the loop after q of the ray's steps: X and Y, the pending crossings; ac, the
+// last one taken; m, the x steps among the q.
+__device__ __forceinline__ void xy_state_at(const Ray& r, int q, float& X, float& Y, float& ac,
+                                            int& m) {
+  X = r.ax;
+  Y = r.ay;
+  ac = r.ac;
+  m = 0;
+  if (q <= 0) return;
+  bool done = false;
+  if (r.ax == r.ax && r.ay == r.ay) {
+    // x steps among q, on the lines that the chains of additions round; then moved to where the
+    // loop's rule holds: the last x step came at or before the pending Y, the last y step
+    // before the pending X
+    const float e = ((float)(q - 1) * r.ayu + (r.ay - r.ax)) / (r.axu + r.ayu) + 0.5f;
+    int c = !(r.axu < 3.0e38f) ? 0 : (!(r.ayu < 3.0e38f) ? q : (e > 0.f ? (int)(e + 0.5f) : 0));
+    c = c < q ? c : q;
+    for (int t = 0; t <= q; t++) {
+      const int k = q - c;
+      const float Xp = c > 0 ? alpha_after(r.ax, r.axu, c - 1) : 0.f;
+      const float Yp = k > 0 ? alpha_after(r.ay, r.ayu, k - 1) : 0.f;
+      X = c > 0 ? Xp + r.axu : r.ax;
+      Y = k > 0 ? Yp + r.ayu : r.ay;
+      if (c > 0 && !(Xp <= Y)) {
+        c--;
+      } else if (k > 0 && !(Yp < X)) {
+        c++;
+      } else {
+        m = c;
+        ac = c == 0 ? Yp : (k == 0 || Xp > Yp ? Xp : Yp);
+        done = ac <= FLT_MAX;
+        break;
+      }
+    }
+  }
+  if (!done) {  // crossings that are not numbers: step by step
+    Ray w = r;
+    int ci, cj, ck;
+    for (int t = 0; t < q; t++) (void)step(w, ci, cj, ck);
+    X = w.ax;
+    Y = w.ay;
+    ac = w.ac;
+    m = r.iinc ? (w.i - r.i) * r.iinc : 0;
+  }
+}
+
+// 64 rays of a subset projection from ray l0, by the whole workgroup (nw wavefronts; part: 64
+// floats of LDS).  Returns the likelihood term of the ray of this lane in wavefront 0.
+template <bool FUSED>
+__device__ __forceinline__ double project2_rays(
+    const Geo& g, const RayXY* __restrict__ rays, const float* __restrict__ img,
+    const float* __restrict__ imgT, float* __restrict__ sino, int nang_sub, int subset,
+    int nsubsets, long nrays, const FusedRatio& fr, long l0, float* part) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+  const long lidx = l0 + lane;
+  const bool on = lidx < nrays;
+  const int l = (int)(on ? lidx : l0);
+  const int rr = l % g.nr, ka = l / g.nr, a = subset + nsubsets * ka;
+  const RayXY t = rays[(long)a * g.nr + rr];
+  Ray ray;
+  const bool valid = setup_ray<2>(g, t, 0.f, 0.f, ray);
+  const int n = on && valid ? ray.n : 0;
+  int nmax = n;
+#pragma unroll
+  for (int d = 32; d; d >>= 1) {
+    const int o = __shfl_xor(nmax, d);
+    nmax = o > nmax ? o : nmax;
+  }
+  const int nxy = g.nx * g.ny;
+  const bool tr = imgT != nullptr && (t.flags & RAY_XMAJOR);
+  float acc = 0.f;
+  for (int b = 0; b < nmax; b += nw * kSeg2) {
+    const int q = b + wave * kSeg2;
+    float term[kSeg2];
+    if (q < nmax) {
+      float X, Y, ac;
+      int m;
+      xy_state_at(ray, q < n ? q : 0, X, Y, ac, m);
+      int i = ray.i + m * ray.iinc, j = ray.j + ((q < n ? q : 0) - m) * ray.jinc;
+      float wv[kSeg2];
+#pragma unroll
+      for (int u = 0; u < kSeg2; u++) {
+        const bool bx = X <= Y;
+        const float an = bx ? X : Y;
+        wv[u] = (an - ac) * ray.L;
+        ac = an;
+        const float nX = X + ray.axu, nY = Y + ray.ayu;
+        X = bx ? nX : X;
+        Y = bx ? Y : nY;
+        // the reference's read test (Siddon.cpp's 2D list, SiddonProjector.cpp:50-77): columns
+        // past the last read the next row
+        const int li = __mul24(j, g.nx) + i;
+        const bool ok = (i >= 0) & (j >= 0) & (li < nxy) & (q + u < n);
+        const bool T = tr & (i < g.nx);
+        const float* const src = T ? imgT : img;
+        term[u] = src[(unsigned)(ok ? (T ? __mul24(i, g.ny) + j : li) : 0)];
+        wv[u] = ok ? wv[u] : 0.f;
+        term[u] = ok ? term[u] : 0.f;
+        i += bx ? ray.iinc : 0;
+        j += bx ? 0 : ray.jinc;
+      }
+#pragma unroll
+      for (int u = 0; u < kSeg2; u++) term[u] = 1.0f * wv[u] * term[u];
+    }
+    // a term that is not the reference's is 0, which leaves the sum (never -0) as it is
+    for (int w = 0; w < nw && b + w * kSeg2 < nmax; w++) {
+      if (wave == w) {
+        acc = b + w > 0 ? part[lane] : 0.f;
+#pragma unroll
+        for (int u = 0; u < kSeg2; u++) acc = acc + term[u];
+        part[lane] = acc;
+      }
+      __syncthreads();
+    }
+  }
+  double lik = 0.0;
+  if (wave == 0 && on) {
+    if (nmax > 0) acc = part[lane];
+    const long idx = (long)ka * g.nr + rr;
+    if (!FUSED) {
+      if (valid) sino[idx] = acc;
+    } else {
+      // fused EM epilogue, as project_ray's (Sinogram2D.cpp:234-266, 565-581)
+      const long full = (long)a * g.nr + rr;
+      float est = valid ? acc : 0.f;
+      if (fr.additive) est = est + fr.additive[fr.additive_local ? idx : full];
+      const float y = fr.meas[full];
+      const bool lik_term = fr.lik_positive_only ? (est > 0.f) : (est != 0.f);
+      if (lik_term) lik = (double)(y * logf(est) - est);
+      fr.ratio[idx] = (y != 0.f && est != 0.f) ? y / est : 0.f;
+    }
+  }
+  return lik;
+}
+
+template <bool FUSED>
+__global__ __launch_bounds__(64 * kSeg2Waves, 8) void project2_kernel(
+    Geo g, const RayXY* __restrict__ rays, const float* __restrict__ img,
+    const float* __restrict__ imgT, float* __restrict__ sino, int nang_sub, int subset,
+    int nsubsets, long nrays, FusedRatio fr) {
+  __shared__ float part[64];
+  double lik = project2_rays<FUSED>(g, rays, img, imgT, sino, nang_sub, subset, nsubsets, nrays,
+                                    fr, (long)blockIdx.x * 64, part);
+  if (FUSED && fr.lik_partials && threadIdx.x < 64) {
+    // deterministic reduction of the likelihood partials (fixed tree)
+#pragma unroll
+    for (int d = 32; d; d >>= 1) lik += __shfl_down(lik, d);
+    if (threadIdx.x == 0) fr.lik_partials[blockIdx.x] = lik;
+  }
+}
+
 // Ray-driven scatter backprojection with fp32 atomics.
 //   BP_PLAIN : term = w * b; 3D skips b == 0 (SiddonProjector.cpp:496) with a full
 //              bounds check (:541-548); 2D keeps every bin (:50-77) and writes
@@ -901,23 +1073,23 @@ __global__ __launch_bounds__(kBlock) void transpose_xy_kernel(const float* __res
 }
 
 // ---- grouped (multi-job) launches --------------------------------------------
-static_assert(kGroupBlock == kBlock, "grouped launches use the projector's block size");
+static_assert(kGroupRays == 64, "a virtual block of a projection is project2_rays' 64 rays");
 
 // Grouped-launch helpers (also used by gather_kernels.hip through group_common.h).
 #include "group_common.h"
 
-__global__ __launch_bounds__(kBlock) void project_group_kernel(BatchHeader* __restrict__ hdr,
-                                                               const ProjJob* __restrict__ jobs) {
+// Each virtual block is 64 rays of one job.
+__global__ __launch_bounds__(kGroupProject, 8) void project_group_kernel(
+    BatchHeader* __restrict__ hdr, const ProjJob* __restrict__ jobs) {
+  __shared__ float part[64];
   const int n = hdr->count[PH_PROJ2];
   const long total = hdr->total[PH_PROJ2];
   const int grab = grab_size(hdr);
   for (long v0 = first_vb(grab); v0 < total; v0 = next_vb(&hdr->next[PH_PROJ2], grab, total))
     for (long vb = v0; vb < v0 + grab && vb < total; vb++) {
       const ProjJob& J = jobs[find_job(jobs, n, vb)];
-      const long lidx = (vb - J.first) * kBlock + threadIdx.x;
-      (void)project_ray<APIRL_PREC_REFERENCE, true, 2>(J.g, J.rays, nullptr, J.img, nullptr,
-                                                       J.nang_sub, J.subset, J.nsubsets, J.nrays,
-                                                       J.fr, nullptr, nullptr, lidx);
+      (void)project2_rays<true>(J.g, J.rays, J.img, nullptr, nullptr, J.nang_sub, J.subset,
+                                J.nsubsets, J.nrays, J.fr, (vb - J.first) * kGroupRays, part);
     }
 }
 
@@ -1326,11 +1498,27 @@ size_t path_image_floats(const Geo& g) {
   return (size_t)g.nx * g.ny * path_pitch(g) + kPathGuard;
 }
 
-int project_partials(const apirl_plan* p, int subset, int nsubsets, bool path) {
+// project2_kernel's launches: rays counted in 32 bits, one likelihood partial per 64 of them
+// (kNoallocPartials at the most).
+static bool split2_ok(const apirl_plan* p, int precision, long nrays) {
+  const Geo& g = p->geo;
+  return g.dims == 2 && precision == APIRL_PREC_REFERENCE && g.ns * g.nas == 1 && g.walk24 &&
+         nrays <= 64L * kNoallocPartials;
+}
+// Voxels from which project2_kernel reads a transposed copy for the rays along x: theirs then lie
+// in a few lines too, which pays for the copy where the image is beyond what the L1s keep
+// (512 x 512: 138 -> 123 us from 252 x 344 bins, 482 -> 432 from 720 x 700; 256 x 256: 65 / 65;
+// 128 x 128: 42 -> 44).
+constexpr long kTransposed2 = 1L << 17;
+
+int project_partials(const apirl_plan* p, int subset, int nsubsets, int precision) {
   const Geo& g = p->geo;
   const int nang_sub = subset_num_angles(g.nang, nsubsets, subset);
-  if (path) return nang_sub * g.nr * fwd_path_split(g, nang_sub * g.nr).parts;
-  return (int)grid_for((long)g.nsino * nang_sub * g.nr);
+  const long nrays = (long)g.nsino * nang_sub * g.nr;
+  if (path_forward_ok(p, precision, subset, nsubsets))
+    return nang_sub * g.nr * fwd_path_split(g, nang_sub * g.nr).parts;
+  if (split2_ok(p, precision, nrays)) return (int)((nrays + 63) / 64);
+  return (int)grid_for(nrays);
 }
 
 hipError_t launch_project(const apirl_plan* p, const float* img, float* sino, int subset,
@@ -1371,6 +1559,24 @@ hipError_t launch_project(const apirl_plan* p, const float* img, float* sino, in
       else APIRL_LAUNCH_PATHS(false, APIRL_PREC_REFERENCE);
     }
 #undef APIRL_LAUNCH_PATHS
+    return hipGetLastError();
+  }
+  if (split2_ok(p, precision, nrays)) {
+    const float* t2 = nullptr;
+    if (copy && (long)g.nx * g.ny >= kTransposed2) {
+      const dim3 tg((g.nx + 31) / 32, (g.ny + 31) / 32, 1);
+      hipLaunchKernelGGL(transpose_xy_kernel, tg, dim3(kBlock), 0, st, img, copy, g.nx, g.ny);
+      t2 = copy;
+    }
+    const unsigned nb = (unsigned)((nrays + 63) / 64);
+    const dim3 wg(64 * seg2_waves(g, nb));
+    if (nblocks_out) *nblocks_out = (int)nb;
+    if (f)
+      hipLaunchKernelGGL(project2_kernel<true>, dim3(nb), wg, 0, st, g, p->d_rays, img, t2, sino,
+                         nang_sub, subset, nsubsets, nrays, fr);
+    else
+      hipLaunchKernelGGL(project2_kernel<false>, dim3(nb), wg, 0, st, g, p->d_rays, img, t2, sino,
+                         nang_sub, subset, nsubsets, nrays, fr);
     return hipGetLastError();
   }
   const float* imgT = nullptr;
@@ -1525,7 +1731,7 @@ hipError_t launch_min_nz_max(const float* x, size_t n, float* d_out, hipStream_t
 }
 
 hipError_t launch_group_project(BatchHeader* hdr, const ProjJob* jobs, int grid, hipStream_t st) {
-  hipLaunchKernelGGL(project_group_kernel, dim3(grid), dim3(kBlock), 0, st, hdr, jobs);
+  hipLaunchKernelGGL(project_group_kernel, dim3(grid), dim3(kGroupProject), 0, st, hdr, jobs);
   return hipGetLastError();
 }
 
