@@ -827,34 +827,54 @@ __global__ __launch_bounds__(kGBlock) void gather_kernel(GatherArgs A) {
 
 // ---- 2D gather, reference arithmetic ------------------------------------------------
 //
-// A workgroup takes a patch of 8 x 8 voxels, one per lane.  Its first nw wavefronts take
-// one angle each per round and write every candidate bin's term (0 where the bin does not
-// cross the voxel) to LDS; the next wavefront adds the terms of the round before to the 64
-// sums, in the reference's order (angle, radial bin).  The terms of an angle do not depend
-// on the sums, so an image too small to fill the GPU with one lane per voxel (gather_kernel:
-// 256 wavefronts for 128 x 128, each waiting for the loads of 192 angles in turn) runs 16
-// times the wavefronts with the same sums, bit for bit.  The rays that can cross the patch
-// (17 of an angle there) are staged in LDS by coalesced loads, with their entry crossings of
-// the patch's columns and rows: read by each lane at its own candidates, they took 38 cache
-// lines per load and bounded the kernel.  128x128 from 192 angles x 192 bins: 569 -> 48 us
-// (72 without the staging); 256x256 from 252 x 344: 642 -> 139 us; 64x64 from 48 x 64: 85 ->
-// 14 us.
-constexpr int kPatch = kPatch2;
-constexpr int kG2Waves = 16;   // wavefronts of the workgroup, one of them sums
-constexpr int kG2Rays = 20;    // rays staged at a time, by each wavefront
-// a staged ray: words 4 .. 15 of its RayXY (the bin value in place of lxy) and its crossings
-// into the patch's columns and rows
-constexpr int kG2RayWords = 12 + 2 * kPatch;
-constexpr int kG2LdsFloats = 16 * 1024 - 64;  // 64 KiB less the batch's block number: the
-                                              // staged rays and two rounds of terms
-// Wavefronts that compute terms for plans with up to maxc candidates per (voxel, angle);
-// 0: the terms of one angle do not fit (over 120 bins per voxel).
-__host__ __device__ inline int gather2_waves(int maxc) {
-  const int fit = kG2LdsFloats / (kG2Rays * kG2RayWords + 2 * kWave * (maxc > 0 ? maxc : 1));
-  return fit < kG2Waves - 1 ? fit : kG2Waves - 1;
+// A workgroup takes a patch of P x P voxels.  Its first nw wavefronts walk the rays of a few
+// angles each per round, one ray per lane, through the patch, and write each voxel's term to the
+// LDS slot of the ray's rank among the voxel's candidate bins (a slot no ray writes holds 0);
+// the next wavefront, a voxel per lane, adds the terms of the round before in the reference's
+// order (angle, radial bin).  The sums are gather_kernel's, bit for bit.
+//
+// gather_kernel (one lane per voxel, its angles in turn) waits for its loads with too few
+// wavefronts (256 for 128 x 128: 569 us from 192 x 192 bins).  One voxel per lane and an angle
+// per wavefront, its rays staged in LDS, is VALU-bound: 570 instructions an angle and patch,
+// most for bins that miss the voxel (48 us).  A ray's steps through an 8 x 8 patch are 15 at the
+// most, 23 instructions each, for 3 angles at a time there.  Calls, 17 us of host work
+// included, voxel per lane -> ray per lane: 128 x 128 from 192 x 192 50 -> 33 us, from 252 x 344
+// 118 -> 61; 64 x 64 from 192 x 192 108 -> 29; 32 x 32 from 252 x 344 1575 -> 82; 512 x 512 from
+// 252 x 344 381 -> 212.
+constexpr int kG2Waves = 16;                  // wavefronts of the workgroup, one of them sums
+constexpr int kG2LdsFloats = 16 * 1024 - 64;  // a grouped launch's two rounds of terms: 64 KiB
+                                              // less the batch's block number
+
+struct G2Plan {
+  int slots;   // of a voxel and angle: its candidates and one more (a rank is rounded down)
+  int rays;    // of an angle, that can cross a patch (64: or more)
+  int angles;  // of a wavefront's round
+  int nw;      // wavefronts that walk; 0: one angle's terms do not fit
+};
+// The half-width of a patch's bins: its own, a hundredth of a bin and 2 um more than its voxels'
+// own ranges, whose rounding is far below that.
+template <int P>
+__host__ __device__ inline float gather2_half(const Geo& g, float c, float s) {
+  return 0.5f * P * (g.dx * c + g.dy * s) + 0.5f * fabsf(g.dx - g.dy) + g.rmargin + 0.01f * g.dr +
+         2e-3f;
 }
-inline size_t gather2_lds(int nw, int maxc) {
-  return (size_t)nw * (kG2Rays * kG2RayWords + 2 * kWave * maxc) * sizeof(float);
+template <int P>
+__host__ __device__ inline G2Plan gather2_plan(const Geo& g, int maxc, int nang_sub,
+                                               int lds_floats) {
+  G2Plan q;
+  q.slots = (maxc > 0 ? maxc : 1) + 1;
+  const float r = 2.f * gather2_half<P>(g, 0.7072f, 0.7072f) / g.dr + 2.f;  // widest: 45 degrees
+  q.rays = r < (float)kWave ? (int)r : kWave;
+  q.angles = kWave / q.rays;
+  const int fit = lds_floats / (2 * q.angles * q.slots * P * P);
+  const int need = (nang_sub + q.angles - 1) / q.angles;
+  q.nw = fit < kG2Waves - 1 ? fit : kG2Waves - 1;
+  q.nw = q.nw < need ? q.nw : need;
+  return q;
+}
+template <int P>
+inline size_t gather2_lds(const G2Plan& q) {
+  return (size_t)q.nw * 2 * q.angles * q.slots * P * P * sizeof(float);
 }
 
 // Orders a wavefront's LDS accesses before and after this point (lanes read what
@@ -865,118 +885,168 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The terms of angle ka for the voxels of patch (px, py), this lane's (i, j): T[c * 64] for
-// candidate c < maxc.  st: the wavefront's kG2Rays staged rays.
-__device__ __forceinline__ void gather2_terms(const GatherArgs& A, int ka, int px, int py, int i,
-                                              int j, float inv_dr, float* st, float* T) {
+// The terms of angles ka0 .. ka0 + q.angles - 1 for the voxels of patch (px, py), to
+// T[((angle * q.slots) + rank) * P * P + voxel].
+template <int P>
+__device__ __forceinline__ void gather2_terms(const GatherArgs& A, const G2Plan& q, int ka0, int px,
+                                              int py, float inv_dr, int al, int rl, float* T) {
   const Geo& g = A.g;
   const int lane = threadIdx.x & (kWave - 1);
-  const int a = A.subset + A.nsubsets * ka;
-  const float xc = -g.R + g.dx * ((float)i + 0.5f), yc = -g.R + g.dy * ((float)j + 0.5f);
-  int jlo, jhi, lo1, hi1;
-  candidate_bins<kGridUniform>(A, a, xc, yc, inv_dr, jlo, jhi, lo1, hi1);
-  // the patch's bins: its half-width, a hundredth of a bin and 2 um more than its voxels' own
-  // ranges, whose rounding is far below that
+  for (int c = lane * 4; c < q.angles * q.slots * P * P; c += kWave * 4)
+    *reinterpret_cast<float4*>(T + c) = make_float4(0.f, 0.f, 0.f, 0.f);
+  wave_lds_sync();
+  const int ka = ka0 + al;
+  if (al >= q.angles || ka >= A.nang_sub) return;
+  const int a = A.subset + A.nsubsets * ka, ci0 = px * P, cj0 = py * P;
   const float2 cs = A.angcs[a];
-  const float sp = (-g.R + g.dx * (float)(px * kPatch + kPatch / 2)) * cs.x +
-                   (-g.R + g.dy * (float)(py * kPatch + kPatch / 2)) * cs.y;
-  const float hp = 0.5f * kPatch * (g.dx * fabsf(cs.x) + g.dy * fabsf(cs.y)) +
-                   0.5f * fabsf(g.dx - g.dy) + g.rmargin + 0.01f * g.dr + 2e-3f;
+  // the patch's bins
+  const float sp = (-g.R + g.dx * (float)(ci0 + P / 2)) * cs.x +
+                   (-g.R + g.dy * (float)(cj0 + P / 2)) * cs.y;
+  const float hp = gather2_half<P>(g, fabsf(cs.x), fabsf(cs.y));
   int p0 = (int)ceilf((sp - hp - g.r0) * inv_dr), p1 = (int)floorf((sp + hp - g.r0) * inv_dr);
-  p0 = __builtin_amdgcn_readfirstlane(p0 < 0 ? 0 : p0);
-  p1 = __builtin_amdgcn_readfirstlane(p1 > g.nr - 1 ? g.nr - 1 : p1);
-  const float* bins = A.kind == BP_PLAIN ? A.sino + (long)ka * g.nr
-                                         : (A.kind == BP_MULT ? A.sino + (long)a * g.nr : nullptr);
-  for (int c = 0; c < A.maxc; c++) T[c * kWave] = 0.f;
-  for (int r0 = p0; r0 <= p1; r0 += kG2Rays) {
-    const int nr = p1 - r0 + 1 < kG2Rays ? p1 - r0 + 1 : kG2Rays;
-    wave_lds_sync();  // the rays staged before are read
-    if (lane < 3 * kG2Rays && lane / 3 < nr) {
-      const int r = lane / 3, q = lane - 3 * r;
-      float4 v = reinterpret_cast<const float4*>(A.rays + (long)a * g.nr + r0 + r)[1 + q];
-      if (q == 1) v.z = bins ? bins[r0 + r] : 1.f;
-      *reinterpret_cast<float4*>(st + r * kG2RayWords + 4 * q) = v;
+  p0 = p0 < 0 ? 0 : p0;
+  p1 = p1 > g.nr - 1 ? g.nr - 1 : p1;
+  // a voxel's first candidate is the bin at or after t0 + i tx + j ty (candidate_bins; a
+  // thousandth of a bin early for the rounding here).  In 2^-16 bins, from bin p0: whole
+  // numbers, so a voxel's is the same whatever the path to it.
+  const float hw = 0.5f * g.dx * (fabsf(cs.x) + fabsf(cs.y)) + g.rmargin;
+  const int tx = (int)rintf(g.dx * cs.x * inv_dr * 65536.f);
+  const int ty = (int)rintf(g.dy * cs.y * inv_dr * 65536.f);
+  const float t0 = ((-g.R + g.dx * ((float)ci0 + 0.5f)) * cs.x +
+                    (-g.R + g.dy * ((float)cj0 + 0.5f)) * cs.y - hw - g.r0) * inv_dr - 1e-3f;
+  const int u0 = (int)((float)p0 * 65536.f - t0 * 65536.f);
+  const int ci1 = ci0 + P - 1 < g.nx ? ci0 + P - 1 : g.nx - 1;
+  const int cj1 = cj0 + P - 1 < g.ny ? cj0 + P - 1 : g.ny - 1;
+  // byte addresses in LDS: a rank's terms are kSlot bytes, so that a rank in 2^-16 ranks, shifted
+  // and its fraction replaced by the voxel's offset, is the term's address
+  constexpr int kSlot = P * P * 4, kShift = 16 - (P == 8 ? 8 : 6);
+  constexpr int kRow = 2 * P;  // (row, column) as one number, a guard bit above each
+  constexpr unsigned kGuards = ~(unsigned)((P - 1) | (P - 1) * kRow | 63 << 16);
+  typedef __attribute__((address_space(3))) char* lds_bytes;
+  typedef __attribute__((address_space(3))) float* lds_float;
+  const int slot0 = (int)(unsigned)(uintptr_t)(lds_bytes)(char*)(T + al * q.slots * P * P) / kSlot;
+  const int ulo = slot0 << 16, uhi = ulo + (q.slots << 16) - 1;
+  for (int rr = p0 + rl; rr <= p1; rr += q.rays) {
+    const float4* ray = reinterpret_cast<const float4*>(A.rays + (long)a * g.nr + rr);
+    const float4 q1 = ray[1], q2 = ray[2], q3 = ray[3];
+    const float amin = q1.x, ax = q1.z, ay = q1.w, axu = q2.x, ayu = q2.y, len = q3.w;
+    const int i0 = __float_as_int(q2.w), j0 = __float_as_int(q3.x);
+    const int nxy = __float_as_int(q3.y), flags = __float_as_int(q3.z);
+    const int iinc = ray_iinc(flags), jinc = ray_jinc(flags);
+    // the columns and rows the ray has to come to first, and the steps to them
+    const int ic = iinc > 0 ? (i0 > ci0 ? i0 : ci0) : (i0 < ci1 ? i0 : ci1);
+    const int jc = jinc > 0 ? (j0 > cj0 ? j0 : cj0) : (j0 < cj1 ? j0 : cj1);
+    const int na = (ic - i0) * iinc, nb = (jc - j0) * jinc;
+    int il = ic - ci0, jl = jc - cj0;
+    bool ok = (flags & RAY_VALID) != 0 && (unsigned)(il | jl) < (unsigned)P;
+    ok &= (iinc != 0) | (ic == i0);
+    ok &= (jinc != 0) | (jc == j0);
+    if (!ok) continue;
+    const float b = A.kind == BP_PLAIN ? A.sino[(long)ka * g.nr + rr]
+                                       : (A.kind == BP_MULT ? A.sino[(long)a * g.nr + rr] : 1.f);
+    const float* xytab = A.xytab + ((long)a * g.nr + rr) * (g.nx + g.ny);
+    const float Xi = na > 0 ? xytab[ic] : -FLT_MAX, Yi = nb > 0 ? xytab[g.nx + jc] : -FLT_MAX;
+    float X = na > 0 ? Xi + axu : ax, Y = nb > 0 ? Yi + ayu : ay;
+    // rows, columns and the steps left in the list (of 64) in one number, whose guard bits say
+    // when one runs out; the term's rank; the voxel's offset
+    int left = nxy - na - nb;
+    left = left < 0 ? 0 : (left > 63 ? 63 : left);
+    int at = il + jl * kRow + ((64 - left) << 16);
+    int u = u0 + ((rr - p0) << 16) + ulo - il * tx - jl * ty;
+    int off = (jl * P + il) * 4;
+    const int atx = iinc + (1 << 16), aty = jinc * kRow + (1 << 16);
+    const int ux = -iinc * tx, uy = -jinc * ty, ox = iinc * 4, oy = jinc * P * 4;
+    // the later of the two crossings enters the patch; the other chain's crossings before it
+    // (x first on ties) are taken first
+    float ac = Xi > Yi ? Xi : Yi;
+    if (na + nb == 0) {
+      ac = amin;
+    } else if (Xi > Yi) {
+      while (Y < Xi && !(at & kGuards)) {
+        Y = Y + ayu;
+        at += aty;
+        u += uy;
+        off += oy;
+      }
+    } else {
+      while (X <= Yi && !(at & kGuards)) {
+        X = X + axu;
+        at += atx;
+        u += ux;
+        off += ox;
+      }
     }
-    const float* xytab = A.xytab + ((long)a * g.nr + r0) * (g.nx + g.ny);
-    for (int q = lane; q < nr * 2 * kPatch; q += kWave) {
-      const int r = q / (2 * kPatch), w = q % (2 * kPatch);
-      int e = w < kPatch ? px * kPatch + w : py * kPatch + w - kPatch;
-      e = w < kPatch ? (e < g.nx ? e : g.nx - 1) : g.nx + (e < g.ny ? e : g.ny - 1);
-      st[r * kG2RayWords + 12 + w] = xytab[(long)r * (g.nx + g.ny) + e];
-    }
-    wave_lds_sync();
-    const int rlo = jlo > r0 ? jlo : r0, rhi = jhi < r0 + nr - 1 ? jhi : r0 + nr - 1;
-    for (int rr = rlo; rr <= rhi; rr++) {
-      const float* s = st + (rr - r0) * kG2RayWords;
-      const float4 q1 = *reinterpret_cast<const float4*>(s);
-      const float4 q2 = *reinterpret_cast<const float4*>(s + 4);
-      const float4 q3 = *reinterpret_cast<const float4*>(s + 8);
-      const float xyi = s[12 + (i & (kPatch - 1))], xyj = s[12 + kPatch + (j & (kPatch - 1))];
-      const float amin = q1.x, ax = q1.z, ay = q1.w, axu = q2.x, ayu = q2.y, b = q2.z, len = q3.w;
-      const int i0 = __float_as_int(q2.w), j0 = __float_as_int(q3.x);
-      const int nxy = __float_as_int(q3.y), flags = __float_as_int(q3.z);
-      // the tests of gather_voxel as one predicate
-      const int iinc = ray_iinc(flags), jinc = ray_jinc(flags);
-      const int na = __mul24(i - i0, iinc), nb = __mul24(j - j0, jinc), m = na + nb;
-      bool ok = (flags & RAY_VALID) != 0;
-      ok &= (i == i0) | ((iinc != 0) & (na >= 0));
-      ok &= (j == j0) | ((jinc != 0) & (nb >= 0));
-      ok &= m < nxy;
-      const float Xp = na > 0 ? xyi : -FLT_MAX, Xn = na > 0 ? xyi + axu : ax;
-      const float Yp = nb > 0 ? xyj : -FLT_MAX, Yn = nb > 0 ? xyj + ayu : ay;
-      ok &= ((na <= 0) | (Xp <= Yn)) & ((nb <= 0) | (Yp < Xn));
-      const float ac = m > 0 ? (Xp > Yp ? Xp : Yp) : amin;
-      const float an = Xn < Yn ? Xn : Yn;
+    while (!(at & kGuards)) {
+      const bool bx = X <= Y;
+      const float an = bx ? X : Y;
       const float w = (an - ac) * len;
-      if (ok) T[(rr - jlo) * kWave] = w * b * 1.0f;  // SiddonProjector.cpp:72
+      ac = an;
+      const int c = u < ulo ? ulo : (u > uhi ? uhi : u);
+      *(lds_float)(lds_bytes)(uintptr_t)(unsigned)(((c >> kShift) & ~(kSlot - 1)) |
+                                                   (off & (kSlot - 1))) =
+          w * b * 1.0f;  // SiddonProjector.cpp:72
+      const float nX = X + axu, nY = Y + ayu;
+      X = bx ? nX : X;
+      Y = bx ? Y : nY;
+      at += bx ? atx : aty;
+      u += bx ? ux : uy;
+      off += bx ? ox : oy;
     }
   }
 }
 
-// Patch (px, py) by the whole workgroup (more than nw wavefronts, 1 <= nw <=
-// gather2_waves(A.maxc)); lds: gather2_lds(nw, A.maxc) bytes.
-__device__ __forceinline__ void gather2_patch(const GatherArgs& A, int nw, int px, int py,
+// Patch (px, py) by the whole workgroup (more than q.nw wavefronts, q.nw >= 1); lds:
+// gather2_lds(q) bytes.
+template <int P>
+__device__ __forceinline__ void gather2_patch(const GatherArgs& A, const G2Plan& q, int px, int py,
                                               float* lds) {
   const Geo& g = A.g;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & (kWave - 1);
-  const int ir = px * kPatch + (lane & (kPatch - 1)), jr = py * kPatch + lane / kPatch;
-  const bool in = ir < g.nx && jr < g.ny;
-  const int i = ir < g.nx ? ir : g.nx - 1, j = jr < g.ny ? jr : g.ny - 1;
-  const long v = (long)j * g.nx + i;
-  const float inv_dr = 1.0f / g.dr;
-  float* T = lds + nw * kG2Rays * kG2RayWords;
-  const int buf = nw * A.maxc * kWave, rounds = (A.nang_sub + nw - 1) / nw;
-  float acc = wave == nw && !A.upd_sens ? A.img[v] : 0.f;
-  for (int it = 0; it <= rounds; it++) {
-    if (wave < nw) {
-      const int ka = it * nw + wave;
-      if (ka < A.nang_sub)
-        gather2_terms(A, ka, px, py, i, j, inv_dr, lds + wave * kG2Rays * kG2RayWords,
-                      T + (it & 1) * buf + wave * A.maxc * kWave + lane);
-    } else if (wave == nw && it > 0) {
-      const float* s = T + ((it - 1) & 1) * buf + lane;
-      const int left = A.nang_sub - (it - 1) * nw, n = (left < nw ? left : nw) * A.maxc;
-#pragma unroll 8
-      for (int q = 0; q < n; q++) acc = acc + s[q * kWave];
+  const int mine = q.angles * q.slots * P * P, buf = q.nw * mine, round = q.nw * q.angles;
+  const int rounds = (A.nang_sub + round - 1) / round;
+  // the two kinds of wavefront meet at the same barriers, rounds + 1 of them
+  if (wave < q.nw) {
+    const float inv_dr = 1.0f / g.dr;
+    const int al = lane / q.rays, rl = lane % q.rays;
+    for (int it = 0; it <= rounds; it++) {
+      const int ka0 = it * round + wave * q.angles;
+      if (ka0 < A.nang_sub)
+        gather2_terms<P>(A, q, ka0, px, py, inv_dr, al, rl, lds + (it & 1) * buf + wave * mine);
+      __syncthreads();
     }
-    __syncthreads();
+  } else {
+    const int ir = px * P + lane % P, jr = py * P + lane / P;
+    const bool in = wave == q.nw && lane < P * P && ir < g.nx && jr < g.ny;
+    const long v = (long)jr * g.nx + ir;
+    float acc = in && !A.upd_sens ? A.img[v] : 0.f;
+    for (int it = 0; it <= rounds; it++) {
+      if (it > 0 && in) {
+        const float* s = lds + ((it - 1) & 1) * buf + lane;
+        const int left = A.nang_sub - (it - 1) * round;
+        const int n = (left < round ? left : round) * q.slots;
+#pragma unroll 8
+        for (int c = 0; c < n; c++) acc = acc + s[c * (P * P)];
+      }
+      __syncthreads();
+    }
+    if (in) store_voxel(A, v, acc);
   }
-  if (wave == nw && in) store_voxel(A, v, acc);
 }
 
-__global__ __launch_bounds__(kG2Waves * kWave, 8) void gather2_kernel(GatherArgs A, int nw) {
-  extern __shared__ __align__(16) float g2lds[];
-  gather2_patch(A, nw, blockIdx.x, blockIdx.y, g2lds);
+template <int P>
+__global__ __launch_bounds__(kG2Waves * kWave, 8) void gather2_kernel(GatherArgs A, G2Plan q) {
+  extern __shared__ __align__(256) float g2lds[];  // a slot's alignment (gather2_terms)
+  gather2_patch<P>(A, q, blockIdx.x, blockIdx.y, g2lds);
 }
 
 // ---- grouped (multi-job) launch -----------------------------------------------
 #include "group_common.h"
 
 // Each virtual block is one 8 x 8 patch of one 2D job, by the whole workgroup.
-__global__ __launch_bounds__(kG2Waves * kWave) void gather2_group_kernel(
+__global__ __launch_bounds__(kG2Waves * kWave, 8) void gather2_group_kernel(
     BatchHeader* __restrict__ hdr, const GJob* __restrict__ jobs) {
-  extern __shared__ __align__(16) float g2lds[];
+  extern __shared__ __align__(256) float g2lds[];  // a slot's alignment (gather2_terms)
   const int n = hdr->count[PH_GATHER2];
   const long total = hdr->total[PH_GATHER2];
   const int grab = grab_size(hdr);
@@ -984,12 +1054,12 @@ __global__ __launch_bounds__(kG2Waves * kWave) void gather2_group_kernel(
     for (long vb = v0; vb < v0 + grab && vb < total; vb++) {
       const GJob& J = jobs[find_job(jobs, n, vb)];
       const int lb = (int)(vb - J.first), px = lb % J.ntx, py = lb / J.ntx;
-      const int nw = gather2_waves(J.A.maxc);
-      if (nw > 0) {
-        gather2_patch(J.A, nw, px, py, g2lds);
+      const G2Plan q = gather2_plan<kPatch2>(J.A.g, J.A.maxc, J.A.nang_sub, kG2LdsFloats);
+      if (q.nw > 0) {
+        gather2_patch<kPatch2>(J.A, q, px, py, g2lds);
       } else if (threadIdx.x < kWave) {  // more candidates per angle than the LDS holds
         const int i = px * kPatch2 + threadIdx.x % kPatch2, j = py * kPatch2 + threadIdx.x / kPatch2;
-        if (i < J.A.g.nx && j < J.A.g.ny)
+        if (threadIdx.x < kPatch2 * kPatch2 && i < J.A.g.nx && j < J.A.g.ny)
           gather_voxel<2, APIRL_PREC_REFERENCE>(J.A, nullptr, i, j, 0);
       }
     }
@@ -1040,15 +1110,41 @@ void launch_gather3(const GatherArgs& A, int zlanes, int zvox, hipStream_t st) {
                      A);
 }
 
+// 4 x 4 patches for images of up to this many 8 x 8 ones, which would leave half of the CUs idle
+// (8 x 8 / 4 x 4: 64 x 64 from 192 x 192 bins 68 / 31 us, 252 x 344 108 / 57; 88 x 88 48 / 38);
+// from 96 x 96 on the 8 x 8 patches, whose rays' setup serves more voxels, are ahead (98 / 105 us
+// there, 42 / 52 at 128 x 128).  A grouped launch, which has several images' patches, keeps 8 x 8
+// (17 of 64 x 64: 2.36 / 2.59 ms).
+constexpr int kG2SmallPatches = 128;
+
+// The patches a CU gets share its LDS: more wavefronts at work on one patch while there are few
+// of them (128 x 128, one a CU: 48, 64 and 96 KiB 42, 42 and 37 us), less waiting at the rounds'
+// ends with several workgroups a CU (256 x 256 from 96 x 192: 32, 64 and 96 KiB 34, 39, 51 us).
+inline int gather2_lds_floats(long patches) {
+  constexpr int kCus = 256;
+  const long per = (patches + kCus - 1) / kCus, share = 40 * 1024 / (per > 0 ? per : 1);
+  return (int)(share > 24 * 1024 ? 24 * 1024 : (share < 8 * 1024 ? 8 * 1024 : share));
+}
+
+template <int P>
+bool launch_gather2_patches(const GatherArgs& A, hipStream_t st) {
+  const Geo& g = A.g;
+  const dim3 grid((g.nx + P - 1) / P, (g.ny + P - 1) / P);
+  const int lds = gather2_lds_floats((long)grid.x * grid.y);
+  G2Plan q = gather2_plan<P>(g, A.maxc, A.nang_sub, lds);
+  if (q.nw == 0) q = gather2_plan<P>(g, A.maxc, A.nang_sub, 24 * 1024);
+  if (q.nw == 0) return false;
+  hipLaunchKernelGGL(gather2_kernel<P>, grid, dim3((q.nw + 1) * kWave), gather2_lds<P>(q), st, A,
+                     q);
+  return true;
+}
+
 template <int PREC>
 void launch_gather2(const GatherArgs& A, hipStream_t st) {
   const Geo& g = A.g;
-  if (PREC == APIRL_PREC_REFERENCE && gather2_waves(A.maxc) > 0) {
-    const int nw = gather2_waves(A.maxc) < A.nang_sub ? gather2_waves(A.maxc) : A.nang_sub;
-    hipLaunchKernelGGL(gather2_kernel,
-                       dim3((g.nx + kPatch2 - 1) / kPatch2, (g.ny + kPatch2 - 1) / kPatch2),
-                       dim3((nw + 1) * kWave), gather2_lds(nw, A.maxc), st, A, nw);
-    return;
+  if (PREC == APIRL_PREC_REFERENCE) {
+    const bool small = (g.nx + 7) / 8 * ((g.ny + 7) / 8) <= kG2SmallPatches;
+    if (small ? launch_gather2_patches<4>(A, st) : launch_gather2_patches<8>(A, st)) return;
   }
   const dim3 grid((g.nx + kTile - 1) / kTile, (g.ny + kTile - 1) / kTile, g.nz);
   hipLaunchKernelGGL((gather_kernel<2, PREC>), grid, dim3(kGBlock), 0, st, A);
