@@ -282,6 +282,10 @@ struct EmFuse {
   float thr;
   int strict;
 };
+// The 2D gather by patches runs this subset's backprojection; the scatter form, whose atomics it
+// outruns everywhere (34 / 19 us for 32 x 32 from 8 x 40 bins, 319 / 82 from 252 x 344; 164 / 20
+// for 256 x 256 from 24 x 76, 531 / 99 from 252 x 320), then does too.
+bool gather2_takes(const apirl_plan* p, int subset, int nsubsets);
 hipError_t launch_backproject_gather(const apirl_plan* p, const float* sino, float* img,
                                      int subset, int nsubsets, int kind, int precision,
                                      void* scratch, size_t scratch_bytes, hipStream_t st,

@@ -333,6 +333,11 @@ apirl_status backproject_any(apirl_plan* p, const float* sino, const float* est,
       const apirl_status st = tile_backproject(p, sino, img, subset, nsubsets, kind, nullptr, done);
       if (done) return st;
     }
+    if (kind != apirl::BP_DIVIDE && apirl::gather2_takes(p, subset, nsubsets)) {
+      APIRL_HIP(c, apirl::launch_backproject_gather(p, sino, img, subset, nsubsets, kind,
+                                                    precision, nullptr, 0, c->stream, nullptr));
+      return APIRL_OK;
+    }
     if (!p->d_replicas && !p->replicas_failed) {
       // the per-XCD scatter targets (16 image copies), zeroed here and re-zeroed by
       // the reduction after every use; without them the atomics go to the image

@@ -909,7 +909,7 @@ __device__ __forceinline__ void gather2_terms(const GatherArgs& A, const G2Plan&
   // a voxel's first candidate is the bin at or after t0 + i tx + j ty (candidate_bins; a
   // thousandth of a bin early for the rounding here).  In 2^-16 bins, from bin p0: whole
   // numbers, so a voxel's is the same whatever the path to it.
-  const float hw = 0.5f * g.dx * (fabsf(cs.x) + fabsf(cs.y)) + g.rmargin;
+  const float hw = 0.5f * (g.dx * fabsf(cs.x) + g.dy * fabsf(cs.y)) + g.rmargin;
   const int tx = (int)rintf(g.dx * cs.x * inv_dr * 65536.f);
   const int ty = (int)rintf(g.dy * cs.y * inv_dr * 65536.f);
   const float t0 = ((-g.R + g.dx * ((float)ci0 + 0.5f)) * cs.x +
@@ -1120,31 +1120,45 @@ constexpr int kG2SmallPatches = 128;
 // The patches a CU gets share its LDS: more wavefronts at work on one patch while there are few
 // of them (128 x 128, one a CU: 48, 64 and 96 KiB 42, 42 and 37 us), less waiting at the rounds'
 // ends with several workgroups a CU (256 x 256 from 96 x 192: 32, 64 and 96 KiB 34, 39, 51 us).
+constexpr int kG2MostLds = 24 * 1024;
 inline int gather2_lds_floats(long patches) {
   constexpr int kCus = 256;
   const long per = (patches + kCus - 1) / kCus, share = 40 * 1024 / (per > 0 ? per : 1);
-  return (int)(share > 24 * 1024 ? 24 * 1024 : (share < 8 * 1024 ? 8 * 1024 : share));
+  return (int)(share > kG2MostLds ? kG2MostLds : (share < 8 * 1024 ? 8 * 1024 : share));
 }
 
 template <int P>
-bool launch_gather2_patches(const GatherArgs& A, hipStream_t st) {
+void launch_gather2_patches(const GatherArgs& A, hipStream_t st) {
   const Geo& g = A.g;
   const dim3 grid((g.nx + P - 1) / P, (g.ny + P - 1) / P);
   const int lds = gather2_lds_floats((long)grid.x * grid.y);
   G2Plan q = gather2_plan<P>(g, A.maxc, A.nang_sub, lds);
-  if (q.nw == 0) q = gather2_plan<P>(g, A.maxc, A.nang_sub, 24 * 1024);
-  if (q.nw == 0) return false;
+  if (q.nw == 0) q = gather2_plan<P>(g, A.maxc, A.nang_sub, kG2MostLds);  // gather2_fits: not 0
   hipLaunchKernelGGL(gather2_kernel<P>, grid, dim3((q.nw + 1) * kWave), gather2_lds<P>(q), st, A,
                      q);
-  return true;
+}
+
+// bins within a column's half-width (candidate_bins) of its centre, on a uniform grid
+inline int gather2_candidates(const Geo& g) {
+  return (int)std::min(1e6, std::floor((1.41421357 * std::max(g.dx, g.dy) + 2.0 * g.rmargin) /
+                                           g.dr * 1.0001 + 1e-3) + 1);
+}
+
+inline bool gather2_small(const Geo& g) {
+  return (long)((g.nx + 7) / 8) * ((g.ny + 7) / 8) <= kG2SmallPatches;
+}
+inline bool gather2_fits(const Geo& g, int maxc, int nang_sub) {
+  return (gather2_small(g) ? gather2_plan<4>(g, maxc, nang_sub, kG2MostLds)
+                           : gather2_plan<8>(g, maxc, nang_sub, kG2MostLds)).nw > 0;
 }
 
 template <int PREC>
 void launch_gather2(const GatherArgs& A, hipStream_t st) {
   const Geo& g = A.g;
-  if (PREC == APIRL_PREC_REFERENCE) {
-    const bool small = (g.nx + 7) / 8 * ((g.ny + 7) / 8) <= kG2SmallPatches;
-    if (small ? launch_gather2_patches<4>(A, st) : launch_gather2_patches<8>(A, st)) return;
+  if (PREC == APIRL_PREC_REFERENCE && gather2_fits(g, A.maxc, A.nang_sub)) {
+    if (gather2_small(g)) launch_gather2_patches<4>(A, st);
+    else launch_gather2_patches<8>(A, st);
+    return;
   }
   const dim3 grid((g.nx + kTile - 1) / kTile, (g.ny + kTile - 1) / kTile, g.nz);
   hipLaunchKernelGGL((gather_kernel<2, PREC>), grid, dim3(kGBlock), 0, st, A);
@@ -2063,9 +2077,7 @@ void gather_args_for(const apirl_plan* p, int subset, int nsubsets, int kind, co
   }
   A.zr = zr;
   A.nz_pair = nz_pair;
-  // bins within the column's half-width (candidate_bins) of its centre, on a uniform grid
-  A.maxc = (int)std::min(1e6, std::floor((1.41421357 * std::max(g.dx, g.dy) + 2.0 * g.rmargin) /
-                                             g.dr * 1.0001 + 1e-3) + 1);
+  A.maxc = gather2_candidates(g);
   A.upd_sens = nullptr;
   A.upd_thr = 0.f;
   A.upd_strict = 0;
@@ -2075,6 +2087,13 @@ hipError_t launch_group_gather(BatchHeader* hdr, const GJob* jobs, int grid, hip
   hipLaunchKernelGGL(gather2_group_kernel, dim3(grid), dim3(kG2Waves * kWave),
                      kG2LdsFloats * sizeof(float), st, hdr, jobs);
   return hipGetLastError();
+}
+
+bool gather2_takes(const apirl_plan* p, int subset, int nsubsets) {
+  const Geo& g = p->geo;
+  if (g.dims != 2 || g.ns * g.nas != 1 || !p->gather_ok) return false;
+  const int nang_sub = subset_num_angles(g.nang, nsubsets, subset);
+  return nang_sub > 0 && gather2_fits(g, gather2_candidates(g), nang_sub);
 }
 
 const char* gather_misfit(const apirl_plan* p, int subset, int nsubsets) {

@@ -72,3 +72,17 @@ def test_gather2d_batch_equals_alone(torch, ctx):
         assert np.array_equal(np.isnan(a), np.isnan(b))
         same(np.nan_to_num(a), np.nan_to_num(b))
     batch.close()
+
+
+@pytest.mark.parametrize("g", GEOMS)
+def test_scatter2d_is_the_gather(torch, ctx, g):
+    """The scatter form runs the patches where they fit: the oracle's sums, bit for bit."""
+    log(f"case: 2D scatter form {g}")
+    p, im, ang, r, rfov = build(ctx, g)
+    rng = np.random.default_rng(4)
+    sino = rng.random((1, g[2], g[3]), dtype=np.float32)
+    sd = dev(torch, sino)
+    same(host(p.backproject(sd, mode=hip.BP_SCATTER)),
+         O.backproject2d(im, sino[0], ang, r, rfov, 400.0))
+    same(host(p.sensitivity(mode=hip.BP_SCATTER, force_positive=0)),
+         O.backproject2d(im, np.ones_like(sino[0]), ang, r, rfov, 400.0))
