@@ -1384,16 +1384,22 @@ __device__ __forceinline__ void tile_lane(const TileRay& R, const TileZ& z, floa
   float Zn = z.az0;
   // z crossings taken before the entry: those below its alpha (a z crossing at the
   // alpha of an x or y crossing is taken after it, Siddon.cpp:318-339), by the
-  // loop's own additions, four at a time
+  // loop's own additions, four at a time while all four are (one test in four: 1.08 -> 0.94 ms
+  // for 12 of 252 angles of 344 x 837 bins into 256 x 256 x 81, whose rays cross up to 70 slices)
   if (R.mxy > 0) {
-    while (left > 0 && Zn < ce) {
-      const float z1 = Zn + azu, z2 = z1 + azu, z3 = z2 + azu;
-      const int c = 1 + (z1 < ce ? 1 : 0) + (z2 < ce ? 1 : 0) + (z3 < ce ? 1 : 0);
-      Zn = c == 1 ? z1 : (c == 2 ? z2 : (c == 3 ? z3 : z3 + azu));
-      k += c * kinc;
-      left -= c;
-      if (c < 4) break;
+    int c = 0;
+    float z1 = Zn + azu, z2 = z1 + azu, z3 = z2 + azu;
+    while (z3 < ce && c < left) {
+      Zn = z3 + azu;
+      z1 = Zn + azu;
+      z2 = z1 + azu;
+      z3 = z2 + azu;
+      c += 4;
     }
+    c += (Zn < ce ? 1 : 0) + (z1 < ce ? 1 : 0) + (z2 < ce ? 1 : 0);
+    Zn = z2 < ce ? z3 : (z1 < ce ? z2 : (Zn < ce ? z1 : Zn));
+    k += c * kinc;
+    left -= c;
   }
   unsigned v = (unsigned)((k - kz0) * kTPitch + R.col0);
   const int kstep = kinc * kTPitch;
