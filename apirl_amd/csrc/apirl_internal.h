@@ -269,9 +269,15 @@ void free_os_parts(apirl_plan* p);
 // block partials into `partials`, then a fixed-order sum into *out.
 hipError_t launch_likelihood(const float* x, const float* y, long n, int positive_only,
                              double* partials, double* out, hipStream_t st);
-// d_out: [min_nz, max] and 2 kMinMaxBlocks floats of scratch.
+// The MLEM update threshold from a sensitivity's smallest non-zero and largest value (Mlem.cpp:41).
+__host__ __device__ inline float mlem_threshold(float least, float most) {
+  return least + (most - least) * 0.0001f;
+}
+// d_out: [min_nz, max] and 2 kMinMaxBlocks floats of scratch.  d_thr: null, or where the MLEM
+// threshold of a sensitivity x goes (mlem_threshold).
 constexpr int kMinMaxBlocks = 512;
-hipError_t launch_min_nz_max(const float* x, size_t n, float* d_out, hipStream_t st);
+constexpr size_t kMinMaxFloats = 2 + 2 * (size_t)kMinMaxBlocks;
+hipError_t launch_min_nz_max(const float* x, size_t n, float* d_out, float* d_thr, hipStream_t st);
 hipError_t launch_count_intersections(const apirl_plan* p, int subset, int nsubsets,
                                       unsigned long long* d_out, hipStream_t st);
 
@@ -281,6 +287,7 @@ struct EmFuse {
   const float* sens;
   float thr;
   int strict;
+  const float* thr_at = nullptr;  // device: the threshold, in place of thr
 };
 // The 2D gather by patches runs this subset's backprojection; the scatter form, whose atomics it
 // outruns everywhere (34 / 19 us for 32 x 32 from 8 x 40 bins, 319 / 82 from 252 x 344; 164 / 20
@@ -404,6 +411,7 @@ struct GatherArgs {
   // to (s > thr or, not strict, s >= thr) ? (x b) / s : 0 with s = upd_sens[v]
   const float* upd_sens;
   float upd_thr;
+  const float* upd_thr_at;  // null, or (device) the threshold in place of upd_thr
   int upd_strict;
   int maxc;  // 2D: upper bound on a voxel's candidate bins of one angle
 };

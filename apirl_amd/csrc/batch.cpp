@@ -37,7 +37,8 @@ struct BJob {
   bool active = false;       // scheduled in future rounds
   bool done_recorded = false;
   hipEvent_t done_ev = nullptr;
-  std::vector<float> thr;
+  std::vector<float> thr;   // oversampled jobs: the subsets' thresholds
+  float* thr_at = nullptr;  // the other MLEM jobs: the same on the device (null: 0)
   int strict = 0;
   // device state owned by the job
   float* sens = nullptr;     // S images
@@ -230,10 +231,15 @@ int apirl_batch_job_backprojector(const apirl_plan* p) {
   return APIRL_BP_GATHER;
 }
 
+// The subsets' thresholds and the scratch that finds them, after the sensitivities.
+static size_t thresholds_bytes(int subsets) {
+  return ((size_t)subsets + apirl::kMinMaxFloats) * sizeof(float);
+}
+
 size_t apirl_batch_job_bytes(const apirl_plan* p, int subsets) {
   if (!p || subsets < 1) return 0;
   const size_t nvox = apirl_plan_image_voxels(p);
-  size_t bytes = (size_t)subsets * nvox * sizeof(float) +
+  size_t bytes = (size_t)subsets * nvox * sizeof(float) + thresholds_bytes(subsets) +
                  max_subset_bins(p, subsets) * sizeof(float);
   if (p->geo.dims == 3) {
     // oversampled bins: the largest scratch of the plans of one LOR per bin once they are
@@ -320,7 +326,7 @@ apirl_status apirl_batch_submit(apirl_batch* b, const apirl_job_desc* d, int* jo
   j->nvox = apirl_plan_image_voxels(p);
   j->strict = (!j->osem && j->is2d) ? 1 : 0;
   apirl::ActiveForm form_scope(p, j->form);
-  const size_t sens_b = (size_t)j->S * j->nvox * sizeof(float);
+  const size_t sens_b = (size_t)j->S * j->nvox * sizeof(float) + thresholds_bytes(j->S);
   const size_t ratio_b = max_subset_bins(p, j->S) * sizeof(float);
   size_t z_b = 0;
   if (!j->is2d)
@@ -375,7 +381,17 @@ apirl_status apirl_batch_submit(apirl_batch* b, const apirl_job_desc* d, int* jo
         st = APIRL_ERR_HIP;
       }
     }
-    if (st == APIRL_OK && !j->osem) st = apirl_mlem_threshold(c, sens, j->nvox, &j->thr[s]);
+    if (st != APIRL_OK || j->osem) continue;
+    if (os) {
+      st = apirl_mlem_threshold(c, sens, j->nvox, &j->thr[s]);
+      continue;
+    }
+    // left on the device, where the update reads it: waiting for it here took 30 us a slice of
+    // 64 x 64, which the GPU stood still
+    float* thr = j->sens + (size_t)j->S * j->nvox;
+    j->thr_at = thr;
+    if (launch_min_nz_max(sens, j->nvox, thr + j->S, thr + s, b->stream) != hipSuccess)
+      st = APIRL_ERR_HIP;
   }
   if (st == APIRL_OK &&
       hipMemcpyAsync(j->x, d->d_init, j->nvox * sizeof(float), hipMemcpyDeviceToDevice,
@@ -471,7 +487,7 @@ apirl_status apirl_batch_step(apirl_batch* b, int* active) {
       int* unused_nz = nullptr;
       gather_args_for(p, s, S, BP_PLAIN, j->ratio, j->x, nullptr, q.A, unused_zr, unused_nz);
       q.A.upd_sens = j->sens + (size_t)s * j->nvox;
-      q.A.upd_thr = j->thr[s];
+      if (j->thr_at) q.A.upd_thr_at = j->thr_at + s;
       q.A.upd_strict = j->strict;
       q.ntx = (g.nx + kPatch2 - 1) / kPatch2;
       q.nty = (g.ny + kPatch2 - 1) / kPatch2;
@@ -532,7 +548,7 @@ apirl_status apirl_batch_step(apirl_batch* b, int* active) {
     e = launch_project(j->plan, j->x, nullptr, s, j->S, APIRL_PREC_REFERENCE, &fr, nullptr,
                        b->stream, j->copy);
     if (e == hipSuccess && !j->bp) {
-      const EmFuse fz{sens, j->thr[s], j->strict};
+      const EmFuse fz{sens, 0.f, j->strict, j->thr_at ? j->thr_at + s : nullptr};
       e = backproject_job(j, j->ratio, j->x, s, BP_PLAIN, &fz, b->stream);
     } else if (e == hipSuccess) {
       e = hipMemsetAsync(j->bp, 0, j->nvox * sizeof(float), b->stream);

@@ -455,7 +455,7 @@ apirl_status apirl_ctx_create(int device, apirl_ctx** out) {
   apirl_ctx* c = new apirl_ctx();
   c->device = device;
   DeviceGuard g(device);
-  if (hipMalloc(&c->d_fred, (2 + 2 * apirl::kMinMaxBlocks) * sizeof(float)) != hipSuccess ||
+  if (hipMalloc(&c->d_fred, apirl::kMinMaxFloats * sizeof(float)) != hipSuccess ||
       hipMalloc(&c->d_ured, 8 * sizeof(unsigned long long)) != hipSuccess) {
     delete c;
     return APIRL_ERR_NOMEM;
@@ -1135,12 +1135,11 @@ apirl_status apirl_mlem_threshold(apirl_ctx* c, const float* d_sens, size_t n, f
   if (!c || !d_sens || !h_thr || n == 0) return APIRL_ERR_INVALID;
   DeviceGuard g(c->device);
   float mm[2];
-  APIRL_HIP(c, apirl::launch_min_nz_max(d_sens, n, c->d_fred, c->stream));
+  APIRL_HIP(c, apirl::launch_min_nz_max(d_sens, n, c->d_fred, nullptr, c->stream));
   APIRL_HIP(c, hipMemcpyAsync(mm, c->d_fred, 2 * sizeof(float), hipMemcpyDeviceToHost,
                               c->stream));
   APIRL_HIP(c, hipStreamSynchronize(c->stream));
-  // Mlem.cpp:41
-  *h_thr = mm[0] + (mm[1] - mm[0]) * 0.0001f;
+  *h_thr = apirl::mlem_threshold(mm[0], mm[1]);
   return APIRL_OK;
 }
 

@@ -343,7 +343,8 @@ __device__ __forceinline__ void store_voxel(const GatherArgs& A, long v, float b
     return;
   }
   const float sv = A.upd_sens[v];
-  const bool ok = A.upd_strict ? (sv > A.upd_thr) : (sv >= A.upd_thr);
+  const float thr = A.upd_thr_at ? *A.upd_thr_at : A.upd_thr;
+  const bool ok = A.upd_strict ? (sv > thr) : (sv >= thr);
   A.img[v] = ok ? A.img[v] * b / sv : 0.f;
 }
 
@@ -1807,6 +1808,7 @@ hipError_t launch_backproject_gather(const apirl_plan* p, const float* sino, flo
   if (fuse) {
     A.upd_sens = fuse->sens;
     A.upd_thr = fuse->thr;
+    A.upd_thr_at = fuse->thr_at;
     A.upd_strict = fuse->strict;
   }
   if (g.dims == 3) {
@@ -2010,6 +2012,7 @@ hipError_t launch_backproject_tile(const apirl_plan* p, const float* sino, float
   if (fuse) {
     A.upd_sens = fuse->sens;
     A.upd_thr = fuse->thr;
+    A.upd_thr_at = fuse->thr_at;
     A.upd_strict = fuse->strict;
   }
   // the subset's geometry: the rays of every tile with their paths
@@ -2086,6 +2089,7 @@ void gather_args_for(const apirl_plan* p, int subset, int nsubsets, int kind, co
   A.maxc = gather2_candidates(g);
   A.upd_sens = nullptr;
   A.upd_thr = 0.f;
+  A.upd_thr_at = nullptr;
   A.upd_strict = 0;
 }
 

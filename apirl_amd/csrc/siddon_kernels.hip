@@ -933,9 +933,11 @@ __global__ __launch_bounds__(kBlock) void sum_partials_kernel(const double* __re
 // order-independent, so the result is exact.  A launch of one workgroup gives out[0] = min_nz,
 // out[1] = max; the reference's maximum starts from pixel 0, so a NaN there is kept.  A launch
 // of more leaves a pair per workgroup after them, which a second launch of one takes in place
-// of x (pairs > 0).  One workgroup took 5.7 ms for 256x256x81 voxels, the two launches TT us.
+// of x (pairs > 0).  One workgroup took 5.7 ms for 256x256x81 voxels, the two launches 19 us (128x128x47:
+// 346 and 10 us).
 __global__ __launch_bounds__(kBlock) void min_nz_max_kernel(const float* __restrict__ x, long n,
-                                                            float* __restrict__ out, int pairs) {
+                                                            float* __restrict__ out, int pairs,
+                                                            float* __restrict__ thr) {
   __shared__ float smin[kBlock], smax[kBlock];
   float mn = FLT_MAX, mx = -FLT_MAX;
   if (pairs > 0) {
@@ -965,8 +967,10 @@ __global__ __launch_bounds__(kBlock) void min_nz_max_kernel(const float* __restr
       out[2 + 2 * blockIdx.x] = smin[0];
       out[3 + 2 * blockIdx.x] = smax[0];
     } else {
+      const float most = (x[0] > smax[0] || x[0] != x[0]) ? x[0] : smax[0];
       out[0] = smin[0];
-      out[1] = (x[0] > smax[0] || x[0] != x[0]) ? x[0] : smax[0];
+      out[1] = most;
+      if (thr) *thr = mlem_threshold(smin[0], most);
     }
   }
 }
@@ -1717,16 +1721,18 @@ hipError_t launch_likelihood(const float* x, const float* y, long n, int positiv
   return hipGetLastError();
 }
 
-hipError_t launch_min_nz_max(const float* x, size_t n, float* d_out, hipStream_t st) {
+hipError_t launch_min_nz_max(const float* x, size_t n, float* d_out, float* d_thr, hipStream_t st) {
   if (n == 0) return hipSuccess;
   // 16 values per thread and workgroup; up to two workgroups' worth in one launch
   const size_t blocks = (n + 16 * kBlock - 1) / (16 * kBlock);
   int pairs = 0;
   if (blocks > 2) {
     pairs = (int)(blocks < (size_t)kMinMaxBlocks ? blocks : (size_t)kMinMaxBlocks);
-    hipLaunchKernelGGL(min_nz_max_kernel, dim3(pairs), dim3(kBlock), 0, st, x, (long)n, d_out, 0);
+    hipLaunchKernelGGL(min_nz_max_kernel, dim3(pairs), dim3(kBlock), 0, st, x, (long)n, d_out, 0,
+                       (float*)nullptr);
   }
-  hipLaunchKernelGGL(min_nz_max_kernel, dim3(1), dim3(kBlock), 0, st, x, (long)n, d_out, pairs);
+  hipLaunchKernelGGL(min_nz_max_kernel, dim3(1), dim3(kBlock), 0, st, x, (long)n, d_out, pairs,
+                     d_thr);
   return hipGetLastError();
 }
 
