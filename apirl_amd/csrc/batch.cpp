@@ -47,6 +47,7 @@ struct BJob {
   void* zscr = nullptr;      // 3D: backprojection scratch
   size_t zscr_bytes = 0;
   float* copy = nullptr;     // 3D: the projector's copy of the image
+  hipStream_t st = nullptr;  // where its work is queued (apirl_batch::lane)
   std::vector<std::pair<void*, size_t>> bufs;
 };
 
@@ -63,7 +64,9 @@ size_t align_up(size_t n) {
 
 struct apirl_batch {
   apirl_ctx* ctx = nullptr;
-  hipStream_t stream = nullptr;
+  hipStream_t stream = nullptr;    // the grouped rounds of the 2D jobs, and a lane of the 3D ones
+  std::vector<hipStream_t> lanes;  // the other lanes
+  unsigned next_lane = 0;
   int cap = 0, max_nsino = 0;
   int grid = 2048;
   bool use_graph = true;
@@ -101,6 +104,25 @@ void* balloc(apirl_batch* b, size_t bytes) {
   void* p = nullptr;
   if (hipMalloc(&p, bytes) != hipSuccess) return nullptr;
   return p;
+}
+
+// The next 3D job's stream.  Its whole work is queued there, in its own buffers, so the kernels
+// of one small job run beside those of others: alone, each leaves much of the GPU idle.  Eight
+// jobs of 64 x 64 x 17: 5.5 ms on one stream, 3.3 on two, 2.9 on three, 3.5 on four (a process
+// has four hardware queues, the caller's stream among them).
+constexpr unsigned kLanes = 3;
+hipStream_t lane(apirl_batch* b) {
+  const unsigned k = b->next_lane++ % kLanes;
+  if (k == 0) return b->stream;
+  while (b->lanes.size() < k) {
+    hipStream_t st;
+    if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) {
+      (void)hipGetLastError();
+      return b->stream;
+    }
+    b->lanes.push_back(st);
+  }
+  return b->lanes[k - 1];
 }
 
 void release_bufs(apirl_batch* b, BJob* j) {
@@ -201,6 +223,7 @@ apirl_status apirl_batch_create(apirl_ctx* ctx, int max_jobs, int max_sinograms,
 apirl_status apirl_batch_destroy(apirl_batch* b) {
   if (!b) return APIRL_ERR_INVALID;
   if (b->stream) (void)hipStreamSynchronize(b->stream);
+  for (hipStream_t st : b->lanes) (void)hipStreamSynchronize(st);
   for (BJob* j : b->jobs) {
     if (!j) continue;
     release_bufs(b, j);
@@ -216,6 +239,7 @@ apirl_status apirl_batch_destroy(apirl_batch* b) {
     if (b->copy_ev[i]) (void)hipEventDestroy(b->copy_ev[i]);
   }
   if (b->stream) (void)hipStreamDestroy(b->stream);
+  for (hipStream_t st : b->lanes) (void)hipStreamDestroy(st);
   delete b;
   return APIRL_OK;
 }
@@ -349,7 +373,7 @@ apirl_status apirl_batch_submit(apirl_batch* b, const apirl_job_desc* d, int* jo
     return bfail(b, APIRL_ERR_NOMEM, "cannot allocate the job's device state");
   }
   // Work of the caller's stream (inputs) comes first; the job's set-up then runs on
-  // the batch stream: sensitivity per subset (OsemSinogram3d.cpp:101-117,
+  // its stream: sensitivity per subset (OsemSinogram3d.cpp:101-117,
   // MlemSinogram3d.cpp:312-331), MLEM thresholds, and the initial image.
   apirl_ctx* c = b->ctx;
   hipEvent_t ready;
@@ -359,10 +383,11 @@ apirl_status apirl_batch_submit(apirl_batch* b, const apirl_job_desc* d, int* jo
     return bfail(b, APIRL_ERR_HIP, "event creation failed");
   }
   (void)hipEventRecord(ready, c->stream);
-  (void)hipStreamWaitEvent(b->stream, ready, 0);
+  j->st = j->is2d ? b->stream : lane(b);
+  (void)hipStreamWaitEvent(j->st, ready, 0);
   (void)hipEventDestroy(ready);
   hipStream_t saved = c->stream;
-  c->stream = b->stream;
+  c->stream = j->st;
   apirl_status st = APIRL_OK;
   j->thr.assign(j->S, 0.f);
   for (int s = 0; s < j->S && st == APIRL_OK; s++) {
@@ -371,11 +396,11 @@ apirl_status apirl_batch_submit(apirl_batch* b, const apirl_job_desc* d, int* jo
       st = apirl_sensitivity(p, d->d_mult, sens, s, j->S, APIRL_BP_GATHER, j->osem);
     } else {
       // as apirl_sensitivity computes it, in the job's own scratch
-      hipError_t e = hipMemsetAsync(sens, 0, j->nvox * sizeof(float), b->stream);
+      hipError_t e = hipMemsetAsync(sens, 0, j->nvox * sizeof(float), j->st);
       if (e == hipSuccess)
         e = backproject_job(j, d->d_mult, sens, s, d->d_mult ? BP_MULT : BP_ONES, nullptr,
-                            b->stream);
-      if (e == hipSuccess && j->osem) e = launch_force_positive(sens, j->nvox, b->stream);
+                            j->st);
+      if (e == hipSuccess && j->osem) e = launch_force_positive(sens, j->nvox, j->st);
       if (e != hipSuccess) {
         c->err = std::string("sensitivity: ") + hipGetErrorString(e);
         st = APIRL_ERR_HIP;
@@ -390,15 +415,16 @@ apirl_status apirl_batch_submit(apirl_batch* b, const apirl_job_desc* d, int* jo
     // 64 x 64, which the GPU stood still
     float* thr = j->sens + (size_t)j->S * j->nvox;
     j->thr_at = thr;
-    if (launch_min_nz_max(sens, j->nvox, thr + j->S, thr + s, b->stream) != hipSuccess)
+    if (launch_min_nz_max(sens, j->nvox, thr + j->S, thr + s, j->st) != hipSuccess)
       st = APIRL_ERR_HIP;
   }
   if (st == APIRL_OK &&
       hipMemcpyAsync(j->x, d->d_init, j->nvox * sizeof(float), hipMemcpyDeviceToDevice,
-                     b->stream) != hipSuccess)
+                     j->st) != hipSuccess)
     st = APIRL_ERR_HIP;
   c->stream = saved;
   if (st != APIRL_OK) {
+    (void)hipStreamSynchronize(j->st);  // the buffers may go to a job of another lane
     release_bufs(b, j);
     (void)hipEventDestroy(j->done_ev);
     delete j;
@@ -519,7 +545,7 @@ apirl_status apirl_batch_step(apirl_batch* b, int* active) {
       return bfail(b, APIRL_ERR_HIP, std::string("round launch failed: ") + hipGetErrorString(e));
   }
   // 3D jobs: the sub-iteration apirl_em_reconstruct runs for them (fused projection and
-  // ratio, backprojection with the update fused in), on the batch stream
+  // ratio, backprojection with the update fused in), in the job's lane
   for (auto& pr : direct) {
     BJob* j = pr.first;
     const int s = pr.second;
@@ -546,21 +572,21 @@ apirl_status apirl_batch_step(apirl_batch* b, int* active) {
       j->zscr_bytes = need;
     }
     e = launch_project(j->plan, j->x, nullptr, s, j->S, APIRL_PREC_REFERENCE, &fr, nullptr,
-                       b->stream, j->copy);
+                       j->st, j->copy);
     if (e == hipSuccess && !j->bp) {
       const EmFuse fz{sens, 0.f, j->strict, j->thr_at ? j->thr_at + s : nullptr};
-      e = backproject_job(j, j->ratio, j->x, s, BP_PLAIN, &fz, b->stream);
+      e = backproject_job(j, j->ratio, j->x, s, BP_PLAIN, &fz, j->st);
     } else if (e == hipSuccess) {
-      e = hipMemsetAsync(j->bp, 0, j->nvox * sizeof(float), b->stream);
-      if (e == hipSuccess) e = backproject_job(j, j->ratio, j->bp, s, BP_PLAIN, nullptr, b->stream);
+      e = hipMemsetAsync(j->bp, 0, j->nvox * sizeof(float), j->st);
+      if (e == hipSuccess) e = backproject_job(j, j->ratio, j->bp, s, BP_PLAIN, nullptr, j->st);
       if (e == hipSuccess)
-        e = launch_em_update(j->x, j->bp, sens, j->nvox, j->thr[s], j->strict, b->stream);
+        e = launch_em_update(j->x, j->bp, sens, j->nvox, j->thr[s], j->strict, j->st);
     }
     if (e != hipSuccess)
       return bfail(b, APIRL_ERR_HIP, std::string("3D job launch failed: ") + hipGetErrorString(e));
   }
   for (BJob* j : finishing) {
-    (void)hipEventRecord(j->done_ev, b->stream);
+    (void)hipEventRecord(j->done_ev, j->st);
     j->done_recorded = true;
     j->active = false;
     b->order.erase(std::find(b->order.begin(), b->order.end(), j->id));
@@ -583,7 +609,9 @@ apirl_status apirl_batch_job_done(apirl_batch* b, int id, int* done) {
 
 apirl_status apirl_batch_synchronize(apirl_batch* b) {
   if (!b) return APIRL_ERR_INVALID;
-  return hipStreamSynchronize(b->stream) == hipSuccess ? APIRL_OK : APIRL_ERR_HIP;
+  bool ok = hipStreamSynchronize(b->stream) == hipSuccess;
+  for (hipStream_t st : b->lanes) ok = hipStreamSynchronize(st) == hipSuccess && ok;
+  return ok ? APIRL_OK : APIRL_ERR_HIP;
 }
 
 apirl_status apirl_batch_release(apirl_batch* b, int id) {
