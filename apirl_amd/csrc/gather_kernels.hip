@@ -1920,10 +1920,15 @@ struct TileSizes {
   long nrays, npair, nvox;
 };
 
-// Wavefronts the items should come to: about three for each that the GPU holds, so that the
-// last ones to finish are a small part.
-constexpr int kTWaves = 32768;
-constexpr int kTChunkRays = 8;                   // rays per chunk at least, on average
+// Wavefronts the items should come to, by the pairs of a slot and a sinogram there are to walk.
+// Few of them and the GPU (some 4600 wavefronts with an item's LDS) is not filled, or the last
+// ones to finish are a large part; many of them and each spends its time on its own start, its
+// sums and their way through memory (nchunk images of doubles).  The best of sweeps over 44
+// subsets of 2e5 .. 8e7 pairs lay at 0.5 .. 3 times 4600, about as their 0.36th power: 2.0e5 pairs
+// 32 us at 2300 wavefronts, 52 at 9200; 6.2e6 92, 80 and 90 us at 4600, 6900 and 13800; 8.5e7
+// 1180, 623 and 618 us at 4600, 9200 and 13800.
+constexpr double kTWaves = 30.0, kTWavesPower = 0.36;
+constexpr int kTChunkRays = 4;                   // slots per chunk at least
 constexpr size_t kTPartBytes = size_t(1) << 28;  // the chunks' sums at most
 
 TileSizes tile_sizes(const apirl_plan* p, int subset, int nsubsets) {
@@ -1938,7 +1943,12 @@ TileSizes tile_sizes(const apirl_plan* p, int subset, int nsubsets) {
   z.nslot = z.nang_sub * z.maxc;
   z.zs = tile_slab_depth(p);
   z.nslab = (g.nz + z.zs - 1) / z.zs;
-  long c = kTWaves / ((long)z.ntiles * z.nslab);
+  const double waves = kTWaves * std::pow((double)z.ntiles * z.nslot * g.nsino, kTWavesPower);
+  long c = std::lround(waves / ((double)z.ntiles * z.nslab));
+  // whole eights, where there are some: a tile's chunk k then runs on XCD k % 8 in every tile and
+  // slab, whose L2 has the rays' records (33 chunks against 32: 2.22 against 2.20 ms for the 128 x 128 x
+  // 47 sensitivity, 95 against 90 us for a 55 x 55 x 50 update)
+  if (c >= 12) c = (c + 4) / 8 * 8;
   c = std::min(c, (long)z.nslot / kTChunkRays);
   c = std::min(c, (long)(kTPartBytes / (z.nvox * sizeof(double))));
   z.nchunk = c < 1 ? 1 : (int)c;
