@@ -79,3 +79,24 @@ def test_path_projector_compensated_sums(torch, ctx, name):
                 total, mag = total + t, mag + abs(t)
         # Kahan's bound, 2 eps + O(n eps^2) of the terms' magnitudes, eps = 2^-24
         assert abs(float(got[s, a, q]) - total) <= 3 * 2.0 ** -24 * mag
+
+
+@pytest.mark.parametrize("precision", ["PREC_KAHAN", "PREC_F64_SETUP"])
+def test_path_projector_equals_ray_per_lane(torch, ctx, precision):
+    """A long enough projection of more than 112 sinograms takes the path in these precisions,
+    its single angles a ray per lane: the same bins, bit for bit."""
+    log(f"case: path against ray per lane, {precision}")
+    rng = np.random.default_rng(5)
+    nx, nz, nang, nr, nsino = 190, 21, 9, 240, 130
+    mid = np.sort(rng.uniform(1.0, 41.0, nsino))
+    half = rng.uniform(-15.0, 15.0, nsino)
+    p = hip.Plan(ctx, nx, nx, nz, 2.0, 2.0, nang, nr, nx * 1.0, 300.0,
+                 z1=(mid - half).astype(np.float32), z2=(mid + half).astype(np.float32),
+                 ring_width=np.float32(2.0))
+    assert nsino * nang * nr * 2 * nx >= 1e8 > nsino * nr * 2 * nx
+    x = dev(torch, rng.random((nz, nx, nx), dtype=np.float32))
+    prec = getattr(hip, precision)
+    whole = host(p.project(x, precision=prec))
+    for a in range(nang):
+        one = host(p.project(x, subset=a, nsubsets=nang, precision=prec))
+        assert np.array_equal(one.view(np.int32)[:, 0], whole.view(np.int32)[:, a])
