@@ -252,6 +252,10 @@ hipError_t launch_force_positive(float* x, size_t n, hipStream_t st);
 hipError_t launch_divide_rule(const float* meas, const float* est, float* out, size_t n,
                               int dims, hipStream_t st);
 hipError_t launch_sum_partials(const double* partials, int n, double* out, hipStream_t st);
+// Sums of rows of partials, stride apart: row r's first nmore where r % nsubsets < more, its
+// first nless otherwise, to out[r], each in launch_sum_partials' order.
+hipError_t launch_sum_partials_rows(const double* partials, int rows, long stride, int nsubsets,
+                                    int more, int nmore, int nless, double* out, hipStream_t st);
 // Partials of apirl_project_ratio_noalloc: a file-scope device array of
 // siddon_kernels.hip of kNoallocPartials doubles (one per workgroup of 256 bins).
 constexpr int kNoallocPartials = 1 << 19;

@@ -915,9 +915,15 @@ __global__ __launch_bounds__(kBlock) void force_positive_kernel(float* __restric
 }
 
 // Fixed-order sum of block partials (one block): deterministic for a given count.
+// Row r = blockIdx.x of the partials (stride of them; nmore used where r % nsubsets < more, nless
+// otherwise) to out[r].
 __global__ __launch_bounds__(kBlock) void sum_partials_kernel(const double* __restrict__ p,
-                                                              int n, double* __restrict__ out) {
+                                                              long stride, int nsubsets, int more,
+                                                              int nmore, int nless,
+                                                              double* __restrict__ out) {
   __shared__ double red[kBlock];
+  const int n = (int)(blockIdx.x % nsubsets) < more ? nmore : nless;
+  p += (long)blockIdx.x * stride;
   double acc = 0.0;
   for (int i = threadIdx.x; i < n; i += kBlock) acc += p[i];
   red[threadIdx.x] = acc;
@@ -926,7 +932,7 @@ __global__ __launch_bounds__(kBlock) void sum_partials_kernel(const double* __re
     if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];
     __syncthreads();
   }
-  if (threadIdx.x == 0) *out = red[0];
+  if (threadIdx.x == 0) out[blockIdx.x] = red[0];
 }
 
 // Minimum of the non-zero values and maximum (Images.cpp:397-431).  Both are
@@ -1703,21 +1709,28 @@ hipError_t noalloc_scratch_address(double** out) {
 }
 
 hipError_t launch_sum_partials(const double* partials, int n, double* out, hipStream_t st) {
-  hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(kBlock), 0, st, partials, n, out);
+  return launch_sum_partials_rows(partials, 1, n, 1, 0, n, n, out, st);
+}
+
+hipError_t launch_sum_partials_rows(const double* partials, int rows, long stride, int nsubsets,
+                                    int more, int nmore, int nless, double* out, hipStream_t st) {
+  hipLaunchKernelGGL(sum_partials_kernel, dim3(rows), dim3(kBlock), 0, st, partials, stride,
+                     nsubsets, more, nmore, nless, out);
   return hipGetLastError();
 }
 
 hipError_t launch_likelihood(const float* x, const float* y, long n, int positive_only,
                              double* partials, double* out, hipStream_t st) {
   if (n <= 0) {
-    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(kBlock), 0, st, partials, 0, out);
+    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(kBlock), 0, st, partials, 0L, 1, 0, 0,
+                       0, out);
     return hipGetLastError();
   }
   const unsigned grid = grid_for(n);
   hipLaunchKernelGGL(likelihood_kernel, dim3(grid), dim3(kBlock), 0, st, x, y, n,
                      positive_only, partials);
-  hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(kBlock), 0, st, partials, (int)grid,
-                     out);
+  hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(kBlock), 0, st, partials, 0L, 1, 0, 0,
+                     (int)grid, out);
   return hipGetLastError();
 }
 
