@@ -19,7 +19,7 @@ ARCH = os.environ.get("APIRL_OFFLOAD_ARCH", "gfx950")
 # -ffp-contract=off: no fused multiply-add anywhere, so every floor() at a voxel face
 #   and every weight rounds as in the reference's float code.
 # correctly rounded fp32 division / sqrt (the reference runs on IEEE x86 SSE).
-# packed-fp32 instructions disabled (v_pk_* fp32 forms are avoided on this pool).
+# packed-fp32 instructions disabled: some v_pk_* fp32 forms have given wrong results.
 COMMON = ["-O3", "-fPIC", "-std=c++17", "-ffp-contract=off", "-Wall", "-Wno-unused-function",
           "-I" + os.path.join(ROOT, "include"), "-I" + CSRC]
 DEVICE = ["--offload-arch=" + ARCH, "-fhip-fp32-correctly-rounded-divide-sqrt",

@@ -1,10 +1,13 @@
 // gfx950 kernels of the Siddon projector / backprojector and the EM update.
 //
-// One ray per lane.  Lanes of a wavefront take consecutive radial bins of one
-// (sinogram, angle), so the 64-byte RayXY records, the measured / additive bins and
-// the sinogram writes are contiguous per wavefront, and the 64 rays are parallel
-// neighbours whose voxel gathers hit the same cache lines of the (L2 / MALL
-// resident) image.  The path is gather/scatter bound; no MFMA is involved.
+// Three forward projectors: the path projector (3D; the rays of one angle and bin in
+// every sinogram share a path), the 2D one (64 rays a workgroup, their steps shared out
+// over its wavefronts) and, for what those do not take, one ray per lane: lanes of a
+// wavefront take consecutive radial bins of one (sinogram, angle), so the 64-byte RayXY
+// records, the measured / additive bins and the sinogram writes are contiguous per
+// wavefront, and the 64 rays are parallel neighbours whose voxel gathers hit the same
+// cache lines of the (L2 / MALL resident) image.  No MFMA is involved: a ray's sum has
+// one order.
 //
 // Arithmetic follows recon/src/Siddon.cpp in float, operation by operation, and the
 // file is compiled with -ffp-contract=off and correctly rounded division / sqrt, so
@@ -939,8 +942,8 @@ __global__ __launch_bounds__(kBlock) void sum_partials_kernel(const double* __re
 // order-independent, so the result is exact.  A launch of one workgroup gives out[0] = min_nz,
 // out[1] = max; the reference's maximum starts from pixel 0, so a NaN there is kept.  A launch
 // of more leaves a pair per workgroup after them, which a second launch of one takes in place
-// of x (pairs > 0).  One workgroup took 5.7 ms for 256x256x81 voxels, the two launches 19 us (128x128x47:
-// 346 and 10 us).
+// of x (pairs > 0).  One workgroup took 5.7 ms for 256x256x81 voxels and 346 us for 128x128x47,
+// the two launches 14 and 10 us.
 __global__ __launch_bounds__(kBlock) void min_nz_max_kernel(const float* __restrict__ x, long n,
                                                             float* __restrict__ out, int pairs,
                                                             float* __restrict__ thr) {
@@ -1497,6 +1500,8 @@ bool path_forward_ok(const apirl_plan* p, int precision, int subset, int nsubset
   if (precision != APIRL_PREC_REFERENCE) {
     const double rays = (double)g.nsino * subset_num_angles(g.nang, nsubsets, subset) * g.nr;
     if (g.nsino <= kPathMinSino || rays * (g.nx + g.ny) < kPathMinWork) return false;
+    // a likelihood partial per (angle, bin) then, where a ray per lane has one per 256 bins
+    if (rays > (double)kNoallocPartials * g.nsino) return false;
   }
   // the columns of an entry are kept in 16 bits each, a voxel's byte address in 32
   return g.dims == 3 && precision != APIRL_PREC_F64_ALPHA && g.ns * g.nas == 1 && g.walk24 &&

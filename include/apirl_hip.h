@@ -35,14 +35,19 @@ typedef enum apirl_status {
 
 /* Backprojection forms. */
 enum {
-  APIRL_BP_SCATTER = 0, /* ray-driven, fp32 atomics into image copies: order not fixed */
-  APIRL_BP_GATHER = 1,  /* voxel-driven, fixed order: deterministic; in 2D equal, bit for
-                           bit, to the reference's single-thread result; in 3D the same
-                           float terms summed in (angle, bin, segment, sinogram) order */
+  APIRL_BP_SCATTER = 0, /* any plan.  APIRL_PREC_REFERENCE only: 2D as the gather, 3D as the
+                           tile form, where those take the plan; otherwise (and in the
+                           divide rule) ray-driven, fp32 atomics into image copies, order
+                           not fixed */
+  APIRL_BP_GATHER = 1,  /* deterministic; in 2D equal, bit for bit, to the reference's
+                           single-thread result; in 3D the tile form for
+                           APIRL_PREC_REFERENCE where it takes the plan, and voxel-driven
+                           otherwise: the same float terms in (angle, bin, segment,
+                           sinogram) order */
   APIRL_BP_TILE = 2     /* 3D, APIRL_PREC_REFERENCE: ray-driven walks clipped to tiles of
-                           8 x 8 columns by a slab of slices, summed in LDS by one
-                           wavefront per tile (no global atomics): deterministic, the
-                           same float terms in the wavefront's order */
+                           8 x 8 columns by a slab of slices, summed in LDS in double by
+                           one wavefront per tile, slab and share of the rays (no global
+                           atomics): deterministic, the reference's float terms */
 };
 
 /* Arithmetic of the projector and of the gather backprojector. */
@@ -130,18 +135,16 @@ apirl_status apirl_plan_intersections(apirl_plan* plan, int subset, int nsubsets
  *                  gathers V consecutive voxels of a column, sharing each candidate
  *                  ray's transaxial tests and sinogram search among them (float
  *                  precision modes; APIRL_PREC_F64_ALPHA always uses 1).
- *   tile_zs:       slices per item of the tile backprojector (APIRL_BP_TILE; default
- *                  about 5).
+ *   tile_zs:       slices per item of the tile backprojector (default: all of up to 13,
+ *                  otherwise about 12).
  *   tile_cache_mb: device memory (MiB, default 16384) in which the plan keeps the
  *                  tile backprojector's per-subset geometry from its first call on:
- *                  the candidate rays of every 8 x 8-column tile with their paths, and
- *                  for each (tile, slab, ray) the sinograms that reach the slab inside
- *                  the tile (2 bytes each), which later calls read instead of listing
- *                  them.  -1 keeps none and frees what is kept; a subset beyond the
- *                  budget is rebuilt on every call.  The first call on a subset waits
- *                  for the stream once (to size its lists).
- * Gather results do not depend on these (the per-voxel summation order is fixed);
- * tile results are deterministic for a given tile_zs, kept geometry or not.
+ *                  the rays that enter every 8 x 8-column tile with their paths.  -1
+ *                  keeps none and frees what is kept; a subset beyond the budget is
+ *                  rebuilt on every call.
+ * The gather_ fields shape the voxel-driven kernels, whose results do not depend on them
+ * (the per-voxel summation order is fixed); tile results, which are double sums rounded
+ * once, are deterministic for a given tile_zs, kept geometry or not.
  * Zero in a field leaves it unchanged. */
 typedef struct apirl_tuning {
   int gather_zlanes;
@@ -207,9 +210,10 @@ apirl_status apirl_project(apirl_plan* plan, const float* d_img, float* d_sino, 
 /* Backproject: d_img += A^T d_sino (accumulates; the caller zeroes, Mlem2d.cpp:162).
  * Replaces SiddonProjector::Backproject (2D :34-87, 3D :444-568).  precision applies
  * to the gather form: APIRL_PREC_REFERENCE sums the reference's float weights in
- * float, APIRL_PREC_KAHAN with a compensation term, APIRL_PREC_F64 computes the
- * crossings and sums in double; the scatter form takes APIRL_PREC_REFERENCE only and
- * allocates its 16 per-XCD image copies on its first call on a plan. */
+ * float (2D) or double (3D, the tile form), APIRL_PREC_KAHAN with a compensation term,
+ * APIRL_PREC_F64 computes the crossings and sums in double; the scatter form takes
+ * APIRL_PREC_REFERENCE only and allocates its 16 per-XCD image copies on its first call
+ * on a plan that needs them. */
 apirl_status apirl_backproject(apirl_plan* plan, const float* d_sino, float* d_img, int subset,
                                int nsubsets, int mode, int precision);
 /* The backprojection fused with the EM update that consumes it (Backproject, then
@@ -319,12 +323,13 @@ apirl_status apirl_em_reconstruct_timed(apirl_plan* plan, const apirl_em_options
  * No counterpart in the reference, whose EM drivers run one job at a time
  * (OsemSinogram3d.cpp:36-325, Mlem2d.cpp:60-260).  A batch advances many OSEM / MLEM
  * jobs of different geometries together: each apirl_batch_step enqueues one round,
- * one sub-iteration of every active job, as seven grouped launches (clear, fused
- * projection + ratio, axial setup, gather backprojection, update) replayed from a
- * captured hipGraph.  Jobs may be submitted between steps while others are running.
+ * one sub-iteration of every active job: the 2D jobs' as two grouped launches (fused
+ * projection + ratio, gather backprojection with the update) replayed from a captured
+ * hipGraph, each 3D job's with the single-job kernels in its own buffers, on one of
+ * three streams.  Jobs may be submitted between steps while others are running.
  * A job's image has the same bits as apirl_em_reconstruct with APIRL_BP_GATHER and
  * APIRL_PREC_REFERENCE gives it alone; the likelihood is not evaluated.  The batch
- * runs on its own stream; apirl_batch_submit orders the job after the work already
+ * runs on its own streams; apirl_batch_submit orders the job after the work already
  * enqueued on the context's stream, and the image is final once apirl_batch_job_done
  * reports it. */
 typedef struct apirl_batch apirl_batch;
@@ -339,24 +344,25 @@ typedef struct apirl_job_desc {
   float* d_out;             /* image, updated in place every sub-iteration */
   int additive_own_angles;  /* as apirl_em_options.additive_own_angles */
 } apirl_job_desc;
-/* max_sinograms bounds the 3D jobs' sinogram count (LDS of the gather launch). */
+/* max_sinograms bounds the 3D jobs' sinogram count. */
 apirl_status apirl_batch_create(apirl_ctx* ctx, int max_jobs, int max_sinograms,
                                 apirl_batch** out);
 apirl_status apirl_batch_destroy(apirl_batch* batch);
 const char* apirl_batch_last_error(const apirl_batch* batch);
-/* Device memory a job of this plan holds while admitted (sensitivities, ratio,
- * backprojection, gather records), for admission by HBM footprint. */
+/* Device memory a job of this plan holds while admitted (sensitivities and thresholds,
+ * ratio, 3D: backprojection scratch and a copy of the image), for admission by HBM
+ * footprint. */
 size_t apirl_batch_job_bytes(const apirl_plan* plan, int subsets);
 /* The backprojector a batch runs a job of this plan with: APIRL_BP_TILE for 3D jobs of
- * 2^21 voxels or more with one LOR per bin that the tile form takes (they run with the
- * single-job kernels after each grouped round), else APIRL_BP_GATHER.  A batched job's
+ * 2^21 voxels or more with one LOR per bin that the tile form takes, else
+ * APIRL_BP_GATHER (in 3D the same form where that takes the plan).  A batched job's
  * image equals apirl_em_reconstruct's with that bp_mode, bit for bit. */
 int apirl_batch_job_backprojector(const apirl_plan* plan);
 /* Workgroups per grouped launch (0 keeps the current value) and graph replay on/off. */
 apirl_status apirl_batch_set_launch(apirl_batch* batch, int grid, int use_graph);
 /* Scheduling of the grouped launches (no reference counterpart: the batch engine is
- * this library's own): `grab` virtual blocks (256 rays, 256 voxels or one gather
- * tile each) per draw from a phase's work counter (1..64, default 2), and the order
+ * this library's own): `grab` virtual blocks (64 rays or one 8 x 8 patch of voxels
+ * each) per draw from a phase's work counter (1..64, default 2), and the order
  * in which the jobs' blocks are laid out in a round.  Results do not depend on
  * either; serving.autotune picks them by timing live rounds. */
 #define APIRL_BATCH_ORDER_SUBMISSION 0
