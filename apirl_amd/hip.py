@@ -316,7 +316,8 @@ class Plan:
 
     def set_tuning(self, **fields):
         """Sets apirl_tuning fields (gather_zlanes, gather_zvox, gather_xcd, tile_zs,
-        tile_cache_mb: -1 keeps no tile geometry); gather results do not depend on them."""
+        tile_cache_mb: -1 keeps no tile geometry); the voxel-driven kernels' results do not
+        depend on the gather_ fields."""
         t = Tuning(**{k: int(v) for k, v in fields.items()})
         self.ctx.check(self.ctx.lib.apirl_plan_set_tuning(self.h, ctypes.byref(t)),
                        "apirl_plan_set_tuning")
