@@ -304,7 +304,11 @@ apirl_status tile_backproject(apirl_plan* p, const float* sino, float* img, int 
   const size_t need = apirl::tile_scratch_bytes(p, subset, nsubsets, tg == nullptr);
   if ((need > p->gscratch_bytes || !p->d_tile_order) && capturing(c->stream))
     return fail(c, APIRL_ERR_NOMEM, "the gather scratch cannot be allocated during a capture");
-  if (!ensure_gscratch(p, need))
+  // with room for the geometry of the plan's largest subset, so that a capture of a subset, or
+  // on a stream, whose kept geometry cannot be read in it builds its own
+  const size_t most = apirl::tile_scratch_bytes(p, 0, nsubsets, true);
+  if (need > p->gscratch_bytes && !ensure_gscratch(p, std::max(need, most)) &&
+      !ensure_gscratch(p, need))
     return fail(c, APIRL_ERR_NOMEM, "cannot allocate the gather scratch");
   if (!ensure_tile_order(p))
     return fail(c, APIRL_ERR_NOMEM, "cannot allocate the tile backprojector's item order");
