@@ -1490,15 +1490,26 @@ __global__ __launch_bounds__(kBlock, PREC == APIRL_PREC_REFERENCE ? 8 : 7) void 
 // path at 23 sinograms 137 / 341 us, at 35 84 / 146) and where the whole launch is short, by its
 // rays times the columns of a long one: 61 / 70 us at 5e7, 54 / 61 at 7e7, 60 / 63 at 9e7, against
 // 96 / 96 at 1.4e8, 111 / 98 at 1.5e8, 217 / 110 at 2.0e8, 686 / 431 at 1.0e9 (113 sinograms).
-// The reference arithmetic is ahead on the path at any number (80 / 52 us at 19 sinograms,
-// 372 / 158 at 47).
 constexpr int kPathMinSino = 112;
 constexpr double kPathMinWork = 1.0e8;
+// The reference arithmetic's path is dearer than a ray per lane only where few of its 64 lanes
+// are filled and the 64 neighbouring bins of a ray per lane lie close enough to read the same
+// lines: sinograms times the bins' spacing in voxels up to 40, the spacing up to 1.25.  Ray per
+// lane / path: 121 / 313 us for 27 sinograms of 20100 bins at 0.7 voxels, 33 / 66 for 21 of 10010
+// at 0.2, 96 / 153 for 47 of 9641 at 0.5, 64 / 67 for 57 of 9164 at 0.7; but 104 / 72 for 21 of
+// 2695 at 2.6, 86 / 80 for 113 of 5800 at 0.5, 36 / 32 for 55 of 1020 at 0.9, 383 / 336 for 141 at
+// 0.9.  Short launches, by rays times columns, keep the path (27 / 24 us at 4e6).
+constexpr double kPathMaxBins = 40, kPathMaxSpacing = 1.25, kRayMinWork = 5.0e6;
 
 bool path_forward_ok(const apirl_plan* p, int precision, int subset, int nsubsets) {
   const Geo& g = p->geo;
-  if (precision != APIRL_PREC_REFERENCE) {
-    const double rays = (double)g.nsino * subset_num_angles(g.nang, nsubsets, subset) * g.nr;
+  const double rays = (double)g.nsino * subset_num_angles(g.nang, nsubsets, subset) * g.nr;
+  if (precision == APIRL_PREC_REFERENCE) {
+    const double spacing = (double)g.dr / g.dx;
+    if (spacing <= kPathMaxSpacing && g.nsino * spacing <= kPathMaxBins &&
+        rays * (g.nx + g.ny) >= kRayMinWork)
+      return false;
+  } else {
     if (g.nsino <= kPathMinSino || rays * (g.nx + g.ny) < kPathMinWork) return false;
     // a likelihood partial per (angle, bin) then, where a ray per lane has one per 256 bins
     if (rays > (double)kNoallocPartials * g.nsino) return false;

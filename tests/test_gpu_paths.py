@@ -100,3 +100,30 @@ def test_path_projector_equals_ray_per_lane(torch, ctx, precision):
     for a in range(nang):
         one = host(p.project(x, subset=a, nsubsets=nang, precision=prec))
         assert np.array_equal(one.view(np.int32)[:, 0], whole.view(np.int32)[:, a])
+
+
+def test_few_sinograms_equal_path_and_ray_per_lane(torch, ctx):
+    """A projection of few sinograms of close bins takes a ray per lane, its single angles the
+    path: the same bins, bit for bit."""
+    log("case: path against ray per lane, reference arithmetic")
+    rng = np.random.default_rng(6)
+    nx, nz, nang, nr, nsino = 100, 15, 12, 120, 40
+    mid = np.sort(rng.uniform(1.0, 29.0, nsino))
+    half = rng.uniform(-10.0, 10.0, nsino)
+    p = hip.Plan(ctx, nx, nx, nz, 2.0, 2.0, nang, nr, nx * 1.0, 300.0,
+                 z1=(mid - half).astype(np.float32), z2=(mid + half).astype(np.float32),
+                 ring_width=np.float32(2.0))
+    assert nsino * nang * nr * 2 * nx >= 5e6 > nsino * nr * 2 * nx
+    x = dev(torch, rng.random((nz, nx, nx), dtype=np.float32))
+    whole = host(p.project(x))
+    meas = dev(torch, rng.poisson(3.0, whole.shape).astype(np.float32))
+    ratio, lik = p.project_ratio(x, meas)
+    total = 0.0
+    for a in range(nang):
+        one = host(p.project(x, subset=a, nsubsets=nang))
+        assert np.array_equal(one.view(np.int32)[:, 0], whole.view(np.int32)[:, a])
+        part, l1 = p.project_ratio(x, meas, subset=a, nsubsets=nang)
+        assert np.array_equal(host(part).view(np.int32)[:, 0], host(ratio).view(np.int32)[:, a])
+        total += float(l1)
+    # the same terms summed in double, in another order
+    assert abs(float(lik) - total) <= 1e-9 * abs(total)
