@@ -929,6 +929,9 @@ __device__ __forceinline__ void gather2_terms(const GatherArgs& A, const G2Plan&
   const int slot0 = (int)(unsigned)(uintptr_t)(lds_bytes)(char*)(T + al * q.slots * P * P) / kSlot;
   const int ulo = slot0 << 16, uhi = ulo + (q.slots << 16) - 1;
   for (int rr = p0 + rl; rr <= p1; rr += q.rays) {
+    const float b = A.kind == BP_PLAIN ? A.sino[(long)ka * g.nr + rr]
+                                       : (A.kind == BP_MULT ? A.sino[(long)a * g.nr + rr] : 1.f);
+    if (b == 0.f) continue;  // its terms are 0, as its slots are
     const float4* ray = reinterpret_cast<const float4*>(A.rays + (long)a * g.nr + rr);
     const float4 q1 = ray[1], q2 = ray[2], q3 = ray[3];
     const float amin = q1.x, ax = q1.z, ay = q1.w, axu = q2.x, ayu = q2.y, len = q3.w;
@@ -944,8 +947,6 @@ __device__ __forceinline__ void gather2_terms(const GatherArgs& A, const G2Plan&
     ok &= (iinc != 0) | (ic == i0);
     ok &= (jinc != 0) | (jc == j0);
     if (!ok) continue;
-    const float b = A.kind == BP_PLAIN ? A.sino[(long)ka * g.nr + rr]
-                                       : (A.kind == BP_MULT ? A.sino[(long)a * g.nr + rr] : 1.f);
     const float* xytab = A.xytab + ((long)a * g.nr + rr) * (g.nx + g.ny);
     const float Xi = na > 0 ? xytab[ic] : -FLT_MAX, Yi = nb > 0 ? xytab[g.nx + jc] : -FLT_MAX;
     float X = na > 0 ? Xi + axu : ax, Y = nb > 0 ? Yi + ayu : ay;
