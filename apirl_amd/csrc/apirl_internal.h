@@ -286,13 +286,16 @@ hipError_t launch_count_intersections(const apirl_plan* p, int subset, int nsubs
                                       unsigned long long* d_out, hipStream_t st);
 
 // The EM update a gather can apply to its voxels instead of storing their
-// backprojection (GatherArgs::upd_sens): img is then the image being updated.
+// backprojection (GatherArgs::upd_sens): img is then the image being updated.  Or, with fresh
+// (GatherArgs::fresh) and no sens, how a backprojection is stored whose image need not be cleared.
 struct EmFuse {
   const float* sens;
   float thr;
   int strict;
   const float* thr_at = nullptr;  // device: the threshold, in place of thr
+  int fresh = 0;
 };
+constexpr int kFresh = 1, kFreshPositive = 2;  // as it is; forcePositive applied
 // The 2D gather by patches runs this subset's backprojection; the scatter form, whose atomics it
 // outruns everywhere (34 / 19 us for 32 x 32 from 8 x 40 bins, 319 / 82 from 252 x 344; 164 / 20
 // for 256 x 256 from 24 x 76, 531 / 99 from 252 x 320), then does too.
@@ -414,6 +417,8 @@ struct GatherArgs {
   // then the image x, and each voxel's backprojection b, summed from zero, updates it
   // to (s > thr or, not strict, s >= thr) ? (x b) / s : 0 with s = upd_sens[v]
   const float* upd_sens;
+  // not 0: img takes the backprojection itself, whatever it held (kFresh, kFreshPositive)
+  int fresh;
   float upd_thr;
   const float* upd_thr_at;  // null, or (device) the threshold in place of upd_thr
   int upd_strict;

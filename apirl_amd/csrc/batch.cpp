@@ -396,11 +396,13 @@ apirl_status apirl_batch_submit(apirl_batch* b, const apirl_job_desc* d, int* jo
       st = apirl_sensitivity(p, d->d_mult, sens, s, j->S, APIRL_BP_GATHER, j->osem);
     } else {
       // as apirl_sensitivity computes it, in the job's own scratch
-      hipError_t e = hipMemsetAsync(sens, 0, j->nvox * sizeof(float), j->st);
+      EmFuse fz{nullptr, 0.f, 0};
+      fz.fresh = j->osem ? kFreshPositive : kFresh;
+      hipError_t e = os ? hipMemsetAsync(sens, 0, j->nvox * sizeof(float), j->st) : hipSuccess;
       if (e == hipSuccess)
-        e = backproject_job(j, d->d_mult, sens, s, d->d_mult ? BP_MULT : BP_ONES, nullptr,
-                            j->st);
-      if (e == hipSuccess && j->osem) e = launch_force_positive(sens, j->nvox, j->st);
+        e = backproject_job(j, d->d_mult, sens, s, d->d_mult ? BP_MULT : BP_ONES,
+                            os ? nullptr : &fz, j->st);
+      if (e == hipSuccess && os && j->osem) e = launch_force_positive(sens, j->nvox, j->st);
       if (e != hipSuccess) {
         c->err = std::string("sensitivity: ") + hipGetErrorString(e);
         st = APIRL_ERR_HIP;

@@ -318,8 +318,8 @@ apirl_status tile_backproject(apirl_plan* p, const float* sino, float* img, int 
   return APIRL_OK;
 }
 
-// fuse (gather form, one LOR per bin): img is the EM image, updated by each voxel's
-// backprojection instead of accumulating it
+// fuse (one LOR per bin): img is the EM image (not in the scatter form), updated by each voxel's
+// backprojection instead of accumulating it, or takes the backprojection itself (EmFuse::fresh)
 apirl_status backproject_any(apirl_plan* p, const float* sino, const float* est, float* img,
                              int subset, int nsubsets, int kind, int mode,
                              int precision = APIRL_PREC_REFERENCE,
@@ -334,14 +334,16 @@ apirl_status backproject_any(apirl_plan* p, const float* sino, const float* est,
     if (kind != apirl::BP_DIVIDE && tile_takes(p, subset, nsubsets)) {
       // DivideAndBackproject keeps its own bounds rule (BP_DIVIDE in the scatter kernel)
       bool done = false;
-      const apirl_status st = tile_backproject(p, sino, img, subset, nsubsets, kind, nullptr, done);
+      const apirl_status st = tile_backproject(p, sino, img, subset, nsubsets, kind, fuse, done);
       if (done) return st;
     }
     if (kind != apirl::BP_DIVIDE && apirl::gather2_takes(p, subset, nsubsets)) {
       APIRL_HIP(c, apirl::launch_backproject_gather(p, sino, img, subset, nsubsets, kind,
-                                                    precision, nullptr, 0, c->stream, nullptr));
+                                                    precision, nullptr, 0, c->stream, fuse));
       return APIRL_OK;
     }
+    const size_t nvox = apirl_plan_image_voxels(p);
+    if (fuse) APIRL_HIP(c, hipMemsetAsync(img, 0, nvox * sizeof(float), c->stream));
     if (!p->d_replicas && !p->replicas_failed) {
       // the per-XCD scatter targets (16 image copies), zeroed here and re-zeroed by
       // the reduction after every use; without them the atomics go to the image
@@ -359,6 +361,8 @@ apirl_status backproject_any(apirl_plan* p, const float* sino, const float* est,
     }
     APIRL_HIP(c, apirl::launch_backproject(p, sino, est, img, subset, nsubsets, kind, mode,
                                            c->stream));
+    if (fuse && fuse->fresh == apirl::kFreshPositive)
+      APIRL_HIP(c, apirl::launch_force_positive(img, nvox, c->stream));
     return APIRL_OK;
   }
   if (mode != APIRL_BP_GATHER && mode != APIRL_BP_TILE)
@@ -1121,9 +1125,17 @@ apirl_status sensitivity_impl(apirl_plan* p, const float* d_mult, float* d_sens,
   apirl_ctx* c = p->ctx;
   DeviceGuard g(c->device);
   const size_t nvox = apirl_plan_image_voxels(p);
+  const int kind = d_mult ? apirl::BP_MULT : apirl::BP_ONES;
+  if (p->geo.ns * p->geo.nas == 1 && apirl_plan_subset_bins(p, subset, nsubsets) > 0) {
+    // stored as it is, clamped if asked for: a clear and a pass over the image less
+    apirl::EmFuse fz{nullptr, 0.f, 0};
+    fz.fresh = force_positive ? apirl::kFreshPositive : apirl::kFresh;
+    return backproject_any(p, d_mult, nullptr, d_sens, subset, nsubsets, kind, mode, precision,
+                           &fz);
+  }
   APIRL_HIP(c, hipMemsetAsync(d_sens, 0, nvox * sizeof(float), c->stream));
-  apirl_status st = backproject_any(p, d_mult, nullptr, d_sens, subset, nsubsets,
-                                    d_mult ? apirl::BP_MULT : apirl::BP_ONES, mode, precision);
+  apirl_status st = backproject_any(p, d_mult, nullptr, d_sens, subset, nsubsets, kind, mode,
+                                    precision);
   if (st != APIRL_OK) return st;
   if (force_positive) APIRL_HIP(c, apirl::launch_force_positive(d_sens, nvox, c->stream));
   return APIRL_OK;
