@@ -417,7 +417,8 @@ struct GatherArgs {
   // then the image x, and each voxel's backprojection b, summed from zero, updates it
   // to (s > thr or, not strict, s >= thr) ? (x b) / s : 0 with s = upd_sens[v]
   const float* upd_sens;
-  // not 0: img takes the backprojection itself, whatever it held (kFresh, kFreshPositive)
+  // not 0: the sums start from zero, not from img (kFresh, as with upd_sens; kFreshPositive);
+  // APIRL_PREC_REFERENCE only
   int fresh;
   float upd_thr;
   const float* upd_thr_at;  // null, or (device) the threshold in place of upd_thr

@@ -515,6 +515,7 @@ apirl_status apirl_batch_step(apirl_batch* b, int* active) {
       int* unused_nz = nullptr;
       gather_args_for(p, s, S, BP_PLAIN, j->ratio, j->x, nullptr, q.A, unused_zr, unused_nz);
       q.A.upd_sens = j->sens + (size_t)s * j->nvox;
+      q.A.fresh = kFresh;
       if (j->thr_at) q.A.upd_thr_at = j->thr_at + s;
       q.A.upd_strict = j->strict;
       q.ntx = (g.nx + kPatch2 - 1) / kPatch2;

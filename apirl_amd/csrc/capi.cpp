@@ -1126,7 +1126,8 @@ apirl_status sensitivity_impl(apirl_plan* p, const float* d_mult, float* d_sens,
   DeviceGuard g(c->device);
   const size_t nvox = apirl_plan_image_voxels(p);
   const int kind = d_mult ? apirl::BP_MULT : apirl::BP_ONES;
-  if (p->geo.ns * p->geo.nas == 1 && apirl_plan_subset_bins(p, subset, nsubsets) > 0) {
+  if (precision == APIRL_PREC_REFERENCE && p->geo.ns * p->geo.nas == 1 &&
+      apirl_plan_subset_bins(p, subset, nsubsets) > 0) {
     // stored as it is, clamped if asked for: a clear and a pass over the image less
     apirl::EmFuse fz{nullptr, 0.f, 0};
     fz.fresh = force_positive ? apirl::kFreshPositive : apirl::kFresh;
