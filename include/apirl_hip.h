@@ -140,8 +140,9 @@ apirl_status apirl_plan_intersections(apirl_plan* plan, int subset, int nsubsets
  *   tile_cache_mb: device memory (MiB, default 16384) in which the plan keeps the
  *                  tile backprojector's per-subset geometry from its first call on:
  *                  the rays that enter every 8 x 8-column tile with their paths.  -1
- *                  keeps none and frees what is kept; a subset beyond the budget is
- *                  rebuilt on every call.
+ *                  keeps none and frees what is kept (graphs captured over it must not
+ *                  be replayed then); a subset beyond the budget is rebuilt on every
+ *                  call.
  * The gather_ fields shape the voxel-driven kernels, whose results do not depend on them
  * (the per-voxel summation order is fixed); tile results, which are double sums rounded
  * once, are deterministic for a given tile_zs, kept geometry or not.
