@@ -265,7 +265,7 @@ hipError_t tile_run(apirl_plan* p, const float* sino, float* img, int subset, in
 // A plan's backprojections in the reference arithmetic, whichever form is asked for, are run
 // by the tile backprojector where it takes the plan: it adds the same float terms, in double,
 // in a fixed order.  12-angle subset of the 256x256x81 / 344x252x837 workload, every bin
-// non-zero: 1.8 ms, the gather's column kernel 4.2 ms, the scatter's atomics 22 ms; 12 angles
+// non-zero: 1.5 ms, the gather's column kernel 4.2 ms, the scatter's atomics 22 ms; 12 angles
 // of 122x84x73 on 64x64x17: 0.05, 0.40 and 0.20 ms.
 bool tile_takes(const apirl_plan* p, int subset, int nsubsets) {
   return p->gather_ok && !apirl::gather_misfit(p, subset, nsubsets) && !apirl::tile_misfit(p);

@@ -1,8 +1,8 @@
 // Deterministic backprojectors for gfx950: the voxel-driven gather, the 2D gather by patches and
 // the 3D tile-walk form (each described at its kernels).
 //
-// The voxel-driven gather: one voxel per lane.  For each angle of the subset the lane finds the contiguous
-// radial bins whose LOR can cross its voxel column, and for 3D, per segment, the
+// The voxel-driven gather: one voxel per lane.  For each angle of the subset the lane finds the
+// contiguous radial bins whose LOR can cross its voxel column, and for 3D, per segment, the
 // contiguous range of sinograms whose ray can cross its slice.  For every candidate
 // ray it reconstructs, without walking the ray, the state the reference's Siddon
 // loop would be in when it emits this voxel (recon/src/Siddon.cpp:310-340, 615-639):
