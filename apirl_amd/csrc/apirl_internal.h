@@ -82,6 +82,7 @@ struct LorForm {
   int2* rlut = nullptr;         // radial position -> bin range; null on a uniform grid
   float rl0 = 0.f, rl_inv_h = 0.f;
   int nrl = 0;
+  int tile_maxc = 0;            // with rlut: candidate bins of a tile and angle at most
   bool built = false;
   bool gather = false;          // the gather's tables exist for this form
   // APIRL_PREC_F64_SETUP tables of the gather's column kernel, built on its first
@@ -315,6 +316,9 @@ hipError_t launch_backproject_tile(const apirl_plan* p, const float* sino, float
                                    size_t scratch_bytes, hipStream_t st, const EmFuse* fuse,
                                    void* geo, bool geo_ready);
 const char* tile_misfit(const apirl_plan* p);
+// Candidate bins (even and odd ones counted alike) of one tile and angle at the most, on the
+// radial grid of a lookup table.
+int tile_lut_candidates(const Geo& g, const std::vector<int2>& lut, float inv_h);
 // A batched 3D job's backprojections (one LOR per bin), as apirl_backproject runs them for
 // APIRL_BP_GATHER, on any stream with a scratch of the job's own.  job_scratch_bytes: what a
 // subset needs; prepare also builds the tile order and takes the memory of its kept geometry.

@@ -104,6 +104,7 @@ bool upload_gather_form(apirl_plan* p, const std::vector<apirl::RayXY>& rays,
     }
     apirl::build_radial_lut(r, tab, f.rl0, f.rl_inv_h);
     f.nrl = (int)tab.size();
+    f.tile_maxc = apirl::tile_lut_candidates(p->geo, tab, f.rl_inv_h);
     ok = hipMalloc(&f.angcs_odd, odd.size() * sizeof(float2)) == hipSuccess &&
          hipMemcpy(f.angcs_odd, odd.data(), odd.size() * sizeof(float2),
                    hipMemcpyHostToDevice) == hipSuccess &&

@@ -1508,9 +1508,16 @@ __global__ __launch_bounds__(kGBlock) void tile_rays_kernel(GatherArgs A, int ma
     const int c = idx % maxc, ka = idx / maxc, a = A.subset + A.nsubsets * ka;
     int lo0, hi0, lo1, hi1;
     tile_bins(A, a, xt, yt, hx, hy, 1.0f / g.dr, lo0, hi0, lo1, hi1);
-    const int jlo = lo0 < lo1 ? lo0 : lo1, jhi = hi0 > hi1 ? hi0 : hi1;
-    const int rr = jlo + c;
-    if (rr > jhi || (grid_lut<kGridAny>(A) && !in_parity_range(rr, lo0, hi0, lo1, hi1))) return 0;
+    int rr = lo0 + c, last = hi0;
+    if (grid_lut<kGridAny>(A)) {
+      // even and odd bins in turn, each from its own range's first (the ranges of odd bins half
+      // an angular step away can lie far apart)
+      const int even = lo0 + (lo0 & 1), odds = lo1 + 1 - (lo1 & 1);
+      const bool odd = ((c & 1) != 0) != (odds < even);
+      rr = (odd ? odds : even) + 2 * (c >> 1);
+      last = odd ? hi1 : hi0;
+    }
+    if (rr > last) return 0;
     pair = ka * g.nr + rr;
     t = A.rays[(long)a * g.nr + rr];
     if (!(t.flags & RAY_VALID) ||
@@ -1888,18 +1895,33 @@ int tile_slab_depth(const apirl_plan* p) {
   return (nz + nslab - 1) / nslab;
 }
 
-// Upper bound on the candidate bins of one (tile, angle): the bins within the tile's
-// projected half-width (plus the search margin, and one lookup-table step on each
-// side on a non-uniform grid) of its centre, for each parity.
+// Half-width along r of the bins whose LORs can cross a tile at the widest angle (tile_bins).
+double tile_half_width(const Geo& g) {
+  return 0.5 * kTW * std::max(g.dx, g.dy) * 1.41421357 + g.rmargin + 1e-3;
+}
+
+int tile_lut_candidates(const Geo& g, const std::vector<int2>& lut, float inv_h) {
+  // entries between the two that lut_bins looks up, which rounds outwards and takes one more on
+  // each side; two more for its own rounding
+  const int n = (int)lut.size();
+  const double d = std::ceil(2.0 * tile_half_width(g) * inv_h) + 6;
+  const int step = d < n ? (int)d : n;
+  int most = 0;
+  for (int k = 0; k < n; k++)
+    most = std::max(most, lut[std::min(k + step, n - 1)].y - lut[k].x + 1);
+  return most + 1;  // the parity with one bin more, in turn with the other
+}
+
+// Upper bound on the candidate bins of one (tile, angle) of the active LOR form: counted in its
+// lookup table (LorForm::tile_maxc), whose radial grid need not be the plan's, or the bins within
+// the tile's half-width on the plan's uniform grid.
 int tile_max_candidates(const apirl_plan* p) {
   const Geo& g = p->geo;
+  if (p->d_rlut) return p->forms[p->scanner].tile_maxc;
   double drmin = g.dr > 0 ? g.dr : 1.0;
   for (size_t j = 1; j < p->r.size(); j++) drmin = std::min(drmin, (double)p->r[j] - p->r[j - 1]);
   if (!(drmin > 0)) drmin = 1e-3;
-  const double hw = 0.5 * kTW * std::max(g.dx, g.dy) * 1.41421357 + g.rmargin + 1e-3;
-  const double h = p->rl_inv_h > 0 ? 1.0 / p->rl_inv_h : 0.0;
-  const int one = (int)std::ceil((2 * hw + 2 * h) / drmin) + 3;
-  const int c = p->d_rlut ? 2 * one : one;
+  const int c = (int)std::ceil(2 * tile_half_width(g) / drmin) + 3;
   return c < g.nr ? c : g.nr;
 }
 
