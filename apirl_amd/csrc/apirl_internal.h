@@ -135,7 +135,6 @@ struct apirl_plan {
   int gather_zvox = 3;             // 3D gather voxels per lane along z (1..4, tiles only)
   int gather_xcd = APIRL_GATHER_XCD_WEDGES;  // column kernel's tile order
   int tile_zs = 0;                 // tile backprojector's slab depth (0: about 5 slices)
-  int* d_tile_order = nullptr;     // its tiles, nearest the image centre first
   float* d_zinc = nullptr;         // [nsino] z-crossing increment |dz / Vz|, negative for Vz < 0
   bool slices16 = false;           // every slice index of its rays fits 16 bits
   // its geometry per (LOR form, subset, subsets), kept from the first call on, within
@@ -321,15 +320,13 @@ const char* tile_misfit(const apirl_plan* p);
 int tile_lut_candidates(const Geo& g, const std::vector<int2>& lut, float inv_h);
 // A batched 3D job's backprojections (one LOR per bin), as apirl_backproject runs them for
 // APIRL_BP_GATHER, on any stream with a scratch of the job's own.  job_scratch_bytes: what a
-// subset needs; prepare also builds the tile order and takes the memory of its kept geometry.
+// subset needs; prepare also takes the memory of its kept geometry.
 size_t job_scratch_bytes(apirl_plan* p, int subset, int nsubsets, bool prepare);
 hipError_t job_backproject(apirl_plan* p, const float* sino, float* img, int subset, int nsubsets,
                            int kind, const EmFuse* fuse, void* scratch, size_t scratch_bytes,
                            hipStream_t st);
 size_t tile_geo_bytes(const apirl_plan* p, int subset, int nsubsets);
 size_t tile_scratch_bytes(const apirl_plan* p, int subset, int nsubsets, bool with_geo);
-// the tiles, the ones nearest the image centre first
-void build_tile_order(const apirl_plan* p, std::vector<int>& order);
 size_t gather_scratch_bytes(const apirl_plan* p, int subset, int nsubsets);
 // The 3D gather's 32-bit record and table offsets hold for this subset (fewer than
 // 2^31 subset bins; angle x radial bins, sinograms and crossing-table slots below 2^24).

@@ -2,7 +2,6 @@
 // and the device-resident MLEM / OSEM drivers.
 #include <cfloat>
 #include <cmath>
-#include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <algorithm>
@@ -180,22 +179,6 @@ bool ensure_f64s_tables(apirl_plan* p) {
   return ok;
 }
 
-// The tile backprojector's tile order, built on first use.
-bool ensure_tile_order(apirl_plan* p) {
-  if (p->d_tile_order) return true;
-  std::vector<int> order;
-  apirl::build_tile_order(p, order);
-  if (hipMalloc(&p->d_tile_order, order.size() * sizeof(int)) != hipSuccess ||
-      hipMemcpy(p->d_tile_order, order.data(), order.size() * sizeof(int),
-                hipMemcpyHostToDevice) != hipSuccess) {
-    (void)hipGetLastError();
-    if (p->d_tile_order) (void)hipFree(p->d_tile_order);
-    p->d_tile_order = nullptr;
-    return false;
-  }
-  return true;
-}
-
 // Work enqueued on the stream is being captured into a graph (or its state is unknown).
 bool capturing(hipStream_t st) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -243,7 +226,7 @@ void free_tile_geo(apirl_plan* p) {
 }
 
 // The tile backprojection of one subset on stream st with the geometry tg (null: built in the
-// scratch); the item order is built.
+// scratch).
 hipError_t tile_run(apirl_plan* p, const float* sino, float* img, int subset, int nsubsets,
                     int kind, const apirl::EmFuse* fuse, apirl_plan::TileGeo* tg, void* scratch,
                     size_t scratch_bytes, hipStream_t st) {
@@ -303,7 +286,7 @@ apirl_status tile_backproject(apirl_plan* p, const float* sino, float* img, int 
   apirl_ctx* c = p->ctx;
   apirl_plan::TileGeo* tg = tile_geo_for(p, subset, nsubsets, c->stream);
   const size_t need = apirl::tile_scratch_bytes(p, subset, nsubsets, tg == nullptr);
-  if ((need > p->gscratch_bytes || !p->d_tile_order) && capturing(c->stream))
+  if (need > p->gscratch_bytes && capturing(c->stream))
     return fail(c, APIRL_ERR_NOMEM, "the gather scratch cannot be allocated during a capture");
   // with room for the geometry of the plan's largest subset, so that a capture of a subset, or
   // on a stream, whose kept geometry cannot be read in it builds its own
@@ -311,8 +294,6 @@ apirl_status tile_backproject(apirl_plan* p, const float* sino, float* img, int 
   if (need > p->gscratch_bytes && !ensure_gscratch(p, std::max(need, most)) &&
       !ensure_gscratch(p, need))
     return fail(c, APIRL_ERR_NOMEM, "cannot allocate the gather scratch");
-  if (!ensure_tile_order(p))
-    return fail(c, APIRL_ERR_NOMEM, "cannot allocate the tile backprojector's item order");
   done = true;
   APIRL_HIP(c, tile_run(p, sino, img, subset, nsubsets, kind, fuse, tg, p->d_gscratch,
                         p->gscratch_bytes, c->stream));
@@ -739,7 +720,6 @@ namespace apirl {
 size_t job_scratch_bytes(apirl_plan* p, int subset, int nsubsets, bool prepare) {
   if (!tile_takes(p, subset, nsubsets)) return gather_scratch_bytes(p, subset, nsubsets);
   if (!prepare) return tile_scratch_bytes(p, subset, nsubsets, false);
-  if (!ensure_tile_order(p)) return SIZE_MAX;  // not to be had
   return tile_scratch_bytes(p, subset, nsubsets,
                             tile_geo_for(p, subset, nsubsets, p->ctx->stream) == nullptr);
 }
@@ -748,7 +728,6 @@ hipError_t job_backproject(apirl_plan* p, const float* sino, float* img, int sub
                            int kind, const EmFuse* fuse, void* scratch, size_t scratch_bytes,
                            hipStream_t st) {
   if (tile_takes(p, subset, nsubsets)) {
-    if (!p->d_tile_order) return hipErrorInvalidValue;  // job_scratch_bytes builds it
     apirl_plan::TileGeo* tg = tile_geo_for(p, subset, nsubsets, st);
     if (scratch_bytes >= tile_scratch_bytes(p, subset, nsubsets, tg == nullptr))
       return tile_run(p, sino, img, subset, nsubsets, kind, fuse, tg, scratch, scratch_bytes, st);
@@ -832,7 +811,6 @@ apirl_status apirl_plan_destroy(apirl_plan* p) {
   if (p->d_divbins) (void)hipFree(p->d_divbins);
   for (int* m : p->d_tilemap)
     if (m) (void)hipFree(m);
-  if (p->d_tile_order) (void)hipFree(p->d_tile_order);
   if (p->d_zinc) (void)hipFree(p->d_zinc);
   free_tile_geo(p);
   if (p->d_zsoff) (void)hipFree(p->d_zsoff);

@@ -1481,14 +1481,18 @@ __device__ __forceinline__ int tile_path(const RayXY& t, const TileEntry& E, int
 // The rays of one tile per workgroup: candidate c of angle ka (the c-th bin of the angle's
 // candidate range) is kept when its LOR is valid and its path enters the tile.  The kept rays
 // go to the front of the tile's slots, the longest paths first and in (angle, bin) order among
-// equal ones: the lanes of a pass then walk about equally far.
+// equal ones: the lanes of a pass then walk about equally far.  The workgroup also finds its
+// tile's place in the order of tile_bp_kernel's items: by the distance from the image centre, and
+// by number among equal ones.
 __global__ __launch_bounds__(kGBlock) void tile_rays_kernel(GatherArgs A, int maxc, int nslot,
                                                             TileRay* __restrict__ rays,
                                                             int* __restrict__ pairs,
-                                                            int* __restrict__ count) {
+                                                            int* __restrict__ count,
+                                                            int* __restrict__ order) {
   constexpr int kWaves = kGBlock / kWave;
   __shared__ int place[kTPath];            // next slot of each path length
   __shared__ int wcount[kWaves][kTPath];
+  __shared__ int before;  // tiles before this one in the order
   const Geo& g = A.g;
   const int tile = blockIdx.x, wave = threadIdx.x / kWave;
   const int ntx = (g.nx + kTW - 1) / kTW;
@@ -1526,13 +1530,28 @@ __global__ __launch_bounds__(kGBlock) void tile_rays_kernel(GatherArgs A, int ma
     return tile_path(t, E, ti0, ti1, tj0, tj1, [](int, float, bool) {});
   };
   if (threadIdx.x < kTPath) place[threadIdx.x] = 0;
+  if (threadIdx.x == 0) before = 0;
   __syncthreads();
+  {
+    auto distance = [&](int t) -> long {  // squared, of twice the voxels
+      const long x = (2 * (t % ntx) + 1) * (long)kTW - g.nx, y = (2 * (t / ntx) + 1) * (long)kTW - g.ny;
+      return x * x + y * y;
+    };
+    const long mine = distance(tile);
+    int n = 0;
+    for (int t = threadIdx.x; t < (int)gridDim.x; t += kGBlock) {
+      const long d = distance(t);
+      n += d < mine || (d == mine && t < tile) ? 1 : 0;
+    }
+    if (n > 0) atomicAdd(&before, n);
+  }
   for (int base = 0; base < nslot; base += kGBlock) {
     const int n = candidate(base + threadIdx.x);
     if (n > 0) atomicAdd(&place[n], 1);
   }
   __syncthreads();
   if (threadIdx.x == 0) {
+    order[before] = tile;
     int run = 0;
     for (int n = kTPath - 1; n > 0; n--) {
       const int c = place[n];
@@ -1940,22 +1959,6 @@ int tile_count(const apirl_plan* p) {
   return ((p->geo.nx + kTW - 1) / kTW) * ((p->geo.ny + kTW - 1) / kTW);
 }
 
-void build_tile_order(const apirl_plan* p, std::vector<int>& order) {
-  const int ntx = (p->geo.nx + kTW - 1) / kTW, nty = (p->geo.ny + kTW - 1) / kTW;
-  std::vector<std::pair<double, int>> tiles;
-  for (int ty = 0; ty < nty; ty++)
-    for (int tx = 0; tx < ntx; tx++) {
-      const double cx = (tx + 0.5) * kTW - 0.5 * p->geo.nx, cy = (ty + 0.5) * kTW - 0.5 * p->geo.ny;
-      tiles.push_back({cx * cx + cy * cy, ty * ntx + tx});
-    }
-  std::stable_sort(tiles.begin(), tiles.end(),
-                   [](const std::pair<double, int>& a, const std::pair<double, int>& b) {
-                     return a.first < b.first;
-                   });
-  order.clear();
-  for (const auto& t : tiles) order.push_back(t.second);
-}
-
 namespace {
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
@@ -1999,9 +2002,10 @@ TileSizes tile_sizes(const apirl_plan* p, int subset, int nsubsets) {
   return z;
 }
 
-// geometry: [ray count per tile][ray (angle, bin) pairs][rays]
+// geometry: [ray count per tile][order of the tiles][ray (angle, bin) pairs][rays]
 struct TileGeoPtrs {
   int* count;
+  int* order;
   int* pairs;
   TileRay* rays;
   size_t bytes;
@@ -2013,6 +2017,8 @@ TileGeoPtrs tile_geo_ptrs(const TileSizes& z, void* geo) {
   char* c = (char*)geo;
   size_t o = 0;
   q.count = (int*)(c + o);
+  o += align256((size_t)z.ntiles * sizeof(int));
+  q.order = (int*)(c + o);
   o += align256((size_t)z.ntiles * sizeof(int));
   q.pairs = (int*)(c + o);
   o += align256(nslots * sizeof(int));
@@ -2050,7 +2056,6 @@ hipError_t launch_backproject_tile(const apirl_plan* p, const float* sino, float
   if (z.nrays == 0 || z.nvox == 0) return hipSuccess;
   if (scratch_bytes < tile_scratch_bytes(p, subset, nsubsets, geo == nullptr))
     return hipErrorInvalidValue;
-  if (!p->d_tile_order) return hipErrorInvalidValue;
   char* sp = (char*)scratch;
   TileZ* zr = (TileZ*)sp;
   sp += align256((size_t)z.nrays * sizeof(TileZ));
@@ -2083,12 +2088,12 @@ hipError_t launch_backproject_tile(const apirl_plan* p, const float* sino, float
   // the subset's geometry: the rays of every tile with their paths
   if (!geo_ready)
     hipLaunchKernelGGL(tile_rays_kernel, dim3(z.ntiles), dim3(kGBlock), 0, st, A, z.maxc, z.nslot,
-                       q.rays, q.pairs, q.count);
+                       q.rays, q.pairs, q.count, q.order);
   // the call's axial records with their bin values, and the (angle, r) with a non-zero bin
   hipLaunchKernelGGL(tile_zsetup_kernel, dim3((g.nr + kTZBins - 1) / kTZBins, z.nang_sub),
                      dim3(kGBlock), 0, st, A, zr, nzmask, nzp);
   hipLaunchKernelGGL(tile_bp_kernel, dim3((unsigned)(z.ntiles * z.nslab * z.nchunk)), dim3(kWave),
-                     tile_lds_bytes(z.zs), st, A, z.zs, z.nslab, z.nchunk, p->d_tile_order,
+                     tile_lds_bytes(z.zs), st, A, z.zs, z.nslab, z.nchunk, (const int*)q.order,
                      (const TileRay*)q.rays, (const int*)q.pairs, (const int*)q.count, z.nslot,
                      (const TileZ*)zr, (const unsigned*)nzmask, p->d_zinc, parts);
   if (parts)
