@@ -162,6 +162,7 @@ struct apirl_plan {
   float* d_xytab = nullptr;        // [nang][nr][nx + ny] entry crossings (gather)
   int zblock = 0;                  // z-crossing table entries per (angle, radial bin)
   size_t gscratch_bytes = 0;
+  size_t gscratch_refused = SIZE_MAX;  // as much could not be allocated
   std::vector<float> ang, r;       // host copies of the grids
   std::vector<float2> zab;         // [nsino] one axial sample per bin
   std::vector<float> z1m, z2m;     // [nsino] mean ring coordinates of each sinogram
@@ -244,7 +245,7 @@ hipError_t launch_backproject(const apirl_plan* p, const float* sino, const floa
                               hipStream_t st);
 // zeroes the scatter's n-float image copies (device-scope stores, as the reduction
 // clears them)
-hipError_t launch_zero_replicas(float* rep, size_t n, hipStream_t st);
+hipError_t launch_zero_floats(float* x, size_t n, hipStream_t st);
 hipError_t launch_em_update(float* x, const float* b, const float* s, size_t n, float thr,
                             int strict, hipStream_t st);
 hipError_t launch_force_positive(float* x, size_t n, hipStream_t st);

@@ -44,6 +44,14 @@ struct DeviceGuard {
   }
 };
 
+// Work enqueued on the stream is being captured into a graph (or its state is unknown).
+bool capturing(hipStream_t st) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 apirl_status ensure_red(apirl_ctx* ctx, size_t n) {
   if (ctx->red_cap >= n) return APIRL_OK;
   if (ctx->d_red) (void)hipFree(ctx->d_red);
@@ -179,14 +187,6 @@ bool ensure_f64s_tables(apirl_plan* p) {
   return ok;
 }
 
-// Work enqueued on the stream is being captured into a graph (or its state is unknown).
-bool capturing(hipStream_t st) {
-  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
-  (void)hipGetLastError();
-  return true;
-}
-
 // The kept tile geometry of (the plan's LOR form, subset, subsets) for work on stream st:
 // found, or allocated within the plan's budget (not ready until a call has built it).  Null
 // when it does not fit the budget; the call then builds it in its scratch.  During a capture
@@ -262,9 +262,10 @@ bool os_precision_ok(const apirl_plan* p, int precision) {
   return p->geo.ns * p->geo.nas == 1 || (precision == APIRL_PREC_REFERENCE && p->geo.walk24);
 }
 
-// The plan's backprojection scratch holds at least `need` bytes.
+// The plan's backprojection scratch holds at least `need` bytes.  A capture allocates nothing.
 bool ensure_gscratch(apirl_plan* p, size_t need) {
   if (need <= p->gscratch_bytes) return true;
+  if (capturing(p->ctx->stream)) return false;
   if (p->d_gscratch) {
     if (hipStreamSynchronize(p->ctx->stream) != hipSuccess) return false;
     (void)hipFree(p->d_gscratch);
@@ -273,26 +274,34 @@ bool ensure_gscratch(apirl_plan* p, size_t need) {
   p->gscratch_bytes = 0;
   if (hipMalloc(&p->d_gscratch, need) != hipSuccess) {
     (void)hipGetLastError();
+    p->d_gscratch = nullptr;
     return false;
   }
   p->gscratch_bytes = need;
   return true;
 }
 
+// Room in the scratch, when there is the memory, for what a capture may ask of it: the tile
+// backprojection of the plan's largest subset with its geometry (a capture builds its own when it
+// cannot read the kept one), and for calls of the gather form the voxel-driven one's, which its
+// other precisions run.
+void reserve_gscratch(apirl_plan* p, int nsubsets, int mode) {
+  size_t most = apirl::tile_scratch_bytes(p, 0, nsubsets, true);
+  if (mode == APIRL_BP_GATHER)
+    most = std::max(most, apirl::gather_scratch_bytes(p, 0, nsubsets));
+  if (most <= p->gscratch_bytes || most >= p->gscratch_refused || capturing(p->ctx->stream)) return;
+  if (!ensure_gscratch(p, most)) p->gscratch_refused = most;
+}
+
 // The tile backprojection with the plan's scratch.  done stays false when it cannot be had
 // (no memory, or a capture that would have to allocate): the caller's own form then runs.
 apirl_status tile_backproject(apirl_plan* p, const float* sino, float* img, int subset,
-                              int nsubsets, int kind, const apirl::EmFuse* fuse, bool& done) {
+                              int nsubsets, int kind, int mode, const apirl::EmFuse* fuse,
+                              bool& done) {
   apirl_ctx* c = p->ctx;
   apirl_plan::TileGeo* tg = tile_geo_for(p, subset, nsubsets, c->stream);
-  const size_t need = apirl::tile_scratch_bytes(p, subset, nsubsets, tg == nullptr);
-  if (need > p->gscratch_bytes && capturing(c->stream))
-    return fail(c, APIRL_ERR_NOMEM, "the gather scratch cannot be allocated during a capture");
-  // with room for the geometry of the plan's largest subset, so that a capture of a subset, or
-  // on a stream, whose kept geometry cannot be read in it builds its own
-  const size_t most = apirl::tile_scratch_bytes(p, 0, nsubsets, true);
-  if (need > p->gscratch_bytes && !ensure_gscratch(p, std::max(need, most)) &&
-      !ensure_gscratch(p, need))
+  reserve_gscratch(p, nsubsets, mode);
+  if (!ensure_gscratch(p, apirl::tile_scratch_bytes(p, subset, nsubsets, tg == nullptr)))
     return fail(c, APIRL_ERR_NOMEM, "cannot allocate the gather scratch");
   done = true;
   APIRL_HIP(c, tile_run(p, sino, img, subset, nsubsets, kind, fuse, tg, p->d_gscratch,
@@ -316,7 +325,7 @@ apirl_status backproject_any(apirl_plan* p, const float* sino, const float* est,
     if (kind != apirl::BP_DIVIDE && tile_takes(p, subset, nsubsets)) {
       // DivideAndBackproject keeps its own bounds rule (BP_DIVIDE in the scatter kernel)
       bool done = false;
-      const apirl_status st = tile_backproject(p, sino, img, subset, nsubsets, kind, fuse, done);
+      const apirl_status st = tile_backproject(p, sino, img, subset, nsubsets, kind, mode, fuse, done);
       if (done) return st;
     }
     if (kind != apirl::BP_DIVIDE && apirl::gather2_takes(p, subset, nsubsets)) {
@@ -325,8 +334,9 @@ apirl_status backproject_any(apirl_plan* p, const float* sino, const float* est,
       return APIRL_OK;
     }
     const size_t nvox = apirl_plan_image_voxels(p);
-    if (fuse) APIRL_HIP(c, hipMemsetAsync(img, 0, nvox * sizeof(float), c->stream));
-    if (!p->d_replicas && !p->replicas_failed) {
+    // (a fill kernel, which a graph replays as it is)
+    if (fuse) APIRL_HIP(c, apirl::launch_zero_floats(img, nvox, c->stream));
+    if (!p->d_replicas && !p->replicas_failed && !capturing(c->stream)) {
       // the per-XCD scatter targets (16 image copies), zeroed here and re-zeroed by
       // the reduction after every use; without them the atomics go to the image
       const size_t bytes = (size_t)16 * p->geo.nx * p->geo.ny * p->geo.nz * sizeof(float);
@@ -334,7 +344,7 @@ apirl_status backproject_any(apirl_plan* p, const float* sino, const float* est,
         p->d_replicas = nullptr;
         p->replicas_failed = true;
         (void)hipGetLastError();
-      } else if (apirl::launch_zero_replicas(p->d_replicas, bytes / sizeof(float), c->stream) !=
+      } else if (apirl::launch_zero_floats(p->d_replicas, bytes / sizeof(float), c->stream) !=
                  hipSuccess) {
         (void)hipFree(p->d_replicas);
         p->d_replicas = nullptr;
@@ -399,7 +409,7 @@ apirl_status backproject_any(apirl_plan* p, const float* sino, const float* est,
   }
   if (precision == APIRL_PREC_REFERENCE && tile_takes(p, subset, nsubsets)) {
     bool done = false;
-    const apirl_status st = tile_backproject(p, sino, img, subset, nsubsets, kind, fuse, done);
+    const apirl_status st = tile_backproject(p, sino, img, subset, nsubsets, kind, mode, fuse, done);
     if (done || mode == APIRL_BP_TILE) return st;
   }
   if (!ensure_gscratch(p, apirl::gather_scratch_bytes(p, subset, nsubsets)))
@@ -1113,7 +1123,7 @@ apirl_status sensitivity_impl(apirl_plan* p, const float* d_mult, float* d_sens,
     return backproject_any(p, d_mult, nullptr, d_sens, subset, nsubsets, kind, mode, precision,
                            &fz);
   }
-  APIRL_HIP(c, hipMemsetAsync(d_sens, 0, nvox * sizeof(float), c->stream));
+  APIRL_HIP(c, apirl::launch_zero_floats(d_sens, nvox, c->stream));
   apirl_status st = backproject_any(p, d_mult, nullptr, d_sens, subset, nsubsets, kind, mode,
                                     precision);
   if (st != APIRL_OK) return st;

@@ -1681,9 +1681,9 @@ hipError_t launch_count_intersections(const apirl_plan* p, int subset, int nsubs
   return hipGetLastError();
 }
 
-hipError_t launch_zero_replicas(float* rep, size_t n, hipStream_t st) {
+hipError_t launch_zero_floats(float* x, size_t n, hipStream_t st) {
   if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(zero_floats_kernel, dim3(grid_for((long)n)), dim3(kBlock), 0, st, rep,
+  hipLaunchKernelGGL(zero_floats_kernel, dim3(grid_for((long)n)), dim3(kBlock), 0, st, x,
                      (long)n);
   return hipGetLastError();
 }
