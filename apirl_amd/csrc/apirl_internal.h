@@ -145,6 +145,7 @@ struct apirl_plan {
     void* d;
     size_t bytes;
     bool ready;
+    bool captured;  // a graph reads it
     hipStream_t stream;
     hipEvent_t ev;
   };
@@ -162,7 +163,10 @@ struct apirl_plan {
   float* d_xytab = nullptr;        // [nang][nr][nx + ny] entry crossings (gather)
   int zblock = 0;                  // z-crossing table entries per (angle, radial bin)
   size_t gscratch_bytes = 0;
+  bool gscratch_captured = false;  // a graph reads d_gscratch
   size_t gscratch_refused = SIZE_MAX;  // as much could not be allocated
+  // scratch and tile geometry that graphs read, kept until the plan ends
+  std::vector<void*> retired;
   std::vector<float> ang, r;       // host copies of the grids
   std::vector<float2> zab;         // [nsino] one axial sample per bin
   std::vector<float> z1m, z2m;     // [nsino] mean ring coordinates of each sinogram

@@ -195,12 +195,16 @@ bool ensure_f64s_tables(apirl_plan* p) {
 apirl_plan::TileGeo* tile_geo_for(apirl_plan* p, int subset, int nsubsets, hipStream_t st) {
   const bool cap = capturing(st);
   for (apirl_plan::TileGeo& e : p->tile_geo)
-    if (e.form == p->scanner && e.subset == subset && e.nsubsets == nsubsets)
-      return !cap || (e.ready && e.stream == st) ? &e : nullptr;
+    if (e.form == p->scanner && e.subset == subset && e.nsubsets == nsubsets) {
+      if (cap && !(e.ready && e.stream == st)) return nullptr;
+      e.captured |= cap;
+      return &e;
+    }
   if (cap) return nullptr;
   const size_t bytes = apirl::tile_geo_bytes(p, subset, nsubsets);
   if (bytes == 0 || p->tile_geo_used + bytes > p->tile_geo_budget) return nullptr;
-  apirl_plan::TileGeo e{p->scanner, subset, nsubsets, nullptr, bytes, false, nullptr, nullptr};
+  apirl_plan::TileGeo e{p->scanner, subset, nsubsets, nullptr, bytes,
+                        false,      false,  nullptr,  nullptr};
   if (hipMalloc(&e.d, bytes) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
@@ -218,7 +222,8 @@ apirl_plan::TileGeo* tile_geo_for(apirl_plan* p, int subset, int nsubsets, hipSt
 void free_tile_geo(apirl_plan* p) {
   for (apirl_plan::TileGeo& e : p->tile_geo) {
     (void)hipEventSynchronize(e.ev);
-    (void)hipFree(e.d);
+    if (e.captured) p->retired.push_back(e.d);
+    else (void)hipFree(e.d);
     (void)hipEventDestroy(e.ev);
   }
   p->tile_geo.clear();
@@ -262,16 +267,26 @@ bool os_precision_ok(const apirl_plan* p, int precision) {
   return p->geo.ns * p->geo.nas == 1 || (precision == APIRL_PREC_REFERENCE && p->geo.walk24);
 }
 
-// The plan's backprojection scratch holds at least `need` bytes.  A capture allocates nothing.
+// The plan's backprojection scratch holds at least `need` bytes.  A capture allocates nothing, and
+// scratch that a captured graph reads stays with the plan when a larger one takes its place.
 bool ensure_gscratch(apirl_plan* p, size_t need) {
-  if (need <= p->gscratch_bytes) return true;
-  if (capturing(p->ctx->stream)) return false;
+  const bool cap = capturing(p->ctx->stream);
+  if (need <= p->gscratch_bytes) {
+    p->gscratch_captured |= cap;
+    return true;
+  }
+  if (cap) return false;
   if (p->d_gscratch) {
-    if (hipStreamSynchronize(p->ctx->stream) != hipSuccess) return false;
-    (void)hipFree(p->d_gscratch);
+    if (p->gscratch_captured) {
+      p->retired.push_back(p->d_gscratch);
+    } else {
+      if (hipStreamSynchronize(p->ctx->stream) != hipSuccess) return false;
+      (void)hipFree(p->d_gscratch);
+    }
   }
   p->d_gscratch = nullptr;
   p->gscratch_bytes = 0;
+  p->gscratch_captured = false;
   if (hipMalloc(&p->d_gscratch, need) != hipSuccess) {
     (void)hipGetLastError();
     p->d_gscratch = nullptr;
@@ -818,11 +833,12 @@ apirl_status apirl_plan_destroy(apirl_plan* p) {
   if (p->d_imgT) (void)hipFree(p->d_imgT);
   if (p->d_segs) (void)hipFree(p->d_segs);
   if (p->d_gscratch) (void)hipFree(p->d_gscratch);
+  free_tile_geo(p);
+  for (void* q : p->retired) (void)hipFree(q);
   if (p->d_divbins) (void)hipFree(p->d_divbins);
   for (int* m : p->d_tilemap)
     if (m) (void)hipFree(m);
   if (p->d_zinc) (void)hipFree(p->d_zinc);
-  free_tile_geo(p);
   if (p->d_zsoff) (void)hipFree(p->d_zsoff);
   delete p;
   return APIRL_OK;

@@ -1,7 +1,8 @@
 """Captured calls at the limits of what earlier calls have allocated: a subset larger than any
 before, another form or precision than before, no call before at all.  What can run without an
 allocation does, and every replay gives the eager result; the rest is refused with an error that
-leaves the capture and the plan as they were."""
+leaves the capture and the plan as they were.  A graph outlives the scratch it was captured over:
+a later, larger call leaves it its own."""
 import ctypes
 
 import numpy as np
@@ -134,3 +135,27 @@ def test_refused_capture_leaves_the_plan(torch, mode):
     assert bool((img == 3.0).all())
     want = host(plan3(c).backproject(x, mode=m))
     assert np.array_equal(host(p.backproject(x, mode=m)).view(np.int32), want.view(np.int32))
+
+
+@pytest.mark.parametrize("mode", ["BP_SCATTER", "BP_GATHER", "BP_TILE"])
+def test_graph_outlives_its_scratch(torch, mode):
+    """A larger call replaces the scratch, and a smaller tile_cache_mb the kept geometry, of a
+    captured call; its replays read the ones they were captured over."""
+    log(f"case: replays after the scratch has grown, {mode}")
+    c = hip.Context(0)
+    p = plan3(c)
+    m = getattr(hip, mode)
+    S = 10
+    x, img = bins(torch, p, 1, S), torch.zeros(p.image_shape(), device="cuda")
+    cap = Captured(torch, c)
+    # the geometry kept on the capture's own stream
+    c.check(c.lib.apirl_ctx_set_stream(c.h, ctypes.c_void_p(cap.side.cuda_stream)), "set_stream")
+    torch.cuda.synchronize()
+    p.backproject(x, out=img, subset=1, nsubsets=S, mode=m)
+    with cap:
+        p.backproject(x, out=img, subset=1, nsubsets=S, mode=m)
+    p.backproject(bins(torch, p, 0, 1), mode=m)
+    p.set_tuning(tile_cache_mb=-1)
+    fill = [torch.full((1 << 20,), float("nan"), device="cuda") for _ in range(16)]
+    replays(torch, cap, x, img, lambda: p.backproject(x, subset=1, nsubsets=S, mode=m), True)
+    del fill
