@@ -104,6 +104,8 @@ struct apirl_ctx {
   // scratch owned by the context (likelihood partials, reductions)
   double* d_red = nullptr;
   size_t red_cap = 0;
+  bool red_captured = false;     // a graph reads d_red
+  std::vector<void*> retired;    // ones that graphs read, kept until the context ends
   float* d_fred = nullptr;
   unsigned long long* d_ured = nullptr;
 };

@@ -53,10 +53,19 @@ bool capturing(hipStream_t st) {
 }
 
 apirl_status ensure_red(apirl_ctx* ctx, size_t n) {
-  if (ctx->red_cap >= n) return APIRL_OK;
-  if (ctx->d_red) (void)hipFree(ctx->d_red);
+  const bool captures = capturing(ctx->stream);
+  if (ctx->red_cap >= n) {
+    ctx->red_captured |= captures;
+    return APIRL_OK;
+  }
+  if (captures) return fail(ctx, APIRL_ERR_NOMEM, "the partials cannot be allocated during a capture");
+  if (ctx->d_red) {
+    if (ctx->red_captured) ctx->retired.push_back(ctx->d_red);
+    else (void)hipFree(ctx->d_red);
+  }
   ctx->d_red = nullptr;
   ctx->red_cap = 0;
+  ctx->red_captured = false;
   size_t cap = n < 1024 ? 1024 : n;
   APIRL_HIP(ctx, hipMalloc(&ctx->d_red, (cap + 8) * sizeof(double)));
   ctx->red_cap = cap;
@@ -484,6 +493,7 @@ apirl_status apirl_ctx_destroy(apirl_ctx* ctx) {
   if (!ctx) return APIRL_OK;
   DeviceGuard g(ctx->device);
   if (ctx->d_red) (void)hipFree(ctx->d_red);
+  for (void* q : ctx->retired) (void)hipFree(q);
   if (ctx->d_fred) (void)hipFree(ctx->d_fred);
   if (ctx->d_ured) (void)hipFree(ctx->d_ured);
   delete ctx;
@@ -1085,7 +1095,13 @@ apirl_status project_ratio_impl(apirl_plan* p, const float* d_img, const float* 
         return fail(c, APIRL_ERR_HIP, "the partials array's device address is unavailable");
       fr.lik_partials = c->d_noalloc;
     } else {
-      apirl_status st = ensure_red(c, (size_t)nblocks);
+      // outside a capture, room for every precision and subset: what a capture may ask for
+      size_t most = (size_t)nblocks;
+      if (!capturing(c->stream))
+        for (int q : {APIRL_PREC_REFERENCE, APIRL_PREC_KAHAN, APIRL_PREC_F64_ALPHA})
+          for (int s : {0, nsubsets - 1})
+            most = std::max(most, (size_t)apirl::project_partials(p, s, nsubsets, q));
+      apirl_status st = ensure_red(c, most);
       if (st != APIRL_OK) return st;
       fr.lik_partials = c->d_red;
     }

@@ -159,3 +159,34 @@ def test_graph_outlives_its_scratch(torch, mode):
     fill = [torch.full((1 << 20,), float("nan"), device="cuda") for _ in range(16)]
     replays(torch, cap, x, img, lambda: p.backproject(x, subset=1, nsubsets=S, mode=m), True)
     del fill
+
+
+def test_ratio_after_another_precision(torch):
+    """The likelihood's partials: a captured call of any precision finds room for them, and a
+    graph keeps its own when a larger call takes more."""
+    log("case: captured ratio, other precision, then a larger sinogram")
+    c = hip.Context(0)
+    p = hip.Plan.for_2d(c, 64, 4.0, 600, 200, 128.0, 400.0)
+    x = torch.rand(p.image_shape(), device="cuda")
+    meas = torch.poisson(torch.full(p.subset_shape(), 5.0, device="cuda"))
+    ratio = torch.empty_like(meas)
+    lik = torch.zeros(1, dtype=torch.float64, device="cuda")
+    p.project_ratio(x, meas, precision=hip.PREC_KAHAN)
+
+    def call(r, out):
+        c.check(c.lib.apirl_project_ratio(p.h, x.data_ptr(), meas.data_ptr(), None, r.data_ptr(),
+                                          out.data_ptr(), 0, 1, 0, hip.PREC_REFERENCE), "ratio")
+
+    with Captured(torch, c) as cap:
+        call(ratio, lik)
+    big = hip.Plan.for_2d(c, 64, 4.0, 9000, 600, 128.0, 400.0)
+    big.project_ratio(x, torch.ones(big.subset_shape(), device="cuda"))
+    for _ in range(3):
+        x.copy_(torch.rand_like(x))
+        lik.zero_()
+        torch.cuda.synchronize()
+        cap.graph.replay()
+        torch.cuda.synchronize()
+        r2, l2 = torch.empty_like(meas), torch.zeros_like(lik)
+        call(r2, l2)
+        assert bool((ratio == r2).all()) and float(lik) == float(l2)
