@@ -1309,11 +1309,10 @@ __global__ __launch_bounds__(kBlock, PREC == APIRL_PREC_REFERENCE ? 8 : 7) void 
   const char* const zbytes = (const char*)imgZ;
   const int nxy = g.nx * g.ny, npix = nxy * g.nz;
   double lik = 0.0;
-  const int s0 = (int)blockIdx.y * chunk, s1 = s0 + chunk < g.nsino ? s0 + chunk : g.nsino;
-  for (int s = s0 + (int)threadIdx.x; s < s1; s += nt) {
+  // The traversal state of sinogram s.
+  auto setup = [&](int s, Ray& ray) -> bool {
     const float2 zz = zab[s];
-    Ray ray;
-    bool valid = setup_ray<3>(g, t, zz.x, zz.y, ray);
+    const bool valid = setup_ray<3>(g, t, zz.x, zz.y, ray);
     if (PREC == APIRL_PREC_F64_SETUP) {
       // the axial setup in double too (project_ray's F64_SETUP)
       SetupZ64 zs;
@@ -1326,6 +1325,50 @@ __global__ __launch_bounds__(kBlock, PREC == APIRL_PREC_REFERENCE ? 8 : 7) void 
       ray.kinc = zs.kinc;
       ray.n = abs(xy64.i1 - xy64.i0) + abs(xy64.j1 - xy64.j0) + abs(zs.k1 - zs.k0);
     }
+    return valid;
+  };
+  // The sum of sinogram s to its bin.
+  auto store = [&](int s, bool valid, float sum) {
+    const long idx = ((long)s * nang_sub + ka) * g.nr + rr;
+    if (!FUSED) {
+      if (valid) sino[idx] = sum;
+    } else {
+      // fused EM epilogue, as project_ray's (Sinogram3D.cpp:584-607, 830-870)
+      const long full = ((long)s * g.nang + a) * g.nr + rr;
+      float est = valid ? sum : 0.f;
+      if (fr.additive)
+        est = est + fr.additive[fr.additive_local ? ((long)s * g.nang + ka) * g.nr + rr : full];
+      const float y = fr.meas[full];
+      const bool lik_term = fr.lik_positive_only ? (est > 0.f) : (est != 0.f);
+      if (lik_term) lik += (double)(y * logf(est) - est);
+      fr.ratio[idx] = (y != 0.f && est != 0.f) ? y / est : 0.f;
+    }
+  };
+  const int s0 = (int)blockIdx.y * chunk;
+  int s1 = s0 + chunk < g.nsino ? s0 + chunk : g.nsino;
+  // LORs that miss the image's square have lists of their own: the reference walks on from the
+  // later of the two entries, along columns beside the image, where a negative index can name a
+  // voxel of the row before.  They may run past the path's entries and their z crossings fall
+  // anywhere: the loop step by step, without the path.
+  const bool misses =
+      PREC == APIRL_PREC_F64_SETUP
+          ? xy64.amin > xy64.amax ||
+                abs(xy64.i1 - xy64.i0) + abs(xy64.j1 - xy64.j0) > g.nx + g.ny + 2
+          : t.amin > t.amax || t.nxy > g.nx + g.ny + 2;
+  if (misses) {
+    for (int s = s0 + (int)threadIdx.x; s < s1; s += nt) {
+      Ray ray;
+      const bool valid = setup(s, ray);
+      RaySum<kSum2> acc;
+      for (int m = 0; valid && m < ray.n; m += kUnroll)
+        walk3d_batch<false, kSum2, kStrict>(g, ray, img, nullptr, nxy, m, acc);
+      store(s, valid, acc.s);
+    }
+    s1 = s0;
+  }
+  for (int s = s0 + (int)threadIdx.x; s < s1; s += nt) {
+    Ray ray;
+    const bool valid = setup(s, ray);
     RaySum<kSum2> acc;
     if (valid) {
       // state: the next z crossing, the last crossing taken, the slice (kb: its byte offset
@@ -1455,20 +1498,7 @@ __global__ __launch_bounds__(kBlock, PREC == APIRL_PREC_REFERENCE ? 8 : 7) void 
         kb = k * 4;
       }
     }
-    const long idx = ((long)s * nang_sub + ka) * g.nr + rr;
-    if (!FUSED) {
-      if (valid) sino[idx] = acc.s;
-    } else {
-      // fused EM epilogue, as project_ray's (Sinogram3D.cpp:584-607, 830-870)
-      const long full = ((long)s * g.nang + a) * g.nr + rr;
-      float est = valid ? acc.s : 0.f;
-      if (fr.additive)
-        est = est + fr.additive[fr.additive_local ? ((long)s * g.nang + ka) * g.nr + rr : full];
-      const float y = fr.meas[full];
-      const bool lik_term = fr.lik_positive_only ? (est > 0.f) : (est != 0.f);
-      if (lik_term) lik += (double)(y * logf(est) - est);
-      fr.ratio[idx] = (y != 0.f && est != 0.f) ? y / est : 0.f;
-    }
+    store(s, valid, acc.s);
   }
   if (FUSED && fr.lik_partials) {
     // deterministic block reduction of the likelihood partials (fixed tree)
