@@ -235,17 +235,22 @@ struct FusedRatio {
   // the full additive sinogram, as OsemSinogram3d.cpp:172-173 with
   // Sinogram3D::addBinToBin (Sinogram3D.cpp:857-873) reads it
   int additive_local = 0;
+  int max_partials = 0;
 };
-// The fused form writes project_partials likelihood partials, one per workgroup.
+// The fused form writes project_partials likelihood partials, one per workgroup.  With
+// FusedRatio::max_partials (max_partials below) the path projector, which has one or more per
+// (angle, bin), runs only where that holds them; a ray per lane has one per 256 bins.
 // image_copy: where the projector's copy of the image goes (path_image_floats floats in 3D,
 // the image's in 2D) instead of the plan's own buffer, for work on a stream of its own.
 hipError_t launch_project(const apirl_plan* p, const float* img, float* sino, int subset,
                           int nsubsets, int precision, const FusedRatio* fused, int* nblocks_out,
                           hipStream_t st, float* image_copy = nullptr);
-bool path_forward_ok(const apirl_plan* p, int precision, int subset, int nsubsets);
+bool path_forward_ok(const apirl_plan* p, int precision, int subset, int nsubsets,
+                     int max_partials = 0);
 // Floats of the path forward projector's z-fastest image copy (apirl_plan::d_imgT).
 size_t path_image_floats(const Geo& g);
-int project_partials(const apirl_plan* p, int subset, int nsubsets, int precision);
+int project_partials(const apirl_plan* p, int subset, int nsubsets, int precision,
+                     int max_partials = 0);
 hipError_t launch_backproject(const apirl_plan* p, const float* sino, const float* est,
                               float* img, int subset, int nsubsets, int kind, int mode,
                               hipStream_t st);
@@ -264,7 +269,8 @@ hipError_t launch_sum_partials(const double* partials, int n, double* out, hipSt
 hipError_t launch_sum_partials_rows(const double* partials, int rows, long stride, int nsubsets,
                                     int more, int nmore, int nless, double* out, hipStream_t st);
 // Partials of apirl_project_ratio_noalloc: a file-scope device array of
-// siddon_kernels.hip of kNoallocPartials doubles (one per workgroup of 256 bins).
+// siddon_kernels.hip of kNoallocPartials doubles (one per workgroup, of 256 bins at least where
+// there are as many as APIRL_NOALLOC_MAX_BINS).
 constexpr int kNoallocPartials = 1 << 19;
 // The current device's address of that array (hipGetSymbolAddress).
 hipError_t noalloc_scratch_address(double** out);

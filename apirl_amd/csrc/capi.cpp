@@ -1072,8 +1072,10 @@ apirl_status project_ratio_impl(apirl_plan* p, const float* d_img, const float* 
   if (!os_precision_ok(p, precision))
     return fail(c, APIRL_ERR_UNSUPPORTED, "oversampled LORs use the reference precision");
   DeviceGuard g(c->device);
-  const int nblocks = apirl::project_partials(p, subset, nsubsets, precision);
   apirl::FusedRatio fr;
+  if (noalloc && d_lik) fr.max_partials = apirl::kNoallocPartials;
+  const int nblocks =
+      apirl::project_partials(p, subset, nsubsets, precision, fr.max_partials);
   fr.meas = d_meas;
   fr.additive = d_additive;
   fr.ratio = d_ratio;
@@ -1084,8 +1086,8 @@ apirl_status project_ratio_impl(apirl_plan* p, const float* d_img, const float* 
   fr.lik_partials = d_partials;
   if (d_lik && !d_partials) {
     if (noalloc) {
-      // the documented limit in bins (one partial per 256 bins at most, whichever
-      // projector kernel runs)
+      // the documented limit in bins: a ray per lane writes one partial per 256 of them, and the
+      // other projector kernels run only where theirs fit
       if (apirl_plan_subset_bins(p, subset, nsubsets) > (size_t)APIRL_NOALLOC_MAX_BINS ||
           nblocks > apirl::kNoallocPartials)
         return fail(c, APIRL_ERR_INVALID,

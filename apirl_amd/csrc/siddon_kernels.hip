@@ -1531,7 +1531,8 @@ constexpr double kPathMinWork = 1.0e8;
 // 0.9.  Short launches, by rays times columns, keep the path (27 / 24 us at 4e6).
 constexpr double kPathMaxBins = 40, kPathMaxSpacing = 1.25, kRayMinWork = 5.0e6;
 
-bool path_forward_ok(const apirl_plan* p, int precision, int subset, int nsubsets) {
+bool path_forward_ok(const apirl_plan* p, int precision, int subset, int nsubsets,
+                     int max_partials) {
   const Geo& g = p->geo;
   const double rays = (double)g.nsino * subset_num_angles(g.nang, nsubsets, subset) * g.nr;
   if (precision == APIRL_PREC_REFERENCE) {
@@ -1543,6 +1544,10 @@ bool path_forward_ok(const apirl_plan* p, int precision, int subset, int nsubset
     if (g.nsino <= kPathMinSino || rays * (g.nx + g.ny) < kPathMinWork) return false;
     // a likelihood partial per (angle, bin) then, where a ray per lane has one per 256 bins
     if (rays > (double)kNoallocPartials * g.nsino) return false;
+  }
+  if (max_partials > 0) {
+    const int npair = subset_num_angles(g.nang, nsubsets, subset) * g.nr;
+    if ((long)npair * fwd_path_split(g, npair).parts > max_partials) return false;
   }
   // the columns of an entry are kept in 16 bits each, a voxel's byte address in 32
   return g.dims == 3 && precision != APIRL_PREC_F64_ALPHA && g.ns * g.nas == 1 && g.walk24 &&
@@ -1567,11 +1572,12 @@ static bool split2_ok(const apirl_plan* p, int precision, long nrays) {
 // 128 x 128: 42 -> 44).
 constexpr long kTransposed2 = 1L << 17;
 
-int project_partials(const apirl_plan* p, int subset, int nsubsets, int precision) {
+int project_partials(const apirl_plan* p, int subset, int nsubsets, int precision,
+                     int max_partials) {
   const Geo& g = p->geo;
   const int nang_sub = subset_num_angles(g.nang, nsubsets, subset);
   const long nrays = (long)g.nsino * nang_sub * g.nr;
-  if (path_forward_ok(p, precision, subset, nsubsets))
+  if (path_forward_ok(p, precision, subset, nsubsets, max_partials))
     return nang_sub * g.nr * fwd_path_split(g, nang_sub * g.nr).parts;
   if (split2_ok(p, precision, nrays)) return (int)((nrays + 63) / 64);
   return (int)grid_for(nrays);
@@ -1589,7 +1595,7 @@ hipError_t launch_project(const apirl_plan* p, const float* img, float* sino, in
   if (nrays == 0) return hipSuccess;
   FusedRatio fr = fused ? *fused : FusedRatio{};
   const bool f = fused != nullptr;
-  if (path_forward_ok(p, precision, subset, nsubsets)) {
+  if (path_forward_ok(p, precision, subset, nsubsets, fr.max_partials)) {
     // the path forward projector: the image with z fastest (into the plan's
     // transposed-image buffer), one workgroup per (angle, bin) of the subset
     const int npair = nang_sub * g.nr, qmax = fwd_path_len(g), pitch = path_pitch(g);
