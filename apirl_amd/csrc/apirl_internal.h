@@ -333,8 +333,12 @@ const char* tile_misfit(const apirl_plan* p);
 int tile_lut_candidates(const Geo& g, const std::vector<int2>& lut, float inv_h);
 // A batched 3D job's backprojections (one LOR per bin), as apirl_backproject runs them for
 // APIRL_BP_GATHER, on any stream with a scratch of the job's own.  job_scratch_bytes: what a
-// subset needs; prepare also takes the memory of its kept geometry.
-size_t job_scratch_bytes(apirl_plan* p, int subset, int nsubsets, bool prepare);
+// subset needs, after the memory of its kept geometry has been taken.  job_footprint: what the
+// subsets of a job would need, scratch (their largest) and kept geometry that the plan does not
+// hold yet, for a plan of one LOR per bin (parts: as many plans like it, sharing its budget).
+size_t job_scratch_bytes(apirl_plan* p, int subset, int nsubsets);
+void job_footprint(const apirl_plan* p, int nsubsets, int parts, size_t& scratch,
+                   size_t& geometry);
 hipError_t job_backproject(apirl_plan* p, const float* sino, float* img, int subset, int nsubsets,
                            int kind, const EmFuse* fuse, void* scratch, size_t scratch_bytes,
                            hipStream_t st);

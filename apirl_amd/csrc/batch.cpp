@@ -138,9 +138,9 @@ size_t max_subset_bins(const apirl_plan* p, int S) {
   return m;
 }
 
-size_t job_scratch(apirl_plan* p, int S, bool prepare) {
+size_t job_scratch(apirl_plan* p, int S) {
   size_t m = 0;
-  for (int s = 0; s < S; s++) m = std::max(m, job_scratch_bytes(p, s, S, prepare));
+  for (int s = 0; s < S; s++) m = std::max(m, job_scratch_bytes(p, s, S));
   return m;
 }
 
@@ -266,12 +266,19 @@ size_t apirl_batch_job_bytes(const apirl_plan* p, int subsets) {
   size_t bytes = (size_t)subsets * nvox * sizeof(float) + thresholds_bytes(subsets) +
                  max_subset_bins(p, subsets) * sizeof(float);
   if (p->geo.dims == 3) {
-    // oversampled bins: the largest scratch of the plans of one LOR per bin once they are
-    // built (the job's submission builds them), the plan's own before
-    size_t z = 0;
-    if (p->os_parts.empty()) z = job_scratch(const_cast<apirl_plan*>(p), subsets, false);
-    for (apirl_plan* h : p->os_parts) z = std::max(z, job_scratch(h, subsets, false));
-    bytes += z + path_image_floats(p->geo) * sizeof(float);
+    // oversampled bins: the largest scratch of the plans of one LOR per bin, and their geometry,
+    // once they are built (the job's submission builds them), as many as the plan's own before
+    size_t z = 0, geometry = 0;
+    if (p->os_parts.empty()) {
+      apirl::job_footprint(p, subsets, p->geo.ns * p->geo.nas, z, geometry);
+    }
+    for (const apirl_plan* h : p->os_parts) {
+      size_t zh = 0, gh = 0;
+      apirl::job_footprint(h, subsets, 1, zh, gh);
+      z = std::max(z, zh);
+      geometry += gh;
+    }
+    bytes += z + geometry + path_image_floats(p->geo) * sizeof(float);
     if (p->geo.ns * p->geo.nas > 1) bytes += nvox * sizeof(float);
   }
   return bytes;
@@ -354,7 +361,7 @@ apirl_status apirl_batch_submit(apirl_batch* b, const apirl_job_desc* d, int* jo
   const size_t ratio_b = max_subset_bins(p, j->S) * sizeof(float);
   size_t z_b = 0;
   if (!j->is2d)
-    for (apirl_plan* q : gplans) z_b = std::max(z_b, job_scratch(q, j->S, true));
+    for (apirl_plan* q : gplans) z_b = std::max(z_b, job_scratch(q, j->S));
   auto get = [&](size_t n) -> void* {
     void* q = balloc(b, n);
     if (q) j->bufs.emplace_back(q, n);
@@ -563,10 +570,10 @@ apirl_status apirl_batch_step(apirl_batch* b, int* active) {
     const float* sens = j->sens + (size_t)s * j->nvox;
     // more scratch than at submission only when the plan's tuning has changed since
     size_t need = 0;
-    if (j->plan->geo.ns * j->plan->geo.nas == 1) need = job_scratch_bytes(j->plan, s, j->S, true);
+    if (j->plan->geo.ns * j->plan->geo.nas == 1) need = job_scratch_bytes(j->plan, s, j->S);
     else
       for (apirl_plan* q : j->plan->os_parts)
-        need = std::max(need, job_scratch_bytes(q, s, j->S, true));
+        need = std::max(need, job_scratch_bytes(q, s, j->S));
     if (need > j->zscr_bytes) {
       void* z = balloc(b, need);
       if (!z) return bfail(b, APIRL_ERR_NOMEM, "cannot allocate the job's device state");

@@ -752,11 +752,37 @@ apirl_status apirl_plan_create(apirl_ctx* ctx, const apirl_image_desc* image,
 extern "C++" {
 namespace apirl {
 
-size_t job_scratch_bytes(apirl_plan* p, int subset, int nsubsets, bool prepare) {
+size_t job_scratch_bytes(apirl_plan* p, int subset, int nsubsets) {
   if (!tile_takes(p, subset, nsubsets)) return gather_scratch_bytes(p, subset, nsubsets);
-  if (!prepare) return tile_scratch_bytes(p, subset, nsubsets, false);
   return tile_scratch_bytes(p, subset, nsubsets,
                             tile_geo_for(p, subset, nsubsets, p->ctx->stream) == nullptr);
+}
+
+void job_footprint(const apirl_plan* p, int nsubsets, int parts, size_t& scratch,
+                   size_t& geometry) {
+  // OSEM jobs on the mMR run its subset form, whose radial grid, and with it all sizes, is the
+  // mMR form's (apirl_batch_submit; a job of one subset is taken for MLEM)
+  const int form =
+      p->scanner == APIRL_SCANNER_MMR && nsubsets > 1 ? APIRL_SCANNER_MMR_SUBSET : p->scanner;
+  const size_t budget = p->tile_geo_budget / (size_t)parts;
+  size_t used = p->tile_geo_used;
+  scratch = geometry = 0;
+  for (int s = 0; s < nsubsets; s++) {
+    if (gather_misfit(p, s, nsubsets) || tile_misfit(p)) {
+      scratch = std::max(scratch, gather_scratch_bytes(p, s, nsubsets));
+      continue;
+    }
+    bool kept = false;
+    for (const apirl_plan::TileGeo& e : p->tile_geo)
+      kept |= e.form == form && e.subset == s && e.nsubsets == nsubsets;
+    const size_t bytes = tile_geo_bytes(p, s, nsubsets);
+    if (!kept && used + bytes <= budget) {
+      used += bytes;
+      geometry += bytes * (size_t)parts;
+      kept = true;
+    }
+    scratch = std::max(scratch, tile_scratch_bytes(p, s, nsubsets, !kept));
+  }
 }
 
 hipError_t job_backproject(apirl_plan* p, const float* sino, float* img, int subset, int nsubsets,

@@ -10,8 +10,9 @@
   the batch it tunes -- results do not depend on any of them, so the rounds spent
   tuning are not wasted.
 * serve: open-loop Poisson arrivals; a job is admitted when the batch has a slot and
-  its device state (apirl_batch_job_bytes) fits the HBM budget, joins the next
-  round, and leaves when done; latency = completion - arrival."""
+  its device state (apirl_batch_job_bytes) fits the HBM budget beside the running jobs'
+  and the tile geometry that the plans keep from earlier ones, joins the next round, and
+  leaves when done; latency = completion - arrival."""
 import time
 
 import numpy as np
@@ -109,6 +110,15 @@ def run_batched(ctx, plans, jobs, torch, max_jobs=64, tune=True):
     return dt, choice
 
 
+def _drop_geometry(plans):
+    """Frees the tile geometry that the plans keep; they keep new one as before."""
+    for p in plans.values():
+        mb = p.get_tuning()["tile_cache_mb"]
+        p.set_tuning(tile_cache_mb=-1)
+        if mb > 0:
+            p.set_tuning(tile_cache_mb=mb)
+
+
 def serve(ctx, plans, jobs, rate, torch, max_jobs=64, hbm_budget=200e9, seed=0, grid=0,
           use_graph=True):
     """Open-loop arrivals at `rate` jobs/s of `jobs` (specs with materialised inputs).
@@ -117,10 +127,17 @@ def serve(ctx, plans, jobs, rate, torch, max_jobs=64, hbm_budget=200e9, seed=0, 
     arrivals = np.cumsum(rng.exponential(1.0 / rate, len(jobs)))
     batch = hip.Batch(ctx, max_jobs=max_jobs, max_sinograms=1024)
     batch.set_launch(grid, use_graph)
-    need = [hip.Batch.job_bytes(plans[s["kind"]], s["subsets"]) for s, _ in jobs]
-    if max(need) > hbm_budget:
-        raise ValueError(f"a job needs {max(need)} bytes, above the HBM budget {hbm_budget}")
-    queue, running = [], {}
+
+    def need(k):  # with the tile geometry that its plan does not keep yet
+        spec = jobs[k][0]
+        return hip.Batch.job_bytes(plans[spec["kind"]], spec["subsets"])
+
+    def check(most):
+        if most > hbm_budget:
+            raise ValueError(f"a job needs {most} bytes, above the HBM budget {hbm_budget}")
+
+    check(max(need(k) for k in range(len(jobs))))
+    queue, running, holds = [], {}, {}
     finished = np.full(len(jobs), np.nan)
     used = 0
     nxt = 0
@@ -132,19 +149,30 @@ def serve(ctx, plans, jobs, rate, torch, max_jobs=64, hbm_budget=200e9, seed=0, 
             queue.append(nxt)
             nxt += 1
         # admission: capacity and HBM footprint, in arrival order
-        while queue and len(running) < max_jobs and used + need[queue[0]] <= hbm_budget:
-            k = queue.pop(0)
+        while queue and len(running) < max_jobs:
+            k = queue[0]
+            take = need(k)
+            if used + take > hbm_budget:
+                if running:
+                    break
+                # only geometry that the plans keep from earlier jobs is left: it makes room
+                _drop_geometry(plans)
+                used = 0
+                take = need(k)
+                check(take)
+            queue.pop(0)
             spec, d = jobs[k]
             running[k] = batch.submit(plans[spec["kind"]], d["meas"], d["init"], d["out"],
                                       spec["iterations"], spec["subsets"], mult=d["mult"])
-            used += need[k]
+            used += take
+            holds[k] = need(k)  # without the geometry, which the plan keeps
         if running:
             batch.step()
             for k in list(running):
                 if batch.done(running[k]):
                     finished[k] = time.perf_counter() - t0
                     batch.release(running.pop(k))
-                    used -= need[k]
+                    used -= holds.pop(k)
         elif nxt < len(jobs):
             time.sleep(max(0.0, min(arrivals[nxt] - now, 0.01)))
     batch.synchronize()

@@ -350,9 +350,11 @@ apirl_status apirl_batch_create(apirl_ctx* ctx, int max_jobs, int max_sinograms,
                                 apirl_batch** out);
 apirl_status apirl_batch_destroy(apirl_batch* batch);
 const char* apirl_batch_last_error(const apirl_batch* batch);
-/* Device memory a job of this plan holds while admitted (sensitivities and thresholds,
- * ratio, 3D: backprojection scratch and a copy of the image), for admission by HBM
- * footprint. */
+/* Device memory that admitting a job of this plan takes: what the job holds while admitted
+ * (sensitivities and thresholds, ratio, 3D: backprojection scratch and a copy of the image)
+ * and, in 3D, the tile geometry of its subsets that the plan does not keep yet and holds from
+ * then on (apirl_tuning.tile_cache_mb; a call after the submission no longer counts it), for
+ * admission by HBM footprint. */
 size_t apirl_batch_job_bytes(const apirl_plan* plan, int subsets);
 /* The backprojector a batch runs a job of this plan with: APIRL_BP_TILE for 3D jobs of
  * 2^21 voxels or more with one LOR per bin that the tile form takes, else
