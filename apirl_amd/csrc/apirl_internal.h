@@ -58,8 +58,8 @@ struct Geo {
   int ns, nas;  // LORs per bin: transaxial x axial samples (oversampled 3D Siddon)
 };
 
-// A run of consecutive sinograms with increasing mean axial coordinate (one segment
-// of the reference's enumeration): zmean(first + l) ~ z0 + l h.  The gather
+// A run of consecutive sinograms with increasing mean axial coordinate and ends that do not
+// move back (one segment of the reference's enumeration): zmean(first + l) ~ z0 + l h.  The gather
 // backprojector starts its sinogram scan at the index this line predicts for a ray
 // of typical axial slope dlo (the middle sinogram's zb - za); dhi holds 1 / h.  The
 // tile backprojector bounds the run's axial slopes zb - za by [dmin, dmax] and the

@@ -1100,8 +1100,10 @@ void launch_gather3(const GatherArgs& A, int zlanes, int zvox, hipStream_t st) {
   const Geo& g = A.g;
   const size_t lds =
       (size_t)g.nsino * sizeof(float2) + (size_t)(2 * g.nsino + 1) * sizeof(int);
+  // (the one-voxel kernel where the column kernel's tables, with their runs, exceed the LDS of a
+  // workgroup: from 2700 sinograms of few runs, 1330 of runs of two)
   if (PREC != APIRL_PREC_F64_ALPHA && PREC != APIRL_PREC_F64_SETUP && zlanes <= 1 &&
-      zvox >= 1) {
+      zvox >= 1 && column_lds_bytes(g.nsino, A.nseg) <= 65536) {
     constexpr int P =
         (PREC == APIRL_PREC_F64_ALPHA || PREC == APIRL_PREC_F64_SETUP) ? APIRL_PREC_REFERENCE
                                                                        : PREC;

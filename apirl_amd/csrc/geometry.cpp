@@ -283,8 +283,11 @@ void build_gather_tables(const apirl_plan& p, std::vector<float2>& angcs,
   const int ns = p.geo.nsino;
   int first = 0;
   for (int s = 1; s <= ns; s++) {
+    // a run's rays keep their order in z at every alpha, both ends and the means: the ones that
+    // reach a slab are then neighbours
     const bool split = (s == ns) ||
-                       (0.5f * (p.zab[s].x + p.zab[s].y) <= 0.5f * (p.zab[s - 1].x + p.zab[s - 1].y));
+                       (0.5f * (p.zab[s].x + p.zab[s].y) <= 0.5f * (p.zab[s - 1].x + p.zab[s - 1].y)) ||
+                       p.zab[s].x < p.zab[s - 1].x || p.zab[s].y < p.zab[s - 1].y;
     if (!split) continue;
     GatherSeg g{};
     g.first = first;

@@ -1,0 +1,35 @@
+"""The voxel-driven 3D gather on sinogram tables whose rays cross each other in z (slopes of any
+order among growing means): it and the tile form give the oracle's image.  Tables of more runs
+than the column kernel's LDS holds take the one-voxel kernel."""
+import numpy as np
+import pytest
+
+import _oracle as O
+from apirl_amd import hip
+from test_gpu_parity import assert_voxel_close, ctx, dev, host, log, torch  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nsino,nz,slope", [(60, 40, 16.0), (300, 24, 8.0), (1500, 9, 6.0)])
+def test_crossing_rays(torch, ctx, nsino, nz, slope):
+    log(f"case: gather of {nsino} sinograms of crossing rays")
+    nx, dx, dz, nang, nr = 20, 4.0, 2.0, 5, 22
+    rng = np.random.default_rng(nsino)
+    mid = np.sort(rng.uniform(1.0, nz * dz - 1.0, nsino))
+    half = rng.uniform(-slope, slope, nsino)
+    za, zb = (mid - half).astype(np.float32), (mid + half).astype(np.float32)
+    w = np.float32(2.0)
+    p = hip.Plan(ctx, nx, nx, nz, dx, dz, nang, nr, nx * dx / 2, 300.0, z1=za, z2=zb, ring_width=w)
+    za, zb = (((z - w / 2) + w / 2).astype(np.float32) for z in (za, zb))
+    im = O.image_desc(nx, nx, nz, dx, dz)
+    ang, r = O.sino_grid(nang, nr, nx * dx / 2)
+    sino = rng.uniform(0.5, 1.5, p.subset_shape()).astype(np.float32)
+    ref = O.backproject3d(im, sino, ang, r, 300.0, za, zb)
+    sd = dev(torch, sino)
+    # the oracle's float sums: its rounding over some hundreds of terms is within the forms' bar
+    assert_voxel_close(host(p.backproject(sd, mode=hip.BP_TILE)), ref)
+    for zlanes, zvox in ((1, 1), (1, 3), (2, 3)):
+        p.set_tuning(gather_zlanes=zlanes, gather_zvox=zvox)
+        assert_voxel_close(host(p.backproject(sd, mode=hip.BP_GATHER, precision=hip.PREC_KAHAN)),
+                           ref)
