@@ -78,6 +78,7 @@ struct GatherSeg {
 struct LorForm {
   RayXY* rays = nullptr;        // [nang][nr][ns]
   float* xytab = nullptr;       // [nang][nr][nx + ny] gather entry crossings, or null
+  float2* angcs = nullptr;      // [nang] the angles' (cos, sin); null: the plan's
   float2* angcs_odd = nullptr;  // [nang] odd bins' (cos, sin) (radial lookup search)
   int2* rlut = nullptr;         // radial position -> bin range; null on a uniform grid
   float rl0 = 0.f, rl_inv_h = 0.f;
@@ -359,8 +360,9 @@ size_t ztable_bytes(const apirl_plan* p, int nang_sub);
 void build_xy_crossings(const apirl_image_desc& img, const std::vector<RayXY>& rays,
                         std::vector<float>& out);
 // Radial positions of the mMR's bins (ascending) and the (cos, sin) of each angle's
-// odd bins (half an angular step less), as the mMR LOR endpoints use them.
-void mmr_radial_grid(int nang, int nr, std::vector<float>& r, std::vector<float2>& angcs_odd);
+// even and odd bins (half an angular step less), as the mMR LOR endpoints use them.
+void mmr_radial_grid(int nang, int nr, std::vector<float>& r, std::vector<float2>& angcs,
+                     std::vector<float2>& angcs_odd);
 // Lookup table from a radial position to the range of bins around it, on a grid of
 // spacing h from rl0 covering the ascending positions r with two points to spare:
 // lut[k] = (first j with r[j] >= rl0 + k h, last j with r[j] <= rl0 + k h).

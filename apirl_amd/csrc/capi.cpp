@@ -87,6 +87,7 @@ void free_form(apirl::LorForm& f) {
   free_f64s(f);
   if (f.rays) (void)hipFree(f.rays);
   if (f.xytab) (void)hipFree(f.xytab);
+  if (f.angcs) (void)hipFree(f.angcs);
   if (f.angcs_odd) (void)hipFree(f.angcs_odd);
   if (f.rlut) (void)hipFree(f.rlut);
   f = apirl::LorForm();
@@ -94,22 +95,26 @@ void free_form(apirl::LorForm& f) {
 
 // The gather's tables of one LOR form: the entry-crossing table of its rays and,
 // when the radial grid r is not the plan's uniform one, the radial lookup table and
-// the odd bins' directions (half a step earlier when odd_half_step, the mMR's;
-// the bin's own angle otherwise).  false leaves the form without gather tables.
+// the odd bins' directions (half a step earlier in APIRL_SCANNER_MMR, the angle's own
+// otherwise), in the mMR's forms, whose angles are not the plan's, the even ones' too.
+// false leaves the form without gather tables.
 bool upload_gather_form(apirl_plan* p, const std::vector<apirl::RayXY>& rays,
-                        const std::vector<float>& r, bool lut, bool odd_half_step,
-                        apirl::LorForm& f) {
+                        const std::vector<float>& r, bool lut, int form, apirl::LorForm& f) {
   std::vector<float> xy;
   apirl::build_xy_crossings(p->img, rays, xy);
   bool ok = hipMalloc(&f.xytab, xy.size() * sizeof(float)) == hipSuccess &&
             hipMemcpy(f.xytab, xy.data(), xy.size() * sizeof(float), hipMemcpyHostToDevice) ==
                 hipSuccess;
   if (ok && lut) {
-    std::vector<float2> odd;
+    std::vector<float2> even, odd;
     std::vector<int2> tab;
-    if (odd_half_step) {
+    if (form != APIRL_SCANNER_CYLINDRICAL) {
       std::vector<float> rr;
-      apirl::mmr_radial_grid(p->geo.nang, p->geo.nr, rr, odd);
+      apirl::mmr_radial_grid(p->geo.nang, p->geo.nr, rr, even, odd);
+      if (form == APIRL_SCANNER_MMR_SUBSET) odd = even;
+      ok = hipMalloc(&f.angcs, even.size() * sizeof(float2)) == hipSuccess &&
+           hipMemcpy(f.angcs, even.data(), even.size() * sizeof(float2),
+                     hipMemcpyHostToDevice) == hipSuccess;
     } else {
       odd.resize(p->geo.nang);
       for (int a = 0; a < p->geo.nang; a++) {
@@ -121,7 +126,7 @@ bool upload_gather_form(apirl_plan* p, const std::vector<apirl::RayXY>& rays,
     apirl::build_radial_lut(r, tab, f.rl0, f.rl_inv_h);
     f.nrl = (int)tab.size();
     f.tile_maxc = apirl::tile_lut_candidates(p->geo, tab, f.rl_inv_h);
-    ok = hipMalloc(&f.angcs_odd, odd.size() * sizeof(float2)) == hipSuccess &&
+    ok = ok && hipMalloc(&f.angcs_odd, odd.size() * sizeof(float2)) == hipSuccess &&
          hipMemcpy(f.angcs_odd, odd.data(), odd.size() * sizeof(float2),
                    hipMemcpyHostToDevice) == hipSuccess &&
          hipMalloc(&f.rlut, tab.size() * sizeof(int2)) == hipSuccess &&
@@ -726,7 +731,8 @@ apirl_status plan_create_impl(apirl_ctx* ctx, const apirl_image_desc* image,
     f.rays = p->d_rays;
     f.built = true;
     p->gather_tables = p->gather_ok;  // candidate-search tables common to every form
-    if (p->gather_tables) f.gather = upload_gather_form(p, rays, p->r, !p->uniform_r, false, f);
+    if (p->gather_tables)
+      f.gather = upload_gather_form(p, rays, p->r, !p->uniform_r, APIRL_SCANNER_CYLINDRICAL, f);
     apirl::use_lor_form(p, APIRL_SCANNER_CYLINDRICAL);
   }
   // The gather's tile order for the default depth (without it the column kernel
@@ -1481,8 +1487,8 @@ bool build_lor_form(apirl_plan* p, int form) {
     std::vector<float4> pts;
     if (form == APIRL_SCANNER_MMR) mmr_lor_points(p->geo.nang, p->geo.nr, pts);
     else mmr_subset_lor_points(p->geo.nang, p->geo.nr, pts);
-    std::vector<float2> odd;
-    mmr_radial_grid(p->geo.nang, p->geo.nr, r, odd);
+    std::vector<float2> even, odd;
+    mmr_radial_grid(p->geo.nang, p->geo.nr, r, even, odd);
     std::vector<char> ok(pts.size(), 1);  // the 3D form rejects no LOR
     build_ray_table_pts(p->img, false, pts, ok, rays);
   }
@@ -1495,9 +1501,8 @@ bool build_lor_form(apirl_plan* p, int form) {
     return false;
   }
   if (p->gather_tables) {
-    if (form == APIRL_SCANNER_CYLINDRICAL)
-      f.gather = upload_gather_form(p, rays, p->r, !p->uniform_r, false, f);
-    else f.gather = upload_gather_form(p, rays, r, true, form == APIRL_SCANNER_MMR, f);
+    const bool lut = form != APIRL_SCANNER_CYLINDRICAL || !p->uniform_r;
+    f.gather = upload_gather_form(p, rays, r, lut, form, f);
   }
   f.built = true;
   return true;

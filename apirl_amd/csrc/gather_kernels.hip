@@ -2120,7 +2120,8 @@ void gather_args_for(const apirl_plan* p, int subset, int nsubsets, int kind, co
   A.g = g;
   A.rays = p->d_rays;
   A.zab = p->d_zab;
-  A.angcs = p->d_angcs;
+  const float2* own = p->forms[p->scanner].angcs;
+  A.angcs = own ? own : p->d_angcs;
   A.segs = p->d_segs;
   A.nseg = p->nseg;
   A.sino = sino;

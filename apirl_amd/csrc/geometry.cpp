@@ -80,15 +80,20 @@ void mmr_grid(int nang, int nr, std::vector<float>& r, std::vector<float>& ang, 
 }
 }  // namespace
 
-void mmr_radial_grid(int nang, int nr, std::vector<float>& r, std::vector<float2>& angcs_odd) {
+void mmr_radial_grid(int nang, int nr, std::vector<float>& r, std::vector<float2>& angcs,
+                     std::vector<float2>& angcs_odd) {
   std::vector<float> ang;
   float step;
   mmr_grid(nang, nr, r, ang, step);
+  angcs.resize(nang);
   angcs_odd.resize(nang);
   for (int a = 0; a < nang; a++) {
-    const double rad = ((double)ang[a] - step / 2.0) * (double)kDegToRad;
-    angcs_odd[a].x = (float)cos(rad);
-    angcs_odd[a].y = (float)sin(rad);
+    const double even = (double)ang[a] * (double)kDegToRad;
+    const double odd = ((double)ang[a] - step / 2.0) * (double)kDegToRad;
+    angcs[a].x = (float)cos(even);
+    angcs[a].y = (float)sin(even);
+    angcs_odd[a].x = (float)cos(odd);
+    angcs_odd[a].y = (float)sin(odd);
   }
 }
 

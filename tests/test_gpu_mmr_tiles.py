@@ -59,3 +59,26 @@ def test_mmr_images_do_not_depend_on_rfov(torch, ctx, form):
     for sens, x in out[1:]:
         assert int((sens != out[0][0]).sum()) == 0
         assert int((x != out[0][1]).sum()) == 0
+
+
+@pytest.mark.parametrize("form", ["mmr", "mmr_subset"])
+def test_mmr_on_a_plan_of_other_angles(torch, ctx, form):
+    """The mMR's LORs have angles of their own, whatever the plan's are."""
+    log(f"case: {form} on a plan of explicit angles")
+    nx, nz, dx, nang, nr = 40, 4, 6.0, 20, 120
+    rng = np.random.default_rng(9)
+    z1, z2 = hip.ring_table(RINGS, ZFOV, SPAN, MRD)
+    p = hip.Plan(ctx, nx, nx, nz, dx, ZFOV / nz, nang, nr, 297.0, 328.0, z1=z1, z2=z2,
+                 ring_width=np.float32(ZFOV) / np.float32(RINGS), ang=rng.permutation(180)[:nang])
+    p.set_scanner(form)
+    pts = (O.mmr_lor_table if form == "mmr" else O.mmr_subset_lor_table)(nang, nr)
+    za, zb = O.ring_table(RINGS, ZFOV, SPAN, MRD)
+    sino = rng.uniform(0.5, 1.5, p.subset_shape()).astype(np.float32)
+    im = O.image_desc(nx, nx, nz, dx, ZFOV / nz)
+    want = O.backproject3d_pts(im, sino, pts, za, zb).astype(np.float64)
+    terms = nang * len(za) * (int(1.42 * dx / 0.8) + 2)
+    for mode, prec in ((hip.BP_TILE, hip.PREC_REFERENCE), (hip.BP_GATHER, hip.PREC_REFERENCE),
+                       (hip.BP_SCATTER, hip.PREC_REFERENCE), (hip.BP_GATHER, hip.PREC_KAHAN)):
+        got = host(p.backproject(dev(torch, sino), mode=mode, precision=prec)).reshape(want.shape)
+        off = int((np.abs(got - want) > 2 * terms * 2.0 ** -24 * want).sum())
+        assert off == 0, (mode, prec, off)
