@@ -360,6 +360,12 @@ __device__ __forceinline__ void store_voxel(const GatherArgs& A, long v, float b
   A.img[v] = ok ? A.img[v] * b / sv : 0.f;
 }
 
+// alpha at which a ray leaves a column entered at lo, whose next x or y crossing is next: its list
+// ends by amax, except that of an LOR that misses the image's square (lo > amax), which runs on.
+__device__ __forceinline__ float column_exit(float amax, float lo, float next) {
+  return amax < lo ? next : fminf(amax, next);
+}
+
 // Gather of one voxel (i, j, k): adds its terms to A.img[v] in the fixed order
 // (angle, radial bin, segment, sinogram).  s_zab is the axial table in LDS (3D).
 template <int DIMS, int PREC>
@@ -483,7 +489,7 @@ __device__ __forceinline__ void gather_voxel(const GatherArgs& A, const float2* 
       // [zk0, zk1] inside it form a contiguous run of each segment (the mean ring
       // coordinates grow with the index), found by a short scan from an estimate.
       const float lo = fmaxf((float)tamin, fmaxf((float)Xp, (float)Yp));
-      const float hi = fminf((float)tamax, fminf((float)Xn, (float)Yn));
+      const float hi = column_exit((float)tamax, lo, fminf((float)Xn, (float)Yn));
       const float amid = 0.5f * (lo + hi) - 0.5f;
       const float zlo_t = zk0 - kZMargin, zhi_t = zk1 + kZMargin;
       for (int sg = 0; sg < A.nseg; sg++) {
@@ -678,7 +684,7 @@ __device__ __forceinline__ void gather_column(const GatherArgs& A, const float2*
       okt &= ((na <= 0) | (Xp <= Yn)) & ((nb <= 0) | (Yp < Xn));
       if (!okt) continue;
       const float lo = fmaxf(tamin, fmaxf(Xp, Yp));
-      const float hi = fminf(tamax, fminf(Xn, Yn));
+      const float hi = column_exit(tamax, lo, fminf(Xn, Yn));
       const float amid = 0.5f * (lo + hi) - 0.5f;
       const ZRay* zr_pair = A.zr + pair;            // record of sinogram s: [s * npair]
       const float* zt_pair = A.ztab ? A.ztab + pair : nullptr;  // entry e: [e * npair]
