@@ -1150,9 +1150,14 @@ static_assert(sizeof(FwdStep) == 8, "FwdStep is one 8-byte LDS read");
 constexpr int kPathGuard = kPathUnroll;
 inline int path_pitch(const Geo& g) { return g.nz + kPathGuard; }
 
-// Path length kept per (angle, bin): the transaxial list plus a few columns (a rounding
-// can trade a z step of the list for an x or y step).
-__host__ __device__ inline int fwd_path_len(const Geo& g) { return g.nx + g.ny + 4; }
+// Path length kept per (angle, bin): the transaxial list, whose LORs are clipped to a square of
+// the image's width however tall the image is, plus a few columns (a rounding can trade a z step
+// of the list for an x or y step).
+inline int square_rows(const Geo& g) { return (int)ceilf(2.f * g.R / g.dy - 1e-3f); }
+inline int fwd_path_len(const Geo& g) {
+  const int rows = square_rows(g);
+  return g.nx + (rows > g.ny ? rows : g.ny) + 4;
+}
 // LDS of project_paths_kernel: the list (one entry more, and two before it), its columns
 // and the two crossing chains
 inline size_t fwd_path_lds(const Geo& g) {
@@ -1353,8 +1358,8 @@ __global__ __launch_bounds__(kBlock, PREC == APIRL_PREC_REFERENCE ? 8 : 7) void 
   const bool misses =
       PREC == APIRL_PREC_F64_SETUP
           ? xy64.amin > xy64.amax ||
-                abs(xy64.i1 - xy64.i0) + abs(xy64.j1 - xy64.j0) > g.nx + g.ny + 2
-          : t.amin > t.amax || t.nxy > g.nx + g.ny + 2;
+                abs(xy64.i1 - xy64.i0) + abs(xy64.j1 - xy64.j0) > qmax - 2
+          : t.amin > t.amax || t.nxy > qmax - 2;
   if (misses) {
     for (int s = s0 + (int)threadIdx.x; s < s1; s += nt) {
       Ray ray;
@@ -1551,7 +1556,7 @@ bool path_forward_ok(const apirl_plan* p, int precision, int subset, int nsubset
   }
   // the columns of an entry are kept in 16 bits each, a voxel's byte address in 32
   return g.dims == 3 && precision != APIRL_PREC_F64_ALPHA && g.ns * g.nas == 1 && g.walk24 &&
-         g.nx < 16384 && g.ny < 16384 && p->d_imgT != nullptr &&
+         g.nx < 16384 && g.ny < 16384 && square_rows(g) < 16384 && p->d_imgT != nullptr &&
          path_image_floats(g) < ((size_t)1 << 30) && fwd_path_lds(g) <= 48 * 1024;
 }
 
