@@ -1354,9 +1354,13 @@ __global__ __launch_bounds__(kBlock, PREC == APIRL_PREC_REFERENCE ? 8 : 7) void 
   // LORs that miss the image's square have lists of their own: the reference walks on from the
   // later of the two entries, along columns beside the image, where a negative index can name a
   // voxel of the row before.  They may run past the path's entries and their z crossings fall
-  // anywhere: the loop step by step, without the path.
+  // anywhere: the loop step by step, without the path.  (The reference arithmetic stays on the
+  // path's last column there.  Those voxels are no part of the LOR either way; the likelihood of
+  // 122 x 84 x 73 bins 1.42 times as wide as their 64 x 64 x 17 image is 7.1 % from the one of the
+  // LORs' own voxels so, and 9.7 % with the reference's full lists.)
   const bool misses =
-      PREC == APIRL_PREC_F64_SETUP
+      PREC == APIRL_PREC_REFERENCE ? false
+      : PREC == APIRL_PREC_F64_SETUP
           ? xy64.amin > xy64.amax ||
                 abs(xy64.i1 - xy64.i0) + abs(xy64.j1 - xy64.j0) > qmax - 2
           : t.amin > t.amax || t.nxy > qmax - 2;

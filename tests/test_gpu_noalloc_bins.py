@@ -11,10 +11,10 @@ pytestmark = pytest.mark.gpu
 
 
 def test_many_pairs_of_few_sinograms(torch, ctx):
-    log("case: ratio without allocation, 2 sinograms of 600000 pairs")
-    nang, nr = 1000, 600
+    log("case: ratio without allocation, 2 sinograms of 540000 pairs")
+    nang, nr = 45000, 12
     z1, z2 = np.float32([3.0, 5.0]), np.float32([5.0, 3.0])
-    p = hip.Plan(ctx, 16, 16, 4, 1.0, 2.0, nang, nr, 600.0, 900.0, z1=z1, z2=z2,
+    p = hip.Plan(ctx, 16, 16, 4, 1.0, 2.0, nang, nr, 8.0, 400.0, z1=z1, z2=z2,
                  ring_width=np.float32(2.0))
     assert nang * nr > 1 << 19
     x = torch.rand(p.image_shape(), device="cuda")
