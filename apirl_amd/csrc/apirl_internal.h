@@ -127,7 +127,9 @@ struct apirl_plan {
   // the oversampled backprojection; built on the first gather, freed with the plan or
   // when the oversampling changes
   std::vector<apirl_plan*> os_parts;
-  float* d_imgT = nullptr;         // [nz][nx][ny] transposed copy of the projected image
+  // copy of the projected image: in 3D with z fastest (path_image_floats), or transposed
+  // ([nz][nx][ny]) for a ray per lane
+  float* d_imgT = nullptr;
   int* d_zorder = nullptr;         // [nsino] sinograms sorted by mean axial coordinate
   float2* d_angcs = nullptr;       // [nang] (cos, sin) for the gather candidate search
   apirl::GatherSeg* d_segs = nullptr;
@@ -137,7 +139,7 @@ struct apirl_plan {
                                    // Z slices x 64/Z columns per wavefront)
   int gather_zvox = 3;             // 3D gather voxels per lane along z (1..4, tiles only)
   int gather_xcd = APIRL_GATHER_XCD_WEDGES;  // column kernel's tile order
-  int tile_zs = 0;                 // tile backprojector's slab depth (0: about 5 slices)
+  int tile_zs = 0;                 // tile backprojector's slab depth (0: tile_slab_depth's)
   float* d_zinc = nullptr;         // [nsino] z-crossing increment |dz / Vz|, negative for Vz < 0
   bool slices16 = false;           // every slice index of its rays fits 16 bits
   // its geometry per (LOR form, subset, subsets), kept from the first call on, within

@@ -52,7 +52,8 @@ struct BJob {
 };
 
 // 3D jobs of at least this many voxels are named after the tile form
-// (apirl_batch_job_backprojector).
+// (apirl_batch_job_backprojector), which the smaller ones run too: as they always were, so that
+// a caller's comparison with the single job in the named form keeps its bits.
 constexpr size_t kLargeVoxels = size_t(1) << 21;
 
 template <class T>

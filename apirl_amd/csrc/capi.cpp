@@ -274,7 +274,6 @@ bool tile_takes(const apirl_plan* p, int subset, int nsubsets) {
   return p->gather_ok && !apirl::gather_misfit(p, subset, nsubsets) && !apirl::tile_misfit(p);
 }
 
-// Backprojection of one subset in either form.
 // Oversampled bins are traversed in the reference's arithmetic only (and need the
 // 24-bit index walk).
 bool os_precision_ok(const apirl_plan* p, int precision) {
@@ -338,6 +337,7 @@ apirl_status tile_backproject(apirl_plan* p, const float* sino, float* img, int 
   return APIRL_OK;
 }
 
+// Backprojection of one subset in any form.
 // fuse (one LOR per bin): img is the EM image (not in the scatter form), updated by each voxel's
 // backprojection instead of accumulating it, or takes the backprojection itself (EmFuse::fresh)
 apirl_status backproject_any(apirl_plan* p, const float* sino, const float* est, float* img,

@@ -30,7 +30,6 @@ constexpr int kNumXcd = 8;  // MI355X: 8 XCDs of 32 CUs
 constexpr int kUnroll = 8;  // Siddon steps per batch of voxel loads
 constexpr int kPathUnroll = 12;  // the same for project_paths_kernel's step-by-step batches
 constexpr int kPathCols = 8;     // columns per batch of project_paths_kernel's column walk
-// Marks a batch slot without a term: no Siddon weight is NaN-boxed like this value.
 
 // Per-ray traversal state (Siddon.cpp:253-340).
 struct Ray {
@@ -1119,7 +1118,7 @@ inline unsigned grid_for(long n) { return (unsigned)((n + kBlock - 1) / kBlock);
 // the sinograms one per lane: each lane runs the reference's loop, taking a z step when
 // its next z crossing is below the column's exit alpha and the path's next column
 // otherwise, and adds w * voxel in the loop's order, so the bin is the reference's float
-// sum, bit for bit (as project_kernel's).  Voxels come from a copy of the image with z
+// sum, bit for bit (as project_kernel's; LORs that miss the image: at `misses`).  Voxels come from a copy of the image with z
 // fastest, where the lanes, at one column and neighbouring slices, read neighbouring
 // words; kPathGuard zeros lie between its columns.
 //
@@ -1128,9 +1127,11 @@ inline unsigned grid_for(long n) { return (unsigned)((n + kBlock - 1) / kBlock);
 // lanes: their exit alphas and addresses are one LDS read for the wavefront, a column
 // costs each lane its slice's address, two products and a sum, and the one z step a lane
 // may take among them is put in by selects.  Its loads also touch the lines of one column
-// instead of those of several, as they do where each lane steps on its own (the form kept
-// for the path's ends, and from the first batch on in which a lane would take two z
-// steps).  Fused, 12-angle subset of the 256x256x81 / 344x252x837 workload: 0.86 -> 0.68
+// instead of those of several, as they do where each lane steps on its own.  Only LORs whose
+// list starts inside the image walk so, up to the first batch in which a lane would take two z
+// steps: 24 % of the 256x256x81 workload's, 29 % of 128x128x47's, 7 % of 64x64x17's.  The
+// others' first entry, by a rounding, is the column before the image; they step on their own
+// throughout, which is most of the instructions below (19 a lane and step).  Fused, 12-angle subset of the 256x256x81 / 344x252x837 workload: 0.86 -> 0.68
 // ms (3.3e8 VALU wave-instructions, 0.54 ms of issue); the whole 192x192x233 sinogram of
 // a 128x128x47 image: 1.24 -> 0.74 ms; F64_SETUP, 12 angles of 344x252x357 on 172x172x65:
 // 0.26 -> 0.22 ms.  Stepping every lane by itself with the same 12 instructions a step

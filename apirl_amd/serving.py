@@ -5,7 +5,7 @@
 * run_batched: all jobs submitted to one batch (up to its capacity, later ones as
   slots free up), rounds stepped until every job is done.
 * autotune: picks the batch's persistent grid (workgroups per grouped launch), graph
-  replay on or off, the virtual blocks (256 rays / voxels, or one gather tile) a
+  replay on or off, the virtual blocks (64 rays, or one 8 x 8 patch of voxels) a
   workgroup draws at a time and the jobs' order in a round, by timing real rounds of
   the batch it tunes -- results do not depend on any of them, so the rounds spent
   tuning are not wasted.

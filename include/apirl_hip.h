@@ -140,9 +140,8 @@ apirl_status apirl_plan_intersections(apirl_plan* plan, int subset, int nsubsets
  *   tile_cache_mb: device memory (MiB, default 16384) in which the plan keeps the
  *                  tile backprojector's per-subset geometry from its first call on:
  *                  the rays that enter every 8 x 8-column tile with their paths.  -1
- *                  keeps none and frees what is kept (graphs captured over it must not
- *                  be replayed then); a subset beyond the budget is rebuilt on every
- *                  call.
+ *                  keeps none and frees what is kept (what a captured graph reads stays
+ *                  with the plan); a subset beyond the budget is rebuilt on every call.
  * The gather_ fields shape the voxel-driven kernels, whose results do not depend on them
  * (the per-voxel summation order is fixed); tile results, which are double sums rounded
  * once, are deterministic for a given tile_zs, kept geometry or not.
@@ -285,7 +284,7 @@ apirl_status apirl_mlem_threshold(apirl_ctx* ctx, const float* d_sens, size_t n,
 typedef struct apirl_em_options {
   int iterations;
   int subsets;         /* 1 = MLEM */
-  int bp_mode;         /* APIRL_BP_SCATTER or APIRL_BP_GATHER */
+  int bp_mode;         /* APIRL_BP_SCATTER, APIRL_BP_GATHER or APIRL_BP_TILE */
   int precision;       /* APIRL_PREC_* for the forward step */
   int osem_rules;      /* 1: per-subset sensitivity with forcePositive, threshold 0 with >=
                           (OsemSinogram3d); 0: MLEM rules (threshold min+1e-4(max-min),
